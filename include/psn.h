@@ -289,7 +289,9 @@ int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32
  * 128x256, 256x128 or 256x256), into how many ranges K is cut (1, 2, 4 or 8; with more than one, Y is
  * zeroed by a fill kernel and the partial sums are added atomically, so their order -- and the last bit
  * of a sum -- can vary between runs), and the kernel family:
- *    4  four waves, every wave stages and multiplies (any tile);
+ *    4  the kernels that decode in their loop, every wave staging and multiplying (any tile): eight waves (two to a SIMD,
+ *       the staging spread behind the MFMAs) for tiles of 64 and 128 columns, which are what the planner uses; four
+ *       waves for tiles of 256 columns;
  *   16  eight waves of which four only multiply and four only stage: X by direct-to-LDS loads three K
  *       steps ahead, weights decoded from registers one step ahead (64x64, 64x128, 128x128, 128x256);
  *   32  the wide kernel for large M (256x256 tiles only): four waves, each with all 256 rows x 64 columns

@@ -344,6 +344,7 @@ static int32_t get_fn(psn_module *mod, const char *name, hipFunction_t *out) {
     for (hipModule_t h : mod->m) {
         e = hipModuleGetFunction(&f, h, name);
         if (e == hipSuccess) break;
+        if (e == hipErrorNotFound) (void)hipGetLastError();   /* a miss is no error: it must not be what the thread's next HIP user finds */
     }
     if (e != hipSuccess) return fail(PSN_E_MODULE, "kernel '%s' not found in module: hipError %d (%s)", name, (int)e, hipGetErrorString(e));
     mod->fn.emplace(std::string(name), f);
@@ -1335,21 +1336,22 @@ static int32_t check_prefill(const char *what, psn_module *mod, psn_stream *s, i
     return PSN_OK;
 }
 
-/* per-tile cost model measured on MI355X: microseconds per 64-wide K step of one workgroup, and how
- * many workgroups of that tile one compute unit holds (LDS and registers) */
-static const double k_prefill_step_us[] = {0.87, 1.10, 1.50, 2.00, 2.00, 2.44};
-static const int k_prefill_wgs_per_cu[] = {3, 3, 2, 1, 1, 1};
-/* the producer / consumer kernels (16 = four multiplying + four staging waves) and the wide kernel (32:
- * 256 x 256, four waves decoding their own operands from raw bytes):
- * {tile index, kernel family, step cost, workgroups per compute unit, K steps a workgroup spends filling its load rings} */
-/* the K-quants' four-wave kernels per tile, one workgroup per compute unit (measured over three projection shapes,
- * M = 128 .. 1024, every K split; Q5_K takes Q4_K's figures), what each further workgroup on the same compute unit adds
- * (Q6_K's decode keeps the vector ALUs busy, so two resident workgroups take turns), and the 128 x 256 producer /
- * consumer kernel of Q4_K and Q5_K (one round of workgroups, several rounds) */
-static const double k_q45_K_step_us[] = {0.76, 1.14, 1.33, 1.91, 1.71, 2.60};
-static const double k_q6_K_step_us[] = {0.95, 1.33, 1.51, 2.43, 1.96, 3.10};
-static const double k_kquant_ws_step_us[2] = {1.58, 3.4};
-static const struct { int tile; int waves; double step_us; int per_cu; int fill; } k_prefill_alt[] = {{3, 16, 1.25, 1, 2}, {2, 16, 0.82, 1, 1}, {5, 32, 2.20, 1, 3}};
+/* Family 4 (psn_prefill_pp.hip), measured on MI355X over five formats, eleven matrices and M = 65 .. 4096 (2145 launches; the
+ * estimate is off by 6-11 % rms, and the plan it picks is within 1 % of the best of the family on average):
+ * base + rounds of workgroups x (K steps + prologue) x step cost of the format, workgroups that share a compute unit slowing
+ * each other down by `shared` each, the store of Y, and with K cut the zero fill and the atomic adds. */
+struct prefill_cost {
+    int tile, per_cu;                 /* index into k_prefill_tiles, workgroups a compute unit holds */
+    double base_us, shared, y_us_per_mb, add_us_per_mb, split_us, prologue_steps;
+    double step_us[5];                /* per 64 of K: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
+};
+static const prefill_cost k_prefill_cost[] = {
+    {0, 3, 3.1, 0.76, 0.24, 0.35, 2.8, 1.1, {0.295, 0.386, 0.303, 0.318, 0.396}},
+    {1, 2, 2.8, 1.02, 0.42, 0.60, 2.2, 0.8, {0.428, 0.575, 0.470, 0.513, 0.560}},
+    {2, 1, 2.3, 0.00, 0.52, 0.63, 3.1, 0.0, {0.521, 0.679, 0.556, 0.595, 0.638}},
+    {4, 1, 1.6, 0.00, 0.43, 0.66, 3.1, 1.8, {0.753, 0.903, 0.794, 0.829, 0.862}},
+};
+static int format_index(int32_t t) { return t == PSN_Q4_0 ? 0 : t == PSN_Q8_0 ? 1 : t == PSN_Q4_K ? 2 : t == PSN_Q5_K ? 3 : 4; }
 
 /* zero fill of Y and the atomic adds of `sp` partial sums per element, plus a launch: with few ranges the adds overlap
  * the multiply well enough to count at the fill's 3 TB/s; from `slow_from` ranges on (eight; four for the kernels
@@ -1385,8 +1387,6 @@ static double dense_estimate(int64_t M, int64_t N, int64_t K, int32_t cus, bool 
     return best;
 }
 
-static int32_t plan_q4_0_q8_0(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit, int32_t *waves,
-                              double *t_best);
 extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit,
                                             int32_t *waves) {
     return psn_qmatmul_prefill_plan_for(PSN_Q4_0, M, N, K, cus, tile_m, tile_n, ksplit, waves);
@@ -1402,88 +1402,25 @@ static void plan_weight_stream(int64_t M, int64_t N, int64_t K, int32_t cus, int
     *ksplit = sp;
     *waves = 64;
 }
-static int32_t plan_q4_0_q8_0(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit, int32_t *waves,
-                              double *t_best) {
-    if (!tile_m || !tile_n || !ksplit || !waves) return fail(PSN_E_INVALID_ARG, "psn_qmatmul_prefill_plan: out is null");
-    *waves = 4;
-    *t_best = 0.0;
-    if (M <= 0 || N <= 0 || K <= 0 || K % 256) return fail(PSN_E_SHAPE, "prefill: M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
-    if (cus <= 0) cus = 256;
-    if (M <= 64) {
-        plan_weight_stream(M, N, K, cus, tile_m, tile_n, ksplit, waves);
-        return PSN_OK;
-    }
-    /* estimated time = waves of workgroups over the chip's slots x K steps per workgroup x step cost,
-     * plus, when K is split, zeroing Y and the atomic adds of the partial sums */
+/* family 4: the tile and the K split with the smallest estimate; K ranges hold at least two 256-wide chunks */
+static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
+    const int f = format_index(qtype);
+    const double y_mb = (double)(M * N) * 4e-6;
     double best = 1e300;
-    int bi = 0, bs = 1;
-    for (int i = 0; i < 6; ++i) {
-        const int bm = k_prefill_tiles[i][0], bn = k_prefill_tiles[i][1];
-        const int64_t mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
-        const int64_t slots = (int64_t)cus * k_prefill_wgs_per_cu[i];
+    for (const prefill_cost &c : k_prefill_cost) {
+        const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
+        const int64_t mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn, slots = (int64_t)cus * c.per_cu;
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
-            const bool short_range = sp > 1 && K / 256 < 4 * sp;    /* two or three chunks per range: the producer / consumer kernels only */
+            const double one = ((double)(K / 64) / sp + c.prologue_steps) * c.step_us[f];
+            const auto round_us = [&](int64_t wgs) { return wgs ? one * (1.0 + c.shared * (double)((wgs + cus - 1) / cus - 1)) : 0.0; };
             const int64_t wgs = mt * nt * sp;
-            const int64_t rounds = (wgs + slots - 1) / slots;
-            const double steps = (double)(K / 64) / sp;
-            /* the step costs are those of one workgroup per compute unit; workgroups that share one slow each
-             * other down (measured: 1.45 x with three of the small tiles resident) */
-            const int64_t resident = ((wgs < slots ? wgs : slots) + cus - 1) / cus;
-            double t = (double)rounds * steps * k_prefill_step_us[i] * (1.0 + 0.225 * (double)(resident - 1)) + 5.0;
-            if (sp > 1) t += ksplit_overhead_us(M, N, sp, i == 5 ? 4 : 8);
-            if (!short_range && t < best) { best = t; bi = i; bs = sp; *waves = 4; }
-            for (const auto &v : k_prefill_alt) {
-                if (v.tile != i || (short_range && v.waves != 16)) continue;
-                const int64_t sl = (int64_t)cus * v.per_cu;
-                const int64_t r8 = (wgs + sl - 1) / sl;
-                double t8 = (double)r8 * (steps + v.fill) * v.step_us + 5.0;
-                if (sp > 1) t8 += ksplit_overhead_us(M, N, sp, v.waves == 32 ? 4 : 8);
-                if (t8 < best) { best = t8; bi = i; bs = sp; *waves = v.waves; }
-            }
+            double t = c.base_us + (double)(wgs / slots) * round_us(slots) + round_us(wgs % slots) + c.y_us_per_mb * y_mb;
+            if (sp > 1) t += c.split_us + c.add_us_per_mb * y_mb * sp;
+            if (t > 100.0) t += 0.4 * (t - 100.0);          /* the device lowers its clock under sustained matrix work */
+            if (t < best) { best = t; *tile_m = bm; *tile_n = bn; *ksplit = sp; }
         }
     }
-    *tile_m = k_prefill_tiles[bi][0];
-    *tile_n = k_prefill_tiles[bi][1];
-    *ksplit = bs;
-    *t_best = best;
-    return PSN_OK;
-}
-
-/* The K-quants (Q4_K, Q5_K, Q6_K) have the four-wave family (the same estimate over its six tiles with step costs of
- * their own: the dequantization is fp32 arithmetic per weight) and, Q4_K and
- * Q5_K, the 128 x 256 producer / consumer kernel (its staging waves decode while the others multiply). */
-static double prefill_plan_kquant(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit,
-                                int32_t *waves) {
-    if (cus <= 0) cus = 256;
-    const double *step_us = qtype == PSN_Q6_K ? k_q6_K_step_us : k_q45_K_step_us;
-    const double shared = qtype == PSN_Q6_K ? 1.0 : 0.35;
-    double best = 1e300;
-    int bi = 0, bs = 1;
-    *waves = 4;
-    for (int i = 0; i < 6; ++i) {
-        const int bm = k_prefill_tiles[i][0], bn = k_prefill_tiles[i][1];
-        if (bm > 64 && M <= 64) continue;
-        const int64_t mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
-        const int64_t slots = (int64_t)cus * (k_prefill_wgs_per_cu[i] > 2 ? 2 : k_prefill_wgs_per_cu[i]);
-        for (int sp = 1; sp <= 8; sp *= 2) {
-            if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 4 * sp)) continue;
-            const int64_t wgs = mt * nt * sp, rounds = (wgs + slots - 1) / slots;
-            const int64_t resident = ((wgs < slots ? wgs : slots) + cus - 1) / cus;
-            double t = (double)rounds * ((double)(K / 64) / sp) * step_us[i] * (1.0 + shared * (double)(resident - 1)) + 5.0;
-            if (sp > 1) t += ksplit_overhead_us(M, N, sp, i == 5 ? 4 : 8);
-            if (t < best) { best = t; bi = i; bs = sp; *waves = 4; }
-            if (i == 3 && qtype != PSN_Q6_K && M > 64) {
-                const int64_t r16 = (wgs + cus - 1) / cus;
-                double t16 = (double)r16 * ((double)(K / 64) / sp + 2.0) * (r16 > 1 ? k_kquant_ws_step_us[1] : k_kquant_ws_step_us[0]) + 5.0;
-                if (sp > 1) t16 += ksplit_overhead_us(M, N, sp);
-                if (t16 < best) { best = t16; bi = i; bs = sp; *waves = 16; }
-            }
-        }
-    }
-    *tile_m = k_prefill_tiles[bi][0];
-    *tile_n = k_prefill_tiles[bi][1];
-    *ksplit = bs;
     return best;
 }
 
@@ -1494,25 +1431,16 @@ static int32_t prefill_plan_any(int32_t qtype, int64_t M, int64_t N, int64_t K, 
     if (!tile_m || !tile_n || !ksplit || !waves) return fail(PSN_E_INVALID_ARG, "psn_qmatmul_prefill_plan: null output");
     if (M <= 0 || N <= 0 || K <= 0 || K % 256) return fail(PSN_E_SHAPE, "prefill plan: M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
     if (cus <= 0) cus = 256;
-    double best = 0.0;
-    if (qtype == PSN_Q4_0 || qtype == PSN_Q8_0) {
-        int32_t rc = plan_q4_0_q8_0(M, N, K, cus, tile_m, tile_n, ksplit, waves, &best);
-        if (rc) return rc;
-        if (M <= 64) return PSN_OK;                              /* the weight-streaming kernel */
-        if (qtype == PSN_Q8_0) best *= 1.15;                     /* the step costs above were measured on Q4_0; Q8_0 stages twice the bytes */
-    } else if (M <= 64 && (qtype != PSN_Q6_K || K % 2048 == 0)) {
+    if (M <= 64 && (qtype != PSN_Q6_K || K % 2048 == 0)) {
         plan_weight_stream(M, N, K, cus, tile_m, tile_n, ksplit, waves);
         return PSN_OK;
-    } else {
-        best = prefill_plan_kquant(qtype, M, N, K, cus, tile_m, tile_n, ksplit, waves);
     }
+    *waves = 4;
+    const double best = plan_in_loop(qtype, M, N, K, cus, tile_m, tile_n, ksplit);
     if (allow_dense && M > 64) {
         int sp = 1, bm = 256;
-        /* two more launches and a workspace: only for a clear gain -- except for the K-quants on matrices of 16 M
-         * weights and more, whose in-loop kernels the estimates flatter (their fp32 decode competes with the MFMAs
-         * for issue slots): there the dense family wins ties */
-        const double margin = (qtype == PSN_Q4_0 || qtype == PSN_Q8_0 || N * K < ((int64_t)1 << 24)) ? 0.95 : 1.05;
-        if (dense_estimate(M, N, K, cus, true, &bm, &sp) < margin * best) {
+        /* (two launches more and a trip of the weights through memory: 8 us where the estimate is tight) */
+        if (dense_estimate(M, N, K, cus, true, &bm, &sp) + 8.0 < best) {
             *tile_m = bm;
             *tile_n = 256;
             *ksplit = sp;
@@ -1651,7 +1579,9 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
      * 8 x 16 KB reduction */
     const int skinny_rings = 3 * 32768 + (qtype == PSN_Q4_0 || qtype == PSN_Q4_K ? 6 * 64 * 144 : qtype == PSN_Q5_K ? 5 * 64 * 176 : qtype == PSN_Q6_K ? 4 * 64 * 240 : 3 * 64 * 304);
     const int wide_rings = 3 * (32768 + 256 * (qtype == PSN_Q4_0 ? 36 : 68));   /* three stages of X (256 rows x 64 k) and of raw blocks (two per row) */
-    const int lds = skinny ? (skinny_rings > 8 * 16384 ? skinny_rings : 8 * 16384) : wide ? wide_rings : waves == 16 ? 0 : 2 * (bm + bn) * 128;
+    /* the eight-wave kernels: a ring of four stages of X and two fp16 weight tiles, 128 bytes per row */
+    const bool pp = waves == 4 && bn <= 128;
+    const int lds = pp ? (4 * bm + 2 * bn) * 128 : skinny ? (skinny_rings > 8 * 16384 ? skinny_rings : 8 * 16384) : wide ? wide_rings : waves == 16 ? 0 : 2 * (bm + bn) * 128;
     if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: tile %dx%d needs %d bytes of LDS, device offers %d", bm, bn, lds, mod->ctx->max_lds);
     if ((rc = bind(mod->ctx))) return rc;
     if (ksplit > 1) {
@@ -1682,8 +1612,8 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
         snprintf(name, sizeof name, "psn_prefill_%s_wide", fmt_name(qtype));
         return launch(mod, s, name, (unsigned)blocks, 256, (unsigned)lds, &a);
     }
-    snprintf(name, sizeof name, "psn_prefill_%s_m%d_n%d%s", fmt_name(qtype), bm, bn, waves == 16 ? "_ws" : "");
-    return launch(mod, s, name, (unsigned)blocks, (unsigned)(64 * (waves == 16 ? 8 : 4)), (unsigned)lds, &a);
+    snprintf(name, sizeof name, "psn_prefill_%s_m%d_n%d%s", fmt_name(qtype), bm, bn, waves == 16 ? "_ws" : pp ? "_pp" : "");
+    return launch(mod, s, name, (unsigned)blocks, (unsigned)(64 * (waves == 16 || pp ? 8 : 4)), (unsigned)lds, &a);
 }
 
 extern "C" int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32_t layout, const psn_buf *W,

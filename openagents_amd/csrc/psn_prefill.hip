@@ -1,7 +1,10 @@
 /*
- * psn_prefill.hip -- gfx950 quantized prefill matmul  Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k]
- * for GGUF Q4_0 / Q8_0 weights (every kernel family) and Q4_K / Q5_K / Q6_K weights (the four-wave base family),
- * fp16 activations, fp32 accumulation on v_mfma_f32_32x32x16_f16.
+ * psn_prefill.hip -- gfx950 quantized prefill matmul  Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k],
+ * fp16 activations, fp32 accumulation on v_mfma_f32_32x32x16_f16: the weight-streaming kernels for M <= 64, the dense
+ * family for large M, and the kernels of explicit plans (producer / consumer, wide, and the four-wave tiles of 256
+ * columns).  What the planner picks between 64 rows and the dense family is in psn_prefill_pp.hip.
+ *
+ * The four-wave kernels:
  *
  * A workgroup of 256 threads owns a BM x BN tile of Y and walks K in steps of 64.  Per step
  *   - the X tile (BM x 64 fp16) goes global -> LDS with 16-byte direct-to-LDS loads;
@@ -12,7 +15,7 @@
  *   - each wave multiplies its (BM/WM) x (BN/WN) part with 32x32x16 MFMAs, operands read from LDS
  *     as 16-byte fragments (8 consecutive k per lane for both A = X rows and B = W rows).
  * LDS rows are 128 bytes (64 fp16); the eight 16-byte chunks of a row are stored XOR-swizzled by
- * (row & 7) so that the 32 rows a fragment read touches fall into distinct banks.  Two LDS
+ * tile_swz(row) so that the 32 rows a fragment read touches fall into distinct banks.  Two LDS
  * buffers alternate; one barrier per K step.
  *
  * Workgroup -> tile mapping is XCD-aware: workgroup b runs on XCD b % 8, and all M tiles of one
@@ -21,26 +24,7 @@
 #include "psn_args.h"
 #include "psn_device.h"
 
-#define UNROLL _Pragma("unroll")
-
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-
-/* byte offset of 16-byte chunk `chunk` (0..7) of tile row `row` */
-PSN_DEV int tile_off(int row, int chunk) { return row * 128 + ((chunk ^ (row & 7)) << 4); }
-
-PSN_DEV u32 h2_bits(half2_t v) { return __builtin_bit_cast(u32, v); }
-PSN_DEV half2_t bits_h2(u32 v) { return __builtin_bit_cast(half2_t, v); }
-
-/* four bytes of v (already masked to the wanted 0..255 values) -> four fp16 (1024 + byte) in element
- * order, minus `bias`, times the block scale */
-PSN_DEV void bytes_to_h4(u32 v, u32 keep, half2_t bias, half2_t d2, u32 &lo, u32 &hi) {
-    const u32 t01 = __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u) & keep;   /* [b0, 0x64, b1, 0x64] */
-    const u32 t23 = __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u) & keep;   /* [b2, 0x64, b3, 0x64] */
-    lo = h2_bits((bits_h2(t01) - bias) * d2);
-    hi = h2_bits((bits_h2(t23) - bias) * d2);
-}
+#include "psn_prefill_common.h"
 
 struct PfQ4_0 {
     static constexpr int DW = 36, BYTES = 144;
@@ -134,25 +118,6 @@ struct PfQ8_0 {
  *      round-to-nearest-even is the second rounding (the compiler emits v_cvt_f32_ubyteN + v_fma_mix{lo,hi}_f16:
  *      two instructions per weight).  Q6_K: d * scale (19 bits) * (q - 32) (5 bits, or the power of two 32) is
  *      exact; written as fma(ds, q, -32 ds) the unsigned byte converts directly. ---- */
-PSN_DEV u32 pack_h2_rn(float a, float b) {
-    const half2_t v = {(_Float16)a, (_Float16)b};
-    return h2_bits(v);
-}
-PSN_DEV void pf_kq_scales(u32 s0, u32 s1, u32 s2, u32 (&sc)[2], u32 (&mn)[2]) {
-    sc[0] = s0 & 0x3f3f3f3fu;
-    mn[0] = s1 & 0x3f3f3f3fu;
-    sc[1] = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
-    mn[1] = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
-}
-template <int I> PSN_DEV float pf_byte(const u32 (&v)[2]) { return (float)((v[I >> 2] >> (8 * (I & 3))) & 0xffu); }
-/* four unsigned byte values of q -> d1 * q - m1, two packed pairs */
-PSN_DEV void pf_affine4(u32 q, float d1, float m1, u32 &lo, u32 &hi) {
-    const float v0 = __builtin_fmaf(d1, (float)(q & 0xffu), -m1), v1 = __builtin_fmaf(d1, (float)((q >> 8) & 0xffu), -m1);
-    const float v2 = __builtin_fmaf(d1, (float)((q >> 16) & 0xffu), -m1), v3 = __builtin_fmaf(d1, (float)(q >> 24), -m1);
-    lo = pack_h2_rn(v0, v1);
-    hi = pack_h2_rn(v2, v3);
-}
-
 /* Q4_K: dword 0 = d | dmin << 16, dwords 1..3 = scales, dwords 4..35 = nibbles (sub-block 2g in the low,
  * 2g+1 in the high nibbles of bytes 32g .. 32g+31) */
 struct PfQ4_K {
@@ -298,7 +263,7 @@ PSN_DEV void prefill_body(const psn_prefill_args &a) {
     auto stage_x = [&](char *tile, int k0) {
         /* slot s = 16-byte word s of the tile in LDS order: row s/8, position s%8 holds chunk (s%8)^(row&7) */
         UNROLL for (int i = 0; i < BM * 8 / NT; ++i) {
-            const int s = i * NT + tid, row = s >> 3, chunk = (s & 7) ^ (row & 7);
+            const int s = i * NT + tid, row = s >> 3, chunk = (s & 7) ^ tile_swz(row);
             const uint16_t *src = a.X + (int64_t)min(m0 + row, M - 1) * K + k0 + chunk * 8;
             __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(tile + (i * NT + __builtin_amdgcn_readfirstlane(wave) * 64) * 16), 16, 0, 0);
         }
@@ -522,7 +487,7 @@ PSN_DEV void prefill_body_ws(const psn_prefill_args &a) {
         auto stage_x = [&](uint4 *tile, int k0) {
             k0 = min(k0, k_last);
             UNROLL for (int i = 0; i < NX; ++i) {
-                const int s_ = i * NP + ptid, row = s_ >> 3, chunk = (s_ & 7) ^ (row & 7);
+                const int s_ = i * NP + ptid, row = s_ >> 3, chunk = (s_ & 7) ^ tile_swz(row);
                 const uint16_t *src = a.X + (int64_t)min(m0 + row, M - 1) * K + k0 + chunk * 8;
                 __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(tile + i * NP + pwave * 64), 16, 0, 0);
             }
@@ -684,8 +649,8 @@ PSN_DEV void prefill_skinny_loop(const psn_prefill_args &a, int wave, int lane, 
             const int k0 = c * 256;
             __attribute__((address_space(3))) char *dst = lds_ptr + (xs_base - lds0) + (q % XR) * XBYTES;
             UNROLL for (int u = 0; u < CX; ++u) {
-                /* 16-byte word s_ of the stage in LDS order: step s_/512, row (s_%512)/8, position s_%8 holds chunk pos^(row&7) */
-                const int i = wave * CX + u, s_ = i * 64 + lane, step = s_ >> 9, row = (s_ >> 3) & 63, chunk = (s_ & 7) ^ (row & 7);
+                /* 16-byte word s_ of the stage in LDS order: step s_/512, row (s_%512)/8, position s_%8 holds chunk pos^tile_swz(row) */
+                const int i = wave * CX + u, s_ = i * 64 + lane, step = s_ >> 9, row = (s_ >> 3) & 63, chunk = (s_ & 7) ^ tile_swz(row);
                 const uint16_t *src = a.X + (int64_t)min(row, M - 1) * K + k0 + step * 64 + chunk * 8;
                 __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(dst + i * 1024), 16, 0, 0);
             }
@@ -1003,8 +968,6 @@ PSN_DEV void prefill_skinny_body(const psn_prefill_args &a) {
  *     per MFMA ride along for free);
  *   - one workgroup barrier per 64 of K; every wave first waits for its own share of the next stage's
  *     loads (loads complete in issue order, so "at most n outstanding" identifies them). */
-template <int N> struct pf_int { static constexpr int value = N; };
-
 template <typename WF>
 PSN_DEV void prefill_wide_body(const psn_prefill_args &a) {
     constexpr int BM = 256, BN = 256, TM = 8, TN = 2, NS = 3;     /* a wave: all 256 rows x 64 columns */
@@ -1045,7 +1008,7 @@ PSN_DEV void prefill_wide_body(const psn_prefill_args &a) {
      * issues the same number of loads. */
     u32 xoff_g[NX], woff_g[NR];
     UNROLL for (int u = 0; u < NX; ++u) {
-        const int s_ = (wave * NX + u) * 64 + lane, row = s_ >> 3, chunk = (s_ & 7) ^ (row & 7);
+        const int s_ = (wave * NX + u) * 64 + lane, row = s_ >> 3, chunk = (s_ & 7) ^ tile_swz(row);
         xoff_g[u] = (u32)min(m0 + row, M - 1) * (u32)(K * 2) + (u32)(chunk * 16);
     }
     UNROLL for (int u = 0; u < NR; ++u) {
@@ -1066,7 +1029,7 @@ PSN_DEV void prefill_wide_body(const psn_prefill_args &a) {
     /* per-lane LDS offsets: the X fragment of K slice kk (row base + swizzled 16-byte position; the four
      * 32-row blocks of the wave's tile are 4096 bytes apart), the raw bytes of weight row block j */
     u32 xsw[4], rrow[TN];
-    UNROLL for (int kk = 0; kk < 4; ++kk) xsw[kk] = (u32)((lane & 31) * 128) + ((((u32)(2 * kk + h)) ^ (u32)(lane & 7)) << 4);
+    UNROLL for (int kk = 0; kk < 4; ++kk) xsw[kk] = (u32)((lane & 31) * 128) + ((((u32)(2 * kk + h)) ^ (u32)tile_swz(lane & 31)) << 4);
     UNROLL for (int j = 0; j < TN; ++j) rrow[j] = (u32)((wn * 64 + 32 * j + (lane & 31)) * SB);
     const u32 hq = 8u * (u32)h;
 
@@ -1464,11 +1427,7 @@ template <int TM> PSN_DEV void prefill_dense_body(const psn_prefill_args &a) {
     PSN_PREFILL_KERNEL_WS(fmt, WF, 128, 128)     \
     PSN_PREFILL_KERNEL_WS(fmt, WF, 128, 256)
 #define PSN_PREFILL_FAMILY_BASE(fmt, WF)         \
-    PSN_PREFILL_KERNEL(fmt, WF, 64, 64, 2, 2)    \
-    PSN_PREFILL_KERNEL(fmt, WF, 64, 128, 2, 2)   \
-    PSN_PREFILL_KERNEL(fmt, WF, 128, 128, 2, 2)  \
     PSN_PREFILL_KERNEL(fmt, WF, 128, 256, 2, 2)  \
-    PSN_PREFILL_KERNEL(fmt, WF, 256, 128, 2, 2)  \
     PSN_PREFILL_KERNEL(fmt, WF, 256, 256, 2, 2)
 
 /* The build compiles this file once per (format, kernel family) -- -DPSN_BUILD_ONLY -DPSN_BUILD_PF=<n>

@@ -1,0 +1,538 @@
+/*
+ * psn_prefill_pp.hip -- gfx950 quantized prefill matmul, the kernels that decode in their loop:
+ * Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k], fp16 MFMA, fp32 accumulation.
+ *
+ * A workgroup of eight waves (two to a SIMD) owns a BM x BN tile of Y and walks K in steps of 64.  Every wave does every
+ * kind of work, a little of it behind each of its MFMAs, so that the two waves of a SIMD fill each other's gaps: while
+ * step s is multiplied out of LDS, the wave
+ *   - reads the step's operand fragments, half a step before they are multiplied,
+ *   - asks for its share of the X tile NS - 1 steps on (direct-to-LDS loads into a ring of NS stages; spread over the
+ *     step because four in a row stall their wave for 500 cycles),
+ *   - decodes its share of the weights of step s + 1 into the other one of two fp16 tiles.  A weight is decoded once per
+ *     workgroup: a thread owns BN / 8 weights of one row per step, and their raw bytes come straight from memory into
+ *     registers, asked for a whole 256-wide chunk ahead.
+ * One barrier per step.
+ *
+ * What bounds it (counters, Q4_K 512 x 14336 x 4096, 256 x 128 tiles): of 121 k cycles 66 k are MFMA, and the device runs at
+ * 2.1 GHz under them; the same instructions on zero weights take 45 us instead of 59, so from M = 512 on it is power
+ * (operand reads, decode arithmetic and MFMAs together), below that the decode's vector instructions (60 per wave and
+ * step, of which six per MFMA ride along for free).  Against the kernels that served these shapes before (producer /
+ * consumer and dequantize-first): 14336 x 4096 at M = 203: Q4_0 52 -> 40 us, Q8_0 74 -> 52, Q4_K 65 -> 43, Q6_K 91 -> 48; at
+ * M = 512: Q4_0 80 -> 64, Q8_0 99 -> 73, Q4_K 94 -> 67, Q6_K 105 -> 71.  Splitting the roles (eight multiplying and eight
+ * staging waves) measured 2-8 % slower, running the two waves of a SIMD in strictly opposite phases 10-15 % slower.
+ */
+#include "psn_args.h"
+#include "psn_device.h"
+#include "psn_prefill_common.h"
+
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+/* ---- raw bytes of a thread, in one to five registers, loaded without a wait.  Every load is aligned to four bytes: 16- and
+ *      8-byte loads from odd halfwords (where the quants of Q4_0, Q8_0 and Q6_K blocks start) take two to three times as long
+ *      (a whole 14336 x 4096 matrix streamed by 112 workgroups: Q4_0 22.5 us against 9.9, Q8_0 32.9 against 22.4), so those
+ *      formats fetch the aligned words around their bytes and pick the bytes out with v_perm.  ("+v": the load's target is the
+ *      very register the variable lives in, so that no copy of it is made while the bytes are still on their way.) ---- */
+typedef u32 u32x3 __attribute__((ext_vector_type(3)));
+template <int NB> struct raw_bytes;
+template <> struct raw_bytes<4> { typedef u32 t; };
+template <> struct raw_bytes<8> { typedef u32x2 t; };
+template <> struct raw_bytes<12> { typedef u32x3 t; };
+template <> struct raw_bytes<16> { typedef u32x4 t; };
+PSN_DEV u32 raw_word(u32 v, int) { return v; }
+PSN_DEV u32 raw_word(u32x2 v, int i) { return v[i]; }
+PSN_DEV u32 raw_word(u32x3 v, int i) { return v[i]; }
+PSN_DEV u32 raw_word(u32x4 v, int i) { return v[i]; }
+template <int OFF> PSN_DEV void raw_load(const uint8_t *p, u32 &v) { asm volatile("global_load_dword %0, %1, off offset:%2" : "+v"(v) : "v"(p), "n"(OFF) : "memory"); }
+template <int OFF> PSN_DEV void raw_load(const uint8_t *p, u32x2 &v) { asm volatile("global_load_dwordx2 %0, %1, off offset:%2" : "+v"(v) : "v"(p), "n"(OFF) : "memory"); }
+template <int OFF> PSN_DEV void raw_load(const uint8_t *p, u32x3 &v) { asm volatile("global_load_dwordx3 %0, %1, off offset:%2" : "+v"(v) : "v"(p), "n"(OFF) : "memory"); }
+template <int OFF> PSN_DEV void raw_load(const uint8_t *p, u32x4 &v) { asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "+v"(v) : "v"(p), "n"(OFF) : "memory"); }
+template <int OFF> PSN_DEV void raw_load_u16(const uint8_t *p, u32 &v) { asm volatile("global_load_ushort %0, %1, off offset:%2" : "+v"(v) : "v"(p), "n"(OFF) : "memory"); }
+template <typename T> PSN_DEV void raw_tie(T &v) { asm volatile("" : "+v"(v)); }
+
+/* ---- four weights in two pieces of about five instructions each (what fits behind an MFMA): bytes -> `half_done`, then
+ *      half_done -> four fp16.  K-quants: the bytes as floats, then d * q - m and the conversion to fp16 (fused multiply-add
+ *      and v_cvt_pk_f16_f32 issue in half the cycles of v_fma_mix).  Q4_0 / Q8_0: 1024 + byte as fp16, then minus the bias,
+ *      times the scale. ---- */
+struct half_done { float f[4]; u32 h[2]; };
+PSN_DEV void kq_floats(u32 q, half_done &t) {
+    asm volatile("" : "+v"(q));                          /* (else the mask becomes a bit-field extract per byte instead of v_cvt_f32_ubyteN) */
+    UNROLL for (int i = 0; i < 4; ++i) t.f[i] = (float)((q >> (8 * i)) & 0xffu);
+}
+typedef float float2_t __attribute__((ext_vector_type(2)));
+PSN_DEV void kq_finish(const half_done &t, float d, float m, u32 &o0, u32 &o1) {
+    const float2_t a = {__builtin_fmaf(d, t.f[0], -m), __builtin_fmaf(d, t.f[1], -m)}, b = {__builtin_fmaf(d, t.f[2], -m), __builtin_fmaf(d, t.f[3], -m)};
+    o0 = h2_bits(__builtin_convertvector(a, half2_t));
+    o1 = h2_bits(__builtin_convertvector(b, half2_t));
+}
+PSN_DEV void q0_halves(u32 v, u32 keep, half_done &t) {
+    t.h[0] = __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u) & keep;
+    t.h[1] = __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u) & keep;
+}
+PSN_DEV void q0_finish(const half_done &t, u32 bias, u32 d2, u32 &o0, u32 &o1) {
+    o0 = h2_bits((bits_h2(t.h[0]) - bits_h2(bias)) * bits_h2(d2));
+    o1 = h2_bits((bits_h2(t.h[1]) - bits_h2(bias)) * bits_h2(d2));
+}
+
+/* ---- a format's share of one thread: part `part` of 32 / NB parts of a row.  `base` is the row's chunk plus lane_off(part);
+ *      load() asks for everything the four steps of the chunk need (LOADS instructions); step J's bytes are two groups
+ *      (HI = 0, 1) of NB weights, which belong at k = k_lo(part) and k_hi(part) of the 64-wide step; first() and second() turn
+ *      word i of a group into four fp16, with the step's scales from scales0() and scales1().  SPREAD (for NB = 4, 8): see row_of below. ---- */
+struct PpQ4_K {
+    static constexpr int BYTES = 144, LOADS = 5;
+    template <int NB> struct raw { u32x4 h; typename raw_bytes<NB>::t q[4]; };
+    template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
+    template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
+        raw_load<0>(row, r.h);
+        const uint8_t *p = row + lane;
+        raw_load<16>(p, r.q[0]); raw_load<48>(p, r.q[1]); raw_load<80>(p, r.q[2]); raw_load<112>(p, r.q[3]);
+    }
+    template <int NB> static PSN_DEV void clear(raw<NB> &r) { r.h = (u32x4)(0u); UNROLL for (int j = 0; j < 4; ++j) r.q[j] = 0u; }
+    template <int NB> static PSN_DEV void landed(raw<NB> &r) { raw_tie(r.h); UNROLL for (int j = 0; j < 4; ++j) raw_tie(r.q[j]); }
+    struct scale { float d[2], m[2]; };
+    template <int J, int NB> static PSN_DEV void scales0(const raw<NB> &r, int, scale &s) {
+        u32 sc[2], mn[2];
+        pf_kq_scales(r.h.y, r.h.z, r.h.w, sc, mn);
+        s.d[0] = pf_byte<2 * J>(sc); s.d[1] = pf_byte<2 * J + 1>(sc);
+        s.m[0] = pf_byte<2 * J>(mn); s.m[1] = pf_byte<2 * J + 1>(mn);
+    }
+    template <int NB> static PSN_DEV void scales1(const raw<NB> &r, scale &s) {
+        const float d = h2f_lo(r.h.x), dm = h2f_hi(r.h.x);
+        UNROLL for (int i = 0; i < 2; ++i) { s.d[i] = __fmul_rn(d, s.d[i]); s.m[i] = __fmul_rn(dm, s.m[i]); }
+    }
+    template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &r, const scale &, int i, half_done &t) { kq_floats((raw_word(r.q[J], i) >> (4 * HI)) & 0x0f0f0f0fu, t); }
+    template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
+    template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
+    template <int NB> static PSN_DEV int k_hi(int part) { return 32 + NB * part; }
+    static constexpr int SPREAD[2] = {0, 3};
+};
+struct PpQ5_K {
+    static constexpr int BYTES = 176, LOADS = 6;
+    template <int NB> struct raw { u32x4 h; typename raw_bytes<NB>::t top, q[4]; };
+    template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
+    template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
+        raw_load<0>(row, r.h);
+        const uint8_t *p = row + lane;
+        raw_load<16>(p, r.top);
+        raw_load<48>(p, r.q[0]); raw_load<80>(p, r.q[1]); raw_load<112>(p, r.q[2]); raw_load<144>(p, r.q[3]);
+    }
+    template <int NB> static PSN_DEV void clear(raw<NB> &r) { r.h = (u32x4)(0u); r.top = 0u; UNROLL for (int j = 0; j < 4; ++j) r.q[j] = 0u; }
+    template <int NB> static PSN_DEV void landed(raw<NB> &r) { raw_tie(r.h); raw_tie(r.top); UNROLL for (int j = 0; j < 4; ++j) raw_tie(r.q[j]); }
+    struct scale { float d[2], m[2]; };
+    template <int J, int NB> static PSN_DEV void scales0(const raw<NB> &r, int, scale &s) {
+        u32 sc[2], mn[2];
+        pf_kq_scales(r.h.y, r.h.z, r.h.w, sc, mn);
+        s.d[0] = pf_byte<2 * J>(sc); s.d[1] = pf_byte<2 * J + 1>(sc);
+        s.m[0] = pf_byte<2 * J>(mn); s.m[1] = pf_byte<2 * J + 1>(mn);
+    }
+    template <int NB> static PSN_DEV void scales1(const raw<NB> &r, scale &s) {
+        const float d = h2f_lo(r.h.x), dm = h2f_hi(r.h.x);
+        UNROLL for (int i = 0; i < 2; ++i) { s.d[i] = __fmul_rn(d, s.d[i]); s.m[i] = __fmul_rn(dm, s.m[i]); }
+    }
+    template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &r, const scale &, int i, half_done &t) { kq_floats(((raw_word(r.q[J], i) >> (4 * HI)) & 0x0f0f0f0fu) | (((raw_word(r.top, i) >> (2 * J + HI)) & 0x01010101u) << 4), t); }
+    template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
+    template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
+    template <int NB> static PSN_DEV int k_hi(int part) { return 32 + NB * part; }
+    static constexpr int SPREAD[2] = {0, 3};
+};
+/* step J = half J / 2 of the super-block, quarters t = 2 (J & 1) and 2 (J & 1) + 1: the first 32 and the second 32 of
+ * the half's 64 low-bit bytes, their low (J even) or high nibbles; bits 4..5 from the half's 32 high-bit bytes.  A
+ * super-block (210 bytes) starts on a dword or two bytes behind one: `pick` takes four bytes out of two dwords accordingly. */
+struct PpQ6_K {
+    static constexpr int BYTES = 210, LOADS = 9;
+    template <int NB> struct raw { typename raw_bytes<NB + 4>::t ql[4], qh[2]; u32x4 sc; u32 sc4, d, pick; };
+    template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
+    template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
+        const uint8_t *d = (const uint8_t *)((uintptr_t)row & ~(uintptr_t)3), *p = d + lane;
+        r.pick = ((uintptr_t)row & 2) ? 0x05040302u : 0x03020100u;
+        raw_load<0>(p, r.ql[0]); raw_load<32>(p, r.ql[1]); raw_load<64>(p, r.ql[2]); raw_load<96>(p, r.ql[3]);
+        raw_load<128>(p, r.qh[0]); raw_load<160>(p, r.qh[1]);
+        raw_load<192>(d, r.sc);
+        /* the scales' last two bytes where the super-block starts two bytes late (else a dword inside it that nobody uses) */
+        raw_load<204>((const uint8_t *)((uintptr_t)(row + 2) & ~(uintptr_t)3), r.sc4);
+        raw_load_u16<208>(row, r.d);
+    }
+    template <int NB> static PSN_DEV void clear(raw<NB> &r) { r.sc = (u32x4)(0u); r.sc4 = r.d = r.pick = 0u; r.qh[0] = r.qh[1] = 0u; UNROLL for (int j = 0; j < 4; ++j) r.ql[j] = 0u; }
+    template <int NB> static PSN_DEV void landed(raw<NB> &r) {
+        UNROLL for (int j = 0; j < 4; ++j) raw_tie(r.ql[j]);
+        raw_tie(r.qh[0]); raw_tie(r.qh[1]); raw_tie(r.sc); raw_tie(r.sc4); raw_tie(r.d);
+    }
+    struct scale { float d[2], m[2]; };
+    template <int J, int NB> static PSN_DEV void scales0(const raw<NB> &r, int part, scale &s) {
+        /* the scales of quarter t and (16 bits on) of quarter t + 1, each of this part's half */
+        constexpr int I = 2 * (J >> 1) + (J & 1);
+        const u32 v = __builtin_amdgcn_perm(I == 3 ? r.sc4 : r.sc[(I + 1) & 3], r.sc[I], r.pick) >> (8 * ((NB * part) >> 4));
+        s.d[0] = (float)(int)(int8_t)(v & 0xffu);
+        s.d[1] = (float)(int)(int8_t)((v >> 16) & 0xffu);
+    }
+    template <int NB> static PSN_DEV void scales1(const raw<NB> &r, scale &s) {
+        const float d = h2f_lo(r.d);
+        UNROLL for (int i = 0; i < 2; ++i) { s.d[i] = __fmul_rn(d, s.d[i]); s.m[i] = s.d[i] * 32.f; }
+    }
+    template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &r, const scale &, int i, half_done &t) {
+        constexpr int H = J >> 1, T = 2 * (J & 1);
+        const u32 a = __builtin_amdgcn_perm(raw_word(r.ql[2 * H + HI], i + 1), raw_word(r.ql[2 * H + HI], i), r.pick);
+        const u32 b = __builtin_amdgcn_perm(raw_word(r.qh[H], i + 1), raw_word(r.qh[H], i), r.pick);
+        kq_floats(((a >> (2 * T)) & 0x0f0f0f0fu) | (((b >> (2 * T + 2 * HI)) & 0x03030303u) << 4), t);
+    }
+    template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
+    template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
+    template <int NB> static PSN_DEV int k_hi(int part) { return 32 + NB * part; }
+    static constexpr int SPREAD[2] = {0, 3};
+};
+/* Q4_0 and Q8_0: step J = blocks 2 J and 2 J + 1, 36 (68) bytes from a dword on.  The first block's quants start two bytes
+ * into its first dword, the second one's on a dword; so the dwords from DW * part on hold a part's bytes two (first block) or
+ * four bytes in, its block's scale sits in the low (first block) or high half of the first dword of the block's first
+ * part, and one v_perm selector per thread picks either. */
+template <int PB, int NB> struct pp_blocks {               /* PB: bytes per part (NB or 2 NB) */
+    static constexpr int PARTS = 32 / NB;
+    static PSN_DEV bool second_block(int part) { return part >= PARTS / 2; }
+    static PSN_DEV u32 pick(int part) { return second_block(part) ? 0x07060504u : 0x05040302u; }
+    static PSN_DEV u32 scale(u32 first_dword, int part) {   /* the block's scale in both halves */
+        /* quad_perm: lanes of a quad read their block's first part (parts 0, 0, 2, 2, or 0 of quads that are one block) */
+        const u32 v = (u32)__builtin_amdgcn_mov_dpp((int)first_dword, PARTS == 4 ? 0xA0 : 0x00, 0xf, 0xf, false);
+        return __builtin_amdgcn_perm(v, v, second_block(part) ? 0x03020302u : 0x01000100u);
+    }
+};
+struct PpQ4_0 {
+    static constexpr int BYTES = 144, LOADS = 4;
+    template <int NB> struct raw { typename raw_bytes<NB + 4>::t q[4]; };
+    template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
+    template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
+        const uint8_t *p = row + lane;
+        raw_load<0>(p, r.q[0]); raw_load<36>(p, r.q[1]); raw_load<72>(p, r.q[2]); raw_load<108>(p, r.q[3]);
+    }
+    template <int NB> static PSN_DEV void clear(raw<NB> &r) { UNROLL for (int j = 0; j < 4; ++j) r.q[j] = 0u; }
+    template <int NB> static PSN_DEV void landed(raw<NB> &r) { UNROLL for (int j = 0; j < 4; ++j) raw_tie(r.q[j]); }
+    struct scale { u32 d, q[2]; };
+    template <int J, int NB> static PSN_DEV void scales0(const raw<NB> &r, int part, scale &s) {
+        typedef pp_blocks<NB, NB> B;
+        s.d = B::scale(raw_word(r.q[J], 0), part);
+        UNROLL for (int i = 0; i < NB / 4; ++i) s.q[i] = __builtin_amdgcn_perm(raw_word(r.q[J], i + 1), raw_word(r.q[J], i), B::pick(part));
+    }
+    template <int NB> static PSN_DEV void scales1(const raw<NB> &, scale &) {}
+    template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &, const scale &s, int i, half_done &t) { q0_halves(s.q[i] >> (4 * HI), 0x640f640fu, t); }
+    template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { q0_finish(t, 0x64086408u, s.d, o0, o1); }
+    /* low nibbles first, high nibbles sixteen further on */
+    template <int NB> static PSN_DEV int k_lo(int part) { return 32 * ((NB * part) >> 4) + ((NB * part) & 15); }
+    template <int NB> static PSN_DEV int k_hi(int part) { return k_lo<NB>(part) + 16; }
+    static constexpr int SPREAD[2] = {0, 2};
+};
+struct PpQ8_0 {
+    static constexpr int BYTES = 272, LOADS = 8;
+    template <int NB> struct raw { typename raw_bytes<2 * NB>::t q[4]; u32 e[4]; };    /* e: the dword behind them */
+    template <int NB> static PSN_DEV int lane_off(int part) { return 2 * NB * part; }
+    template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
+        const uint8_t *p = row + lane;
+        raw_load<0>(p, r.q[0]); raw_load<2 * NB>(p, r.e[0]); raw_load<68>(p, r.q[1]); raw_load<68 + 2 * NB>(p, r.e[1]);
+        raw_load<136>(p, r.q[2]); raw_load<136 + 2 * NB>(p, r.e[2]); raw_load<204>(p, r.q[3]); raw_load<204 + 2 * NB>(p, r.e[3]);
+    }
+    template <int NB> static PSN_DEV void clear(raw<NB> &r) { UNROLL for (int j = 0; j < 4; ++j) { r.q[j] = 0u; r.e[j] = 0u; } }
+    template <int NB> static PSN_DEV void landed(raw<NB> &r) { UNROLL for (int j = 0; j < 4; ++j) { raw_tie(r.q[j]); raw_tie(r.e[j]); } }
+    struct scale { u32 d, pick; };
+    template <int J, int NB> static PSN_DEV void scales0(const raw<NB> &r, int part, scale &s) {
+        typedef pp_blocks<2 * NB, NB> B;
+        s.d = B::scale(raw_word(r.q[J], 0), part);
+        s.pick = B::pick(part);
+    }
+    template <int NB> static PSN_DEV void scales1(const raw<NB> &, scale &) {}
+    template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &r, const scale &s, int i, half_done &t) {
+        const int w = HI * (NB / 4) + i;
+        const u32 next = w + 1 < NB / 2 ? raw_word(r.q[J], w + 1 < NB / 2 ? w + 1 : 0) : r.e[J];
+        q0_halves(__builtin_amdgcn_perm(next, raw_word(r.q[J], w), s.pick) ^ 0x80808080u, 0x64ff64ffu, t);
+    }
+    template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { q0_finish(t, 0x64806480u, s.d, o0, o1); }
+    template <int NB> static PSN_DEV int k_lo(int part) { return 2 * NB * part; }
+    template <int NB> static PSN_DEV int k_hi(int part) { return 2 * NB * part + NB; }
+    static constexpr int SPREAD[2] = {0, 0};
+};
+
+/* Which weight row a group of 32 / NB threads decodes.  The lanes that write to LDS together (sixteen of 16 bytes) should
+ * hit sixteen different columns, (row & 1) * 8 + (chunk ^ row bits 1..3); the lanes of one row hold chunks that leave one
+ * or two chunk bits to the rows.  So the low bits of the group's number go to row bit 0 and to the row bits that scatter
+ * those: SPREAD 0: bits 1, 2, 3 in order; 2: bit 2 first; 3: bit 3 first. */
+template <int SPREAD> PSN_DEV int row_of(int idx) {
+    const int b0 = idx & 1, b1 = (idx >> 1) & 1, b2 = (idx >> 2) & 1, b3 = (idx >> 3) & 1, high = idx & ~15;
+    if constexpr (SPREAD == 2) return high | b0 | (b1 << 2) | (b2 << 1) | (b3 << 3);
+    if constexpr (SPREAD == 3) return high | b0 | (b1 << 3) | (b2 << 1) | (b3 << 2);
+    return idx;
+}
+
+template <int MF> struct pp_mfma;
+template <> struct pp_mfma<32> {
+    typedef float16_t acc;
+    static constexpr int R = 16, KK = 4;                    /* registers per tile, K slices per step */
+    static PSN_DEV acc mul(u32x4 a, u32x4 b, acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0); }
+    static PSN_DEV int row(int lane, int r) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+};
+template <> struct pp_mfma<16> {
+    typedef float4_t acc;
+    static constexpr int R = 4, KK = 2;
+    static PSN_DEV acc mul(u32x4 a, u32x4 b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0); }
+    static PSN_DEV int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+
+template <int OFF> PSN_DEV void lds_write64o(u32 addr, u32x2 v) { asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory"); }
+template <int OFF> PSN_DEV void lds_write128o(u32 addr, u32x4 v) { asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory"); }
+
+/* does piece p of a decode (see there) end in an LDS write? */
+template <int NB> constexpr bool pp_piece_writes(int p) { return p >= 2 && (p & 1) == 1 && (NB == 4 || ((((p - 2) >> 1) % (NB / 4)) & 1) == 1); }
+
+template <typename WF, int BM, int BN, int WM, int MF, int NS>
+PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
+    typedef pp_mfma<MF> MMA;
+    constexpr int WN = 8 / WM, TM = BM / WM / MF, TN = BN / WN / MF, KK = MMA::KK;
+    constexpr int NB = BN / 16, PARTS = 32 / NB;            /* quant bytes per thread and step, threads per weight row */
+    static_assert(NB == 4 || NB == 8, "64 or 128 weight rows");
+    constexpr int SPREAD = WF::SPREAD[NB == 8];
+    constexpr int XBYTES = BM * 128, WBYTES = BN * 128;
+    constexpr int NX = BM / 64;                             /* X loads per wave and step */
+    static_assert(TM >= 1 && TN >= 1 && NX >= 1 && NS * XBYTES + 2 * WBYTES <= 160 * 1024, "tile");
+    extern __shared__ uint4 psn_smem[];
+    typedef __attribute__((address_space(3))) char lds_char;
+    lds_char *const lds_ptr = (lds_char *)psn_smem;
+    const u32 lds0 = (u32)(uintptr_t)lds_ptr;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    const int M = a.M, N = a.N, K = a.K, C = K >> 8;
+
+    /* workgroups b, b + 8, b + 16, ... share an XCD: they get the M tiles (and K ranges) of one N tile in a row, so that a
+     * weight panel is fetched into a single L2 */
+    const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
+    const int S = a.ksplit;
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+    const int per_xcd_n = (nt + 7) >> 3;
+    const int tile_m = local % mt, split = (local / mt) % S, tn_local = local / (mt * S);
+    const int tile_n = xcd + 8 * tn_local;
+    if (tn_local >= per_xcd_n || tile_n >= nt) return;      /* whole workgroup leaves together */
+    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int per_split = (C + S - 1) / S;
+    const int c_begin = split * per_split, c_end = min(c_begin + per_split, C);
+    if (c_begin >= c_end) return;                           /* an empty K range adds nothing */
+    const int nq = c_end - c_begin, nsteps = nq * 4;
+
+    typename MMA::acc acc[TM][TN];
+    UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int j = 0; j < TN; ++j) UNROLL for (int r = 0; r < MMA::R; ++r) acc[i][j][r] = 0.f;
+
+    /* X: 16-byte word s of a stage in LDS order is row s / 8, position s % 8, which holds chunk (s % 8) ^ tile_swz(row) */
+    u32 xoff[NX];
+    UNROLL for (int u = 0; u < NX; ++u) {
+        const int s_ = (wave * NX + u) * 64 + lane, row = s_ >> 3, chunk = (s_ & 7) ^ tile_swz(row);
+        xoff[u] = (u32)min(m0 + row, M - 1) * (u32)(K * 2) + (u32)(chunk * 16);
+    }
+    const char *xbase = reinterpret_cast<const char *>(a.X) + (int64_t)c_begin * 512;
+    auto issue_x = [&](int g, int u) {                      /* stages past the end repeat the last one, into a slot nothing reads any more */
+        const char *xb = xbase + (int64_t)min(g, nsteps - 1) * 128;
+        lds_char *xd = lds_ptr + (g % NS) * XBYTES + wave * (NX * 1024);
+        __builtin_amdgcn_global_load_lds((const void *)(xb + xoff[u]), (__attribute__((address_space(3))) void *)(xd + u * 1024), 16, 0, 0);
+    };
+
+    /* W: this thread's part of its row */
+    const int part = tid % PARTS, wrow = row_of<SPREAD>(tid / PARTS);
+    const uint8_t *wsrc = a.W + (int64_t)min(n0 + wrow, N - 1) * a.row_bytes + (int64_t)c_begin * WF::BYTES;
+    const int woff = WF::template lane_off<NB>(part);
+    const u32 wtile = lds0 + (u32)(NS * XBYTES);
+    const int kl = WF::template k_lo<NB>(part), kh = WF::template k_hi<NB>(part);
+    const u32 wr_lo = wtile + (u32)tile_off(wrow, kl >> 3) + (u32)((kl & 7) * 2), wr_hi = wtile + (u32)tile_off(wrow, kh >> 3) + (u32)((kh & 7) * 2);
+    typename WF::template raw<NB> wa, wb;                   /* chunks of even and of odd number */
+    WF::template clear<NB>(wa);
+    WF::template clear<NB>(wb);
+    auto load_chunk = [&](int c, typename WF::template raw<NB> &r) {
+        WF::template load<NB>(wsrc + (int64_t)min(c, nq - 1) * WF::BYTES, woff, r);
+    };
+    /* The decode of step J of a chunk, in pieces: the scales (two), then two per word of four weights; a finished 16 bytes (8
+     * with NB = 4) goes to fp16 tile J % 2. */
+    constexpr int NW = NB / 4, PIECES = 2 + 4 * NW;
+    u32 dec[4];
+    half_done dhalf;
+    typename WF::scale wscale;
+    auto decode = [&](const typename WF::template raw<NB> &w, auto jc, auto pc) {
+        constexpr int J = decltype(jc)::value, P = decltype(pc)::value, OFF = (J & 1) * WBYTES;
+        if constexpr (P == 0) {
+            WF::template scales0<J, NB>(w, part, wscale);
+        } else if constexpr (P == 1) {
+            WF::template scales1<NB>(w, wscale);
+        } else {
+            constexpr int WORD = (P - 2) >> 1, HI = WORD / NW, I = WORD % NW, B = 2 * I;
+            if constexpr ((P & 1) == 0) {
+                WF::template first<J, NB, HI>(w, wscale, I, dhalf);
+            } else {
+                WF::template second<HI>(wscale, dhalf, dec[B], dec[B + 1]);
+                if constexpr (NB == 4) lds_write64o<OFF>(HI ? wr_hi : wr_lo, (u32x2){dec[0], dec[1]});
+                else if constexpr (B == 2) lds_write128o<OFF>(HI ? wr_hi : wr_lo, (u32x4){dec[0], dec[1], dec[2], dec[3]});
+            }
+        }
+    };
+
+    /* fragment addresses: row (lane % MF) of the wave tile, 16-byte chunk KF kk + lane / MF, swizzled */
+    constexpr int KF = 64 / MF;                             /* chunks per K slice: 2 or 4 */
+    u32 fx[KK], fw[KK];
+    UNROLL for (int kk = 0; kk < KK; ++kk) {
+        fx[kk] = lds0 + (u32)tile_off(wm * (BM / WM) + lane % MF, KF * kk + lane / MF);
+        fw[kk] = wtile + (u32)tile_off(wn * (BN / WN) + lane % MF, KF * kk + lane / MF);
+    }
+    /* Operands of a whole step: K slices 0 .. KK - 1 in sets of their own.  They run half a step behind the reads: period p
+     * reads step p and multiplies the second half of step p - 1, then the first half of step p, so that a fragment has the
+     * time of KK / 2 slices to arrive. */
+    constexpr int HK = KK / 2;
+    u32x4 xf[KK][TM], wf[KK][TN];
+    UNROLL for (int kk = 0; kk < KK; ++kk) { UNROLL for (int i = 0; i < TM; ++i) xf[kk][i] = (u32x4)(0u); UNROLL for (int j = 0; j < TN; ++j) wf[kk][j] = (u32x4)(0u); }
+    constexpr int FR = TM + TN, READS = KK * FR;            /* fragments per slice (those of W first) and per step */
+    auto read_frag = [&](u32 xslot, auto jc, auto rc) {
+        constexpr int R = decltype(rc)::value, kk = R / FR, I = R % FR, OFF = (decltype(jc)::value & 1) * WBYTES;
+        if constexpr (I < TN) wf[kk][I] = lds_read128<OFF + I * 128 * MF>(fw[kk]);
+        else xf[kk][I - TN] = lds_read128<(I - TN) * 128 * MF>(fx[kk] + xslot);
+    };
+
+    /* What rides behind the NPOS MFMAs of a period, spread evenly (a wave that issues several LDS or memory instructions in a
+     * row waits for the queue they go into, and its SIMD's matrix pipe with it): the fragment reads of step p, its share of
+     * the X loads of step p + NS - 1, the pieces of the decode of step p + 1.  The last few MFMAs carry nothing, so that what
+     * the barrier waits for has come in. */
+    constexpr int NPOS = KK * TM * TN, NRIDE = NPOS - (NPOS >= 8 ? 2 : 0);
+    constexpr auto read_pos = [](int r) constexpr { return r * NRIDE / READS; };
+    constexpr auto piece_pos = [](int p) constexpr { return p * NRIDE / PIECES; };
+    /* LDS operations issued in front of MFMA `pos` that are younger than the reads of slice kk (in a position: reads first) */
+    constexpr auto younger = [](int kk, int pos) constexpr {
+        const int last = (kk + 1) * FR - 1, from = last * NRIDE / READS;
+        int n = 0;
+        for (int r = last + 1; r < READS; ++r) n += r * NRIDE / READS < pos;
+        for (int p = 0; p < PIECES; ++p) {
+            const int at = p * NRIDE / PIECES;
+            n += pp_piece_writes<NB>(p) && at >= from && at < pos;
+        }
+        return n > 15 ? 15 : n;                             /* (four bits of counter: waiting for more than needed is harmless) */
+    };
+    auto ride = [&](int c, const typename WF::template raw<NB> &w, auto jc, auto qc) {
+        constexpr int J = decltype(jc)::value, Q = decltype(qc)::value, NEXT = (J + 1) & 3;
+        const u32 xslot = (u32)(((4 * c + J) % NS) * XBYTES);
+#define PSN_PP_READ(R) if constexpr (R < READS && read_pos(R) == Q) read_frag(xslot, jc, pf_int<R>());
+        PSN_PP_READ(0) PSN_PP_READ(1) PSN_PP_READ(2) PSN_PP_READ(3) PSN_PP_READ(4) PSN_PP_READ(5) PSN_PP_READ(6) PSN_PP_READ(7)
+        PSN_PP_READ(8) PSN_PP_READ(9) PSN_PP_READ(10) PSN_PP_READ(11) PSN_PP_READ(12) PSN_PP_READ(13) PSN_PP_READ(14) PSN_PP_READ(15)
+#undef PSN_PP_READ
+        UNROLL for (int u = 0; u < NX; ++u)
+            if (u * NRIDE / NX == Q) issue_x(4 * c + J + NS - 1, u);
+#define PSN_PP_PIECE(P) if constexpr (P < PIECES && piece_pos(P) == Q) decode(w, pf_int<NEXT>(), pf_int<P>());
+        PSN_PP_PIECE(0) PSN_PP_PIECE(1) PSN_PP_PIECE(2) PSN_PP_PIECE(3) PSN_PP_PIECE(4) PSN_PP_PIECE(5) PSN_PP_PIECE(6) PSN_PP_PIECE(7) PSN_PP_PIECE(8) PSN_PP_PIECE(9)
+#undef PSN_PP_PIECE
+    };
+    static_assert(READS <= 16 && PIECES <= 10, "rides");
+    auto multiply = [&](auto kc, auto &&behind) {
+        constexpr int kk = decltype(kc)::value;
+        UNROLL for (int j = 0; j < TN; ++j) UNROLL for (int i = 0; i < TM; ++i) {
+            __builtin_amdgcn_sched_barrier(0);
+            acc[i][j] = MMA::mul(xf[kk][i], wf[kk][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+            behind(j * TM + i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    /* slice Q of period p = 4 c + J: multiplies K slice (Q + HK) % KK, of step p - 1 while Q < HK */
+    auto slice = [&](int c, const typename WF::template raw<NB> &w, auto jc, auto qc) {
+        constexpr int Q = decltype(qc)::value, kk = (Q + HK) % KK;
+        if constexpr (Q >= HK) {
+            static_assert(((kk + 1) * FR - 1) * NRIDE / READS < Q * TM * TN, "read before it is multiplied");
+            asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(younger(kk, Q * TM * TN)) : "memory");
+            tie(xf[kk]);
+            tie(wf[kk]);
+        }
+        multiply(pf_int<kk>(), [&](int pos) {
+#define PSN_PP_RIDE(P) if (pos == P) { if constexpr (P < TM * TN) ride(c, w, jc, pf_int<Q * TM * TN + P>()); }
+            PSN_PP_RIDE(0) PSN_PP_RIDE(1) PSN_PP_RIDE(2) PSN_PP_RIDE(3) PSN_PP_RIDE(4) PSN_PP_RIDE(5) PSN_PP_RIDE(6) PSN_PP_RIDE(7)
+#undef PSN_PP_RIDE
+        });
+    };
+    /* (a set is read into only after its last use: slice kk >= HK is multiplied in slices 0 .. KK - HK - 1 of the period) */
+    UNROLL for (int kk = HK; kk < KK; ++kk) {
+        constexpr auto ok = [](int k) constexpr { return k * FR * NRIDE / READS >= (k - HK + 1) * TM * TN - 1; };
+        static_assert(ok(HK) && ok(KK - 1), "fragment sets overlap");
+    }
+
+    load_chunk(0, wa);
+    UNROLL for (int g = 0; g < NS - 1; ++g) UNROLL for (int u = 0; u < NX; ++u) issue_x(g, u);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    WF::template landed<NB>(wa);
+    load_chunk(1, wb);
+#define PSN_PP_PIECE(P) if constexpr (P < PIECES) decode(wa, pf_int<0>(), pf_int<P>());
+    PSN_PP_PIECE(0) PSN_PP_PIECE(1) PSN_PP_PIECE(2) PSN_PP_PIECE(3) PSN_PP_PIECE(4) PSN_PP_PIECE(5) PSN_PP_PIECE(6) PSN_PP_PIECE(7) PSN_PP_PIECE(8) PSN_PP_PIECE(9)
+#undef PSN_PP_PIECE
+    lds_barrier();
+
+    /* Period p = 4 c + J, between two barriers.  Nobody touches the stage of X of step p - 1 nor the fp16 tile of step p - 1
+     * any more, which are the ones that X of step p + NS - 1 and the weights of step p + 1 go to.  Its end: X of step p + 1 has
+     * landed -- everything but the X loads of the NS - 2 steps after it and, where they are younger, the raw loads (which go
+     * first in periods J = 3) -- and this wave's reads and writes of LDS are done. */
+#define PSN_PP_STEP(J, w, wother)                                                                                          \
+    {                                                                                                                      \
+        if constexpr (J == 3) {                                                                                            \
+            load_chunk(c + 2, w);                                                                                          \
+            WF::template landed<NB>(wother);                                                                               \
+        }                                                                                                                  \
+        slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<0>());                                                           \
+        slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<1>());                                                           \
+        if constexpr (KK > 2) {                                                                                            \
+            slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<(KK > 2 ? 2 : 0)>());                                        \
+            slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<(KK > 2 ? 3 : 0)>());                                        \
+        }                                                                                                                  \
+        constexpr int KEEP = (NS - 2) * NX + ((J + 1) % 4 < NS - 2 ? WF::LOADS : 0);                                       \
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(KEEP) : "memory");                               \
+        UNROLL for (int kk = HK; kk < KK; ++kk) { tie(xf[kk]); tie(wf[kk]); }                                              \
+    }
+#define PSN_PP_CHUNK(w, wother) PSN_PP_STEP(0, w, wother) PSN_PP_STEP(1, w, wother) PSN_PP_STEP(2, w, wother) PSN_PP_STEP(3, w, wother)
+    int c = 0;
+    for (; c + 1 < nq; ++c) {
+        PSN_PP_CHUNK(wa, wb)
+        ++c;
+        PSN_PP_CHUNK(wb, wa)
+    }
+    if (c < nq) { PSN_PP_CHUNK(wa, wb) }
+#undef PSN_PP_CHUNK
+#undef PSN_PP_STEP
+    multiply(pf_int<HK>(), [](int) {});
+    if constexpr (KK > 2) multiply(pf_int<(KK > 2 ? HK + 1 : HK)>(), [](int) {});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    /* the last raw loads were for nothing, but their registers belong to them until they have landed */
+    WF::template landed<NB>(wa);
+    WF::template landed<NB>(wb);
+
+    /* (worked out again from an opaque thread index, so that nothing of it stays in a register through the loop) */
+    int tid_out = threadIdx.x;
+    asm volatile("" : "+v"(tid_out));
+    const int wm_o = (tid_out >> 6) / WN, wn_o = (tid_out >> 6) % WN, lane_o = tid_out & 63;
+    UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int j = 0; j < TN; ++j) {
+        const int col = n0 + wn_o * (BN / WN) + MF * j + lane_o % MF;
+        UNROLL for (int r = 0; r < MMA::R; ++r) {
+            const int row = m0 + wm_o * (BM / WM) + MF * i + MMA::row(lane_o, r);
+            if (row < M && col < N) {
+                if (S == 1) a.Y[(int64_t)row * N + col] = acc[i][j][r];
+                else unsafeAtomicAdd(&a.Y[(int64_t)row * N + col], acc[i][j][r]);
+            }
+        }
+    }
+}
+
+
+#define PSN_PP(fmt, WF, BM, BN, WM, MF, NS)                                                                                  \
+    extern "C" __global__ void __launch_bounds__(512) psn_prefill_##fmt##_m##BM##_n##BN##_pp(const psn_prefill_args a) {    \
+        prefill_pp_body<WF, BM, BN, WM, MF, NS>(a);                                                                          \
+    }
+#define PSN_PP_FAMILY(fmt, WF)           \
+    PSN_PP(fmt, WF, 64, 64, 2, 16, 4)    \
+    PSN_PP(fmt, WF, 64, 128, 2, 32, 4)   \
+    PSN_PP(fmt, WF, 128, 128, 2, 32, 4)  \
+    PSN_PP(fmt, WF, 256, 128, 4, 32, 4)
+
+#ifdef PSN_BUILD_PP_Q4_0
+PSN_PP_FAMILY(q4_0, PpQ4_0)
+#endif
+#ifdef PSN_BUILD_PP_Q8_0
+PSN_PP_FAMILY(q8_0, PpQ8_0)
+#endif
+#ifdef PSN_BUILD_PP_Q4_K
+PSN_PP_FAMILY(q4_K, PpQ4_K)
+#endif
+#ifdef PSN_BUILD_PP_Q5_K
+PSN_PP_FAMILY(q5_K, PpQ5_K)
+#endif
+#ifdef PSN_BUILD_PP_Q6_K
+PSN_PP_FAMILY(q6_K, PpQ6_K)
+#endif

@@ -390,3 +390,22 @@ def test_prefill_refuses_operands_beyond_32_bit_offsets(hip, orc):
     with pytest.raises(backend.PsnError) as e:
         hip.quantized_matmul_packed(x, x, y, 1 << 20, 64, 4096)
     assert e.value.name == "PSN_E_SHAPE"
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
+def test_in_loop_kernels_at_tile_and_range_edges(hip, orc, qname):
+    """The eight-wave kernels (family 4, tiles of 64 and 128 columns) one row and column either side of their tiles, with K
+    ranges of one, two, an odd and an even number of 256-wide chunks (their loop takes chunks in pairs and asks for raw
+    bytes two chunks ahead), and a K split that leaves a range empty.  fp16 products are exact in fp32, so only the order
+    of at most 2048 sums differs from the oracle: PARITY_TOL is far above 2048 * 2^-24."""
+    t = getattr(orc, qname)
+    for tile in ((64, 64), (64, 128), (128, 128), (256, 128)):
+        for m, n, k in ((tile[0] - 1, tile[1] + 1, 256), (tile[0] + 1, tile[1] - 1, 512), (tile[0], tile[1], 768), (65, 3 * tile[1], 2048)):
+            say(f"in-loop {qname} tile={tile} m={m} n={n} k={k}")
+            W = weights(orc, qname, 880, n, k)
+            X = G.seeded_acts(881 + m, m, k).astype(np.float16)
+            ref = orc.prefill(t, W, X, n, k)
+            for ksplit in (1, 4) if (m * n) % 4 == 0 else (1,):
+                y = hip.matmul_host(t, W, X, n, k, tile + (ksplit, 4))
+                err = G.max_rel_err(y, ref)
+                assert np.all(np.isfinite(y)) and err < PARITY_TOL, (tile, ksplit, m, n, k, err)
