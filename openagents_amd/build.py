@@ -40,6 +40,7 @@ CODE_OBJECTS = [
     *[(f"psn_pf_{fmt}_base", "psn_prefill.hip", ["-DPSN_BUILD_ONLY", "-DPSN_BUILD_PF=4", f"-DPSN_BUILD_PF_{fmt.upper()}"])
       for fmt in ("q4_K", "q5_K", "q6_K")],
     *[(f"psn_pp_{fmt}", "psn_prefill_pp.hip", [f"-DPSN_BUILD_PP_{fmt.upper()}"]) for fmt in ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K")],
+    *[(f"psn_th_{fmt}", "psn_prefill_thin.hip", [f"-DPSN_BUILD_TH_{fmt.upper()}"]) for fmt in ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K")],
     ("psn_decode", "psn_decode.hip", []),
     ("psn_calib", "psn_calib.hip", []),
 ]
@@ -75,7 +76,7 @@ def build(jobs: int = 0, verbose: bool = True, reuse_device: bool = False) -> st
     jobs = jobs or min(8, os.cpu_count() or 1)
     todo = [(stem, src, defs) for stem, src, defs in CODE_OBJECTS if os.path.exists(os.path.join(CSRC, src))]
 
-    device_headers = ["psn_args.h", "psn_device.h", "psn_prefill_common.h"]
+    device_headers = ["psn_args.h", "psn_device.h", "psn_prefill_common.h", "psn_prefill_formats.h"]
 
     def compile_co(item):
         stem, src, defs = item

@@ -1391,16 +1391,46 @@ extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int
                                             int32_t *waves) {
     return psn_qmatmul_prefill_plan_for(PSN_Q4_0, M, N, K, cus, tile_m, tile_n, ksplit, waves);
 }
-/* at most 64 rows (every format; Q6_K when its rows are whole 16-byte words): the weight-streaming kernel on 64 x 64 tiles; K is cut (atomic adds) only
- * while the weight rows alone leave half of the compute units without a workgroup, down to two chunks per range */
-static void plan_weight_stream(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit, int32_t *waves) {
-    const int64_t nt = (N + 63) / 64, C = K / 256;
-    int sp = 1;
-    while (sp < 8 && nt * sp * 2 <= cus && C / (sp * 2) >= 2 && (M * N) % 4 == 0) sp *= 2;
-    *tile_m = 64;
-    *tile_n = 64;
-    *ksplit = sp;
-    *waves = 64;
+/* At most 64 rows: which kernel streams the weights.  psn_prefill_<fmt>_thin_<tm>_<rt> (psn_prefill_thin.hip, 16 tm rows of X and 16 rt
+ * of W per workgroup) against the 64 x 64 kernel (psn_prefill_<fmt>_skinny; rt = 0 here; with Q6_K only for rows of whole 16-byte
+ * words).  Measured on MI355X over five formats, fifteen matrices and M = 16 .. 64 (2300 launches; the estimates are off by 6 % rms,
+ * and what they pick is within 0.5 % of the fastest on average): a launch, then per round of workgroups the first loads, a chain
+ * per chunk of a wave, and the work that the waves of a SIMD share: decode per weight row, X per row of it.  The 64 x 64 kernel stays
+ * the faster one from about 48 rows on where the matrix is large (Q4_0 8192 x 28672 M = 64: 62 us against 65-75), with Q8_0, whose raw
+ * chunks leave no LDS for four tiles, from 17 on (14336 x 4096 M = 32: 23.4 against 26); it cuts K only while the weight rows
+ * alone leave half of the compute units without a workgroup.  At rt = 4 a cut of K did not pay. */
+struct weight_stream_plan { int rt, ksplit; double us; };
+static const double k_thin_row_us[5] = {0.719, 1.348, 0.878, 1.062, 1.695};       /* decode of 16 rows x 256: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
+static const double k_stream64_chunk_us[5] = {0.963, 1.196, 1.175, 1.242, 1.519}; /* 64 rows x 256 in the 64 x 64 kernel */
+static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus) {
+    const int f = format_index(qtype), tm = (int)((M + 15) / 16);
+    const int64_t C = K / 256;
+    const double y_mb = (double)(M * N) * 4e-6;
+    const auto cut_us = [&](int sp) { return sp > 1 ? 1.87 + 0.79 * y_mb * sp : 0.0; };   /* zero fill and atomic adds */
+    const auto may_cut = [&](int sp) { return sp == 1 || ((M * N) % 4 == 0 && C >= 2 * sp); };
+    weight_stream_plan best = {-1, 1, 1e300};
+    if (qtype != PSN_Q6_K || K % 2048 == 0) {
+        const int64_t nt = (N + 63) / 64;
+        int sp = 1;
+        while (sp < 8 && nt * sp * 2 <= cus && may_cut(sp * 2)) sp *= 2;
+        const double rounds = (double)((nt * sp + cus - 1) / cus);
+        best = {0, sp, 0.97 * (3.8 + rounds * (double)((C + sp - 1) / sp) * k_stream64_chunk_us[f] + cut_us(sp) + 0.19 * y_mb)};
+    }
+    for (int rt = 1; rt <= 4; rt *= 2) {
+        const bool big = qtype == PSN_Q8_0 || qtype == PSN_Q6_K;     /* raw chunks of five or six registers a lane instead of three */
+        /* kernels that exist: LDS and registers end at 48 rows of X (Q8_0: 16); at 16 the others' rt = 2 shares compute units */
+        if (rt == 4 && (tm > (qtype == PSN_Q8_0 ? 1 : 3) || (tm == 1 && !big))) continue;
+        const int per_cu = tm == 1 && (rt == 1 || (rt == 2 && !big)) ? 2 : 1;          /* up to 128 registers */
+        for (int sp = 1; sp <= (rt == 4 ? 1 : 4); sp *= 2) {
+            if (!may_cut(sp)) continue;
+            const int64_t wgs = (N + 16 * rt - 1) / (16 * rt) * sp, per = (C + sp - 1) / sp;
+            const double rounds = (double)((wgs + cus * per_cu - 1) / (cus * per_cu)), shared = (double)((wgs + cus - 1) / cus);
+            const double us = 0.9 + rounds * (1.22 + 0.316 * rt * (double)((per + 7) / 8)) +
+                              shared * (double)per * (rt * (k_thin_row_us[f] + 0.04 * tm) + 0.604 * tm) / 8 + cut_us(sp) + 1.52 * y_mb;
+            if (us < best.us) best = {rt, sp, us};
+        }
+    }
+    return best;
 }
 /* family 4: the tile and the K split with the smallest estimate; K ranges hold at least two 256-wide chunks */
 static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
@@ -1432,7 +1462,8 @@ static int32_t prefill_plan_any(int32_t qtype, int64_t M, int64_t N, int64_t K, 
     if (M <= 0 || N <= 0 || K <= 0 || K % 256) return fail(PSN_E_SHAPE, "prefill plan: M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
     if (cus <= 0) cus = 256;
     if (M <= 64 && (qtype != PSN_Q6_K || K % 2048 == 0)) {
-        plan_weight_stream(M, N, K, cus, tile_m, tile_n, ksplit, waves);
+        *tile_m = *tile_n = *waves = 64;
+        *ksplit = plan_weight_stream(qtype, M, N, K, cus).ksplit;
         return PSN_OK;
     }
     *waves = 4;
@@ -1471,27 +1502,46 @@ static int32_t launch_unpack(psn_module *mod, psn_stream *s, int32_t qtype, cons
     snprintf(name, sizeof name, "psn_prefill_%s_unpack", fmt_name(qtype));
     return launch(mod, s, name, (unsigned)((N + 255) / 256 * (K / 256)), 256, 0, &u);
 }
+static int32_t fill_zero_y(psn_module *mod, psn_stream *s, psn_buf *Y, int64_t M, int64_t N) {
+    psn_fill_args f;
+    f.p = (uint32_t *)Y->p;
+    f.n16 = M * N / 4;
+    const int64_t fb = (f.n16 + 255) / 256;
+    return launch(mod, s, "psn_fill_zero", (unsigned)(fb > 2048 ? 2048 : fb), 256, 0, &f);
+}
+static void prefill_args(psn_prefill_args *a, const void *W, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N, int64_t K, int32_t ksplit, int64_t row_bytes) {
+    memset(a, 0, sizeof *a);
+    a->W = (const uint8_t *)W;
+    a->X = (const uint16_t *)X->p;
+    a->Y = (float *)Y->p;
+    a->M = (int32_t)M;
+    a->N = (int32_t)N;
+    a->K = (int32_t)K;
+    a->ksplit = ksplit;
+    a->row_bytes = row_bytes;
+}
+static int32_t launch_thin(psn_module *mod, psn_stream *s, int32_t qtype, const psn_buf *W, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N,
+                           int64_t K, int rt, int32_t ksplit) {
+    static const int lds_row[5] = {144, 272, 144, 176, 224};    /* a row's chunk in LDS */
+    const int tm = (int)((M + 15) / 16), rings = 8 * (16 * rt * lds_row[format_index(qtype)] + tm * 2048), sums = 8 * 1024 * rt * tm;
+    const int lds = rings > sums ? rings : sums;
+    if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: %d x %d rows need %d bytes of LDS, device offers %d", 16 * tm, 16 * rt, lds, mod->ctx->max_lds);
+    int32_t rc = bind(mod->ctx);
+    if (rc) return rc;
+    if (ksplit > 1 && (rc = fill_zero_y(mod, s, Y, M, N))) return rc;
+    psn_prefill_args a;
+    prefill_args(&a, W->p, X, Y, M, N, K, ksplit, psn_row_bytes(qtype, K));
+    char name[96];
+    snprintf(name, sizeof name, "psn_prefill_%s_thin_%d_%d", fmt_name(qtype), tm, rt);
+    return launch(mod, s, name, (unsigned)((N + 16 * rt - 1) / (16 * rt) * ksplit), 512, (unsigned)lds, &a);
+}
 static int32_t launch_dense(psn_module *mod, psn_stream *s, const void *packed, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N, int64_t K,
                             int32_t bm, int32_t ksplit) {
     int32_t rc;
-    if (ksplit > 1) {
-        psn_fill_args f;
-        f.p = (uint32_t *)Y->p;
-        f.n16 = M * N / 4;
-        const int64_t fb = (f.n16 + 255) / 256;
-        if ((rc = launch(mod, s, "psn_fill_zero", (unsigned)(fb > 2048 ? 2048 : fb), 256, 0, &f))) return rc;
-    }
+    if (ksplit > 1 && (rc = fill_zero_y(mod, s, Y, M, N))) return rc;
     const int64_t nt = (N + 255) / 256, mt = (M + bm - 1) / bm;
     psn_prefill_args a;
-    memset(&a, 0, sizeof a);
-    a.W = (const uint8_t *)packed;
-    a.X = (const uint16_t *)X->p;
-    a.Y = (float *)Y->p;
-    a.M = (int32_t)M;
-    a.N = (int32_t)N;
-    a.K = (int32_t)K;
-    a.ksplit = ksplit;
-    a.row_bytes = K * 2;
+    prefill_args(&a, packed, X, Y, M, N, K, ksplit, K * 2);
     /* LDS: a ring of four stages of X, bm rows x 32 k fp16 each */
     return launch(mod, s, bm == 128 ? "psn_prefill_dense_f16_m128" : "psn_prefill_dense_f16", (unsigned)(8 * ((nt + 7) / 8) * mt * ksplit), 256, 4 * bm * 64, &a);
 }
@@ -1584,23 +1634,9 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
     const int lds = pp ? (4 * bm + 2 * bn) * 128 : skinny ? (skinny_rings > 8 * 16384 ? skinny_rings : 8 * 16384) : wide ? wide_rings : waves == 16 ? 0 : 2 * (bm + bn) * 128;
     if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: tile %dx%d needs %d bytes of LDS, device offers %d", bm, bn, lds, mod->ctx->max_lds);
     if ((rc = bind(mod->ctx))) return rc;
-    if (ksplit > 1) {
-        psn_fill_args f;
-        f.p = (uint32_t *)Y->p;
-        f.n16 = M * N / 4;
-        const int64_t fb = (f.n16 + 255) / 256;
-        if ((rc = launch(mod, s, "psn_fill_zero", (unsigned)(fb > 2048 ? 2048 : fb), 256, 0, &f))) return rc;
-    }
+    if (ksplit > 1 && (rc = fill_zero_y(mod, s, Y, M, N))) return rc;
     psn_prefill_args a;
-    memset(&a, 0, sizeof a);
-    a.W = (const uint8_t *)W->p;
-    a.X = (const uint16_t *)X->p;
-    a.Y = (float *)Y->p;
-    a.M = (int32_t)M;
-    a.N = (int32_t)N;
-    a.K = (int32_t)K;
-    a.ksplit = ksplit;
-    a.row_bytes = psn_row_bytes(qtype, K);
+    prefill_args(&a, W->p, X, Y, M, N, K, ksplit, psn_row_bytes(qtype, K));
     const int64_t mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
     char name[96];
     if (skinny) {
@@ -1622,6 +1658,12 @@ extern "C" int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t q
     int32_t rc = check_prefill("psn_qmatmul_prefill", mod, s, qtype, W, X, Y, M, N, K);
     if (rc) return rc;
     int32_t bm = 0, bn = 0, sp = 1, wv = 4;
+    if (M <= 64) {
+        const weight_stream_plan p = plan_weight_stream(qtype, M, N, K, mod->ctx->compute_units);
+        /* (Q6_K rows that are not whole 16-byte words: the kernels that decode in their loop are what it competes with) */
+        const bool thin = p.rt > 0 && ((qtype != PSN_Q6_K || K % 2048 == 0) || p.us < plan_in_loop(qtype, M, N, K, mod->ctx->compute_units, &bm, &bn, &sp));
+        if (thin) return launch_thin(mod, s, qtype, W, X, Y, M, N, K, p.rt, p.ksplit);
+    }
     /* the dense family needs nt * 256 * K fp16 values of workspace on this stream: it competes when that is
      * there already or may still be allocated (not while capturing, not once a graph holds the workspace) */
     bool cap = false;

@@ -409,3 +409,26 @@ def test_in_loop_kernels_at_tile_and_range_edges(hip, orc, qname):
                 y = hip.matmul_host(t, W, X, n, k, tile + (ksplit, 4))
                 err = G.max_rel_err(y, ref)
                 assert np.all(np.isfinite(y)) and err < PARITY_TOL, (tile, ksplit, m, n, k, err)
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
+def test_thin_kernels_at_tile_and_range_edges(hip, orc, qname):
+    """The kernels for at most 64 rows of X that the library picks by itself (16 to 64 rows of X, 16 to 64 of W): X at either
+    end of its sixteens, fewer weight rows than a tile, ragged last tiles, K ranges in which no, some and all of the eight
+    waves have a chunk, one and several, with and without a cut of K -- every kernel of the format (the launch log tells).  fp16 products
+    are exact in fp32, so only the order of at most 4096 sums differs from the oracle: PARITY_TOL is far above 2^-24 sqrt(4096)."""
+    t = getattr(orc, qname)
+    ran = set()
+    for n, k, ms in ((5, 256, (1, 17, 33, 49)), (17, 768, (16, 32, 48, 64)), (300, 2304, (1, 31, 40, 64)), (516, 4096, (15, 33, 63)),
+                     (4104, 1280, (1, 17, 33, 49)), (4109, 512, (16, 32, 48, 64)), (8209, 256, (1, 17, 33)), (8209, 1024, (16, 18, 33))):
+        W = weights(orc, qname, 890, n, k)
+        for m in ms:
+            say(f"thin {qname} m={m} n={n} k={k}")
+            X = G.seeded_acts(891 + m, m, k).astype(np.float16)
+            hip.lib.psn_launch_log_clear()
+            y = hip.matmul_host(t, W, X, n, k)
+            ran |= {name for name in hip.lib.psn_launch_log().decode().split(";") if "_thin_" in name}
+            err = G.max_rel_err(y, orc.prefill(t, W, X, n, k))
+            assert np.all(np.isfinite(y)) and err < PARITY_TOL, (m, n, k, err)
+    tall = {"Q8_0": (1,), "Q6_K": (1, 2, 3)}.get(qname, (2, 3))
+    assert ran == {f"psn_prefill_{qname[0].lower() + qname[1:]}_thin_{tm}_{rt}" for rt in (1, 2, 4) for tm in (tall if rt == 4 else (1, 2, 3, 4))}
