@@ -331,6 +331,12 @@ PSN_DEV void tie1(u32 &v) { asm volatile("" : "+v"(v)); }
 /* workgroup barrier that waits for this wave's LDS traffic only, not for loads still in flight */
 PSN_DEV void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+/* ---- memory access the compiler sees (it places the waits), with the alignment a format guarantees ---- */
+template <typename T, int A> struct __attribute__((packed, aligned(A))) at_least { T v; };
+template <int A, typename T> PSN_DEV void fetch(const uint8_t *p, T &v) { v = reinterpret_cast<const at_least<T, A> *>(p)->v; }
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+template <int A, typename T> PSN_DEV void fetch(const lds_u8 *p, T &v) { v = reinterpret_cast<const __attribute__((address_space(3))) at_least<T, A> *>(p)->v; }
+template <int A, typename T> PSN_DEV void store(lds_u8 *p, T v) { reinterpret_cast<__attribute__((address_space(3))) at_least<T, A> *>(p)->v = v; }
 
 PSN_DEV void unpack4(const uint4 v, u32 *dst) { dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; dst[3] = v.w; }
 

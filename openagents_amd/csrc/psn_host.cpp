@@ -1054,28 +1054,56 @@ struct norm_fusion {
     bool pair;      /* two matrices, a gate and an up projection: the launch stores silu(W0 x) * (W1 x) into y[0] */
 };
 
+static void matvec_args(psn_matvec_args *a, int32_t qtype, const seg_list &sg, int64_t K, int32_t batch, int32_t threads, int32_t blocks) {
+    memset(a, 0, sizeof *a);
+    int64_t end = 0;
+    for (int i = 0; i < PSN_MAX_SEGMENTS; ++i) {
+        const int j = i < sg.count ? i : sg.count - 1;
+        if (i < sg.count) end += sg.N[i];
+        a->W[i] = (const uint8_t *)sg.W[j];
+        a->y[i] = sg.y[j];
+        a->row_end[i] = (int32_t)end;
+    }
+    a->N = (int32_t)sg.total;
+    a->K = (int32_t)K;
+    a->batch = batch;
+    a->nseg = sg.count;
+    a->row_bytes = psn_row_bytes(qtype, K);
+    a->threads = threads;
+    a->blocks = blocks;
+}
+/* psn_mvb_<fmt>_q8 (psn_matvec_batch.hip), on quantized activations.  Its cost does not grow with the batch; the register kernels' does.
+ * Measured on MI355X against them over 200 .. 40000 rows and K = 256 .. 16384: from five columns on 1.0-6 x faster throughout.  With three or
+ * four it is the slower one for long rows (0.66-0.96 x from K = 8192 on: eight waves to a tile make a long chain), for Q4_0 rows of 4096
+ * (0.97-1.07 x) and for many short Q8_0 rows (14336 x 2560: 1.00-1.01 x, 40000 x 1024: 0.88 x), otherwise 1.0-1.8 x. */
+static bool use_batch_kernel(int32_t qtype, int64_t rows, int64_t K, int32_t batch) {
+    if (qtype != PSN_Q4_0 && qtype != PSN_Q8_0) return false;
+    if (batch >= 5) return true;
+    return batch >= 3 && (qtype == PSN_Q4_0 ? K < 4096 : K <= 4096 && (K > 2560 || rows <= 8192));
+}
+static int32_t run_batch(psn_module *mod, psn_stream *s, int32_t qtype, const seg_list &sg, const void *xq, int64_t K, int32_t batch) {
+    psn_actq_info li;
+    int32_t rc = psn_actq_layout(psn_act_type_for(qtype), K, batch, &li);
+    if (rc) return rc;
+    int64_t blocks = 0;
+    for (int i = 0; i < sg.count; ++i) blocks += (sg.N[i] + 15) / 16;
+    psn_matvec_args a;
+    matvec_args(&a, qtype, sg, K, batch, 512, (int32_t)blocks);
+    a.xqs = (const int8_t *)xq + li.off_qs;
+    a.xd = (const float *)((const char *)xq + li.off_d);
+    a.xs = (const char *)xq + li.off_s;
+    const unsigned lds = 8 * (unsigned)(16 * (qtype == PSN_Q4_0 ? 144 : 272) + 8 * 272 + 512);   /* a chunk of the rows and of the columns per wave */
+    char name[96];
+    snprintf(name, sizeof name, "psn_mvb_%s_q8", fmt_name(qtype));
+    return launch(mod, s, name, (unsigned)blocks, 512, lds, &a);
+}
 static int32_t run_matvec(psn_module *mod, psn_stream *s, int32_t qtype, int32_t scheme, const seg_list &sg, const void *x,
                           int64_t K, int32_t batch, const psn_matvec_plan *plan, const norm_fusion *norm = nullptr) {
     int32_t lds = 0;
     int32_t rc = plan->mfma ? PSN_OK : plan_is_valid(plan, qtype, scheme, K, batch, mod->ctx->max_lds, &lds);
     if (rc) return rc;
     psn_matvec_args a;
-    memset(&a, 0, sizeof a);
-    int64_t end = 0;
-    for (int i = 0; i < PSN_MAX_SEGMENTS; ++i) {
-        const int j = i < sg.count ? i : sg.count - 1;
-        if (i < sg.count) end += sg.N[i];
-        a.W[i] = (const uint8_t *)sg.W[j];
-        a.y[i] = sg.y[j];
-        a.row_end[i] = (int32_t)end;
-    }
-    a.N = (int32_t)sg.total;
-    a.K = (int32_t)K;
-    a.batch = batch;
-    a.nseg = sg.count;
-    a.row_bytes = psn_row_bytes(qtype, K);
-    a.threads = plan->threads;
-    a.blocks = plan->blocks;
+    matvec_args(&a, qtype, sg, K, batch, plan->threads, plan->blocks);
     char name[96];
     if (plan->mfma) {
         int64_t total = 0;
@@ -1196,6 +1224,10 @@ extern "C" int32_t psn_qmatvec_q8_multi(psn_module *mod, psn_stream *s, int32_t 
     int32_t rc = gather_segments("psn_qmatvec_q8_multi", mod, s, qtype, PSN_ACT_Q8, count, W, xq, y, N, K, batch, &sg);
     if (rc) return rc;
     if ((rc = check_x_q8("psn_qmatvec_q8_multi", qtype, xq, K, batch))) return rc;
+    if (use_batch_kernel(qtype, sg.total, K, batch)) {
+        if ((rc = bind(mod->ctx))) return rc;
+        return run_batch(mod, s, qtype, sg, xq->p, K, batch);
+    }
     psn_matvec_plan plan;
     if ((rc = make_plan(qtype, PSN_ACT_Q8, sg.total, K, batch, mod->ctx->compute_units, false, sg.N, sg.count, &plan))) return rc;
     if ((rc = bind(mod->ctx))) return rc;
@@ -1227,6 +1259,7 @@ extern "C" int32_t psn_qmatvec_multi(psn_module *mod, psn_stream *s, int32_t qty
     if ((rc = ensure_workspace(s, li.bytes))) return rc;
     if ((rc = note_workspace_use(s))) return rc;    /* a graph being recorded bakes the workspace address into its nodes */
     if ((rc = quantize_into(mod, s, at, (const float *)x->p, s->ws->p, K, batch))) return rc;
+    if (use_batch_kernel(qtype, sg.total, K, batch)) return run_batch(mod, s, qtype, sg, s->ws->p, K, batch);
     return run_matvec(mod, s, qtype, scheme, sg, s->ws->p, K, batch, &plan);
 }
 

@@ -27,13 +27,6 @@
 
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-/* ---- memory access the compiler sees (it places the waits), with the alignment a format guarantees ---- */
-template <typename T, int A> struct __attribute__((packed, aligned(A))) at_least { T v; };
-template <int A, typename T> PSN_DEV void fetch(const uint8_t *p, T &v) { v = reinterpret_cast<const at_least<T, A> *>(p)->v; }
-typedef __attribute__((address_space(3))) uint8_t lds_u8;
-template <int A, typename T> PSN_DEV void fetch(const lds_u8 *p, T &v) { v = reinterpret_cast<const __attribute__((address_space(3))) at_least<T, A> *>(p)->v; }
-template <int A, typename T> PSN_DEV void store(lds_u8 *p, T v) { reinterpret_cast<__attribute__((address_space(3))) at_least<T, A> *>(p)->v = v; }
-
 /* A row's chunk: WORDS 16-byte words are copied to LDS as they are, rows STRIDE bytes apart; read() takes what step J of part g
  * needs from there. */
 template <typename WF> struct Feed;

@@ -954,3 +954,37 @@ def test_default_plans_over_seeded_random_shapes(hip, orc):
             y = hip.alloc(batch * n * 4)
             hip.quantized_matvec_q8(w, xq, y, batch)
             assert G.max_rel_err(y.download(np.float32, (batch, n)), ref) < 2e-5, (qname, n, k, batch, "q8 in")
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0"])
+def test_batch_kernel_at_tile_and_range_edges(hip, orc, qname):
+    """The int8-MFMA kernel for three to eight columns: fewer rows than a tile, ragged last tiles, K ranges in which no, some and all of the
+    eight waves have a chunk, one and several; several ragged matrices in a launch; activations quantized by the call and before it.  The
+    integer dot products are exact, so only the order of at most 512 fp32 sums of three roundings each differs: far below PARITY_TOL."""
+    t = getattr(orc, qname)
+    name = f"psn_mvb_{qname.lower()}_q8"
+    for n, k in ((5, 256), (16, 768), (300, 2304), (1000, 2560), (70, 16384)):
+        W = orc.quantize(t, G.seeded_weights(9300, n, k))
+        w = hip.upload_weight(t, W, n, k)
+        for b in (3, 4, 5, 8):
+            if b < 5 and k > 4096:
+                continue                                    # the register kernels' range
+            x = G.seeded_acts(9301 + b, b, k)
+            ref = orc.matvec(t, orc.ACT_Q8, W, x, n, k)
+            xb, y = hip.upload(x), hip.alloc(b * n * 4)
+            xq = hip.quantize_activations(xb, k, b, backend.act_type_for(t))
+            for call in (lambda: hip.quantized_matvec(w, xb, y, b, _ffi.ACT_Q8), lambda: hip.quantized_matvec_q8(w, xq, y, b)):
+                y.fill_zero()
+                hip.lib.psn_launch_log_clear()
+                call()
+                assert name in hip.lib.psn_launch_log().decode().split(";"), (n, k, b)
+                err = G.max_rel_err(y.download(np.float32, (b, n)), ref)
+                assert err < PARITY_TOL, (n, k, b, err)
+    k, b, rows = 1280, 7, (33, 16, 5, 130)
+    Ws = [orc.quantize(t, G.seeded_weights(9310 + i, n, k)) for i, n in enumerate(rows)]
+    x = G.seeded_acts(9320, b, k)
+    for count in (2, 3, 4):
+        ys = [hip.alloc(b * n * 4) for n in rows[:count]]
+        hip.quantized_matvec_multi([hip.upload_weight(t, W, n, k) for W, n in zip(Ws, rows[:count])], hip.upload(x), ys, b, _ffi.ACT_Q8)
+        for W, n, y in zip(Ws, rows, ys):
+            assert G.max_rel_err(y.download(np.float32, (b, n)), orc.matvec(t, orc.ACT_Q8, W, x, n, k)) < PARITY_TOL, (count, n)
