@@ -228,8 +228,8 @@ int32_t psn_qmatvec_noalloc(psn_module *mod, psn_stream *s, int32_t qtype, int32
                             const psn_buf *x_f32, psn_buf *y_f32, int64_t N, int64_t K, int32_t batch);
 int64_t psn_noalloc_max_bytes(void);
 
-/* Launch geometry of one matvec.  With Q4_0 and Q8_0 weights, scheme Q8 and three to eight columns (three and four: rows of at most
- * 4096) psn_qmatvec(_multi) and psn_qmatvec_q8(_multi) run an int8-MFMA kernel that has no plan; the plan then names the
+/* Launch geometry of one matvec.  With Q4_0 and Q8_0 weights, scheme Q8 and three to eight columns (three and four: short rows, K < 4096
+ * or with Q8_0 K <= 4096) psn_qmatvec(_multi), psn_qmatvec_q8(_multi) and psn_qmatvec_noalloc run an int8-MFMA kernel that has no plan; the plan then names the
  * fastest of those that psn_qmatvec_planned can run.  psn_qmatvec_plan fills in the library's choice for a shape
  * (pure host arithmetic, usable without a device; x_is_f32 != 0 asks for the plan psn_qmatvec uses
  * when it quantizes fp32 activations inside the matvec launch); psn_qmatvec_planned runs with a

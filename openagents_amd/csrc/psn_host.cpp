@@ -1300,6 +1300,7 @@ extern "C" int32_t psn_qmatvec_noalloc(psn_module *mod, psn_stream *s, int32_t q
     /* the quantize launch overwrites every byte the matvec reads (qs, scales, sums of batch x K), so
      * nothing left behind by an earlier, larger call can be seen: no clearing is needed */
     if ((rc = quantize_into(mod, s, at, (const float *)x->p, scratch_ptr, K, batch))) return rc;
+    if (use_batch_kernel(qtype, sg.total, K, batch)) return run_batch(mod, s, qtype, sg, scratch_ptr, K, batch);
     return run_matvec(mod, s, qtype, scheme, sg, scratch_ptr, K, batch, &plan);
 }
 

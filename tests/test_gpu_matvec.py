@@ -959,7 +959,7 @@ def test_default_plans_over_seeded_random_shapes(hip, orc):
 @pytest.mark.parametrize("qname", ["Q4_0", "Q8_0"])
 def test_batch_kernel_at_tile_and_range_edges(hip, orc, qname):
     """The int8-MFMA kernel for three to eight columns: fewer rows than a tile, ragged last tiles, K ranges in which no, some and all of the
-    eight waves have a chunk, one and several; several ragged matrices in a launch; activations quantized by the call and before it.  The
+    eight waves have a chunk, one and several; several ragged matrices in a launch; activations quantized by the call (with and without the stream's workspace) and before it.  The
     integer dot products are exact, so only the order of at most 512 fp32 sums of three roundings each differs: far below PARITY_TOL."""
     t = getattr(orc, qname)
     name = f"psn_mvb_{qname.lower()}_q8"
@@ -973,7 +973,8 @@ def test_batch_kernel_at_tile_and_range_edges(hip, orc, qname):
             ref = orc.matvec(t, orc.ACT_Q8, W, x, n, k)
             xb, y = hip.upload(x), hip.alloc(b * n * 4)
             xq = hip.quantize_activations(xb, k, b, backend.act_type_for(t))
-            for call in (lambda: hip.quantized_matvec(w, xb, y, b, _ffi.ACT_Q8), lambda: hip.quantized_matvec_q8(w, xq, y, b)):
+            for call in (lambda: hip.quantized_matvec(w, xb, y, b, _ffi.ACT_Q8), lambda: hip.quantized_matvec_q8(w, xq, y, b),
+                         lambda: hip.quantized_matvec_noalloc(w, xb, y, b)):
                 y.fill_zero()
                 hip.lib.psn_launch_log_clear()
                 call()
