@@ -330,6 +330,13 @@ template <int N> PSN_DEV void tie(u32x4 (&v)[N]) { _Pragma("unroll") for (int i 
 PSN_DEV void tie1(u32 &v) { asm volatile("" : "+v"(v)); }
 /* workgroup barrier that waits for this wave's LDS traffic only, not for loads still in flight */
 PSN_DEV void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+/* what the lanes of one wave put into LDS for each other stays in order on both sides of this.  The hardware executes one wave's LDS
+ * operations in the order it was given, so it costs no instruction; the compiler may swap a load and a store that one lane cannot have
+ * in common unless a fence stands between them. */
+PSN_DEV void lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 /* ---- memory access the compiler sees (it places the waits), with the alignment a format guarantees ---- */
 template <typename T, int A> struct __attribute__((packed, aligned(A))) at_least { T v; };

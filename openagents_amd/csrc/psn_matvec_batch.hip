@@ -150,10 +150,12 @@ PSN_DEV void mv_batch(const psn_matvec_args &a) {
     if (wave < C) {
         load(wave);
         for (int c = wave; c < C; c += 8) {
+            lds_order();                                    /* the reads of the chunk before */
             UNROLL for (int i = 0; i < NI; ++i) store<16>(wl + wdst[i], w[i]);
             UNROLL for (int u = 0; u < 2; ++u) store<16>(xl + u * 4 * XCOL + xdst, x[u]);
             store<4>(dl + ddst, xd);
             if constexpr (F::SUMS) store<4>(dl + 256 + ddst, (u32)(-8 * (int)xs));
+            lds_order();
             __builtin_amdgcn_sched_barrier(0);
             load(c + 8);
             __builtin_amdgcn_sched_barrier(0);

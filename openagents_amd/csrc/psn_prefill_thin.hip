@@ -9,7 +9,7 @@
  *   - W and X are loaded with consecutive lanes on consecutive 16-byte words (asked for in the order the MFMA wants them,
  *     neighbouring lanes sit on different rows and a load takes 64 cycles instead of 16: X alone then cost 10 us per 16 rows of
  *     it at 14336 x 4096), W a whole chunk ahead, X one to four steps of 64 ahead, in registers;
- *   - put into LDS behind the wave's own earlier reads (LDS operations of one wave keep their order), read back as MFMA
+ *   - put into LDS behind the wave's own earlier reads (lds_order() keeps them there), read back as MFMA
  *     operands, W's raw bytes one tile ahead of their decode.
  * The loop has one body: past the last chunk every lane asks for the start of the buffer, which costs no traffic.
  *
@@ -137,6 +137,7 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
         }
     };
     auto put_w = [&]() {
+        lds_order();                                        /* the reads of the chunk before */
         UNROLL for (int t = 0; t < RT; ++t) {
             UNROLL for (int i = 0; i < NI; ++i) store<16>(wl + t * WTILE + wdst[i], w[t][i]);
             if constexpr (ODD) {
@@ -144,6 +145,7 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
                 store<4>(wl + t * WTILE + row * F::STRIDE + 212, dd[t]);
             }
         }
+        lds_order();
     };
 
     /* X: eight rows of 128 bytes per instruction */
@@ -166,7 +168,9 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
     u32x4 xf[2][2][TM];
     auto stage_x = [&](int c, int next, bool more, auto jc) {
         constexpr int J = decltype(jc)::value, SLOT = J % XD;
+        lds_order();                                        /* the reads of the step before */
         UNROLL for (int u = 0; u < 2 * TM; ++u) store<16>(xl + (u >> 1) * 2048 + (u & 1 ? xdst_odd : xdst), x[SLOT][u]);
+        lds_order();
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (J + XD < 4) load_x(c, true, pf_int<J + XD>(), pf_int<SLOT>());
         else load_x(next, more, pf_int<(J + XD) & 3>(), pf_int<SLOT>());
