@@ -303,7 +303,7 @@ int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32
  *       2048 so that its rows are whole 16-byte words): X and the raw GGUF bytes arrive in LDS rings by
  *       direct-to-LDS loads, every wave decodes its own MFMA operand, one barrier per 256 of K.  For M <= 64
  *       psn_qmatmul_prefill itself (no explicit shape) also has kernels for 16 to 64 rows of X and 16, 32 or 64 of W (every
- *       format and K), and takes whichever is estimated to be faster; the plan's ksplit is that of its choice;
+ *       format and K), and takes whichever is estimated to be faster; the plan names this one, with the cut of K that it needs;
  *  128  the dense family for large M (256x256 or 128x256 tiles, every format): one pass writes h(deq(W)) for the whole
  *       matrix as fp16 into the stream's workspace (ceil(N/256) * 256 * K * 2 bytes, see
  *       psn_prefill_reserve), in the order the multiply kernel's MFMA operands are read; that kernel has no

@@ -1434,6 +1434,12 @@ extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int
  * chunks leave no LDS for four tiles, from 17 on (14336 x 4096 M = 32: 23.4 against 26); it cuts K only while the weight rows
  * alone leave half of the compute units without a workgroup.  At rt = 4 a cut of K did not pay. */
 struct weight_stream_plan { int rt, ksplit; double us; };
+static bool may_cut_k(int64_t M, int64_t N, int64_t K, int sp) { return sp == 1 || ((M * N) % 4 == 0 && K / 256 >= 2 * sp); }
+static int stream64_ksplit(int64_t M, int64_t N, int64_t K, int32_t cus) {
+    int sp = 1;
+    while (sp < 8 && (N + 63) / 64 * sp * 2 <= cus && may_cut_k(M, N, K, sp * 2)) sp *= 2;
+    return sp;
+}
 static const double k_thin_row_us[5] = {0.719, 1.348, 0.878, 1.062, 1.695};       /* decode of 16 rows x 256: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
 static const double k_stream64_chunk_us[5] = {0.963, 1.196, 1.175, 1.242, 1.519}; /* 64 rows x 256 in the 64 x 64 kernel */
 static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus) {
@@ -1441,12 +1447,10 @@ static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N
     const int64_t C = K / 256;
     const double y_mb = (double)(M * N) * 4e-6;
     const auto cut_us = [&](int sp) { return sp > 1 ? 1.87 + 0.79 * y_mb * sp : 0.0; };   /* zero fill and atomic adds */
-    const auto may_cut = [&](int sp) { return sp == 1 || ((M * N) % 4 == 0 && C >= 2 * sp); };
     weight_stream_plan best = {-1, 1, 1e300};
     if (qtype != PSN_Q6_K || K % 2048 == 0) {
         const int64_t nt = (N + 63) / 64;
-        int sp = 1;
-        while (sp < 8 && nt * sp * 2 <= cus && may_cut(sp * 2)) sp *= 2;
+        const int sp = stream64_ksplit(M, N, K, cus);
         const double rounds = (double)((nt * sp + cus - 1) / cus);
         best = {0, sp, 0.97 * (3.8 + rounds * (double)((C + sp - 1) / sp) * k_stream64_chunk_us[f] + cut_us(sp) + 0.19 * y_mb)};
     }
@@ -1456,7 +1460,7 @@ static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N
         if (rt == 4 && (tm > (qtype == PSN_Q8_0 ? 1 : 3) || (tm == 1 && !big))) continue;
         const int per_cu = tm == 1 && (rt == 1 || (rt == 2 && !big)) ? 2 : 1;          /* up to 128 registers */
         for (int sp = 1; sp <= (rt == 4 ? 1 : 4); sp *= 2) {
-            if (!may_cut(sp)) continue;
+            if (!may_cut_k(M, N, K, sp)) continue;
             const int64_t wgs = (N + 16 * rt - 1) / (16 * rt) * sp, per = (C + sp - 1) / sp;
             const double rounds = (double)((wgs + cus * per_cu - 1) / (cus * per_cu)), shared = (double)((wgs + cus - 1) / cus);
             const double us = 0.9 + rounds * (1.22 + 0.316 * rt * (double)((per + 7) / 8)) +
@@ -1497,7 +1501,7 @@ static int32_t prefill_plan_any(int32_t qtype, int64_t M, int64_t N, int64_t K, 
     if (cus <= 0) cus = 256;
     if (M <= 64 && (qtype != PSN_Q6_K || K % 2048 == 0)) {
         *tile_m = *tile_n = *waves = 64;
-        *ksplit = plan_weight_stream(qtype, M, N, K, cus).ksplit;
+        *ksplit = stream64_ksplit(M, N, K, cus);
         return PSN_OK;
     }
     *waves = 4;

@@ -153,6 +153,20 @@ def test_prefill_plans_are_consistent_over_many_shapes(lib):
                         assert wv in (4, 64), tag
 
 
+def test_plans_for_at_most_64_rows_cut_k_for_the_kernel_they_name(lib):
+    """The plan for M <= 64 names the 64 x 64 kernel: its K split is the one that kernel needs, doubled only while the workgroups leave half
+    of the compute units idle, whatever psn_qmatmul_prefill runs there itself."""
+    for qt in (_ffi.Q4_0, _ffi.Q8_0, _ffi.Q4_K, _ffi.Q5_K, _ffi.Q6_K):
+        for n, k in ((1024, 4096), (4096, 4096), (4096, 14336), (14336, 4096), (1000, 2048), (17, 8192), (300, 2304)):
+            if qt == _ffi.Q6_K and k % 2048:
+                continue
+            for m in (1, 16, 33, 48, 64):
+                want = 1
+                while want < 8 and -(-n // 64) * want * 2 <= 256 and k // 256 >= 4 * want and (m * n) % 4 == 0:
+                    want *= 2
+                assert backend.prefill_plan(m, n, k, 256, qt) == (64, 64, want, 64), (qt, m, n, k)
+
+
 def test_null_handles_are_rejected_without_a_device(lib):
     assert lib.psn_stream_sync(None) == _ffi.E_INVALID_ARG
     assert lib.psn_buf_free(None) == _ffi.E_INVALID_ARG
