@@ -282,13 +282,13 @@ int32_t psn_selftest_arith(psn_module *mod, psn_stream *s, psn_buf *out);
 /* Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k]; X fp16 [M][K], Y fp32 [M][N], weight tiles are
  * dequantized to fp16 (h = round to nearest even) in LDS and fed to fp16 MFMA with fp32
  * accumulation.  qtype PSN_Q4_0 or PSN_Q8_0 (every kernel family below), PSN_Q4_K, PSN_Q5_K or PSN_Q6_K
- * (families 4, 64 and 128, and for Q4_K / Q5_K family 16 on the 128x256 tile; planned by psn_qmatmul_prefill_plan_for;
+ * (families 4, 8, 64 and 128, and for Q4_K / Q5_K family 16 on the 128x256 tile; planned by psn_qmatmul_prefill_plan_for;
  * their fp32 dequantization is restated operation by operation before the rounding to fp16).  Replaces the CUDA backend's quantized prefill
  * matmul op. */
 int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32_t layout, const psn_buf *W,
                             const psn_buf *X_f16, psn_buf *Y_f32, int64_t M, int64_t N, int64_t K);
-/* The launch shape the library picks for a prefill: the workgroup tile of Y (64x64, 64x128, 128x128,
- * 128x256, 256x128 or 256x256), into how many ranges K is cut (1, 2, 4 or 8; with more than one, Y is
+/* A launch shape for a prefill (psn_qmatmul_prefill_choice says which the library itself picks): the workgroup tile of Y (64x64,
+ * 64x128, 128x128, 128x256, 256x128 or 256x256; family 8: below), into how many ranges K is cut (1, 2, 4 or 8; with more than one, Y is
  * zeroed by a fill kernel and the partial sums are added atomically, so their order -- and the last bit
  * of a sum -- can vary between runs), and the kernel family:
  *    4  the kernels that decode in their loop, every wave staging and multiplying (any tile): eight waves (two to a SIMD,
@@ -301,9 +301,10 @@ int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32
  *       a wave decodes the operand of its own columns one K slice ahead, interleaved with its MFMAs;
  *   64  the weight-streaming kernel for M <= 64 (64x64 tiles; every format, Q6_K only when K is a multiple of
  *       2048 so that its rows are whole 16-byte words): X and the raw GGUF bytes arrive in LDS rings by
- *       direct-to-LDS loads, every wave decodes its own MFMA operand, one barrier per 256 of K.  For M <= 64
- *       psn_qmatmul_prefill itself (no explicit shape) also has kernels for 16 to 64 rows of X and 16, 32 or 64 of W (every
- *       format and K), and takes whichever is estimated to be faster; the plan names this one, with the cut of K that it needs;
+ *       direct-to-LDS loads, every wave decodes its own MFMA operand, one barrier per 256 of K;
+ *    8  the thin kernels for M <= 64 (every format and K): all of X, padded to 16, 32, 48 or 64 rows (tile_m >= M), by 16, 32 or
+ *       64 rows of W (tile_n; 64 only with tile_m <= 48, Q8_0 16, and not for 16 rows of Q4_0, Q4_K and Q5_K), eight waves with chunks of
+ *       K of their own and no barrier between them.  psn_qmatmul_prefill_plan and _plan_for never name them;
  *  128  the dense family for large M (256x256 or 128x256 tiles, every format): one pass writes h(deq(W)) for the whole
  *       matrix as fp16 into the stream's workspace (ceil(N/256) * 256 * K * 2 bytes, see
  *       psn_prefill_reserve), in the order the multiply kernel's MFMA operands are read; that kernel has no
@@ -311,13 +312,17 @@ int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32
  * Host arithmetic only ... */
 int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t *tile_m, int32_t *tile_n,
                                  int32_t *ksplit, int32_t *waves);
-/* The same for a given weight type: what psn_qmatmul_prefill runs when the dense family's workspace is
- * available (psn_qmatmul_prefill_plan answers for Q4_0 / Q8_0; the K-quants have families 4, 16 on the
- * 128x256 tile, 128, and 64 for M <= 64).  While a stream is capturing, or while a captured graph refers to its workspace,
+/* The same for a given weight type: for M > 64 what psn_qmatmul_prefill runs when the dense family's workspace is
+ * available (psn_qmatmul_prefill_plan answers for Q4_0; the planner uses families 4 and 128 there), for M <= 64 the best shape of family 64 (Q6_K with
+ * K not a multiple of 2048: of family 4), which every format can run.  While a stream is capturing, or while a captured graph refers to its workspace,
  * the workspace cannot grow: psn_qmatmul_prefill then takes the best plan without family 128 unless
  * psn_prefill_reserve (or an earlier dense call of that size) has sized it. */
 int32_t psn_qmatmul_prefill_plan_for(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t *tile_m,
                                      int32_t *tile_n, int32_t *ksplit, int32_t *waves);
+/* What psn_qmatmul_prefill runs, for any M: the plan above, or for M <= 64 a shape of family 8 where that is estimated to be faster.
+ * workspace == 0: what it runs where the dense family's workspace is missing and cannot be allocated. */
+int32_t psn_qmatmul_prefill_choice(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t workspace, int32_t *tile_m,
+                                   int32_t *tile_n, int32_t *ksplit, int32_t *waves);
 /* Sizes the stream's workspace for the dense family on an [N][K] matrix (and keeps whatever the decode
  * matvecs reserved: the workspace only grows).  Call before capturing a graph that should contain it. */
 int32_t psn_prefill_reserve(psn_stream *s, int64_t N, int64_t K);

@@ -92,6 +92,7 @@ SIGNATURES = {
     "psn_qmatmul_prefill": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _i64]),
     "psn_qmatmul_prefill_plan": (_i32, [_i64, _i64, _i64, _i32, C.POINTER(_i32), C.POINTER(_i32), C.POINTER(_i32), C.POINTER(_i32)]),
     "psn_qmatmul_prefill_plan_for": (_i32, [_i32, _i64, _i64, _i64, _i32, C.POINTER(_i32), C.POINTER(_i32), C.POINTER(_i32), C.POINTER(_i32)]),
+    "psn_qmatmul_prefill_choice": (_i32, [_i32, _i64, _i64, _i64, _i32, _i32, C.POINTER(_i32), C.POINTER(_i32), C.POINTER(_i32), C.POINTER(_i32)]),
     "psn_qmatmul_prefill_tiled": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _i32]),
     "psn_prefill_reserve": (_i32, [_vp, _i64, _i64]),
     "psn_prefill_packed_bytes": (_i64, [_i64, _i64]),

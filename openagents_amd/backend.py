@@ -54,12 +54,20 @@ def actq_layout(act_type: int, k: int, batch: int) -> _ffi.ActqInfo:
 
 
 def prefill_plan(m: int, n: int, k: int, compute_units: int = 256, qtype: int | None = None):
-    """(tile_m, tile_n, ksplit, waves) the library picks for a prefill shape (qtype None: the Q4_0 / Q8_0 plan)."""
+    """(tile_m, tile_n, ksplit, family) for a prefill shape (qtype None: Q4_0's plan): what the library picks for more than 64 rows, the best
+    shape of the 64 x 64 kernel for fewer."""
     tm, tn, sp, wv = C.c_int32(), C.c_int32(), C.c_int32(), C.c_int32()
     if qtype is None:
         _check(_ffi.load().psn_qmatmul_prefill_plan(m, n, k, compute_units, C.byref(tm), C.byref(tn), C.byref(sp), C.byref(wv)))
     else:
         _check(_ffi.load().psn_qmatmul_prefill_plan_for(qtype, m, n, k, compute_units, C.byref(tm), C.byref(tn), C.byref(sp), C.byref(wv)))
+    return int(tm.value), int(tn.value), int(sp.value), int(wv.value)
+
+
+def prefill_choice(m: int, n: int, k: int, qtype: int, compute_units: int = 256, workspace: bool = True):
+    """(tile_m, tile_n, ksplit, family) that quantized_matmul runs without an explicit tile; passing it as `tile` runs the same."""
+    tm, tn, sp, wv = C.c_int32(), C.c_int32(), C.c_int32(), C.c_int32()
+    _check(_ffi.load().psn_qmatmul_prefill_choice(qtype, m, n, k, compute_units, int(workspace), C.byref(tm), C.byref(tn), C.byref(sp), C.byref(wv)))
     return int(tm.value), int(tn.value), int(sp.value), int(wv.value)
 
 

@@ -1442,6 +1442,12 @@ static int stream64_ksplit(int64_t M, int64_t N, int64_t K, int32_t cus) {
 }
 static const double k_thin_row_us[5] = {0.719, 1.348, 0.878, 1.062, 1.695};       /* decode of 16 rows x 256: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
 static const double k_stream64_chunk_us[5] = {0.963, 1.196, 1.175, 1.242, 1.519}; /* 64 rows x 256 in the 64 x 64 kernel */
+static bool big_chunk(int32_t qtype) { return qtype == PSN_Q8_0 || qtype == PSN_Q6_K; }    /* raw chunks of five or six registers a lane instead of three */
+/* rt = 4: LDS and registers end at 48 rows of X (Q8_0: 16); at 16 rows the others' rt = 2 shares compute units */
+static bool thin_exists(int32_t qtype, int tm, int rt) {
+    if (tm < 1 || tm > 4) return false;
+    return rt == 1 || rt == 2 || (rt == 4 && tm <= (qtype == PSN_Q8_0 ? 1 : 3) && (tm > 1 || big_chunk(qtype)));
+}
 static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus) {
     const int f = format_index(qtype), tm = (int)((M + 15) / 16);
     const int64_t C = K / 256;
@@ -1455,10 +1461,8 @@ static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N
         best = {0, sp, 0.97 * (3.8 + rounds * (double)((C + sp - 1) / sp) * k_stream64_chunk_us[f] + cut_us(sp) + 0.19 * y_mb)};
     }
     for (int rt = 1; rt <= 4; rt *= 2) {
-        const bool big = qtype == PSN_Q8_0 || qtype == PSN_Q6_K;     /* raw chunks of five or six registers a lane instead of three */
-        /* kernels that exist: LDS and registers end at 48 rows of X (Q8_0: 16); at 16 the others' rt = 2 shares compute units */
-        if (rt == 4 && (tm > (qtype == PSN_Q8_0 ? 1 : 3) || (tm == 1 && !big))) continue;
-        const int per_cu = tm == 1 && (rt == 1 || (rt == 2 && !big)) ? 2 : 1;          /* up to 128 registers */
+        if (!thin_exists(qtype, tm, rt)) continue;
+        const int per_cu = tm == 1 && (rt == 1 || (rt == 2 && !big_chunk(qtype))) ? 2 : 1;          /* up to 128 registers */
         for (int sp = 1; sp <= (rt == 4 ? 1 : 4); sp *= 2) {
             if (!may_cut_k(M, N, K, sp)) continue;
             const int64_t wgs = (N + 16 * rt - 1) / (16 * rt) * sp, per = (C + sp - 1) / sp;
@@ -1524,6 +1528,27 @@ extern "C" int32_t psn_qmatmul_prefill_plan_for(int32_t qtype, int64_t M, int64_
     return prefill_plan_any(qtype, M, N, K, cus, true, tile_m, tile_n, ksplit, waves);
 }
 
+/* what psn_qmatmul_prefill launches, in psn_qmatmul_prefill_tiled's terms */
+static int32_t prefill_choice(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, bool workspace, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit,
+                              int32_t *waves) {
+    const int32_t rc = prefill_plan_any(qtype, M, N, K, cus, workspace, tile_m, tile_n, ksplit, waves);
+    if (rc || M > 64) return rc;
+    if (cus <= 0) cus = 256;
+    const weight_stream_plan p = plan_weight_stream(qtype, M, N, K, cus);
+    int32_t bm, bn, sp;
+    /* (Q6_K rows that are not whole 16-byte words: the kernels that decode in their loop are what it competes with) */
+    if (p.rt == 0 || (*waves == 4 && p.us >= plan_in_loop(qtype, M, N, K, cus, &bm, &bn, &sp))) return PSN_OK;
+    *tile_m = 16 * (int32_t)((M + 15) / 16);
+    *tile_n = 16 * p.rt;
+    *ksplit = p.ksplit;
+    *waves = 8;
+    return PSN_OK;
+}
+extern "C" int32_t psn_qmatmul_prefill_choice(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t workspace, int32_t *tile_m, int32_t *tile_n,
+                                              int32_t *ksplit, int32_t *waves) {
+    return prefill_choice(qtype, M, N, K, cus, workspace != 0, tile_m, tile_n, ksplit, waves);
+}
+
 static int32_t need(const psn_buf *b, int64_t bytes, const char *what, const char *name);
 /* the dense family's two steps: GGUF blocks -> fp16 MFMA fragments ([ceil(N/32)][K/16][64 lanes][8 halves], rows
  * padded to whole 256-row panels), and the fp16 multiply on 256 x 256 tiles over such a buffer */
@@ -1559,9 +1584,9 @@ static void prefill_args(psn_prefill_args *a, const void *W, const psn_buf *X, p
     a->row_bytes = row_bytes;
 }
 static int32_t launch_thin(psn_module *mod, psn_stream *s, int32_t qtype, const psn_buf *W, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N,
-                           int64_t K, int rt, int32_t ksplit) {
+                           int64_t K, int tm, int rt, int32_t ksplit) {
     static const int lds_row[5] = {144, 272, 144, 176, 224};    /* a row's chunk in LDS */
-    const int tm = (int)((M + 15) / 16), rings = 8 * (16 * rt * lds_row[format_index(qtype)] + tm * 2048), sums = 8 * 1024 * rt * tm;
+    const int rings = 8 * (16 * rt * lds_row[format_index(qtype)] + tm * 2048), sums = 8 * 1024 * rt * tm;
     const int lds = rings > sums ? rings : sums;
     if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: %d x %d rows need %d bytes of LDS, device offers %d", 16 * tm, 16 * rt, lds, mod->ctx->max_lds);
     int32_t rc = bind(mod->ctx);
@@ -1642,9 +1667,17 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
         if ((rc = launch_unpack(mod, s, qtype, W->p, s->ws->p, N, K))) return rc;
         return launch_dense(mod, s, s->ws->p, X, Y, M, N, K, bm, ksplit);
     }
+    /* waves == 8 selects the thin kernels: tile_m (16 .. 64) rows of X, all of them, and tile_n (16, 32, 64) rows of W */
+    if (waves == 8) {
+        if (bm % 16 || bn % 16 || M > bm || !thin_exists(qtype, bm / 16, bn / 16))
+            return fail(PSN_E_UNSUPPORTED, "prefill: no thin kernel of %s with a %dx%d tile for M=%lld", fmt_name(qtype), bm, bn, (long long)M);
+        if (ksplit < 1 || ksplit > 64) return fail(PSN_E_UNSUPPORTED, "prefill: ksplit=%d outside 1..64", ksplit);
+        if (ksplit > 1 && (M * N) % 4 != 0) return fail(PSN_E_UNSUPPORTED, "prefill: splitting K needs M*N to be a multiple of 4");
+        return launch_thin(mod, s, qtype, W, X, Y, M, N, K, bm / 16, bn / 16, ksplit);
+    }
     if (qtype != PSN_Q4_0 && qtype != PSN_Q8_0 && waves != 4 && waves != 64 && !(waves == 16 && bm == 128 && bn == 256 && qtype != PSN_Q6_K))
-        return fail(PSN_E_UNSUPPORTED, "prefill: %s has the four-wave kernel family, the weight-streaming kernel for M <= 64 (waves = 64)%s", fmt_name(qtype),
-                    qtype == PSN_Q6_K ? "" : " and the 128x256 producer / consumer kernel (waves = 16)");
+        return fail(PSN_E_UNSUPPORTED, "prefill: %s has families 4, 8 and 64 (M <= 64), 128%s", fmt_name(qtype),
+                    qtype == PSN_Q6_K ? "" : " and 16 on the 128x256 tile");
     /* waves == 64 selects the skinny kernel (M <= 64, 64 x 64 tiles, deep LDS rings) */
     const bool skinny = waves == 64;
     if (skinny && (bm != 64 || bn != 64 || M > 64)) return fail(PSN_E_UNSUPPORTED, "prefill: the skinny kernel serves M <= 64 with a 64x64 tile");
@@ -1696,24 +1729,17 @@ extern "C" int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t q
     int32_t rc = check_prefill("psn_qmatmul_prefill", mod, s, qtype, W, X, Y, M, N, K);
     if (rc) return rc;
     int32_t bm = 0, bn = 0, sp = 1, wv = 4;
-    if (M <= 64) {
-        const weight_stream_plan p = plan_weight_stream(qtype, M, N, K, mod->ctx->compute_units);
-        /* (Q6_K rows that are not whole 16-byte words: the kernels that decode in their loop are what it competes with) */
-        const bool thin = p.rt > 0 && ((qtype != PSN_Q6_K || K % 2048 == 0) || p.us < plan_in_loop(qtype, M, N, K, mod->ctx->compute_units, &bm, &bn, &sp));
-        if (thin) return launch_thin(mod, s, qtype, W, X, Y, M, N, K, p.rt, p.ksplit);
-    }
-    /* the dense family needs nt * 256 * K fp16 values of workspace on this stream: it competes when that is
-     * there already or may still be allocated (not while capturing, not once a graph holds the workspace) */
-    bool cap = false;
-    if ((rc = is_capturing(s, &cap))) return rc;
-    const int64_t dense_ws = packed_bytes(N, K);
-    bool ws_pinned;
-    {
+    /* the dense family (never for 64 rows and fewer) needs nt * 256 * K fp16 values of workspace on this stream: it competes when
+     * that is there already or may still be allocated (not while capturing, not once a graph holds the workspace) */
+    bool dense_ok = false;
+    if (M > 64) {
+        bool cap = false;
+        if ((rc = is_capturing(s, &cap))) return rc;
         std::lock_guard<std::mutex> lk(g_cap_mu);
-        ws_pinned = s->ws->graph_refs > 0 || s->ws->capture_refs > 0;
+        const bool ws_pinned = s->ws->graph_refs > 0 || s->ws->capture_refs > 0;
+        dense_ok = s->ws->bytes >= (size_t)packed_bytes(N, K) || (!cap && !ws_pinned);
     }
-    const bool dense_ok = s->ws->bytes >= (size_t)dense_ws || (!cap && !ws_pinned);
-    if ((rc = prefill_plan_any(qtype, M, N, K, mod->ctx->compute_units, dense_ok, &bm, &bn, &sp, &wv))) return rc;
+    if ((rc = prefill_choice(qtype, M, N, K, mod->ctx->compute_units, dense_ok, &bm, &bn, &sp, &wv))) return rc;
     return psn_qmatmul_prefill_tiled(mod, s, qtype, W, X, Y, M, N, K, bm, bn, sp, wv);
 }
 

@@ -30,11 +30,13 @@ import numpy as np
 
 from . import quantize
 from ._ffi import Q4_0, Q4_K, Q5_K, Q6_K, Q8_0
-from .backend import HipBackend, PsnError, prefill_plan, row_bytes
+from .backend import HipBackend, PsnError, prefill_choice, row_bytes
+from .records import launched_kernels
 
-# (tile_m, tile_n, ksplit, family): the explicit plans --compare-plans tries (family 4 = four waves, 16 = producer / consumer,
-# 32 = wide, 64 = weight-streaming for M <= 64, 128 = dense)
-EXPLICIT_PLANS = [(64, 64, 1, 64), (64, 64, 2, 64), (64, 64, 4, 64), (64, 64, 8, 64),
+# (tile_m, tile_n, ksplit, family): the explicit plans --compare-plans tries (family 4 = decoding in the loop, 8 = thin for M <= 64,
+# 16 = producer / consumer, 32 = wide, 64 = weight-streaming for M <= 64, 128 = dense)
+EXPLICIT_PLANS = [*((16 * tm, 16 * rt, sp, 8) for tm in (1, 2, 3, 4) for rt in (1, 2, 4) for sp in (1, 2, 4)),
+                  (64, 64, 1, 64), (64, 64, 2, 64), (64, 64, 4, 64), (64, 64, 8, 64),
                   (64, 64, 2, 4), (64, 64, 4, 4), (64, 64, 8, 4), (64, 128, 2, 4), (64, 128, 4, 4), (64, 128, 8, 4), (256, 128, 2, 4), (256, 128, 4, 4), (256, 128, 8, 4),
                   (128, 128, 1, 4), (256, 128, 1, 4), (256, 256, 1, 4), (256, 256, 2, 4), (256, 256, 4, 4),
                   (128, 128, 1, 16), (128, 128, 2, 16), (128, 128, 4, 16), (128, 128, 8, 16),
@@ -143,7 +145,8 @@ def main(argv=None):
                 tflops, gbs = flops / us / 1e6, nbytes / us / 1e3
                 bound = "mfma" if flops / nbytes >= MFMA_PEAK_TFLOPS * 1e3 / HBM_PEAK_GBS else "hbm"
                 frac = tflops / MFMA_PEAK_TFLOPS if bound == "mfma" else gbs / HBM_PEAK_GBS
-                tm, tn, sp, wv = prefill_plan(m, n, k, be.compute_units, qt)
+                sp = prefill_choice(m, n, k, qt, be.compute_units)[2]
+                kernel = launched_kernels(be, lambda: be.quantized_matmul(ws[0], x, y, m))
                 sustained = {}
                 if args.sample_clock > 0:
                     with ClockSampler() as cs:
@@ -165,7 +168,7 @@ def main(argv=None):
                         sustained["frac_of_mfma_rate_at_that_clock"] = round(flops / sus_us / 1e6 / (MFMA_PEAK_TFLOPS * mhz / MFMA_PEAK_CLOCK_MHZ), 4)
                 print(json.dumps({"op": "quantized prefill matmul", "format": fname, "M": m, "N": n, "K": k, "us": round(us, 1),
                                   "TFLOPs": round(tflops, 1), "GBps": round(gbs, 1), "bound": bound, "frac_of_roofline": round(frac, 4),
-                                  "kernel": {64: f"psn_prefill_{fname}_skinny", 32: f"psn_prefill_{fname}_wide", 128: f"psn_prefill_{fname}_unpack + psn_prefill_dense_f16" + ("_m128" if tm == 128 else "")}.get(wv, f"psn_prefill_{fname}_m{tm}_n{tn}" + {4: "", 16: "_ws"}.get(wv, "")),
+                                  "kernel": kernel,
                                   "ksplit": sp, "iters": args.iters, **sustained, **compared}), flush=True)
             for w in ws:
                 w.buf.free()

@@ -38,7 +38,7 @@ import numpy as np
 
 from . import _ffi, quantize
 from ._ffi import ACT_Q8, Q4_0, Q4_K, Q6_K, Q8_0
-from .backend import HipBackend, act_type_for, prefill_plan, row_bytes
+from .backend import HipBackend, act_type_for, prefill_choice, row_bytes
 
 HBM_PEAK_GBS = 8000.0
 MFMA_F16_PEAK_TFLOPS = 2500.0
@@ -250,7 +250,7 @@ def config4(be: HipBackend, samples: int = 7, seed: int = 41, weights=None, ms=(
                 x = be.upload(x_host)
                 y = be.alloc(m * n * 4)
                 kname = launched_kernels(be, lambda: be.quantized_matmul(ws[0], x, y, m))
-                sp = prefill_plan(m, n, k, be.compute_units, qtype)[2]
+                sp = prefill_choice(m, n, k, qtype, be.compute_units)[2]
                 be.begin_capture()
                 for w in ws:
                     be.quantized_matmul(w, x, y, m)

@@ -413,22 +413,48 @@ def test_in_loop_kernels_at_tile_and_range_edges(hip, orc, qname):
 
 @pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
 def test_thin_kernels_at_tile_and_range_edges(hip, orc, qname):
-    """The kernels for at most 64 rows of X that the library picks by itself (16 to 64 rows of X, 16 to 64 of W): X at either
-    end of its sixteens, fewer weight rows than a tile, ragged last tiles, K ranges in which no, some and all of the eight
-    waves have a chunk, one and several, with and without a cut of K -- every kernel of the format (the launch log tells).  fp16 products
-    are exact in fp32, so only the order of at most 4096 sums differs from the oracle: PARITY_TOL is far above 2^-24 sqrt(4096)."""
+    """Family 8 (16 to 64 rows of X, 16 to 64 of W), every kernel of the format by name: X at either end of its sixteens and below, fewer weight
+    rows than a tile, ragged last tiles, K ranges in which no, some and all of the eight waves have a chunk, one and several, with and without
+    a cut of K (one that leaves ranges empty, too).  fp16 products are exact in fp32, so only the order of at most 4096 sums differs from the
+    oracle: PARITY_TOL is far above 2^-24 sqrt(4096)."""
     t = getattr(orc, qname)
-    ran = set()
-    for n, k, ms in ((5, 256, (1, 17, 33, 49)), (17, 768, (16, 32, 48, 64)), (300, 2304, (1, 31, 40, 64)), (516, 4096, (15, 33, 63)),
-                     (4104, 1280, (1, 17, 33, 49)), (4109, 512, (16, 32, 48, 64)), (8209, 256, (1, 17, 33)), (8209, 1024, (16, 18, 33))):
+    kernels = [(tm, rt) for tm in (1, 2, 3, 4) for rt in (1, 2, 4) if rt < 4 or tm in {"Q8_0": (1,), "Q6_K": (1, 2, 3)}.get(qname, (2, 3))]
+    for n, k in ((5, 256), (17, 768), (300, 2304), (132, 4096)):
         W = weights(orc, qname, 890, n, k)
+        X = G.seeded_acts(891, 64, k).astype(np.float16)
+        ref = orc.prefill(t, W, X, n, k)
+        for tm, rt in kernels:
+            for m in sorted({1, 16 * tm - 15, 16 * tm - 4, 16 * tm}):
+                for ksplit in (1, 2, 5) if (m * n) % 4 == 0 else (1,):
+                    say(f"thin {qname} {tm} {rt} m={m} n={n} k={k} ksplit={ksplit}")
+                    hip.lib.psn_launch_log_clear()
+                    y = hip.matmul_host(t, W, X[:m], n, k, (16 * tm, 16 * rt, ksplit, 8))
+                    assert f"psn_prefill_{qname[0].lower() + qname[1:]}_thin_{tm}_{rt}" in hip.lib.psn_launch_log().decode().split(";")
+                    err = G.max_rel_err(y, ref[:m])
+                    assert np.all(np.isfinite(y)) and err < PARITY_TOL, (tm, rt, ksplit, m, n, k, err)
+    for tile in {(16 * tm, 16 * rt) for tm in (1, 2, 3, 4) for rt in (1, 2, 4)} - {(16 * tm, 16 * rt) for tm, rt in kernels} | {(0, 16), (80, 16), (24, 16), (16, 128), (-16, 16)}:
+        with pytest.raises(backend.PsnError) as e:
+            hip.matmul_host(t, W, X[:1], n, k, tile + (1, 8))
+        assert e.value.name == "PSN_E_UNSUPPORTED"
+    for tile, m in (((16, 16, 1, 8), 17), ((64, 32, 0, 8), 64), ((64, 32, 65, 8), 64)):                     # more rows than the tile, cuts outside 1..64
+        with pytest.raises(backend.PsnError) as e:
+            hip.matmul_host(t, W, X[:m], n, k, tile)
+        assert e.value.name == "PSN_E_UNSUPPORTED"
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
+def test_the_choice_is_what_runs(hip, orc, qname):
+    """psn_qmatmul_prefill_choice names the launch of psn_qmatmul_prefill: the same kernels with and without it as an explicit tile."""
+    t = getattr(orc, qname)
+    for n, k, ms in ((300, 2304, (1, 17, 33, 49, 64, 65)), (4104, 1280, (1, 33, 64)), (8209, 1024, (16, 18, 48)), (2048, 2048, (64, 200, 2048))):
+        w = hip.upload_weight(t, weights(orc, qname, 895, n, k), n, k)
         for m in ms:
-            say(f"thin {qname} m={m} n={n} k={k}")
-            X = G.seeded_acts(891 + m, m, k).astype(np.float16)
-            hip.lib.psn_launch_log_clear()
-            y = hip.matmul_host(t, W, X, n, k)
-            ran |= {name for name in hip.lib.psn_launch_log().decode().split(";") if "_thin_" in name}
-            err = G.max_rel_err(y, orc.prefill(t, W, X, n, k))
-            assert np.all(np.isfinite(y)) and err < PARITY_TOL, (m, n, k, err)
-    tall = {"Q8_0": (1,), "Q6_K": (1, 2, 3)}.get(qname, (2, 3))
-    assert ran == {f"psn_prefill_{qname[0].lower() + qname[1:]}_thin_{tm}_{rt}" for rt in (1, 2, 4) for tm in (tall if rt == 4 else (1, 2, 3, 4))}
+            x, y = hip.upload(G.seeded_acts(896, m, k).astype(np.float16)), hip.alloc(m * n * 4)
+            say(f"choice {qname} m={m} n={n} k={k}")
+            ran = []
+            for tile in (None, backend.prefill_choice(m, n, k, t, hip.compute_units)):
+                hip.lib.psn_launch_log_clear()
+                hip.quantized_matmul(w, x, y, m, tile)
+                ran.append(hip.lib.psn_launch_log().decode())
+            hip.sync()
+            assert ran[0] == ran[1], (m, n, k, ran, tile)

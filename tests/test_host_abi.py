@@ -167,6 +167,28 @@ def test_plans_for_at_most_64_rows_cut_k_for_the_kernel_they_name(lib):
                 assert backend.prefill_plan(m, n, k, 256, qt) == (64, 64, want, 64), (qt, m, n, k)
 
 
+def test_prefill_choice_is_the_plan_or_a_thin_kernel(lib):
+    """Host arithmetic: for more than 64 rows the choice is the plan; for fewer it is that or a thin kernel that exists, tall enough for X, with
+    a K split that leaves two whole chunks per range; without a workspace it is never the dense family."""
+    thin = 0
+    for qt in (_ffi.Q4_0, _ffi.Q8_0, _ffi.Q4_K, _ffi.Q5_K, _ffi.Q6_K):
+        for k in (256, 768, 2048, 4096, 11008, 14336):
+            for n in (1, 17, 1000, 1024, 4096, 14336):
+                for m in (1, 16, 17, 33, 64, 65, 512, 4096):
+                    tm, tn, sp, wv = c = backend.prefill_choice(m, n, k, qt)
+                    if wv == 8:
+                        thin += 1
+                        assert m <= tm <= 64 and tm - m < 16 and tn in (16, 32, 64), (qt, m, n, k, c)
+                        assert tn < 64 or tm in {_ffi.Q8_0: (16,), _ffi.Q6_K: (16, 32, 48)}.get(qt, (32, 48)), (qt, m, n, k, c)
+                        assert sp == 1 or ((m * n) % 4 == 0 and k // 256 >= 2 * sp), (qt, m, n, k, c)
+                    else:
+                        assert c == backend.prefill_plan(m, n, k, 256, qt), (qt, m, n, k, c)
+                    assert backend.prefill_choice(m, n, k, qt, workspace=False)[3] != 128
+    assert thin
+    assert lib.psn_qmatmul_prefill_choice(_ffi.Q4_0, 1, 1, 100, 256, 1, *[C.byref(C.c_int32()) for _ in range(4)]) == _ffi.E_SHAPE
+    assert lib.psn_qmatmul_prefill_choice(_ffi.Q4_0, 1, 1, 256, 256, 1, None, None, None, None) == _ffi.E_INVALID_ARG
+
+
 def test_null_handles_are_rejected_without_a_device(lib):
     assert lib.psn_stream_sync(None) == _ffi.E_INVALID_ARG
     assert lib.psn_buf_free(None) == _ffi.E_INVALID_ARG
