@@ -1370,55 +1370,62 @@ static int32_t check_prefill(const char *what, psn_module *mod, psn_stream *s, i
     return PSN_OK;
 }
 
-/* Family 4 (psn_prefill_pp.hip), measured on MI355X over five formats, eleven matrices and M = 65 .. 4096 (2145 launches; the
- * estimate is off by 6-11 % rms, and the plan it picks is within 1 % of the best of the family on average):
- * base + rounds of workgroups x (K steps + prologue) x step cost of the format, workgroups that share a compute unit slowing
- * each other down by `shared` each, the store of Y, and with K cut the zero fill and the atomic adds. */
+/* Cost models of family 4 (psn_prefill_pp.hip) and of the dense family, fitted to launches timed on MI355X: five formats, 22 matrices (1000 x 2560 ..
+ * 28672 x 8192), M = 65 .. 4096, 22848 launches of family 4 and 9296 of the dense one.  Weight lies on plans near the fastest, whose estimates are
+ * off by 3-6 % rms; what they pick is 0.35 % off the fastest plan of any family on average over 1555 shapes and more than 10 % off in 3.
+ *
+ * Both families deal N tiles to the eight XCDs in turn and give an XCD all M tiles and K ranges of its own, so that the XCDs with one N tile
+ * more set the rounds of workgroups: 5120 columns are 20 tiles of 256, three for four of the XCDs, whose 36 workgroups at M = 3072 take
+ * two rounds on 32 compute units (Q4_K: dense 689 us; 256 x 128 tiles, five for each XCD, 467).  A round in which nearly every compute unit multiplies runs at
+ * a lower clock than an emptier one (8192 x 8192 M = 2048, two full rounds: 1.2 x the step cost of half-filled ones). */
+static int format_index(int32_t t) { return t == PSN_Q4_0 ? 0 : t == PSN_Q8_0 ? 1 : t == PSN_Q4_K ? 2 : t == PSN_Q5_K ? 3 : 4; }
+struct prefill_rounds {
+    int64_t per_xcd;        /* workgroups of an XCD with the most N tiles */
+    double share;           /* workgroups of all XCDs over eight times that */
+    int xcd_cus;
+    prefill_rounds(int64_t mt, int64_t nt, int sp, int32_t cus) : per_xcd((nt + 7) / 8 * mt * sp), share((double)nt / (double)((nt + 7) / 8 * 8)), xcd_cus(cus < 8 ? 1 : cus / 8) {}
+    double busy(double clock, int64_t wgs) const {                 /* the clock's part of a round of wgs workgroups per XCD */
+        const double filled = (wgs < xcd_cus ? (double)wgs / xcd_cus : 1.0) * share, u = (filled - 0.7) / 0.2;
+        return 1.0 + clock * (u < 0.0 ? 0.0 : u > 1.0 ? 1.0 : u);
+    }
+};
+/* plans that cut K come out too low where all ranges of an element add at the same moment (Q8_0 4096 x 4096 M = 128 in four: 26.9 us, 20.2 by the
+ * rest of the model) */
+static double cut_bias(double per_doubling, int sp) { return 1.0 + per_doubling * (sp >= 8 ? 3 : sp >= 4 ? 2 : sp >= 2 ? 1 : 0); }
+
+/* Family 4: base + rounds x (K steps + prologue) x step cost, workgroups that share a compute unit slowing each other down by `shared` each, the
+ * store of Y, and with K cut the zero fill and the atomic adds.  per_cu: workgroups a compute unit holds by LDS and registers, per_cu_q6_K of Q6_K's
+ * kernel. */
 struct prefill_cost {
-    int tile, per_cu;                 /* index into k_prefill_tiles, workgroups a compute unit holds */
-    double base_us, shared, y_us_per_mb, add_us_per_mb, split_us, prologue_steps;
+    int tile, per_cu, per_cu_q6_K;    /* index into k_prefill_tiles */
+    double base_us, shared, y_us_per_mb, add_us_per_mb[2], split_us, prologue_steps, clock;   /* adds: K in two, in four and more */
     double step_us[5];                /* per 64 of K: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
 };
 static const prefill_cost k_prefill_cost[] = {
-    {0, 3, 3.1, 0.76, 0.24, 0.35, 2.8, 1.1, {0.295, 0.386, 0.303, 0.318, 0.396}},
-    {1, 2, 2.8, 1.02, 0.42, 0.60, 2.2, 0.8, {0.428, 0.575, 0.470, 0.513, 0.560}},
-    {2, 1, 2.3, 0.00, 0.52, 0.63, 3.1, 0.0, {0.521, 0.679, 0.556, 0.595, 0.638}},
-    {4, 1, 1.6, 0.00, 0.43, 0.66, 3.1, 1.8, {0.753, 0.903, 0.794, 0.829, 0.862}},
+    {0, 3, 2, 3.66, 0.690, 0.257, {0.439, 0.439}, 2.23, 0.20, 0.025, {0.296, 0.396, 0.304, 0.327, 0.387}},
+    {1, 1, 1, 3.15, 0.000, 0.139, {0.645, 0.645}, 1.12, 2.44, 0.053, {0.418, 0.597, 0.470, 0.505, 0.577}},
+    {2, 1, 1, 3.45, 0.000, 0.222, {0.613, 0.613}, 1.21, 2.55, 0.193, {0.503, 0.659, 0.557, 0.555, 0.631}},
+    {4, 1, 1, 3.25, 0.000, 0.263, {0.547, 0.727}, 2.55, 0.60, 0.269, {0.743, 0.862, 0.794, 0.788, 0.818}},
 };
-static int format_index(int32_t t) { return t == PSN_Q4_0 ? 0 : t == PSN_Q8_0 ? 1 : t == PSN_Q4_K ? 2 : t == PSN_Q5_K ? 3 : 4; }
-
-/* zero fill of Y and the atomic adds of `sp` partial sums per element, plus a launch: with few ranges the adds overlap
- * the multiply well enough to count at the fill's 3 TB/s; from `slow_from` ranges on (eight; four for the kernels
- * whose four waves hold a whole 256 x 256 tile) they run at the measured 1.6 TB/s */
-static double ksplit_overhead_us(int64_t M, int64_t N, int sp, int slow_from = 8) {
-    const double bytes = (double)(M * N) * 4.0;
-    return (sp >= slow_from ? bytes * (1.0 / 3.0e6 + sp / 1.6e6) : bytes * (1.0 + sp) / 3.0e6) + 4.0;
-}
-/* The dense family's estimate: one pass that rewrites the matrix as fp16 (0.45 us per million weights + a
- * launch, measured; none when the caller holds packed weights) and the multiply on 256 x 256 or 128 x 256 tiles,
- * round by round of workgroups. */
-static const double k_dense_step_us[2][3] = {{1.85, 1.5, 1.4}, {0.96, 0.78, 0.72}};   /* {256, 128 rows} x {full round, 60-80 % filled, emptier} */
-static double dense_estimate(int64_t M, int64_t N, int64_t K, int32_t cus, bool with_unpack, int *bm_out, int *ksplit_out) {
-    const int64_t nt = (N + 255) / 256;
-    const double unpack = with_unpack ? 4.0 + (double)N * (double)K * 0.45e-6 : 0.0;
+/* The dense family: one pass that rewrites the matrix as fp16 (none when the caller holds packed weights) and the multiply on 256 x 256 or
+ * 128 x 256 tiles. */
+static const struct { int bm; double base_us, step_us, clock, add_us_per_mb; } k_dense_cost[] = {{256, 4.50, 1.358, 0.236, 0.612}, {128, 4.16, 0.697, 0.288, 0.382}};
+static const double k_unpack_us[5] = {0.427, 0.591, 0.469, 0.399, 0.519};      /* per million weights, from the fit */
+static double dense_estimate(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, bool with_unpack, int *bm_out, int *ksplit_out) {
+    const double y_mb = (double)(M * N) * 4e-6;
     double best = 1e300;
-    for (int v = 0; v < 2; ++v) {
-        const int bm = v ? 128 : 256;
-        const int64_t mt = (M + bm - 1) / bm;
+    for (const auto &c : k_dense_cost) {
         for (int sp = 1; sp <= 4; sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 4 * sp)) continue;
-            const int64_t wgs = mt * nt * sp, full = wgs / cus, rest = wgs % cus;
-            const double steps = (double)(K / 64) / sp;
-            /* a round that fills the chip runs at a lower clock than a partly filled one */
-            const double fill = (double)rest / cus;
-            double t = unpack + (double)full * steps * k_dense_step_us[v][0] +
-                       (rest ? steps * k_dense_step_us[v][fill >= 0.8 ? 0 : fill >= 0.6 ? 1 : 2] : 0.0) + 5.0;
-            /* four contributors per element of a 128-row tile all finish together: their adds cost more than two do */
-            if (sp > 1) t += (v && sp == 4) ? (double)(M * N) * 4.0 * (1.0 / 3.0e6 + 4.0 / 2.0e6) + 4.0 : ksplit_overhead_us(M, N, sp, v ? 8 : 4);
-            if (t < best) { best = t; *bm_out = bm; *ksplit_out = sp; }
+            const prefill_rounds r((M + c.bm - 1) / c.bm, (N + 255) / 256, sp, cus);
+            const int64_t full = r.per_xcd / r.xcd_cus, rest = r.per_xcd % r.xcd_cus;
+            double t = c.base_us + (double)((K / 256 + sp - 1) / sp * 4) * c.step_us * ((double)full * r.busy(c.clock, r.xcd_cus) + (rest ? r.busy(c.clock, rest) : 0.0)) + 0.164 * y_mb;
+            if (sp > 1) t += (c.bm == 128 ? 2.20 : 0.0) + c.add_us_per_mb * y_mb * sp;
+            t *= cut_bias(0.070, sp);
+            if (t < best) { best = t; *bm_out = c.bm; *ksplit_out = sp; }
         }
     }
-    return best;
+    return best + (with_unpack ? 4.46 + (double)N * (double)K * 1e-6 * k_unpack_us[format_index(qtype)] : 0.0);
 }
 
 extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit,
@@ -1481,15 +1488,17 @@ static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32
     double best = 1e300;
     for (const prefill_cost &c : k_prefill_cost) {
         const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
-        const int64_t mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn, slots = (int64_t)cus * c.per_cu;
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
-            const double one = ((double)(K / 64) / sp + c.prologue_steps) * c.step_us[f];
-            const auto round_us = [&](int64_t wgs) { return wgs ? one * (1.0 + c.shared * (double)((wgs + cus - 1) / cus - 1)) : 0.0; };
-            const int64_t wgs = mt * nt * sp;
-            double t = c.base_us + (double)(wgs / slots) * round_us(slots) + round_us(wgs % slots) + c.y_us_per_mb * y_mb;
-            if (sp > 1) t += c.split_us + c.add_us_per_mb * y_mb * sp;
-            if (t > 100.0) t += 0.4 * (t - 100.0);          /* the device lowers its clock under sustained matrix work */
+            const prefill_rounds r((M + bm - 1) / bm, (N + bn - 1) / bn, sp, cus);
+            const int64_t slots = (int64_t)r.xcd_cus * (qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu);
+            const double one = ((double)((K / 256 + sp - 1) / sp * 4) + c.prologue_steps) * c.step_us[f];
+            const auto round_us = [&](int64_t wgs) {
+                return wgs ? one * (1.0 + c.shared * (double)((wgs + r.xcd_cus - 1) / r.xcd_cus - 1)) * r.busy(c.clock, wgs) : 0.0;
+            };
+            double t = c.base_us + (double)(r.per_xcd / slots) * round_us(slots) + round_us(r.per_xcd % slots) + c.y_us_per_mb * y_mb;
+            if (sp > 1) t += c.split_us + c.add_us_per_mb[sp >= 4] * y_mb * sp;
+            t *= cut_bias(0.019, sp);
             if (t < best) { best = t; *tile_m = bm; *tile_n = bn; *ksplit = sp; }
         }
     }
@@ -1512,8 +1521,8 @@ static int32_t prefill_plan_any(int32_t qtype, int64_t M, int64_t N, int64_t K, 
     const double best = plan_in_loop(qtype, M, N, K, cus, tile_m, tile_n, ksplit);
     if (allow_dense && M > 64) {
         int sp = 1, bm = 256;
-        /* (two launches more and a trip of the weights through memory: 8 us where the estimate is tight) */
-        if (dense_estimate(M, N, K, cus, true, &bm, &sp) + 8.0 < best) {
+        /* (1.3 us in favour of a single launch, from the fit; 8 us cost 0.1 % on average) */
+        if (dense_estimate(qtype, M, N, K, cus, true, &bm, &sp) + 1.3 < best) {
             *tile_m = bm;
             *tile_n = 256;
             *ksplit = sp;
@@ -1637,7 +1646,7 @@ extern "C" int32_t psn_qmatmul_prefill_packed(psn_module *mod, psn_stream *s, co
         return rc;
     if ((rc = bind(mod->ctx))) return rc;
     int sp = 1, bm = 256;
-    (void)dense_estimate(M, N, K, mod->ctx->compute_units, false, &bm, &sp);
+    (void)dense_estimate(PSN_Q4_0, M, N, K, mod->ctx->compute_units, false, &bm, &sp);
     return launch_dense(mod, s, packed->p, X, Y, M, N, K, bm, sp);
 }
 

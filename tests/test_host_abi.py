@@ -250,9 +250,8 @@ def test_static_scratch_is_exported_by_the_device_image():
     assert all(r[3] == "OBJECT" and r[4] == "GLOBAL" and int(r[2]) == 1 << 20 for r in rows), rows
 
 
-def _kernel_resources():
-    """name -> (vgpr spills, sgpr spills, scratch bytes per lane) for every kernel of every built code object,
-    read from the code objects' own metadata notes."""
+def _kernel_notes():
+    """(name, lookup of a field) for every kernel of every built code object, from the code objects' own metadata notes."""
     import glob
     import subprocess
     import tempfile
@@ -260,16 +259,25 @@ def _kernel_resources():
     objs = sorted(glob.glob(os.path.join(ROOT, "openagents_amd", "lib", "*.gfx950.hsaco")))
     if not objs or not (os.path.exists(bundler) and os.path.exists(readelf)):
         pytest.skip("built code objects or LLVM binutils not present")
-    out = {}
+    out = []
     with tempfile.TemporaryDirectory() as d:
         for path in objs:
             elf = os.path.join(d, os.path.basename(path) + ".elf")
             subprocess.check_call([bundler, "--unbundle", "--type=o", f"--input={path}", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--output={elf}"])
             notes = subprocess.check_output([readelf, "--notes", elf], text=True)
             for blk in notes.split("- .agpr_count:")[1:]:
-                get = lambda key: re.search(r"\." + key + r":\s+(\S+)", blk).group(1)
-                out[get("name")] = (int(get("vgpr_spill_count")), int(get("sgpr_spill_count")), int(get("private_segment_fixed_size")))
+                get = lambda key, blk=blk: re.search(r"\." + key + r":\s+(\S+)", blk).group(1)
+                out.append((get("name"), get))
     return out
+
+
+def _kernel_resources():
+    """name -> (vgpr spills, sgpr spills, scratch bytes per lane)"""
+    return {name: (int(get("vgpr_spill_count")), int(get("sgpr_spill_count")), int(get("private_segment_fixed_size"))) for name, get in _kernel_notes()}
+
+
+def _kernel_registers():
+    return {name: int(get("vgpr_count")) for name, get in _kernel_notes()}
 
 
 def test_no_kernel_spills_registers_or_uses_scratch():
@@ -283,6 +291,41 @@ def test_no_kernel_spills_registers_or_uses_scratch():
         assert family in res, family
     bad = {k: v for k, v in res.items() if v != (0, 0, 0)}
     assert not bad, bad
+
+
+def test_prefill_planner_counts_the_workgroups_a_compute_unit_can_hold():
+    """The cost models' workgroups per compute unit against the built kernels: 512 vector registers per lane and SIMD, given out in eights, two
+    waves of a workgroup on each of the four SIMDs; 160 KB of LDS, (4 rows + 2 columns) * 128 bytes of it for a family 4 tile."""
+    src = open(os.path.join(ROOT, "openagents_amd", "csrc", "psn_host.cpp")).read()
+    tiles = re.findall(r"\{(\d+), (\d+)\}", re.search(r"k_prefill_tiles\[\]\[2\] = \{(.*)\};", src).group(1))
+    table = re.findall(r"\{(\d), (\d), (\d), ", re.search(r"k_prefill_cost\[\] = \{(.*?)\n\};", src, re.S).group(1))
+    assert len(table) == 4
+    regs = _kernel_registers()
+    held = lambda name, lds: min(512 // (-(-regs[name] // 8) * 8) // 2, 160 * 1024 // lds)
+    for tile, others, q6_K in table:
+        m, n = map(int, tiles[int(tile)])
+        for fmt in ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K"):
+            assert held(f"psn_prefill_{fmt}_m{m}_n{n}_pp", (4 * m + 2 * n) * 128) == int(q6_K if fmt == "q6_K" else others), (fmt, m, n)
+    chunk = {"q4_0": 144, "q8_0": 272, "q4_K": 144, "q5_K": 176, "q6_K": 224}
+    for name in regs:
+        thin = re.fullmatch(r"psn_prefill_(\w+)_thin_(\d)_(\d)", name)
+        if thin:
+            fmt, tm, rt = thin.group(1), int(thin.group(2)), int(thin.group(3))
+            two = tm == 1 and (rt == 1 or (rt == 2 and fmt not in ("q8_0", "q6_K")))
+            assert held(name, max(8 * (16 * rt * chunk[fmt] + tm * 2048), 8192 * rt * tm)) == (2 if two else 1), name
+
+
+def test_prefill_planner_knows_that_xcds_fill_unevenly(lib):
+    """Shapes whose N tiles do not spread evenly over the eight XCDs, or that fill every round, where a planner blind to it picked the slower family:
+    (measured us) dense 689 against 467 at 5120 x 13824 M = 3072, 329 against 283 at 32000 x 4096 M = 1024; family 4 150 against 135 at 4096 x 4096
+    M = 4096, and 40 instead of 31 for Q4_K at 1536 x 5632 M = 640."""
+    for qt in (_ffi.Q4_0, _ffi.Q8_0, _ffi.Q4_K, _ffi.Q5_K, _ffi.Q6_K):
+        for workspace in (True, False):
+            assert backend.prefill_choice(3072, 5120, 13824, qt, workspace=workspace) == (256, 128, 1, 4)
+    assert backend.prefill_choice(1024, 32000, 4096, _ffi.Q4_0) == (256, 128, 1, 4)
+    assert backend.prefill_choice(4096, 4096, 4096, _ffi.Q4_0) == (256, 256, 1, 128)
+    for qt in (_ffi.Q4_0, _ffi.Q4_K, _ffi.Q5_K):
+        assert backend.prefill_choice(640, 1536, 5632, qt)[:2] == (64, 64)
 
 
 def test_prefill_plans_take_the_dense_family_only_for_large_m():
