@@ -1073,13 +1073,19 @@ static void matvec_args(psn_matvec_args *a, int32_t qtype, const seg_list &sg, i
     a->blocks = blocks;
 }
 /* psn_mvb_<fmt>_q8 (psn_matvec_batch.hip), on quantized activations.  Its cost does not grow with the batch; the register kernels' does.
- * Measured on MI355X against them over 200 .. 40000 rows and K = 256 .. 16384: from five columns on 1.0-6 x faster throughout.  With three or
- * four it is the slower one for long rows (0.66-0.96 x from K = 8192 on: eight waves to a tile make a long chain), for Q4_0 rows of 4096
- * (0.97-1.07 x) and for many short Q8_0 rows (14336 x 2560: 1.00-1.01 x, 40000 x 1024: 0.88 x), otherwise 1.0-1.8 x. */
+ * Measured on MI355X against them (register / batch kernel time) over 16 .. 80000 rows and K = 256 .. 28672:
+ *   three and four columns: long rows are a long chain for eight waves to a tile (0.66-0.96 from K = 8192 on; Q4_0 0.98-1.07 at K = 4096).  Many rows
+ *   of K = 1280 .. 2048 fill the register kernels' lane groups (Q4_0 from 14336 rows on 0.86-1.03, below 1.1-1.5); Q8_0 has 1.0-1.8 up to 8192 rows,
+ *   0.83-1.05 beyond, save K > 2560 from 14336 rows on, 0.98-1.10;
+ *   from five on: 1.0-6, but few long rows, whose register kernels still stage their columns in LDS, leave it the chain without the
+ *   bandwidth to hide it: Q4_0 below 1000 rows, five columns 0.87-0.97 at K = 12288 .. 16384 (1.03-1.05 at 11008), six 0.89-1.03 from 13824, seven
+ *   0.92-0.98 from 16128; Q8_0 up to 200 rows, five columns 0.95-0.98 from 16128. */
 static bool use_batch_kernel(int32_t qtype, int64_t rows, int64_t K, int32_t batch) {
-    if (qtype != PSN_Q4_0 && qtype != PSN_Q8_0) return false;
-    if (batch >= 5) return true;
-    return batch >= 3 && (qtype == PSN_Q4_0 ? K < 4096 : K <= 4096 && (K > 2560 || rows <= 8192));
+    if ((qtype != PSN_Q4_0 && qtype != PSN_Q8_0) || batch < 3) return false;
+    const bool q4_0 = qtype == PSN_Q4_0;
+    if (batch >= 5) return !(rows < (q4_0 ? 1000 : 256) && K >= (q4_0 ? 2304 : 3200) * batch && K <= 16384 && batch < 8);
+    if (q4_0) return K < 4096 && !(rows > 12288 && K > 1024 && K <= 2048);
+    return K <= 4096 && (rows <= 8192 || (rows > 12288 && K > 2560));
 }
 static int32_t run_batch(psn_module *mod, psn_stream *s, int32_t qtype, const seg_list &sg, const void *xq, int64_t K, int32_t batch) {
     psn_actq_info li;

@@ -967,8 +967,8 @@ def test_batch_kernel_at_tile_and_range_edges(hip, orc, qname):
         W = orc.quantize(t, G.seeded_weights(9300, n, k))
         w = hip.upload_weight(t, W, n, k)
         for b in (3, 4, 5, 8):
-            if b < 5 and k > 4096:
-                continue                                    # the register kernels' range
+            if b < 8 and k > 4096:
+                continue                                    # the register kernels' range (that few rows of that length)
             x = G.seeded_acts(9301 + b, b, k)
             ref = orc.matvec(t, orc.ACT_Q8, W, x, n, k)
             xb, y = hip.upload(x), hip.alloc(b * n * 4)
@@ -989,3 +989,23 @@ def test_batch_kernel_at_tile_and_range_edges(hip, orc, qname):
         hip.quantized_matvec_multi([hip.upload_weight(t, W, n, k) for W, n in zip(Ws, rows[:count])], hip.upload(x), ys, b, _ffi.ACT_Q8)
         for W, n, y in zip(Ws, rows, ys):
             assert G.max_rel_err(y.download(np.float32, (b, n)), orc.matvec(t, orc.ACT_Q8, W, x, n, k)) < PARITY_TOL, (count, n)
+
+
+@pytest.mark.parametrize("qname,n,k,batch,batch_kernel", [
+    ("Q4_0", 40000, 2048, 3, False), ("Q4_0", 14336, 1280, 4, False), ("Q4_0", 12288, 2048, 4, True), ("Q4_0", 40000, 1024, 3, True),
+    ("Q4_0", 40000, 2304, 4, True), ("Q8_0", 11008, 3072, 3, False), ("Q8_0", 8192, 3072, 3, True), ("Q8_0", 14336, 2816, 4, True),
+    ("Q8_0", 14336, 2560, 4, False), ("Q4_0", 600, 14336, 5, False), ("Q4_0", 1000, 14336, 5, True), ("Q4_0", 600, 13568, 6, True),
+    ("Q4_0", 600, 16384, 7, False), ("Q4_0", 600, 16384, 8, True), ("Q4_0", 600, 18432, 5, True), ("Q8_0", 200, 16384, 5, False),
+    ("Q8_0", 256, 16384, 5, True), ("Q8_0", 200, 16384, 6, True)])
+def test_batch_kernel_runs_where_it_is_the_faster_one(hip, orc, qname, n, k, batch, batch_kernel):
+    """Either side of the lines between the int8-MFMA kernel and the register kernels, for every call that draws them (the launch log tells)."""
+    t = getattr(orc, qname)
+    w = backend.QuantizedTensor(hip.alloc(n * backend.row_bytes(t, k)).fill_zero(), t, n, k)
+    x, y = hip.alloc(batch * k * 4).fill_zero(), hip.alloc(batch * n * 4)
+    xq = hip.quantize_activations(x, k, batch, backend.act_type_for(t))
+    for call in (lambda: hip.quantized_matvec(w, x, y, batch, _ffi.ACT_Q8), lambda: hip.quantized_matvec_q8(w, xq, y, batch),
+                 lambda: hip.quantized_matvec_noalloc(w, x, y, batch), lambda: hip.quantized_matvec_multi([w], x, [y], batch, _ffi.ACT_Q8)):
+        hip.lib.psn_launch_log_clear()
+        call()
+        assert (f"psn_mvb_{qname.lower()}_q8" in hip.lib.psn_launch_log().decode().split(";")) == batch_kernel
+    hip.sync()
