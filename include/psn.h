@@ -229,7 +229,7 @@ int32_t psn_qmatvec_noalloc(psn_module *mod, psn_stream *s, int32_t qtype, int32
 int64_t psn_noalloc_max_bytes(void);
 
 /* Launch geometry of one matvec.  With Q4_0 and Q8_0 weights, scheme Q8 and three to eight columns psn_qmatvec(_multi),
- * psn_qmatvec_q8(_multi) and psn_qmatvec_noalloc run an int8-MFMA kernel that has no plan where that is the faster one (R rows in the launch):
+ * psn_qmatvec_q8(_multi) and psn_qmatvec_noalloc run an int8-MFMA kernel that has no plan where that is the faster one (R rows in the launch, at most 2^26):
  * five and more columns always, except (fewer than eight columns, K <= 16384) Q4_0 with R < 1000 and K >= 2304 * columns and Q8_0 with R < 256
  * and K >= 3200 * columns; three and four columns of Q4_0 with K < 4096, except R > 12288 with 1024 < K <= 2048, and of Q8_0 with K <= 4096
  * and either R <= 8192 or both R > 12288 and K > 2560.  The plan then names the

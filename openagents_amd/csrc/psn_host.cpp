@@ -1082,6 +1082,7 @@ static void matvec_args(psn_matvec_args *a, int32_t qtype, const seg_list &sg, i
  *   0.92-0.98 from 16128; Q8_0 up to 200 rows, five columns 0.95-0.98 from 16128. */
 static bool use_batch_kernel(int32_t qtype, int64_t rows, int64_t K, int32_t batch) {
     if ((qtype != PSN_Q4_0 && qtype != PSN_Q8_0) || batch < 3) return false;
+    if (rows > (1 << 26)) return false;      /* 512 threads to 16 rows: a launch holds fewer than 2^32 of them */
     const bool q4_0 = qtype == PSN_Q4_0;
     if (batch >= 5) return !(rows < (q4_0 ? 1000 : 256) && K >= (q4_0 ? 2304 : 3200) * batch && K <= 16384 && batch < 8);
     if (q4_0) return K < 4096 && !(rows > 12288 && K > 1024 && K <= 2048);

@@ -1009,3 +1009,23 @@ def test_batch_kernel_runs_where_it_is_the_faster_one(hip, orc, qname, n, k, bat
         call()
         assert (f"psn_mvb_{qname.lower()}_q8" in hip.lib.psn_launch_log().decode().split(";")) == batch_kernel
     hip.sync()
+
+
+def test_more_rows_than_the_batch_kernel_can_launch(hip, orc):
+    """The int8-MFMA kernel takes 512 threads for 16 rows, and a launch holds fewer than 2^32 threads: beyond 2^27 rows the register kernels, whose
+    workgroups walk the rows, take the call as they do for two columns."""
+    n, k, b = (1 << 27) + 16, 256, 3
+    rb = backend.row_bytes(orc.Q4_0, k)
+    W = orc.quantize(orc.Q4_0, G.seeded_weights(9400, 16, k))
+    x = G.seeded_acts(9401, b, k)
+    w = backend.QuantizedTensor(hip.alloc(n * rb).fill_zero(), orc.Q4_0, n, k)
+    y = hip.alloc(b * n * 4)
+    try:
+        w.buf.upload(W, (n - 16) * rb)
+        hip.quantized_matvec(w, hip.upload(x), y, b, _ffi.ACT_Q8)
+        ref = orc.matvec(orc.Q4_0, orc.ACT_Q8, W, x, 16, k)
+        for i in range(b):
+            assert G.max_rel_err(y.download(np.float32, (16,), (i * n + n - 16) * 4), ref[i]) < PARITY_TOL, i
+    finally:
+        w.buf.free()
+        y.free()
