@@ -1029,3 +1029,38 @@ def test_more_rows_than_the_batch_kernel_can_launch(hip, orc):
     finally:
         w.buf.free()
         y.free()
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0"])
+def test_batch_kernel_keeps_values_that_are_not_finite_in_their_row(hip, orc, qname):
+    """A block scale that is infinite or NaN spoils its weight row and nothing else changes by a bit, ragged last tile included."""
+    t = getattr(orc, qname)
+    n, k, b = 37, 2304, 5
+    clean = orc.quantize(t, G.seeded_weights(9330, n, k))
+    bad = clean.copy().reshape(n, -1)
+    rows = [0, 16, 33, n - 1]
+    for r, bits in zip(rows, (0x7c00, 0x7e00, 0xfc00, 0x7c01)):
+        at = bad.shape[1] - {"Q4_0": 18, "Q8_0": 34}[qname]            # its last block
+        bad[r, at:at + 2] = np.array([bits], np.uint16).view(np.uint8)
+    x, out = hip.upload(G.seeded_acts(9331, b, k)), []
+    for W in (clean, bad):
+        w, y = hip.upload_weight(t, W, n, k), hip.alloc(b * n * 4)
+        hip.lib.psn_launch_log_clear()
+        hip.quantized_matvec(w, x, y, b, _ffi.ACT_Q8)
+        assert f"psn_mvb_{qname.lower()}_q8" in hip.lib.psn_launch_log().decode().split(";")
+        out.append(y.download(np.float32, (b, n)))
+    assert not np.isfinite(out[1][:, rows]).any()
+    keep = np.setdiff1d(np.arange(n), rows)
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0][:, keep], out[1][:, keep])
+
+
+def test_looking_a_kernel_up_leaves_no_error_behind(hip, orc):
+    """The library asks one code object after the other for a kernel's name; what HIP notes about the misses must not be the next thing that a
+    program on this thread reads as its own error."""
+    be = backend.HipBackend(0)                                          # a module of its own: nothing has been looked up in it yet
+    try:
+        be.lib.hipGetLastError()
+        be.matmul_host(orc.Q5_K, orc.quantize(orc.Q5_K, G.seeded_weights(9340, 64, 256)), G.seeded_acts(9341, 3, 256).astype(np.float16), 64, 256)
+        assert be.lib.hipPeekAtLastError() == 0
+    finally:
+        be.close()

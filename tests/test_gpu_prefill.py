@@ -458,3 +458,29 @@ def test_the_choice_is_what_runs(hip, orc, qname):
                 ran.append(hip.lib.psn_launch_log().decode())
             hip.sync()
             assert ran[0] == ran[1], (m, n, k, ran, tile)
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
+def test_values_that_are_not_finite_stay_in_their_row_and_column(hip, orc, qname):
+    """A block scale that is infinite or NaN spoils its weight row's column of Y, an infinity or NaN in X its row, and nothing else changes by a
+    bit: thin and in-loop kernels, ragged against every tile (rows past the end repeat the last one, tiles past it are moved back)."""
+    t = getattr(orc, qname)
+    n, k = 300, 768
+    clean_w = weights(orc, qname, 897, n, k)
+    bad_w = clean_w.copy().reshape(n, -1)
+    d_at = 208 if qname == "Q6_K" else 0
+    cols, size = [0, 17, 250, n - 1], len(bad_w[0])
+    for i, c in enumerate(cols):
+        block = size - 210 if qname == "Q6_K" and i == 3 else 0
+        bad_w[c, block + d_at:block + d_at + 2] = np.array([0x7c00, 0x7e00, 0xfc00, 0x7c01], np.uint16)[i:i + 1].view(np.uint8)
+    for tile, m in (((16, 16), 13), ((48, 16), 37), ((64, 32), 62), ((64, 64), 70), ((64, 128), 70), ((128, 128), 150), ((256, 128), 270)):
+        say(f"not finite {qname} tile={tile}")
+        x = G.seeded_acts(898, m, k).astype(np.float16)
+        bad_x = x.copy()
+        rows = [2, m - 1]
+        bad_x[2, 5], bad_x[m - 1, k - 1] = np.inf, np.nan
+        tile = tile + (1, 4 if m > 64 else 8)
+        clean, y = hip.matmul_host(t, clean_w, x, n, k, tile), hip.matmul_host(t, bad_w, bad_x, n, k, tile)
+        assert not np.isfinite(y[rows]).any() and not np.isfinite(y[:, cols]).any(), tile
+        keep = np.ix_(np.setdiff1d(np.arange(m), rows), np.setdiff1d(np.arange(n), cols))
+        assert np.isfinite(clean).all() and np.array_equal(clean[keep], y[keep]), tile
