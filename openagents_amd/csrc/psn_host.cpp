@@ -1441,11 +1441,12 @@ extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int
 }
 /* At most 64 rows: which kernel streams the weights.  psn_prefill_<fmt>_thin_<tm>_<rt> (psn_prefill_thin.hip, 16 tm rows of X and 16 rt
  * of W per workgroup) against the 64 x 64 kernel (psn_prefill_<fmt>_skinny; rt = 0 here; with Q6_K only for rows of whole 16-byte
- * words).  Measured on MI355X over five formats, fifteen matrices and M = 16 .. 64 (2300 launches; the estimates are off by 6 % rms,
- * and what they pick is within 0.5 % of the fastest on average): a launch, then per round of workgroups the first loads, a chain
+ * words).  Checked on MI355X against every explicit plan over five formats, sixteen matrices and M = 1 .. 64 (11304 launches): what the estimates
+ * pick is 1.3 % off the fastest on average and more than 10 % off in 35 of 720 shapes (a handful of rows of X on large matrices; the 64 x 64
+ * kernel where family 4, which is considered here for Q6_K only, would do better).  An estimate is a launch, then per round of workgroups the first loads, a chain
  * per chunk of a wave, and the work that the waves of a SIMD share: decode per weight row, X per row of it.  The 64 x 64 kernel stays
- * the faster one from about 48 rows on where the matrix is large (Q4_0 8192 x 28672 M = 64: 62 us against 65-75), with Q8_0, whose raw
- * chunks leave no LDS for four tiles, from 17 on (14336 x 4096 M = 32: 23.4 against 26); it cuts K only while the weight rows
+ * the faster one from about 48 rows on where the matrix is large (Q4_0 8192 x 28672 M = 64: 62 us against 74), with Q8_0, whose raw
+ * chunks leave no LDS for four tiles, from 17 on (14336 x 4096 M = 32: 23.0 against 25.4); it cuts K only while the weight rows
  * alone leave half of the compute units without a workgroup.  At rt = 4 a cut of K did not pay. */
 struct weight_stream_plan { int rt, ksplit; double us; };
 static bool may_cut_k(int64_t M, int64_t N, int64_t K, int sp) { return sp == 1 || ((M * N) % 4 == 0 && K / 256 >= 2 * sp); }

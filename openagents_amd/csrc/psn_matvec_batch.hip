@@ -1,5 +1,5 @@
 /*
- * psn_matvec_batch.hip -- gfx950 decode matvec for two to eight columns, scheme Q8, formats whose blocks of 32 carry one scale
+ * psn_matvec_batch.hip -- gfx950 decode matvec for up to eight columns (used from three on), scheme Q8, formats whose blocks of 32 carry one scale
  * (Q4_0, Q8_0; Q8_0 activations, quantized beforehand).
  *
  * v_mfma_i32_16x16x32_i8 multiplies one block of 16 weight rows with up to 16 columns (A = the columns' int8, B = the rows'):
@@ -12,7 +12,8 @@
  * lanes on consecutive 16-byte words, and go through the wave's own piece of LDS to the lanes that multiply them.
  *
  * What bounds it: a chunk of a wave is a chain of about 1 us (LDS to MFMA to scaling, eight blocks of it), hidden by the waves of three
- * or four workgroups on a compute unit; the weight stream where rows are many (Q8_0 40000 x 8192, batch 8: 348 MB in 79 us).  Against the
+ * workgroups on a compute unit with Q4_0 (72 registers) and of two with Q8_0 (55 KB of LDS each, a third would fit without the 2 KB that
+ * its activation sums, which it has no use for, are given); the weight stream where rows are many (Q8_0 40000 x 8192, batch 8: 348 MB in 79 us).  Against the
  * register kernels at batch 8: Q4_0 14336 x 4096 21.0 -> 15.7 us, 1000 x 4096 11.2 -> 7.5, 4100 x 16384 92 -> 23.5; Q8_0 25.5 -> 20.1,
  * 11.0 -> 7.5, 90 -> 28.3.  Two tiles per workgroup measured 25-45 % slower (fewer waves), a second chunk on its way 2-15 % slower,
  * rows and columns swapped in the products (fewer LDS reads, 96 registers instead of 68) 0-20 % slower.

@@ -14,8 +14,9 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 /* An fp16 tile in LDS: rows of 128 bytes (64 k), the eight 16-byte chunks of a row stored at chunk ^ tile_swz(row).  A
  * fragment read takes the same chunk of 16 consecutive rows at a time: over the 64 banks (256 bytes) they must fall into
  * sixteen different 16-byte columns, (row & 1) * 8 + position -- so it is row bits 1..3 that scatter, not bits 0..2, which
- * put rows r and r + 8 into one column and cost every read four extra cycles (SQ_LDS_BANK_CONFLICT 7.3e6 of 1.65e7 active
- * cycles at 512 x 14336 x 4096, 0 now). */
+ * put rows r and r + 8 into one column and cost every read four extra cycles.  (Q4_K 512 x 14336 x 4096, SQ_LDS_BANK_CONFLICT of
+ * SQ_LDS_IDX_ACTIVE: four-wave 128 x 256 kernel 5.5e6 of 1.47e7 with bits 0..2, 3.7e6 of 1.28e7 with bits 1..3; the eight-wave 256 x 128 kernel
+ * 1.9e6 of 1.11e7.) */
 PSN_DEV int tile_swz(int row) { return (row >> 1) & 7; }
 PSN_DEV int tile_off(int row, int chunk) { return row * 128 + ((chunk ^ tile_swz(row)) << 4); }
 

@@ -57,7 +57,7 @@ PSN_DEV void q0_finish(const half_done &t, u32 bias, u32 d2, u32 &o0, u32 &o1) {
 /* ---- a format's share of one thread: part `part` of 32 / NB parts of a row.  `base` is the row's chunk plus lane_off(part);
  *      load() asks for everything the four steps of the chunk need (LOADS instructions); step J's bytes are two groups
  *      (HI = 0, 1) of NB weights, which belong at k = k_lo(part) and k_hi(part) of the 64-wide step; first() and second() turn
- *      word i of a group into four fp16, with the step's scales from scales0() and scales1().  SPREAD (for NB = 4, 8): see row_of below. ---- */
+ *      word i of a group into four fp16, with the step's scales from scales0() and scales1().  SPREAD (for NB = 4, 8): row_of() in psn_prefill_pp.hip. ---- */
 struct PpQ4_K {
     static constexpr int BYTES = 144, LOADS = 5;
     template <int NB> struct raw { u32x4 h; typename raw_bytes<NB>::t q[4]; };

@@ -13,12 +13,12 @@
  *     registers, asked for a whole 256-wide chunk ahead.
  * One barrier per step.
  *
- * What bounds it (counters, Q4_K 512 x 14336 x 4096, 256 x 128 tiles): of 121 k cycles 66 k are MFMA, and the device runs at
- * 2.1 GHz under them; the same instructions on zero weights take 45 us instead of 59, so from M = 512 on it is power
- * (operand reads, decode arithmetic and MFMAs together), below that the decode's vector instructions (60 per wave and
+ * What bounds it (counters, Q4_K 512 x 14336 x 4096, 256 x 128 tiles): of 123 k cycles 66 k are MFMA on the 224 compute units that have a
+ * tile; launches back to back take 80 us, on zero weights (the same instructions) 64, so from M = 512 on it is power
+ * (operand reads, decode arithmetic and MFMAs together), below that the decode's vector instructions (72 per wave and
  * step, of which six per MFMA ride along for free).  Against the kernels that served these shapes before (producer /
- * consumer and dequantize-first): 14336 x 4096 at M = 203: Q4_0 52 -> 40 us, Q8_0 74 -> 52, Q4_K 65 -> 43, Q6_K 91 -> 48; at
- * M = 512: Q4_0 80 -> 64, Q8_0 99 -> 73, Q4_K 94 -> 67, Q6_K 105 -> 71.  Splitting the roles (eight multiplying and eight
+ * consumer and dequantize-first): 14336 x 4096 at M = 203: Q4_0 55 -> 44 us, Q8_0 75 -> 55, Q4_K 69 -> 47, Q6_K 92 -> 52; at
+ * M = 512: Q4_0 82 -> 68, Q8_0 98 -> 78, Q4_K 97 -> 72, Q6_K 106 -> 77.  Splitting the roles (eight multiplying and eight
  * staging waves) measured 2-8 % slower, running the two waves of a SIMD in strictly opposite phases 10-15 % slower.
  */
 #include "psn_args.h"

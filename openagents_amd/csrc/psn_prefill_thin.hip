@@ -16,8 +16,8 @@
  * What bounds it: a weight costs about four vector instructions (fp32 d * q - m per weight, then the rounding to fp16), which
  * is 8 us of a 14336 x 4096 launch over all SIMDs, and X, which every workgroup reads whole (RT trades it against workgroups).
  * Two chunks of W on their way instead of one changed nothing (-1 .. +4 %), nor did more of X.  Against the 64 x 64 kernel
- * (psn_prefill.hip), us: Q4_K 4096 x 4096 M = 16 11.8 -> 6.8, M = 33 12.6 -> 10.0, M = 64 14.1 -> 11.2; 1024 x 4096 M = 16 8.6 -> 5.4,
- * M = 48 9.3 -> 6.7; 14336 x 4096 M = 16 23 -> 16, M = 48 23.3 -> 21.1; 4096 x 14336 M = 16 23.3 -> 15.5.  At 64 rows of a large
+ * (psn_prefill.hip), us: Q4_K 4096 x 4096 M = 16 11.4 -> 6.5, M = 33 12.2 -> 9.6, M = 64 13.9 -> 11.3; 1024 x 4096 M = 16 8.8 -> 5.3,
+ * M = 48 9.4 -> 6.6; 14336 x 4096 M = 16 21.7 -> 15.1, M = 48 22.4 -> 20.8; 4096 x 14336 M = 16 22.2 -> 16.5.  At 64 rows of a large
  * matrix both take as long.
  */
 #include "psn_args.h"
