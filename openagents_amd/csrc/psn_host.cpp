@@ -1377,20 +1377,25 @@ static int32_t check_prefill(const char *what, psn_module *mod, psn_stream *s, i
     return PSN_OK;
 }
 
-/* Cost models of family 4 (psn_prefill_pp.hip) and of the dense family, fitted to launches timed on MI355X: five formats, 22 matrices (1000 x 2560 ..
- * 28672 x 8192), M = 65 .. 4096, 22848 launches of family 4 and 9296 of the dense one.  Weight lies on plans near the fastest, whose estimates are
- * off by 3-6 % rms; what they pick is 0.35 % off the fastest plan of any family on average over 1555 shapes and more than 10 % off in 3.
+/* Cost models of family 4 (psn_prefill_pp.hip) and of the dense family, fitted to launches timed on MI355X: five formats, 28 matrices (1000 x 2560,
+ * 512 x 4096 .. 32000 x 4096), M = 65 .. 4096, 33348 launches of family 4 and 13760 of the dense one.  Weight lies on plans near the fastest, whose
+ * estimates are off by 4-6 % rms; what they pick is 0.4 % off the fastest plan of any family on average over 2315 shapes and more than 10 % off in 3.
  *
  * Both families deal N tiles to the eight XCDs in turn and give an XCD all M tiles and K ranges of its own, so that the XCDs with one N tile
  * more set the rounds of workgroups: 5120 columns are 20 tiles of 256, three for four of the XCDs, whose 36 workgroups at M = 3072 take
- * two rounds on 32 compute units (Q4_K: dense 689 us; 256 x 128 tiles, five for each XCD, 467).  A round in which nearly every compute unit multiplies runs at
- * a lower clock than an emptier one (8192 x 8192 M = 2048, two full rounds: 1.2 x the step cost of half-filled ones). */
+ * two rounds on 32 compute units (Q4_K: dense 689 us; 256 x 128 tiles, five for each XCD, 467).  A round in which nearly every compute unit multiplies rows
+ * of its own (those past the end repeat the last one) runs at a lower clock than an emptier one (8192 x 8192 M = 2048, two full rounds: 1.2 x the
+ * step cost of half-filled ones). */
 static int format_index(int32_t t) { return t == PSN_Q4_0 ? 0 : t == PSN_Q8_0 ? 1 : t == PSN_Q4_K ? 2 : t == PSN_Q5_K ? 3 : 4; }
 struct prefill_rounds {
     int64_t per_xcd;        /* workgroups of an XCD with the most N tiles */
-    double share;           /* workgroups of all XCDs over eight times that */
+    double share;           /* workgroups of all XCDs over eight times that; rows of tiles past the end of X count half */
     int xcd_cus;
-    prefill_rounds(int64_t mt, int64_t nt, int sp, int32_t cus) : per_xcd((nt + 7) / 8 * mt * sp), share((double)nt / (double)((nt + 7) / 8 * 8)), xcd_cus(cus < 8 ? 1 : cus / 8) {}
+    prefill_rounds(int64_t M, int64_t N, int bm, int bn, int sp, int32_t cus) : xcd_cus(cus < 8 ? 1 : cus / 8) {
+        const int64_t mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn, most = (nt + 7) / 8;
+        per_xcd = most * mt * sp;
+        share = (double)nt / (double)(8 * most) * (0.5 + 0.5 * (double)M / (double)(mt * bm));
+    }
     double busy(double clock, int64_t wgs) const {                 /* the clock's part of a round of wgs workgroups per XCD */
         const double filled = (wgs < xcd_cus ? (double)wgs / xcd_cus : 1.0) * share, u = (filled - 0.7) / 0.2;
         return 1.0 + clock * (u < 0.0 ? 0.0 : u > 1.0 ? 1.0 : u);
@@ -1409,26 +1414,26 @@ struct prefill_cost {
     double step_us[5];                /* per 64 of K: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
 };
 static const prefill_cost k_prefill_cost[] = {
-    {0, 3, 2, 3.66, 0.690, 0.257, {0.439, 0.439}, 2.23, 0.20, 0.025, {0.296, 0.396, 0.304, 0.327, 0.387}},
-    {1, 1, 1, 3.15, 0.000, 0.139, {0.645, 0.645}, 1.12, 2.44, 0.053, {0.418, 0.597, 0.470, 0.505, 0.577}},
-    {2, 1, 1, 3.45, 0.000, 0.222, {0.613, 0.613}, 1.21, 2.55, 0.193, {0.503, 0.659, 0.557, 0.555, 0.631}},
-    {4, 1, 1, 3.25, 0.000, 0.263, {0.547, 0.727}, 2.55, 0.60, 0.269, {0.743, 0.862, 0.794, 0.788, 0.818}},
+    {0, 3, 2, 3.59, 0.690, 0.296, {0.465, 0.465}, 2.14, 0.20, 0.021, {0.290, 0.372, 0.304, 0.314, 0.387}},
+    {1, 1, 1, 3.21, 0.000, 0.128, {0.658, 0.658}, 1.12, 2.29, 0.045, {0.426, 0.597, 0.470, 0.525, 0.577}},
+    {2, 1, 1, 3.52, 0.000, 0.222, {0.613, 0.613}, 1.19, 2.45, 0.209, {0.503, 0.659, 0.546, 0.566, 0.619}},
+    {4, 1, 1, 3.25, 0.000, 0.263, {0.580, 0.760}, 2.55, 0.55, 0.269, {0.743, 0.862, 0.794, 0.788, 0.818}},
 };
 /* The dense family: one pass that rewrites the matrix as fp16 (none when the caller holds packed weights) and the multiply on 256 x 256 or
  * 128 x 256 tiles. */
-static const struct { int bm; double base_us, step_us, clock, add_us_per_mb; } k_dense_cost[] = {{256, 4.50, 1.358, 0.236, 0.612}, {128, 4.16, 0.697, 0.288, 0.382}};
-static const double k_unpack_us[5] = {0.427, 0.591, 0.469, 0.399, 0.519};      /* per million weights, from the fit */
+static const struct { int bm; double base_us, step_us, clock, add_us_per_mb; } k_dense_cost[] = {{256, 4.50, 1.358, 0.271, 0.612}, {128, 4.41, 0.697, 0.288, 0.422}};
+static const double k_unpack_us[5] = {0.427, 0.778, 0.460, 0.375, 0.519};      /* per million weights, from the fit */
 static double dense_estimate(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, bool with_unpack, int *bm_out, int *ksplit_out) {
     const double y_mb = (double)(M * N) * 4e-6;
     double best = 1e300;
     for (const auto &c : k_dense_cost) {
         for (int sp = 1; sp <= 4; sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 4 * sp)) continue;
-            const prefill_rounds r((M + c.bm - 1) / c.bm, (N + 255) / 256, sp, cus);
+            const prefill_rounds r(M, N, c.bm, 256, sp, cus);
             const int64_t full = r.per_xcd / r.xcd_cus, rest = r.per_xcd % r.xcd_cus;
             double t = c.base_us + (double)((K / 256 + sp - 1) / sp * 4) * c.step_us * ((double)full * r.busy(c.clock, r.xcd_cus) + (rest ? r.busy(c.clock, rest) : 0.0)) + 0.164 * y_mb;
-            if (sp > 1) t += (c.bm == 128 ? 2.20 : 0.0) + c.add_us_per_mb * y_mb * sp;
-            t *= cut_bias(0.070, sp);
+            if (sp > 1) t += (c.bm == 128 ? 1.87 : 0.0) + c.add_us_per_mb * y_mb * sp;
+            t *= cut_bias(0.085, sp);
             if (t < best) { best = t; *bm_out = c.bm; *ksplit_out = sp; }
         }
     }
@@ -1498,7 +1503,7 @@ static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32
         const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
-            const prefill_rounds r((M + bm - 1) / bm, (N + bn - 1) / bn, sp, cus);
+            const prefill_rounds r(M, N, bm, bn, sp, cus);
             const int64_t slots = (int64_t)r.xcd_cus * (qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu);
             const double one = ((double)((K / 256 + sp - 1) / sp * 4) + c.prologue_steps) * c.step_us[f];
             const auto round_us = [&](int64_t wgs) {
@@ -1506,7 +1511,7 @@ static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32
             };
             double t = c.base_us + (double)(r.per_xcd / slots) * round_us(slots) + round_us(r.per_xcd % slots) + c.y_us_per_mb * y_mb;
             if (sp > 1) t += c.split_us + c.add_us_per_mb[sp >= 4] * y_mb * sp;
-            t *= cut_bias(0.019, sp);
+            t *= cut_bias(0.020, sp);
             if (t < best) { best = t; *tile_m = bm; *tile_n = bn; *ksplit = sp; }
         }
     }
@@ -1529,8 +1534,8 @@ static int32_t prefill_plan_any(int32_t qtype, int64_t M, int64_t N, int64_t K, 
     const double best = plan_in_loop(qtype, M, N, K, cus, tile_m, tile_n, ksplit);
     if (allow_dense && M > 64) {
         int sp = 1, bm = 256;
-        /* (1.3 us in favour of a single launch, from the fit; 8 us cost 0.1 % on average) */
-        if (dense_estimate(qtype, M, N, K, cus, true, &bm, &sp) + 1.3 < best) {
+        /* (1.1 us in favour of a single launch, from the fit; 8 us cost 0.1 % on average) */
+        if (dense_estimate(qtype, M, N, K, cus, true, &bm, &sp) + 1.1 < best) {
             *tile_m = bm;
             *tile_n = 256;
             *ksplit = sp;
