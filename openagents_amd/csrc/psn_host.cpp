@@ -1419,26 +1419,52 @@ static const prefill_cost k_prefill_cost[] = {
     {2, 1, 1, 3.52, 0.000, 0.222, {0.613, 0.613}, 1.19, 2.45, 0.209, {0.503, 0.659, 0.546, 0.566, 0.619}},
     {4, 1, 1, 3.25, 0.000, 0.263, {0.580, 0.760}, 2.55, 0.55, 0.269, {0.743, 0.862, 0.794, 0.788, 0.818}},
 };
-/* The dense family: one pass that rewrites the matrix as fp16 (none when the caller holds packed weights) and the multiply on 256 x 256 or
- * 128 x 256 tiles. */
-static const struct { int bm; double base_us, step_us, clock, add_us_per_mb; } k_dense_cost[] = {{256, 4.50, 1.358, 0.271, 0.612}, {128, 4.41, 0.697, 0.288, 0.422}};
+/* The dense family (psn_prefill_dense.hip): one pass that rewrites the matrix as fp16 (none when the caller holds packed weights) and the multiply, whose tiles are dealt evenly
+ * to the XCDs.  Fitted to 3175 launches of the multiply (18 matrices, M = 16 .. 4096, K in one to eight ranges): what the estimates pick among the five tiles is 0.5 % off the
+ * fastest on average and more than 10 % off in 2 of 262 shapes.  The tiles below 256 columns are for packed weights only (explicit plans cannot name them, and a plan of
+ * psn_qmatmul_prefill is one that can be run explicitly). */
+static const struct dense_cost {
+    int bm, bn, per_cu;
+    double base_us, step_us, clock, busy_from, shared, prologue_steps, split_us, add_us_per_mb, y_us_per_mb, w_us_per_mb;     /* steps of 64 of K */
+} k_dense_cost[] = {
+    {256, 256, 1, 2.04, 1.038, 0.232, 0.688, 0.016, 9.23, 3.60, 0.54, 0.026, 0.008},
+    {128, 256, 1, 2.23, 0.455, 0.639, 0.328, 0.890, 7.57, 2.04, 0.54, 0.021, 0.050},
+    {128, 128, 1, 2.15, 0.258, 0.696, 0.318, 0.014, 9.71, 2.01, 0.45, 0.006, 0.042},
+    {64, 128, 1, 2.04, 0.179, 0.379, 0.198, 0.014, 8.71, 2.02, 0.43, 0.036, 0.066},
+    {64, 64, 2, 2.60, 0.135, 0.180, 0.442, 0.981, 2.28, 1.98, 0.50, 0.192, 0.057},
+};
 static const double k_unpack_us[5] = {0.427, 0.778, 0.460, 0.375, 0.519};      /* per million weights, from the fit */
-static double dense_estimate(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, bool with_unpack, int *bm_out, int *ksplit_out) {
-    const double y_mb = (double)(M * N) * 4e-6;
-    double best = 1e300;
-    for (const auto &c : k_dense_cost) {
-        for (int sp = 1; sp <= 4; sp *= 2) {
-            if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 4 * sp)) continue;
-            const prefill_rounds r(M, N, c.bm, 256, sp, cus);
-            const int64_t full = r.per_xcd / r.xcd_cus, rest = r.per_xcd % r.xcd_cus;
-            double t = c.base_us + (double)((K / 256 + sp - 1) / sp * 4) * c.step_us * ((double)full * r.busy(c.clock, r.xcd_cus) + (rest ? r.busy(c.clock, rest) : 0.0)) + 0.164 * y_mb;
-            if (sp > 1) t += (c.bm == 128 ? 1.87 : 0.0) + c.add_us_per_mb * y_mb * sp;
-            t *= cut_bias(0.085, sp);
-            if (t < best) { best = t; *bm_out = c.bm; *ksplit_out = sp; }
+struct dense_plan { int bm, bn, ksplit; double us; };
+static dense_plan plan_dense(int64_t M, int64_t N, int64_t K, int32_t cus, bool packed) {
+    const double y_mb = (double)(M * N) * 4e-6, w_mb = (double)(N * K) * 2e-6;
+    const int64_t per_xcd = cus < 8 ? 1 : cus / 8;
+    /* A copy of more than 128 MiB is workspace that a stream holds for good: there the choice between the families stays what it was when N tiles were dealt to the XCDs in
+     * turn and the multiply took a fifth longer, so that more shapes do not start to ask for it (5120 x 13824, M = 3072: 344 us, 389-431 in the loop). */
+    const bool large = !packed && N * K * 2 > ((int64_t)128 << 20);
+    dense_plan best = {256, 256, 1, 1e300};
+    for (const dense_cost &c : k_dense_cost) {
+        if (!packed && c.bn != 256) continue;
+        const int64_t mt = (M + c.bm - 1) / c.bm, tiles = mt * ((N + c.bn - 1) / c.bn), slots = per_xcd * c.per_cu;
+        for (int sp = 1; sp <= (packed ? 8 : 4); sp *= 2) {
+            if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
+            if (tiles * sp > (1 << 22)) continue;                          /* a launch holds fewer than 2^32 threads */
+            const int64_t most = large ? (tiles / mt + 7) / 8 * mt * sp : (tiles * sp + 7) / 8;
+            const double share = (double)(tiles * sp) / (double)(8 * most) * (0.5 + 0.5 * (double)M / (double)(mt * c.bm));   /* rows of tiles past the end of X count half */
+            const double one = ((double)((K / 256 + sp - 1) / sp * 4) + c.prologue_steps) * c.step_us;
+            const auto round_us = [&](int64_t wgs) {                        /* a fuller chip runs at a lower clock */
+                if (!wgs) return 0.0;
+                const double u = ((wgs < per_xcd ? (double)wgs / (double)per_xcd : 1.0) * share - c.busy_from) / (1.0 - c.busy_from);
+                return one * (1.0 + c.clock * (u < 0.0 ? 0.0 : u > 1.0 ? 1.0 : u)) * (1.0 + c.shared * (double)((wgs + per_xcd - 1) / per_xcd - 1));
+            };
+            double t = c.base_us + (double)(most / slots) * round_us(slots) + round_us(most % slots) + c.y_us_per_mb * y_mb + c.w_us_per_mb * w_mb;
+            if (sp > 1) t += c.split_us + (0.2 + c.add_us_per_mb * sp) * y_mb;
+            if (large) t *= 1.2;
+            if (t < best.us) best = {c.bm, c.bn, sp, t};
         }
     }
-    return best + (with_unpack ? 4.46 + (double)N * (double)K * 1e-6 * k_unpack_us[format_index(qtype)] : 0.0);
+    return best;
 }
+static double unpack_estimate(int32_t qtype, int64_t N, int64_t K) { return 4.46 + (double)N * (double)K * 1e-6 * k_unpack_us[format_index(qtype)]; }
 
 extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit,
                                             int32_t *waves) {
@@ -1533,12 +1559,12 @@ static int32_t prefill_plan_any(int32_t qtype, int64_t M, int64_t N, int64_t K, 
     *waves = 4;
     const double best = plan_in_loop(qtype, M, N, K, cus, tile_m, tile_n, ksplit);
     if (allow_dense && M > 64) {
-        int sp = 1, bm = 256;
+        const dense_plan d = plan_dense(M, N, K, cus, false);
         /* (1.1 us in favour of a single launch, from the fit; 8 us cost 0.1 % on average) */
-        if (dense_estimate(qtype, M, N, K, cus, true, &bm, &sp) + 1.1 < best) {
-            *tile_m = bm;
-            *tile_n = 256;
-            *ksplit = sp;
+        if (d.us + unpack_estimate(qtype, N, K) + 1.1 < best) {
+            *tile_m = d.bm;
+            *tile_n = d.bn;
+            *ksplit = d.ksplit;
             *waves = 128;
         }
     }
@@ -1621,14 +1647,19 @@ static int32_t launch_thin(psn_module *mod, psn_stream *s, int32_t qtype, const 
     return launch(mod, s, name, (unsigned)((N + 16 * rt - 1) / (16 * rt) * ksplit), 512, (unsigned)lds, &a);
 }
 static int32_t launch_dense(psn_module *mod, psn_stream *s, const void *packed, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N, int64_t K,
-                            int32_t bm, int32_t ksplit) {
+                            int32_t bm, int32_t bn, int32_t ksplit) {
     int32_t rc;
     if (ksplit > 1 && (rc = fill_zero_y(mod, s, Y, M, N))) return rc;
-    const int64_t nt = (N + 255) / 256, mt = (M + bm - 1) / bm;
+    const int64_t nt = (N + bn - 1) / bn, mt = (M + bm - 1) / bm;
     psn_prefill_args a;
     prefill_args(&a, packed, X, Y, M, N, K, ksplit, K * 2);
-    /* LDS: a ring of four stages of X, bm rows x 32 k fp16 each */
-    return launch(mod, s, bm == 128 ? "psn_prefill_dense_f16_m128" : "psn_prefill_dense_f16", (unsigned)(8 * ((nt + 7) / 8) * mt * ksplit), 256, 4 * bm * 64, &a);
+    /* LDS: three stages of X (64 k) and four steps of W (32 k) with 256 columns, else a ring of four (64 x 64 tiles: five) stages of both */
+    const int lds = bn == 256 ? 3 * bm * 128 + 4 * bn * 64 : (bm + bn) * 128 * (bn == 64 ? 5 : 4);
+    if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: dense %dx%d tiles need %d bytes of LDS, device offers %d", bm, bn, lds, mod->ctx->max_lds);
+    char name[96];
+    if (bn == 256) snprintf(name, sizeof name, "psn_prefill_dense_f16%s", bm == 128 ? "_m128" : "");
+    else snprintf(name, sizeof name, "psn_prefill_dense_f16_m%d_n%d", bm, bn);
+    return launch(mod, s, name, (unsigned)((mt * nt * ksplit + 7) / 8 * 8), 512, (unsigned)lds, &a);
 }
 
 extern "C" int64_t psn_prefill_packed_bytes(int64_t N, int64_t K) {
@@ -1658,9 +1689,8 @@ extern "C" int32_t psn_qmatmul_prefill_packed(psn_module *mod, psn_stream *s, co
         (rc = need(Y, M * N * 4, "psn_qmatmul_prefill_packed", "Y")))
         return rc;
     if ((rc = bind(mod->ctx))) return rc;
-    int sp = 1, bm = 256;
-    (void)dense_estimate(PSN_Q4_0, M, N, K, mod->ctx->compute_units, false, &bm, &sp);
-    return launch_dense(mod, s, packed->p, X, Y, M, N, K, bm, sp);
+    const dense_plan d = plan_dense(M, N, K, mod->ctx->compute_units, true);
+    return launch_dense(mod, s, packed->p, X, Y, M, N, K, d.bm, d.bn, d.ksplit);
 }
 
 extern "C" int32_t psn_prefill_reserve(psn_stream *s, int64_t N, int64_t K) {
@@ -1687,7 +1717,7 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
         if ((rc = ensure_workspace(s, packed_bytes(N, K)))) return rc;
         if ((rc = note_workspace_use(s))) return rc;
         if ((rc = launch_unpack(mod, s, qtype, W->p, s->ws->p, N, K))) return rc;
-        return launch_dense(mod, s, s->ws->p, X, Y, M, N, K, bm, ksplit);
+        return launch_dense(mod, s, s->ws->p, X, Y, M, N, K, bm, bn, ksplit);
     }
     /* waves == 8 selects the thin kernels: tile_m (16 .. 64) rows of X, all of them, and tile_n (16, 32, 64) rows of W */
     if (waves == 8) {

@@ -5,11 +5,16 @@
 #ifndef PSN_PREFILL_COMMON_H
 #define PSN_PREFILL_COMMON_H
 
+#include "psn_args.h"
+#include "psn_device.h"
+
 #define UNROLL _Pragma("unroll")
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) char lds_char;
 
 /* An fp16 tile in LDS: rows of 128 bytes (64 k), the eight 16-byte chunks of a row stored at chunk ^ tile_swz(row).  A
  * fragment read takes the same chunk of 16 consecutive rows at a time: over the 64 banks (256 bytes) they must fall into
@@ -52,5 +57,67 @@ PSN_DEV void pf_affine4(u32 q, float d1, float m1, u32 &lo, u32 &hi) {
 }
 
 template <int N> struct pf_int { static constexpr int value = N; };
+template <int I, int N, class F> PSN_DEV void static_for(F &&f) {
+    if constexpr (I < N) {
+        f(pf_int<I>());
+        static_for<I + 1, N>(f);
+    }
+}
+
+/* Which tile and K range a workgroup takes (psn_prefill_pp.hip, psn_prefill_dense.hip).  Workgroups b, b + 8, ... share an XCD and its L2: each XCD gets one contiguous piece of the
+ * order "K range, ROWS rows of X, N tile, M tile within the rows", so that the 32 compute units of an XCD share a few panels of X and of W, and no XCD has more than one
+ * workgroup more than another (dealing N tiles to the XCDs in turn left 5120 columns in tiles of 256 with three tiles on four of them and two on the others). */
+struct prefill_place { int m0, n0, c0, chunks; };            /* corner of the tile; first 256-wide chunk of K and how many */
+template <int BM, int BN, int ROWS> PSN_DEV bool place_workgroup(const psn_prefill_args &a, prefill_place &p) {
+    constexpr int GROUP = ROWS / BM;
+    const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN, tiles = mt * nt, total = tiles * a.ksplit;
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, each = total >> 3, more = total & 7;
+    if (local >= each + (xcd < more)) return false;
+    const int idx = xcd * each + min(xcd, more) + local, split = idx / tiles, in = idx % tiles;
+    const int per = GROUP * nt, g = in / per, r = in % per, rows = min(GROUP, mt - g * GROUP);
+    p.m0 = (g * GROUP + r % rows) * BM;
+    p.n0 = r / rows * BN;
+    const int C = a.K >> 8, range = (C + a.ksplit - 1) / a.ksplit, c1 = min((split + 1) * range, C);
+    p.c0 = split * range;
+    p.chunks = c1 - p.c0;
+    return p.chunks > 0;                                     /* an empty K range adds nothing */
+}
+
+/* D = W X^T: lane (q, m) = (lane / 16, lane % 16) ends with rows 4 q .. 4 q + 3 of W for row m of X */
+PSN_DEV f32x4 mfma16(u32x4 w, u32x4 x, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, w), __builtin_bit_cast(half8_t, x), c, 0, 0, 0);
+}
+/* A wave's results of one row of MFMA tiles: lane (q, m) holds columns 16 j + 4 q .. + 3 of row m.  They go through LDS (16 rows of 16 TN + 4 words at `out`, this wave's own), so
+ * that an instruction touches whole runs of a row of Y: 16-byte pieces of it where rows are whole 16-byte words and nothing has to be added (stored straight from the
+ * MFMA's layout, 64 bytes of sixteen rows at a time: 4001 x 14336 x 4096 396 us instead of 389, 4001 x 1024 x 4096 on 256 x 256 tiles 87 instead of 78), else words: atomic adds
+ * from the MFMA's layout take several times as long (512 x 1024 x 4096 in four ranges, 64 x 128 tiles: 33.3 us instead of 13.5). */
+template <int TN> constexpr int wave_out_bytes() { return 16 * (16 * TN + 4) * 4; }
+template <int TN> PSN_DEV void store_tiles(const psn_prefill_args &a, int row0, int col0, int lane, const f32x4 (&v)[TN], u32 out) {
+    constexpr int PITCH = (16 * TN + 4) * 4;
+    UNROLL for (int j = 0; j < TN; ++j) lds_write128(out + (u32)((lane & 15) * PITCH + 64 * j + 16 * (lane >> 4)), __builtin_bit_cast(u32x4, v[j]));
+    lds_wait();
+    if (a.ksplit == 1 && (a.N & 3) == 0) {
+        u32x4 w[TN];
+        UNROLL for (int t = 0; t < TN; ++t) w[t] = lds_read128<0>(out + (u32)((t * 64 + lane) / (4 * TN) * PITCH + (t * 64 + lane) % (4 * TN) * 16));
+        lds_wait();
+        tie(w);
+        UNROLL for (int t = 0; t < TN; ++t) {
+            const int row = row0 + (t * 64 + lane) / (4 * TN), col = col0 + (t * 64 + lane) % (4 * TN) * 4;
+            if (row < a.M && col < a.N) *reinterpret_cast<u32x4 *>(a.Y + (int64_t)row * a.N + col) = w[t];
+        }
+        return;
+    }
+    u32 w[4 * TN];
+    UNROLL for (int t = 0; t < 4 * TN; ++t) w[t] = lds_read32(out + (u32)((t * 64 + lane) / (16 * TN) * PITCH + (t * 64 + lane) % (16 * TN) * 4));
+    lds_wait();
+    UNROLL for (int t = 0; t < 4 * TN; ++t) {
+        tie1(w[t]);
+        const int row = row0 + (t * 64 + lane) / (16 * TN), col = col0 + (t * 64 + lane) % (16 * TN);
+        if (row >= a.M || col >= a.N) continue;
+        float *y = a.Y + (int64_t)row * a.N + col;
+        if (a.ksplit == 1) *y = __uint_as_float(w[t]);
+        else unsafeAtomicAdd(y, __uint_as_float(w[t]));
+    }
+}
 
 #endif

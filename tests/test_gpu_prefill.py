@@ -484,3 +484,18 @@ def test_values_that_are_not_finite_stay_in_their_row_and_column(hip, orc, qname
         assert not np.isfinite(y[rows]).any() and not np.isfinite(y[:, cols]).any(), tile
         keep = np.ix_(np.setdiff1d(np.arange(m), rows), np.setdiff1d(np.arange(n), cols))
         assert np.isfinite(clean).all() and np.array_equal(clean[keep], y[keep]), tile
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (63, 65, 512), (64, 64, 2048), (65, 130, 768), (129, 127, 1280), (128, 1000, 2560), (257, 255, 256), (300, 2050, 512), (1025, 1021, 256),
+                                   (2049, 4100, 256)])
+def test_packed_multiply_at_tile_edges(hip, orc, m, n, k):
+    """Every tile of the multiply (64 x 64 .. 256 x 256; the planner takes the larger ones as the shape grows) a row and a column either side of its edges, odd row lengths of Y
+    (stored word by word), and K in several ranges.  Products are exact in fp32, so only the order of at most 2560 sums differs from the oracle: PARITY_TOL is far above 2560 * 2^-24."""
+    W = weights(orc, "Q4_K", 870, n, k)
+    X = G.seeded_acts(871 + m, m, k).astype(np.float16)
+    packed = hip.pack_for_prefill(hip.upload_weight(orc.Q4_K, W, n, k))
+    y = hip.upload(np.full((m, n), np.nan, np.float32))
+    say(f"packed multiply m={m} n={n} k={k}")
+    hip.quantized_matmul_packed(packed, hip.upload(X), y, m, n, k)
+    err = G.max_rel_err(y.download(np.float32, (m, n)), orc.prefill(orc.Q4_K, W, X, n, k))
+    assert err < PARITY_TOL, (m, n, k, err)
