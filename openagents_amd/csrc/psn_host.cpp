@@ -1633,8 +1633,9 @@ static void prefill_args(psn_prefill_args *a, const void *W, const psn_buf *X, p
 }
 static int32_t launch_thin(psn_module *mod, psn_stream *s, int32_t qtype, const psn_buf *W, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N,
                            int64_t K, int tm, int rt, int32_t ksplit) {
-    static const int lds_row[5] = {144, 272, 144, 176, 224};    /* a row's chunk in LDS */
-    const int rings = 8 * (16 * rt * lds_row[format_index(qtype)] + tm * 2048), sums = 8 * 1024 * rt * tm;
+    static const int lds_row[5] = {144, 272, 208, 240, 224};    /* a row's chunk in LDS, with the unpacked scales of Q4_K and Q5_K */
+    const int row = qtype == PSN_Q5_K && tm == 3 && rt == 4 ? 176 : lds_row[format_index(qtype)];      /* (no room for the scales there) */
+    const int rings = 8 * (16 * rt * row + tm * 2048), sums = 8 * 1024 * rt * tm;
     const int lds = rings > sums ? rings : sums;
     if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: %d x %d rows need %d bytes of LDS, device offers %d", 16 * tm, 16 * rt, lds, mod->ctx->max_lds);
     int32_t rc = bind(mod->ctx);

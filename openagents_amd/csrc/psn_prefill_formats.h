@@ -58,6 +58,40 @@ PSN_DEV void q0_finish(const half_done &t, u32 bias, u32 d2, u32 &o0, u32 &o1) {
  *      load() asks for everything the four steps of the chunk need (LOADS instructions); step J's bytes are two groups
  *      (HI = 0, 1) of NB weights, which belong at k = k_lo(part) and k_hi(part) of the 64-wide step; first() and second() turn
  *      word i of a group into four fp16, with the step's scales from scales0() and scales1().  SPREAD (for NB = 4, 8): row_of() in psn_prefill_pp.hip. ---- */
+/* Scales of Q4_K / Q5_K.  Unpacking the two sub-blocks of a 64-wide step costs twenty instructions, as much as decoding seven weights, and four threads share a row: each does
+ * it for one of the chunk's four steps (kq_pick: the fields of step j; kq_own: d, d', m, m').  Next to each other (pp kernels) they hand the values round by quad_perm in each step; as
+ * the four sixteens of lanes (FAR, thin kernels) through LDS, where the four floats of a step take the header's place in raw. */
+PSN_DEV void kq_pick(u32x4 header, int j, u32 &scales, u32 &mins) {
+    u32 sc[2], mn[2];
+    pf_kq_scales(header.y, header.z, header.w, sc, mn);
+    scales = ((j & 2) ? sc[1] : sc[0]) >> (16 * (j & 1));
+    mins = ((j & 2) ? mn[1] : mn[0]) >> (16 * (j & 1));
+}
+PSN_DEV void kq_own(u32x4 header, u32 scales, u32 mins, float (&own)[4]) {
+    const float d = h2f_lo(header.x), dm = h2f_hi(header.x);
+    own[0] = __fmul_rn(d, (float)(scales & 0xffu));
+    own[1] = __fmul_rn(d, (float)((scales >> 8) & 0xffu));
+    own[2] = __fmul_rn(dm, (float)(mins & 0xffu));
+    own[3] = __fmul_rn(dm, (float)((mins >> 8) & 0xffu));
+}
+template <int J> PSN_DEV float from_quad(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x55 * J, 0xf, 0xf, true)); }
+template <int J, bool FAR, class S> PSN_DEV void kq_scales0(u32x4 header, int part, S &s) {
+    if constexpr (FAR) { s.d[0] = __uint_as_float(header.x); s.d[1] = __uint_as_float(header.y); }
+    else if constexpr (J == 0) kq_pick(header, part & 3, s.sc, s.mn);
+    else { s.d[0] = from_quad<J>(s.own[0]); s.d[1] = from_quad<J>(s.own[1]); }
+}
+template <int J, bool FAR, class S> PSN_DEV void kq_scales1(u32x4 header, S &s) {
+    if constexpr (FAR) { s.m[0] = __uint_as_float(header.z); s.m[1] = __uint_as_float(header.w); }
+    else {
+        if constexpr (J == 0) {
+            kq_own(header, s.sc, s.mn, s.own);
+            s.d[0] = from_quad<J>(s.own[0]);
+            s.d[1] = from_quad<J>(s.own[1]);
+        }
+        s.m[0] = from_quad<J>(s.own[2]);
+        s.m[1] = from_quad<J>(s.own[3]);
+    }
+}
 struct PpQ4_K {
     static constexpr int BYTES = 144, LOADS = 5;
     template <int NB> struct raw { u32x4 h; typename raw_bytes<NB>::t q[4]; };
@@ -69,17 +103,9 @@ struct PpQ4_K {
     }
     template <int NB> static PSN_DEV void clear(raw<NB> &r) { r.h = (u32x4)(0u); UNROLL for (int j = 0; j < 4; ++j) r.q[j] = 0u; }
     template <int NB> static PSN_DEV void landed(raw<NB> &r) { raw_tie(r.h); UNROLL for (int j = 0; j < 4; ++j) raw_tie(r.q[j]); }
-    struct scale { float d[2], m[2]; };
-    template <int J, int NB, bool FAR = false> static PSN_DEV void scales0(const raw<NB> &r, int, scale &s) {
-        u32 sc[2], mn[2];
-        pf_kq_scales(r.h.y, r.h.z, r.h.w, sc, mn);
-        s.d[0] = pf_byte<2 * J>(sc); s.d[1] = pf_byte<2 * J + 1>(sc);
-        s.m[0] = pf_byte<2 * J>(mn); s.m[1] = pf_byte<2 * J + 1>(mn);
-    }
-    template <int NB> static PSN_DEV void scales1(const raw<NB> &r, scale &s) {
-        const float d = h2f_lo(r.h.x), dm = h2f_hi(r.h.x);
-        UNROLL for (int i = 0; i < 2; ++i) { s.d[i] = __fmul_rn(d, s.d[i]); s.m[i] = __fmul_rn(dm, s.m[i]); }
-    }
+    struct scale { float d[2], m[2]; u32 sc, mn; float own[4]; };
+    template <int J, int NB, bool FAR = false> static PSN_DEV void scales0(const raw<NB> &r, int part, scale &s) { kq_scales0<J, FAR>(r.h, part, s); }
+    template <int J, int NB, bool FAR = false> static PSN_DEV void scales1(const raw<NB> &r, scale &s) { kq_scales1<J, FAR>(r.h, s); }
     template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &r, const scale &, int i, half_done &t) { kq_floats((raw_word(r.q[J], i) >> (4 * HI)) & 0x0f0f0f0fu, t); }
     template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
     template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
@@ -98,17 +124,9 @@ struct PpQ5_K {
     }
     template <int NB> static PSN_DEV void clear(raw<NB> &r) { r.h = (u32x4)(0u); r.top = 0u; UNROLL for (int j = 0; j < 4; ++j) r.q[j] = 0u; }
     template <int NB> static PSN_DEV void landed(raw<NB> &r) { raw_tie(r.h); raw_tie(r.top); UNROLL for (int j = 0; j < 4; ++j) raw_tie(r.q[j]); }
-    struct scale { float d[2], m[2]; };
-    template <int J, int NB, bool FAR = false> static PSN_DEV void scales0(const raw<NB> &r, int, scale &s) {
-        u32 sc[2], mn[2];
-        pf_kq_scales(r.h.y, r.h.z, r.h.w, sc, mn);
-        s.d[0] = pf_byte<2 * J>(sc); s.d[1] = pf_byte<2 * J + 1>(sc);
-        s.m[0] = pf_byte<2 * J>(mn); s.m[1] = pf_byte<2 * J + 1>(mn);
-    }
-    template <int NB> static PSN_DEV void scales1(const raw<NB> &r, scale &s) {
-        const float d = h2f_lo(r.h.x), dm = h2f_hi(r.h.x);
-        UNROLL for (int i = 0; i < 2; ++i) { s.d[i] = __fmul_rn(d, s.d[i]); s.m[i] = __fmul_rn(dm, s.m[i]); }
-    }
+    struct scale { float d[2], m[2]; u32 sc, mn; float own[4]; };
+    template <int J, int NB, bool FAR = false> static PSN_DEV void scales0(const raw<NB> &r, int part, scale &s) { kq_scales0<J, FAR>(r.h, part, s); }
+    template <int J, int NB, bool FAR = false> static PSN_DEV void scales1(const raw<NB> &r, scale &s) { kq_scales1<J, FAR>(r.h, s); }
     template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &r, const scale &, int i, half_done &t) { kq_floats(((raw_word(r.q[J], i) >> (4 * HI)) & 0x0f0f0f0fu) | (((raw_word(r.top, i) >> (2 * J + HI)) & 0x01010101u) << 4), t); }
     template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
     template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
@@ -145,7 +163,7 @@ struct PpQ6_K {
         s.d[0] = (float)(int)(int8_t)(v & 0xffu);
         s.d[1] = (float)(int)(int8_t)((v >> 16) & 0xffu);
     }
-    template <int NB> static PSN_DEV void scales1(const raw<NB> &r, scale &s) {
+    template <int J, int NB, bool FAR = false> static PSN_DEV void scales1(const raw<NB> &r, scale &s) {
         const float d = h2f_lo(r.d);
         UNROLL for (int i = 0; i < 2; ++i) { s.d[i] = __fmul_rn(d, s.d[i]); s.m[i] = s.d[i] * 32.f; }
     }
@@ -197,7 +215,7 @@ struct PpQ4_0 {
         s.d = B::template scale<FAR>(raw_word(r.q[J], 0), part);
         UNROLL for (int i = 0; i < NB / 4; ++i) s.q[i] = __builtin_amdgcn_perm(raw_word(r.q[J], i + 1), raw_word(r.q[J], i), B::pick(part));
     }
-    template <int NB> static PSN_DEV void scales1(const raw<NB> &, scale &) {}
+    template <int J, int NB, bool FAR = false> static PSN_DEV void scales1(const raw<NB> &, scale &) {}
     template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &, const scale &s, int i, half_done &t) { q0_halves(s.q[i] >> (4 * HI), 0x640f640fu, t); }
     template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { q0_finish(t, 0x64086408u, s.d, o0, o1); }
     /* low nibbles first, high nibbles sixteen further on */
@@ -222,7 +240,7 @@ struct PpQ8_0 {
         s.d = B::template scale<FAR>(raw_word(r.q[J], 0), part);
         s.pick = B::pick(part);
     }
-    template <int NB> static PSN_DEV void scales1(const raw<NB> &, scale &) {}
+    template <int J, int NB, bool FAR = false> static PSN_DEV void scales1(const raw<NB> &, scale &) {}
     template <int J, int NB, int HI> static PSN_DEV void first(const raw<NB> &r, const scale &s, int i, half_done &t) {
         const int w = HI * (NB / 4) + i;
         const u32 next = w + 1 < NB / 2 ? raw_word(r.q[J], w + 1 < NB / 2 ? w + 1 : 0) : r.e[J];

@@ -133,7 +133,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
         if constexpr (P == 0) {
             WF::template scales0<J, NB>(w, part, wscale);
         } else if constexpr (P == 1) {
-            WF::template scales1<NB>(w, wscale);
+            WF::template scales1<J, NB>(w, wscale);
         } else {
             constexpr int WORD = (P - 2) >> 1, HI = WORD / NW, I = WORD % NW, B = 2 * I;
             if constexpr ((P & 1) == 0) {

@@ -11,10 +11,12 @@
  *     it at 14336 x 4096), W a whole chunk ahead, X one to four steps of 64 ahead, in registers;
  *   - put into LDS behind the wave's own earlier reads (lds_order() keeps them there), read back as MFMA
  *     operands, W's raw bytes one tile ahead of their decode.
+ * Q4_K, Q5_K: a lane unpacks the scales of one of the chunk's four steps for its row and hands them to the row's other lanes through LDS (a sixth of the vector
+ * instructions; 14336 x 4096, M = 16: Q4_K 13.6 -> 13.1 us, Q5_K 14.9 -> 14.1; M = 48: Q4_K 18.8 -> 18.0).
  * The loop has one body: past the last chunk every lane asks for the start of the buffer, which costs no traffic.
  *
  * What bounds it: a weight costs about four vector instructions (fp32 d * q - m per weight, then the rounding to fp16), which
- * is 8 us of a 14336 x 4096 launch over all SIMDs, and X, which every workgroup reads whole (RT trades it against workgroups).
+ * is 7 us of a 14336 x 4096 launch over all SIMDs, and X, which every workgroup reads whole (RT trades it against workgroups).
  * Two chunks of W on their way instead of one changed nothing (-1 .. +4 %), nor did more of X.  Against the 64 x 64 kernel
  * (psn_prefill.hip), us: Q4_K 4096 x 4096 M = 16 11.4 -> 6.5, M = 33 12.2 -> 9.6, M = 64 13.9 -> 11.3; 1024 x 4096 M = 16 8.8 -> 5.3,
  * M = 48 9.4 -> 6.6; 14336 x 4096 M = 16 21.7 -> 15.1, M = 48 22.4 -> 20.8; 4096 x 14336 M = 16 22.2 -> 16.5.  At 64 rows of a large
@@ -32,17 +34,17 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 template <typename WF> struct Feed;
 template <> struct Feed<PpQ4_K> {
     typedef PpQ4_K::raw<8> raw;
-    static constexpr int WORDS = 9, STRIDE = 144;
-    template <int J> static PSN_DEV void read(const lds_u8 *row, int g, raw &r) {
-        fetch<16>(row, r.h);
+    static constexpr int WORDS = 9, STRIDE = 144, SCALES = 1024;
+    template <int J, bool SHARED> static PSN_DEV void read(const lds_u8 *row, const lds_u8 *scales, int g, raw &r) {
+        fetch<16>(SHARED ? scales + 256 * J : row, r.h);
         fetch<8>(row + 8 * g + (16 + 32 * J), r.q[J]);
     }
 };
 template <> struct Feed<PpQ5_K> {
     typedef PpQ5_K::raw<8> raw;
-    static constexpr int WORDS = 11, STRIDE = 176;
-    template <int J> static PSN_DEV void read(const lds_u8 *row, int g, raw &r) {
-        fetch<16>(row, r.h);
+    static constexpr int WORDS = 11, STRIDE = 176, SCALES = 1024;
+    template <int J, bool SHARED> static PSN_DEV void read(const lds_u8 *row, const lds_u8 *scales, int g, raw &r) {
+        fetch<16>(SHARED ? scales + 256 * J : row, r.h);
         fetch<8>(row + 8 * g + 16, r.top);
         fetch<8>(row + 8 * g + (48 + 32 * J), r.q[J]);
     }
@@ -51,8 +53,8 @@ template <> struct Feed<PpQ5_K> {
  * starts two bytes late, and its d */
 template <> struct Feed<PpQ6_K> {
     typedef PpQ6_K::raw<8> raw;
-    static constexpr int WORDS = 13, STRIDE = 224;
-    template <int J> static PSN_DEV void read(const lds_u8 *row, int g, raw &r) {
+    static constexpr int WORDS = 13, STRIDE = 224, SCALES = 0;
+    template <int J, bool> static PSN_DEV void read(const lds_u8 *row, const lds_u8 *, int g, raw &r) {
         constexpr int H = J >> 1;
         const lds_u8 *const p = row + 8 * g;
         fetch<4>(p + 64 * H, r.ql[2 * H]);
@@ -65,13 +67,13 @@ template <> struct Feed<PpQ6_K> {
 };
 template <> struct Feed<PpQ4_0> {
     typedef PpQ4_0::raw<8> raw;
-    static constexpr int WORDS = 9, STRIDE = 144;
-    template <int J> static PSN_DEV void read(const lds_u8 *row, int g, raw &r) { fetch<4>(row + 8 * g + 36 * J, r.q[J]); }
+    static constexpr int WORDS = 9, STRIDE = 144, SCALES = 0;
+    template <int J, bool> static PSN_DEV void read(const lds_u8 *row, const lds_u8 *, int g, raw &r) { fetch<4>(row + 8 * g + 36 * J, r.q[J]); }
 };
 template <> struct Feed<PpQ8_0> {
     typedef PpQ8_0::raw<8> raw;
-    static constexpr int WORDS = 17, STRIDE = 272;
-    template <int J> static PSN_DEV void read(const lds_u8 *row, int g, raw &r) {
+    static constexpr int WORDS = 17, STRIDE = 272, SCALES = 0;
+    template <int J, bool> static PSN_DEV void read(const lds_u8 *row, const lds_u8 *, int g, raw &r) {
         fetch<4>(row + 16 * g + 68 * J, r.q[J]);
         fetch<4>(row + 16 * g + (68 * J + 16), r.e[J]);
     }
@@ -85,7 +87,9 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
     constexpr int XD = RT * TM <= 3 ? 4 : RT * TM <= 8 ? 2 : 1;   /* steps of X on their way */
     constexpr bool AHEAD = TM * (RT + 2) < (BIG ? 16 : 24);       /* registers for the next step's fragments of X */
     constexpr int NI = (16 * F::WORDS + 63) / 64;           /* load instructions per 16 rows and chunk */
-    constexpr int WTILE = 16 * F::STRIDE, MINE = RT * WTILE + TM * 2048;
+    constexpr int WTILE = 16 * F::STRIDE, SHARED_BYTES = RT * (WTILE + F::SCALES) + TM * 2048;
+    constexpr bool SHARED = F::SCALES != 0 && 8 * SHARED_BYTES <= 160 * 1024;             /* (Q5_K's 48 rows of X by 64 of W are too large) */
+    constexpr int MINE = SHARED ? SHARED_BYTES : RT * WTILE + TM * 2048;
     extern __shared__ uint4 psn_smem[];
     const int tid = threadIdx.x, lane = tid & 63, row = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -100,7 +104,7 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
     const int rot = (int)((blockIdx.x * 5u) % (unsigned)nq);
     auto chunk_of = [&](int i) { const int r = i + rot; return c_begin + (r >= nq ? r - nq : r); };
 
-    lds_u8 *const wl = (lds_u8 *)(__attribute__((address_space(3))) void *)psn_smem + wave * MINE, *const xl = wl + RT * WTILE;
+    lds_u8 *const wl = (lds_u8 *)(__attribute__((address_space(3))) void *)psn_smem + wave * MINE, *const xl = wl + RT * WTILE, *const sl = xl + TM * 2048;
 
     float4_t acc[RT][TM];
     UNROLL for (int t = 0; t < RT; ++t) UNROLL for (int i = 0; i < TM; ++i) acc[t][i] = (float4_t)(0.f);
@@ -146,6 +150,19 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
             }
         }
         lds_order();
+        if constexpr (SHARED) {                             /* lane (g, row): the scales of step g */
+            u32x4 header[RT];
+            UNROLL for (int t = 0; t < RT; ++t) fetch<16>((const lds_u8 *)(wl + t * WTILE + row * F::STRIDE), header[t]);
+            lds_order();
+            UNROLL for (int t = 0; t < RT; ++t) {
+                u32 sc, mn;
+                float own[4];
+                kq_pick(header[t], g, sc, mn);
+                kq_own(header[t], sc, mn, own);
+                store<16>(sl + t * F::SCALES + lane * 16, (f32x4){own[0], own[1], own[2], own[3]});
+            }
+            lds_order();
+        }
     };
 
     /* X: eight rows of 128 bytes per instruction */
@@ -178,7 +195,7 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
         __builtin_amdgcn_sched_barrier(0);
     };
     typename F::raw r[2];
-    const lds_u8 *const wrow = wl + row * F::STRIDE;
+    const lds_u8 *const wrow = wl + row * F::STRIDE, *const srow = sl + row * 16;
     /* step J of chunk c; `more`: chunk `next` follows.  What a tile's decode needs is read from LDS one tile, X one step ahead. */
     auto step = [&](int c, int next, bool more, auto jc) {
         constexpr int J = decltype(jc)::value;
@@ -186,15 +203,22 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
         else if constexpr (J < 3) stage_x(c, next, more, pf_int<(J + 1) & 3>());
         UNROLL for (int t = 0; t < RT; ++t) {
             typename F::raw &now = r[(J * RT + t) & 1], &then = r[(J * RT + t + 1) & 1];
-            if (t + 1 < RT) F::template read<J>(wrow + (t + 1) * WTILE, g, then);
-            else if constexpr (J < 3) F::template read<(J + 1) & 3>(wrow, g, then);
+            if (t + 1 < RT) F::template read<J, SHARED>(wrow + (t + 1) * WTILE, srow + (t + 1) * F::SCALES, g, then);
+            else if constexpr (J < 3) F::template read<(J + 1) & 3, SHARED>(wrow, srow, g, then);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (ODD) now.pick = ((u32)nb[t] * (u32)a.row_bytes + (u32)(c * WF::BYTES) + rowoff) & 2u ? 0x05040302u : 0x03020100u;
             u32 lo[4], hi[4];
             typename WF::scale s;
             half_done h;
+            if constexpr (F::SCALES != 0 && !SHARED) {
+                u32 sc, mn;
+                float own[4];
+                kq_pick(now.h, J, sc, mn);
+                kq_own(now.h, sc, mn, own);
+                now.h = __builtin_bit_cast(u32x4, (f32x4){own[0], own[1], own[2], own[3]});
+            }
             WF::template scales0<J, 8, true>(now, g, s);
-            WF::template scales1<8>(now, s);
+            WF::template scales1<J, 8, true>(now, s);
             UNROLL for (int i = 0; i < 2; ++i) {
                 WF::template first<J, 8, 0>(now, s, i, h);
                 WF::template second<0>(s, h, lo[2 * i], lo[2 * i + 1]);
@@ -223,7 +247,7 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
             put_w();
             __builtin_amdgcn_sched_barrier(0);
             load_w(next, more);
-            F::template read<0>(wrow, g, r[0]);
+            F::template read<0, SHARED>(wrow, srow, g, r[0]);
             if constexpr (AHEAD) stage_x(c, next, more, pf_int<0>());
             __builtin_amdgcn_sched_barrier(0);
             step(c, next, more, pf_int<0>());
