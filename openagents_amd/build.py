@@ -42,6 +42,7 @@ CODE_OBJECTS = [
     *[(f"psn_pf_{fmt}_base", "psn_prefill.hip", ["-DPSN_BUILD_ONLY", "-DPSN_BUILD_PF=4", f"-DPSN_BUILD_PF_{fmt.upper()}"])
       for fmt in ("q4_K", "q5_K", "q6_K")],
     *[(f"psn_pp_{fmt}", "psn_prefill_pp.hip", [f"-DPSN_BUILD_PP_{fmt.upper()}"]) for fmt in ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K")],
+    *[(f"psn_fr_{fmt}", "psn_prefill_frag.hip", [f"-DPSN_BUILD_FR_{fmt.upper()}"]) for fmt in ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K")],
     *[(f"psn_th_{fmt}", "psn_prefill_thin.hip", [f"-DPSN_BUILD_TH_{fmt.upper()}"]) for fmt in ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K")],
     ("psn_decode", "psn_decode.hip", []),
     ("psn_calib", "psn_calib.hip", []),

@@ -1377,94 +1377,86 @@ static int32_t check_prefill(const char *what, psn_module *mod, psn_stream *s, i
     return PSN_OK;
 }
 
-/* Cost models of family 4 (psn_prefill_pp.hip) and of the dense family, fitted to launches timed on MI355X: five formats, 28 matrices (1000 x 2560,
- * 512 x 4096 .. 32000 x 4096), M = 65 .. 4096, 33348 launches of family 4 and 13760 of the dense one.  Weight lies on plans near the fastest, whose
- * estimates are off by 4-6 % rms; what they pick is 0.4 % off the fastest plan of any family on average over 2315 shapes and more than 10 % off in 3.
+/* Cost models of family 4 (psn_prefill_frag.hip, psn_prefill_pp.hip) and of the dense family, fitted to launches timed on MI355X.  Family 4 and the dense family against each other: five
+ * formats, 14 matrices (1000 x 2560, 2048 x 2048 .. 32000 x 4096), M = 65 .. 4096, 13135 calls, zero fill and dequantization pass included; weight lies on plans near the
+ * fastest, whose estimates are off by 4 % rms; what they pick is 0.4 % off the fastest plan on average over 910 shapes and more than 10 % off in 11.
  *
- * Both families deal N tiles to the eight XCDs in turn and give an XCD all M tiles and K ranges of its own, so that the XCDs with one N tile
- * more set the rounds of workgroups: 5120 columns are 20 tiles of 256, three for four of the XCDs, whose 36 workgroups at M = 3072 take
- * two rounds on 32 compute units (Q4_K: dense 689 us; 256 x 128 tiles, five for each XCD, 467).  A round in which nearly every compute unit multiplies rows
- * of its own (those past the end repeat the last one) runs at a lower clock than an emptier one (8192 x 8192 M = 2048, two full rounds: 1.2 x the
- * step cost of half-filled ones). */
+ * Both families deal tiles evenly to the eight XCDs: rounds of workgroups on the XCD with most of them x (K steps + prologue) x a step cost per tile and format; a round in which nearly
+ * every compute unit multiplies rows of its own (those past the end repeat the last one, and count half) runs at a lower clock than an emptier one; workgroups that share a
+ * compute unit slow each other down; then the store of Y, the weights from memory, and with K cut the zero fill and the adds. */
 static int format_index(int32_t t) { return t == PSN_Q4_0 ? 0 : t == PSN_Q8_0 ? 1 : t == PSN_Q4_K ? 2 : t == PSN_Q5_K ? 3 : 4; }
-struct prefill_rounds {
-    int64_t per_xcd;        /* workgroups of an XCD with the most N tiles */
-    double share;           /* workgroups of all XCDs over eight times that; rows of tiles past the end of X count half */
-    int xcd_cus;
-    prefill_rounds(int64_t M, int64_t N, int bm, int bn, int sp, int32_t cus) : xcd_cus(cus < 8 ? 1 : cus / 8) {
-        const int64_t mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn, most = (nt + 7) / 8;
-        per_xcd = most * mt * sp;
-        share = (double)nt / (double)(8 * most) * (0.5 + 0.5 * (double)M / (double)(mt * bm));
-    }
-    double busy(double clock, int64_t wgs) const {                 /* the clock's part of a round of wgs workgroups per XCD */
-        const double filled = (wgs < xcd_cus ? (double)wgs / xcd_cus : 1.0) * share, u = (filled - 0.7) / 0.2;
-        return 1.0 + clock * (u < 0.0 ? 0.0 : u > 1.0 ? 1.0 : u);
-    }
-};
-/* plans that cut K come out too low where all ranges of an element add at the same moment (Q8_0 4096 x 4096 M = 128 in four: 26.9 us, 20.2 by the
- * rest of the model) */
-static double cut_bias(double per_doubling, int sp) { return 1.0 + per_doubling * (sp >= 8 ? 3 : sp >= 4 ? 2 : sp >= 2 ? 1 : 0); }
+struct tile_cost { double base_us, clock, busy_from, shared, prologue_steps, split_us, add_us_per_mb, y_us_per_mb, w_us_per_million; };     /* steps of 64 of K */
+static double tile_estimate(const tile_cost &c, double step_us, int64_t M, int64_t N, int64_t K, int bm, int bn, int sp, int per_cu, int32_t cus, bool in_turn) {
+    const double y_mb = (double)(M * N) * 4e-6;
+    const int64_t per_xcd = cus < 8 ? 1 : cus / 8, mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn, slots = per_xcd * per_cu;
+    const int64_t most = in_turn ? (nt + 7) / 8 * mt * sp : (mt * nt * sp + 7) / 8;
+    const double share = (double)(mt * nt * sp) / (double)(8 * most) * (0.5 + 0.5 * (double)M / (double)(mt * bm));
+    const double one = ((double)((K / 256 + sp - 1) / sp * 4) + c.prologue_steps) * step_us;
+    const auto round_us = [&](int64_t wgs) {
+        if (!wgs) return 0.0;
+        const double u = ((wgs < per_xcd ? (double)wgs / (double)per_xcd : 1.0) * share - c.busy_from) / (1.0 - c.busy_from);
+        return one * (1.0 + c.clock * (u < 0.0 ? 0.0 : u > 1.0 ? 1.0 : u)) * (1.0 + c.shared * (double)((wgs + per_xcd - 1) / per_xcd - 1));
+    };
+    const double t = c.base_us + (double)(most / slots) * round_us(slots) + round_us(most % slots) + c.y_us_per_mb * y_mb + c.w_us_per_million * (double)(N * K) * 1e-6;
+    return sp > 1 ? t + c.split_us + (0.2 + c.add_us_per_mb * sp) * y_mb : t;
+}
 
-/* Family 4: base + rounds x (K steps + prologue) x step cost, workgroups that share a compute unit slowing each other down by `shared` each, the
- * store of Y, and with K cut the zero fill and the atomic adds.  per_cu: workgroups a compute unit holds by LDS and registers, per_cu_q6_K of Q6_K's
- * kernel. */
+/* LDS of family 4's eight-wave kernels.  256 rows (psn_prefill_pp.hip): a ring of four stages of X and two fp16 weight tiles, 128 bytes per row.  Fewer
+ * (psn_prefill_frag.hip): two stages of X of 256 bytes per row, two chunks of the weight rows in 1 KB pieces and one piece that nobody reads, Q6_K's last words of a row apart,
+ * the unpacked scales of Q4_K and Q5_K. */
+static int in_loop_lds(int32_t qtype, int bm, int bn) {
+    static const int words[5] = {9, 17, 9, 11, 13};
+    const int f = format_index(qtype);
+    if (bm == 256) return (4 * bm + 2 * bn) * 128;
+    return 2 * (bm * 256 + ((bn * words[f] + 63) / 64 + 1) * 1024 + (f == 4 ? bn * 8 : 0)) + (f == 2 || f == 3 ? bn * 64 : 0);
+}
+/* Family 4.  per_cu: workgroups a compute unit holds by its registers, per_cu_q6_K of Q6_K's kernel. */
 struct prefill_cost {
     int tile, per_cu, per_cu_q6_K;    /* index into k_prefill_tiles */
-    double base_us, shared, y_us_per_mb, add_us_per_mb[2], split_us, prologue_steps, clock;   /* adds: K in two, in four and more */
+    tile_cost cost;
     double step_us[5];                /* per 64 of K: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
 };
 static const prefill_cost k_prefill_cost[] = {
-    {0, 3, 2, 3.59, 0.690, 0.296, {0.465, 0.465}, 2.14, 0.20, 0.021, {0.290, 0.372, 0.304, 0.314, 0.387}},
-    {1, 1, 1, 3.21, 0.000, 0.128, {0.658, 0.658}, 1.12, 2.29, 0.045, {0.426, 0.597, 0.470, 0.525, 0.577}},
-    {2, 1, 1, 3.52, 0.000, 0.222, {0.613, 0.613}, 1.19, 2.45, 0.209, {0.503, 0.659, 0.546, 0.566, 0.619}},
-    {4, 1, 1, 3.25, 0.000, 0.263, {0.580, 0.760}, 2.55, 0.55, 0.269, {0.743, 0.862, 0.794, 0.788, 0.818}},
+    {0, 2, 2, {3.51, 0.194, 0.296, 0.667, 5.44, 1.90, 0.449, 0.109, 0.0082}, {0.176, 0.214, 0.200, 0.214, 0.226}},
+    {1, 2, 1, {4.17, 0.172, 0.160, 0.798, 4.28, 1.90, 0.520, 0.093, 0.0073}, {0.255, 0.319, 0.288, 0.329, 0.409}},
+    {2, 1, 1, {3.22, 0.224, 0.511, 0.100, 7.83, 1.90, 0.533, 0.112, 0.0125}, {0.354, 0.420, 0.387, 0.409, 0.481}},
+    {4, 1, 1, {3.83, 0.187, 0.630, 0.100, 5.90, 2.19, 0.544, 0.042, 0.0199}, {0.702, 0.806, 0.757, 0.782, 0.814}},
 };
-/* The dense family (psn_prefill_dense.hip): one pass that rewrites the matrix as fp16 (none when the caller holds packed weights) and the multiply, whose tiles are dealt evenly
- * to the XCDs.  Fitted to 3175 launches of the multiply (18 matrices, M = 16 .. 4096, K in one to eight ranges): what the estimates pick among the five tiles is 0.5 % off the
- * fastest on average and more than 10 % off in 2 of 262 shapes.  The tiles below 256 columns are for packed weights only (explicit plans cannot name them, and a plan of
- * psn_qmatmul_prefill is one that can be run explicitly). */
-static const struct dense_cost {
-    int bm, bn, per_cu;
-    double base_us, step_us, clock, busy_from, shared, prologue_steps, split_us, add_us_per_mb, y_us_per_mb, w_us_per_mb;     /* steps of 64 of K */
-} k_dense_cost[] = {
-    {256, 256, 1, 2.04, 1.038, 0.232, 0.688, 0.016, 9.23, 3.60, 0.54, 0.026, 0.008},
-    {128, 256, 1, 2.23, 0.455, 0.639, 0.328, 0.890, 7.57, 2.04, 0.54, 0.021, 0.050},
-    {128, 128, 1, 2.15, 0.258, 0.696, 0.318, 0.014, 9.71, 2.01, 0.45, 0.006, 0.042},
-    {64, 128, 1, 2.04, 0.179, 0.379, 0.198, 0.014, 8.71, 2.02, 0.43, 0.036, 0.066},
-    {64, 64, 2, 2.60, 0.135, 0.180, 0.442, 0.981, 2.28, 1.98, 0.50, 0.192, 0.057},
+/* The dense family (psn_prefill_dense.hip) behind a pass that rewrites the matrix as fp16, and over packed weights: there all five tiles, fitted to 3175 launches of
+ * the multiply alone (18 matrices, M = 16 .. 4096; what the estimates pick is 0.7 % off the fastest on average, more than 10 % off in 4 of 262 shapes).  The tiles below 256
+ * columns are for packed weights only: explicit plans cannot name them, and a plan of psn_qmatmul_prefill is one that can be run explicitly. */
+struct dense_cost { int bm, bn, per_cu; tile_cost cost; double step_us; };
+static const dense_cost k_dense_cost[] = {
+    {256, 256, 1, {2.38, 0.430, 0.673, 0.016, 4.04, 4.03, 0.462, 0.126, 0.0791}, 0.920},
+    {128, 256, 1, {2.11, 0.517, 0.627, 0.890, 1.85, 4.32, 0.417, 0.162, 0.0058}, 0.512},
 };
-static const double k_unpack_us[5] = {0.427, 0.778, 0.460, 0.375, 0.519};      /* per million weights, from the fit */
+static const dense_cost k_packed_cost[] = {
+    {256, 256, 1, {2.04, 0.232, 0.688, 0.016, 9.23, 3.60, 0.543, 0.026, 0.0170}, 1.038},
+    {128, 256, 1, {2.23, 0.639, 0.328, 0.890, 7.57, 2.04, 0.539, 0.021, 0.0992}, 0.455},
+    {128, 128, 1, {2.15, 0.696, 0.318, 0.014, 9.71, 2.01, 0.452, 0.006, 0.0842}, 0.258},
+    {64, 128, 1, {2.04, 0.379, 0.198, 0.014, 8.71, 2.02, 0.434, 0.036, 0.1321}, 0.179},
+    {64, 64, 2, {2.60, 0.180, 0.442, 0.981, 2.28, 1.98, 0.499, 0.192, 0.1146}, 0.135},
+};
+static const double k_unpack_base_us = 7.03, k_unpack_us[5] = {0.400, 0.554, 0.385, 0.427, 0.530};      /* per million weights */
 struct dense_plan { int bm, bn, ksplit; double us; };
 static dense_plan plan_dense(int64_t M, int64_t N, int64_t K, int32_t cus, bool packed) {
-    const double y_mb = (double)(M * N) * 4e-6, w_mb = (double)(N * K) * 2e-6;
-    const int64_t per_xcd = cus < 8 ? 1 : cus / 8;
     /* A copy of more than 128 MiB is workspace that a stream holds for good: there the choice between the families stays what it was when N tiles were dealt to the XCDs in
-     * turn and the multiply took a fifth longer, so that more shapes do not start to ask for it (5120 x 13824, M = 3072: 344 us, 389-431 in the loop). */
-    const bool large = !packed && N * K * 2 > ((int64_t)128 << 20);
+     * turn, so that shapes whose tiles come out uneven do not start to ask for it (5120 x 13824, M = 3072: 344 us, 389-428 in the loop). */
+    const bool in_turn = !packed && N * K * 2 > ((int64_t)128 << 20);
     dense_plan best = {256, 256, 1, 1e300};
-    for (const dense_cost &c : k_dense_cost) {
-        if (!packed && c.bn != 256) continue;
-        const int64_t mt = (M + c.bm - 1) / c.bm, tiles = mt * ((N + c.bn - 1) / c.bn), slots = per_xcd * c.per_cu;
+    const dense_cost *const from = packed ? k_packed_cost : k_dense_cost, *const to = packed ? k_packed_cost + 5 : k_dense_cost + 2;
+    for (const dense_cost *c = from; c != to; ++c) {
+        const int64_t tiles = (M + c->bm - 1) / c->bm * ((N + c->bn - 1) / c->bn);
         for (int sp = 1; sp <= (packed ? 8 : 4); sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
             if (tiles * sp > (1 << 22)) continue;                          /* a launch holds fewer than 2^32 threads */
-            const int64_t most = large ? (tiles / mt + 7) / 8 * mt * sp : (tiles * sp + 7) / 8;
-            const double share = (double)(tiles * sp) / (double)(8 * most) * (0.5 + 0.5 * (double)M / (double)(mt * c.bm));   /* rows of tiles past the end of X count half */
-            const double one = ((double)((K / 256 + sp - 1) / sp * 4) + c.prologue_steps) * c.step_us;
-            const auto round_us = [&](int64_t wgs) {                        /* a fuller chip runs at a lower clock */
-                if (!wgs) return 0.0;
-                const double u = ((wgs < per_xcd ? (double)wgs / (double)per_xcd : 1.0) * share - c.busy_from) / (1.0 - c.busy_from);
-                return one * (1.0 + c.clock * (u < 0.0 ? 0.0 : u > 1.0 ? 1.0 : u)) * (1.0 + c.shared * (double)((wgs + per_xcd - 1) / per_xcd - 1));
-            };
-            double t = c.base_us + (double)(most / slots) * round_us(slots) + round_us(most % slots) + c.y_us_per_mb * y_mb + c.w_us_per_mb * w_mb;
-            if (sp > 1) t += c.split_us + (0.2 + c.add_us_per_mb * sp) * y_mb;
-            if (large) t *= 1.2;
-            if (t < best.us) best = {c.bm, c.bn, sp, t};
+            const double t = tile_estimate(c->cost, c->step_us, M, N, K, c->bm, c->bn, sp, c->per_cu, cus, in_turn);
+            if (t < best.us) best = {c->bm, c->bn, sp, t};
         }
     }
     return best;
 }
-static double unpack_estimate(int32_t qtype, int64_t N, int64_t K) { return 4.46 + (double)N * (double)K * 1e-6 * k_unpack_us[format_index(qtype)]; }
+static double unpack_estimate(int32_t qtype, int64_t N, int64_t K) { return k_unpack_base_us + (double)N * (double)K * 1e-6 * k_unpack_us[format_index(qtype)]; }
 
 extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit,
                                             int32_t *waves) {
@@ -1522,22 +1514,13 @@ static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N
 }
 /* family 4: the tile and the K split with the smallest estimate; K ranges hold at least two 256-wide chunks */
 static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
-    const int f = format_index(qtype);
-    const double y_mb = (double)(M * N) * 4e-6;
     double best = 1e300;
     for (const prefill_cost &c : k_prefill_cost) {
         const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
+        const int by_regs = qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu, by_lds = 160 * 1024 / in_loop_lds(qtype, bm, bn);
         for (int sp = 1; sp <= 8; sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
-            const prefill_rounds r(M, N, bm, bn, sp, cus);
-            const int64_t slots = (int64_t)r.xcd_cus * (qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu);
-            const double one = ((double)((K / 256 + sp - 1) / sp * 4) + c.prologue_steps) * c.step_us[f];
-            const auto round_us = [&](int64_t wgs) {
-                return wgs ? one * (1.0 + c.shared * (double)((wgs + r.xcd_cus - 1) / r.xcd_cus - 1)) * r.busy(c.clock, wgs) : 0.0;
-            };
-            double t = c.base_us + (double)(r.per_xcd / slots) * round_us(slots) + round_us(r.per_xcd % slots) + c.y_us_per_mb * y_mb;
-            if (sp > 1) t += c.split_us + c.add_us_per_mb[sp >= 4] * y_mb * sp;
-            t *= cut_bias(0.020, sp);
+            const double t = tile_estimate(c.cost, c.step_us[format_index(qtype)], M, N, K, bm, bn, sp, by_regs < by_lds ? by_regs : by_lds, cus, false);
             if (t < best) { best = t; *tile_m = bm; *tile_n = bn; *ksplit = sp; }
         }
     }
@@ -1560,7 +1543,7 @@ static int32_t prefill_plan_any(int32_t qtype, int64_t M, int64_t N, int64_t K, 
     const double best = plan_in_loop(qtype, M, N, K, cus, tile_m, tile_n, ksplit);
     if (allow_dense && M > 64) {
         const dense_plan d = plan_dense(M, N, K, cus, false);
-        /* (1.1 us in favour of a single launch, from the fit; 8 us cost 0.1 % on average) */
+        /* (1.1 us in favour of a single launch, as in the fit) */
         if (d.us + unpack_estimate(qtype, N, K) + 1.1 < best) {
             *tile_m = d.bm;
             *tile_n = d.bn;
@@ -1753,9 +1736,8 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
      * 8 x 16 KB reduction */
     const int skinny_rings = 3 * 32768 + (qtype == PSN_Q4_0 || qtype == PSN_Q4_K ? 6 * 64 * 144 : qtype == PSN_Q5_K ? 5 * 64 * 176 : qtype == PSN_Q6_K ? 4 * 64 * 240 : 3 * 64 * 304);
     const int wide_rings = 3 * (32768 + 256 * (qtype == PSN_Q4_0 ? 36 : 68));   /* three stages of X (256 rows x 64 k) and of raw blocks (two per row) */
-    /* the eight-wave kernels: a ring of four stages of X and two fp16 weight tiles, 128 bytes per row */
     const bool pp = waves == 4 && bn <= 128;
-    const int lds = pp ? (4 * bm + 2 * bn) * 128 : skinny ? (skinny_rings > 8 * 16384 ? skinny_rings : 8 * 16384) : wide ? wide_rings : waves == 16 ? 0 : 2 * (bm + bn) * 128;
+    const int lds = pp ? in_loop_lds(qtype, bm, bn) : skinny ? (skinny_rings > 8 * 16384 ? skinny_rings : 8 * 16384) : wide ? wide_rings : waves == 16 ? 0 : 2 * (bm + bn) * 128;
     if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: tile %dx%d needs %d bytes of LDS, device offers %d", bm, bn, lds, mod->ctx->max_lds);
     if ((rc = bind(mod->ctx))) return rc;
     if (ksplit > 1 && (rc = fill_zero_y(mod, s, Y, M, N))) return rc;
@@ -1767,7 +1749,8 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
         snprintf(name, sizeof name, "psn_prefill_%s_skinny", fmt_name(qtype));
         return launch(mod, s, name, (unsigned)(nt * ksplit), 512, (unsigned)lds, &a);
     }
-    const int64_t blocks = 8 * ((nt + 7) / 8) * mt * ksplit;      /* the kernel spreads N tiles over 8 XCDs */
+    /* the eight-wave kernels spread workgroups evenly over the 8 XCDs, the others N tiles */
+    const int64_t blocks = pp ? (nt * mt * ksplit + 7) / 8 * 8 : 8 * ((nt + 7) / 8) * mt * ksplit;
     if (wide) {
         snprintf(name, sizeof name, "psn_prefill_%s_wide", fmt_name(qtype));
         return launch(mod, s, name, (unsigned)blocks, 256, (unsigned)lds, &a);

@@ -2,7 +2,7 @@
  * psn_prefill.hip -- gfx950 quantized prefill matmul  Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k],
  * fp16 activations, fp32 accumulation on v_mfma_f32_32x32x16_f16: the weight-streaming kernels for M <= 64, the
  * dequantization pass of the dense family, and the kernels of explicit plans (producer / consumer, wide, and the four-wave tiles of 256
- * columns).  What the planner picks between 64 rows and the dense family is in psn_prefill_pp.hip.
+ * columns).  What the planner picks between 64 rows and the dense family is in psn_prefill_frag.hip and psn_prefill_pp.hip.
  *
  * The four-wave kernels:
  *

@@ -64,7 +64,12 @@ template <int I, int N, class F> PSN_DEV void static_for(F &&f) {
     }
 }
 
-/* Which tile and K range a workgroup takes (psn_prefill_pp.hip, psn_prefill_dense.hip).  Workgroups b, b + 8, ... share an XCD and its L2: each XCD gets one contiguous piece of the
+/* 16 bytes per lane from memory to 1 KB of LDS, in the order of the lanes */
+PSN_DEV void load_to_lds(const char *from, lds_char *to) {
+    __builtin_amdgcn_global_load_lds((const void *)from, (__attribute__((address_space(3))) void *)to, 16, 0, 0);
+}
+
+/* Which tile and K range a workgroup takes (kernels of psn_prefill_frag.hip, psn_prefill_pp.hip and psn_prefill_dense.hip).  Workgroups b, b + 8, ... share an XCD and its L2: each XCD gets one contiguous piece of the
  * order "K range, ROWS rows of X, N tile, M tile within the rows", so that the 32 compute units of an XCD share a few panels of X and of W, and no XCD has more than one
  * workgroup more than another (dealing N tiles to the XCDs in turn left 5120 columns in tiles of 256 with three tiles on four of them and two on the others). */
 struct prefill_place { int m0, n0, c0, chunks; };            /* corner of the tile; first 256-wide chunk of K and how many */

@@ -36,10 +36,6 @@ PSN_DEV u32 dense_w_offset(int lane) {
     return (u32)((q >> 1) * 1024 + (q & 1) * 512 + (lane & 15) * 16);
 }
 
-PSN_DEV void load_to_lds(const char *from, lds_char *to) {
-    __builtin_amdgcn_global_load_lds((const void *)from, (__attribute__((address_space(3))) void *)to, 16, 0, 0);
-}
-
 /* Large tiles: WM x WN waves with TM x TN MFMA tiles each, K in steps of 32.  X comes in stages of 64 k (whole lines), a ring of three, W in steps of 32 k, a ring
  * of four: for 256 x 256 tiles that is all 160 KB of LDS.  Step t multiplies what was read during step t - 1, reads the fragments of step t + 1 and asks for W of step t + 4 and
  * half of the stage of X that takes the place of the one read last: the first half of stage (t + 5) / 2 in odd steps, the second of (t + 4) / 2 in even ones.

@@ -15,7 +15,6 @@
  *      very register the variable lives in, so that no copy of it is made while the bytes are still on their way.) ---- */
 typedef u32 u32x3 __attribute__((ext_vector_type(3)));
 template <int NB> struct raw_bytes;
-template <> struct raw_bytes<4> { typedef u32 t; };
 template <> struct raw_bytes<8> { typedef u32x2 t; };
 template <> struct raw_bytes<12> { typedef u32x3 t; };
 template <> struct raw_bytes<16> { typedef u32x4 t; };
@@ -54,10 +53,10 @@ PSN_DEV void q0_finish(const half_done &t, u32 bias, u32 d2, u32 &o0, u32 &o1) {
     o1 = h2_bits((bits_h2(t.h[1]) - bits_h2(bias)) * bits_h2(d2));
 }
 
-/* ---- a format's share of one thread: part `part` of 32 / NB parts of a row.  `base` is the row's chunk plus lane_off(part);
+/* ---- a format's share of one thread: part `part` of 32 / NB parts of a row (NB = 8: four).  `base` is the row's chunk plus lane_off(part);
  *      load() asks for everything the four steps of the chunk need (LOADS instructions); step J's bytes are two groups
  *      (HI = 0, 1) of NB weights, which belong at k = k_lo(part) and k_hi(part) of the 64-wide step; first() and second() turn
- *      word i of a group into four fp16, with the step's scales from scales0() and scales1().  SPREAD (for NB = 4, 8): row_of() in psn_prefill_pp.hip. ---- */
+ *      word i of a group into four fp16, with the step's scales from scales0() and scales1().  SPREAD: row_of() in psn_prefill_pp.hip. ---- */
 /* Scales of Q4_K / Q5_K.  Unpacking the two sub-blocks of a 64-wide step costs twenty instructions, as much as decoding seven weights, and four threads share a row: each does
  * it for one of the chunk's four steps (kq_pick: the fields of step j; kq_own: d, d', m, m').  Next to each other (pp kernels) they hand the values round by quad_perm in each step; as
  * the four sixteens of lanes (FAR, thin kernels) through LDS, where the four floats of a step take the header's place in raw. */
@@ -110,7 +109,7 @@ struct PpQ4_K {
     template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
     template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
     template <int NB> static PSN_DEV int k_hi(int part) { return 32 + NB * part; }
-    static constexpr int SPREAD[2] = {0, 3};
+    static constexpr int SPREAD = 3;
 };
 struct PpQ5_K {
     static constexpr int BYTES = 176, LOADS = 6;
@@ -131,7 +130,7 @@ struct PpQ5_K {
     template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
     template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
     template <int NB> static PSN_DEV int k_hi(int part) { return 32 + NB * part; }
-    static constexpr int SPREAD[2] = {0, 3};
+    static constexpr int SPREAD = 3;
 };
 /* step J = half J / 2 of the super-block, quarters t = 2 (J & 1) and 2 (J & 1) + 1: the first 32 and the second 32 of
  * the half's 64 low-bit bytes, their low (J even) or high nibbles; bits 4..5 from the half's 32 high-bit bytes.  A
@@ -176,7 +175,7 @@ struct PpQ6_K {
     template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { kq_finish(t, s.d[HI], s.m[HI], o0, o1); }
     template <int NB> static PSN_DEV int k_lo(int part) { return NB * part; }
     template <int NB> static PSN_DEV int k_hi(int part) { return 32 + NB * part; }
-    static constexpr int SPREAD[2] = {0, 3};
+    static constexpr int SPREAD = 3;
 };
 /* Q4_0 and Q8_0: step J = blocks 2 J and 2 J + 1, 36 (68) bytes from a dword on.  The first block's quants start two bytes
  * into its first dword, the second one's on a dword; so the dwords from DW * part on hold a part's bytes two (first block) or
@@ -221,7 +220,7 @@ struct PpQ4_0 {
     /* low nibbles first, high nibbles sixteen further on */
     template <int NB> static PSN_DEV int k_lo(int part) { return 32 * ((NB * part) >> 4) + ((NB * part) & 15); }
     template <int NB> static PSN_DEV int k_hi(int part) { return k_lo<NB>(part) + 16; }
-    static constexpr int SPREAD[2] = {0, 2};
+    static constexpr int SPREAD = 2;
 };
 struct PpQ8_0 {
     static constexpr int BYTES = 272, LOADS = 8;
@@ -249,7 +248,7 @@ struct PpQ8_0 {
     template <int HI> static PSN_DEV void second(const scale &s, const half_done &t, u32 &o0, u32 &o1) { q0_finish(t, 0x64806480u, s.d, o0, o1); }
     template <int NB> static PSN_DEV int k_lo(int part) { return 2 * NB * part; }
     template <int NB> static PSN_DEV int k_hi(int part) { return 2 * NB * part + NB; }
-    static constexpr int SPREAD[2] = {0, 0};
+    static constexpr int SPREAD = 0;
 };
 
 #endif

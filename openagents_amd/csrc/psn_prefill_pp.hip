@@ -1,5 +1,5 @@
 /*
- * psn_prefill_pp.hip -- gfx950 quantized prefill matmul, the kernels that decode in their loop:
+ * psn_prefill_pp.hip -- gfx950 quantized prefill matmul, the kernel that decodes in its loop for tiles of 256 rows of X:
  * Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k], fp16 MFMA, fp32 accumulation.
  *
  * A workgroup of eight waves (two to a SIMD) owns a BM x BN tile of Y and walks K in steps of 64.  Every wave does every
@@ -11,24 +11,20 @@
  *   - decodes its share of the weights of step s + 1 into the other one of two fp16 tiles.  A weight is decoded once per
  *     workgroup: a thread owns BN / 8 weights of one row per step, and their raw bytes come straight from memory into
  *     registers, asked for a whole 256-wide chunk ahead.
- * One barrier per step.
+ * One barrier per step.  (Tiles of fewer rows: psn_prefill_frag.hip; its layout needs more registers and LDS than there are for 256 rows.)
  *
- * What bounds it (counters, Q4_K 512 x 14336 x 4096, 256 x 128 tiles): of 123 k cycles 66 k are MFMA on the 224 compute units that have a
- * tile; launches back to back take 80 us, on zero weights (the same instructions) 64, so from M = 512 on it is power
- * (operand reads, decode arithmetic and MFMAs together), below that the decode's vector instructions (72 per wave and
- * step, of which six per MFMA ride along for free).  Against the kernels that served these shapes before (producer /
- * consumer and dequantize-first): 14336 x 4096 at M = 203: Q4_0 55 -> 44 us, Q8_0 75 -> 55, Q4_K 69 -> 47, Q6_K 92 -> 52; at
- * M = 512: Q4_0 82 -> 68, Q8_0 98 -> 78, Q4_K 97 -> 72, Q6_K 106 -> 77.  Splitting the roles (eight multiplying and eight
- * staging waves) measured 2-8 % slower, running the two waves of a SIMD in strictly opposite phases 10-15 % slower.
+ * What bounds it, Q4_K 512 x 14336 x 4096: 69 us; 53 without the decode and its LDS writes, 53 without MFMAs, 57 without loads, so vector instructions, LDS traffic
+ * (176 KB per step, 1.3 times as long as the MFMAs) and MFMAs add up; on a full chip power as well (on zero weights, the same instructions, a fifth faster), which is why the MFMAs
+ * are 16 x 16 x 32: 32 x 32 x 16 took 70 us there and 275 at M = 2048 instead of 257, but 57 instead of 60 on half-filled rounds, which the smaller tiles
+ * serve now.  Splitting the roles (eight multiplying and eight staging waves) measured 2-8 % slower, running the two waves of a SIMD in strictly opposite phases 10-15 %, sixteen
+ * waves with half the tile each 15 %.
  */
 #include "psn_args.h"
 #include "psn_device.h"
 #include "psn_prefill_common.h"
 #include "psn_prefill_formats.h"
 
-typedef float float4_t __attribute__((ext_vector_type(4)));
-
-/* Which weight row a group of 32 / NB threads decodes.  The lanes that write to LDS together (sixteen of 16 bytes) should
+/* Which weight row a group of four threads decodes.  The lanes that write to LDS together (sixteen of 16 bytes) should
  * hit sixteen different columns, (row & 1) * 8 + (chunk ^ row bits 1..3); the lanes of one row hold chunks that leave one
  * or two chunk bits to the rows.  So the low bits of the group's number go to row bit 0 and to the row bits that scatter
  * those: SPREAD 0: bits 1, 2, 3 in order; 2: bit 2 first; 3: bit 3 first. */
@@ -39,62 +35,34 @@ template <int SPREAD> PSN_DEV int row_of(int idx) {
     return idx;
 }
 
-template <int MF> struct pp_mfma;
-template <> struct pp_mfma<32> {
-    typedef float16_t acc;
-    static constexpr int R = 16, KK = 4;                    /* registers per tile, K slices per step */
-    static PSN_DEV acc mul(u32x4 a, u32x4 b, acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0); }
-    static PSN_DEV int row(int lane, int r) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
-};
-template <> struct pp_mfma<16> {
-    typedef float4_t acc;
-    static constexpr int R = 4, KK = 2;
-    static PSN_DEV acc mul(u32x4 a, u32x4 b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0); }
-    static PSN_DEV int row(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
-template <int OFF> PSN_DEV void lds_write64o(u32 addr, u32x2 v) { asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory"); }
 template <int OFF> PSN_DEV void lds_write128o(u32 addr, u32x4 v) { asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory"); }
 
 /* does piece p of a decode (see there) end in an LDS write? */
-template <int NB> constexpr bool pp_piece_writes(int p) { return p >= 2 && (p & 1) == 1 && (NB == 4 || ((((p - 2) >> 1) % (NB / 4)) & 1) == 1); }
+constexpr bool pp_piece_writes(int p) { return p >= 2 && (p & 3) == 1; }
 
-template <typename WF, int BM, int BN, int WM, int MF, int NS>
+template <typename WF, int BM, int BN, int WM, int NS>
 PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
-    typedef pp_mfma<MF> MMA;
-    constexpr int WN = 8 / WM, TM = BM / WM / MF, TN = BN / WN / MF, KK = MMA::KK;
-    constexpr int NB = BN / 16, PARTS = 32 / NB;            /* quant bytes per thread and step, threads per weight row */
-    static_assert(NB == 4 || NB == 8, "64 or 128 weight rows");
-    constexpr int SPREAD = WF::SPREAD[NB == 8];
+    constexpr int MF = 16, WN = 8 / WM, TM = BM / WM / MF, TN = BN / WN / MF, KK = 2;     /* K slices per step */
+    constexpr int NB = 8, PARTS = 4;                        /* quant bytes per thread and step, threads per weight row */
+    static_assert(BN == 128, "512 threads, four to a row");
+    constexpr int SPREAD = WF::SPREAD;
     constexpr int XBYTES = BM * 128, WBYTES = BN * 128;
     constexpr int NX = BM / 64;                             /* X loads per wave and step */
     static_assert(TM >= 1 && TN >= 1 && NX >= 1 && NS * XBYTES + 2 * WBYTES <= 160 * 1024, "tile");
     extern __shared__ uint4 psn_smem[];
-    typedef __attribute__((address_space(3))) char lds_char;
     lds_char *const lds_ptr = (lds_char *)psn_smem;
     const u32 lds0 = (u32)(uintptr_t)lds_ptr;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;
-    const int M = a.M, N = a.N, K = a.K, C = K >> 8;
+    const int M = a.M, N = a.N, K = a.K;
 
-    /* workgroups b, b + 8, b + 16, ... share an XCD: they get the M tiles (and K ranges) of one N tile in a row, so that a
-     * weight panel is fetched into a single L2 */
-    const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
-    const int S = a.ksplit;
-    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-    const int per_xcd_n = (nt + 7) >> 3;
-    const int tile_m = local % mt, split = (local / mt) % S, tn_local = local / (mt * S);
-    const int tile_n = xcd + 8 * tn_local;
-    if (tn_local >= per_xcd_n || tile_n >= nt) return;      /* whole workgroup leaves together */
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const int per_split = (C + S - 1) / S;
-    const int c_begin = split * per_split, c_end = min(c_begin + per_split, C);
-    if (c_begin >= c_end) return;                           /* an empty K range adds nothing */
-    const int nq = c_end - c_begin, nsteps = nq * 4;
+    prefill_place at;
+    if (!place_workgroup<BM, BN, 512>(a, at)) return;       /* whole workgroup leaves together */
+    const int m0 = at.m0, n0 = at.n0, c_begin = at.c0, nq = at.chunks, nsteps = nq * 4;
 
-    typename MMA::acc acc[TM][TN];
-    UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int j = 0; j < TN; ++j) UNROLL for (int r = 0; r < MMA::R; ++r) acc[i][j][r] = 0.f;
+    f32x4 acc[TM][TN];
+    UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4)(0.f);
 
     /* X: 16-byte word s of a stage in LDS order is row s / 8, position s % 8, which holds chunk (s % 8) ^ tile_swz(row) */
     u32 xoff[NX];
@@ -122,8 +90,8 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
     auto load_chunk = [&](int c, typename WF::template raw<NB> &r) {
         WF::template load<NB>(wsrc + (int64_t)min(c, nq - 1) * WF::BYTES, woff, r);
     };
-    /* The decode of step J of a chunk, in pieces: the scales (two), then two per word of four weights; a finished 16 bytes (8
-     * with NB = 4) goes to fp16 tile J % 2. */
+    /* The decode of step J of a chunk, in pieces: the scales (two), then two per word of four weights; a finished 16 bytes
+     * goes to fp16 tile J % 2. */
     constexpr int NW = NB / 4, PIECES = 2 + 4 * NW;
     u32 dec[4];
     half_done dhalf;
@@ -140,8 +108,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
                 WF::template first<J, NB, HI>(w, wscale, I, dhalf);
             } else {
                 WF::template second<HI>(wscale, dhalf, dec[B], dec[B + 1]);
-                if constexpr (NB == 4) lds_write64o<OFF>(HI ? wr_hi : wr_lo, (u32x2){dec[0], dec[1]});
-                else if constexpr (B == 2) lds_write128o<OFF>(HI ? wr_hi : wr_lo, (u32x4){dec[0], dec[1], dec[2], dec[3]});
+                if constexpr (B == 2) lds_write128o<OFF>(HI ? wr_hi : wr_lo, (u32x4){dec[0], dec[1], dec[2], dec[3]});
             }
         }
     };
@@ -180,7 +147,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
         for (int r = last + 1; r < READS; ++r) n += r * NRIDE / READS < pos;
         for (int p = 0; p < PIECES; ++p) {
             const int at = p * NRIDE / PIECES;
-            n += pp_piece_writes<NB>(p) && at >= from && at < pos;
+            n += pp_piece_writes(p) && at >= from && at < pos;
         }
         return n > 15 ? 15 : n;                             /* (four bits of counter: waiting for more than needed is harmless) */
     };
@@ -202,7 +169,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
         constexpr int kk = decltype(kc)::value;
         UNROLL for (int j = 0; j < TN; ++j) UNROLL for (int i = 0; i < TM; ++i) {
             __builtin_amdgcn_sched_barrier(0);
-            acc[i][j] = MMA::mul(xf[kk][i], wf[kk][j], acc[i][j]);
+            acc[i][j] = mfma16(wf[kk][j], xf[kk][i], acc[i][j]);
             __builtin_amdgcn_sched_barrier(0);
             behind(j * TM + i);
         }
@@ -220,6 +187,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
         multiply(pf_int<kk>(), [&](int pos) {
 #define PSN_PP_RIDE(P) if (pos == P) { if constexpr (P < TM * TN) ride(c, w, jc, pf_int<Q * TM * TN + P>()); }
             PSN_PP_RIDE(0) PSN_PP_RIDE(1) PSN_PP_RIDE(2) PSN_PP_RIDE(3) PSN_PP_RIDE(4) PSN_PP_RIDE(5) PSN_PP_RIDE(6) PSN_PP_RIDE(7)
+            PSN_PP_RIDE(8) PSN_PP_RIDE(9) PSN_PP_RIDE(10) PSN_PP_RIDE(11) PSN_PP_RIDE(12) PSN_PP_RIDE(13) PSN_PP_RIDE(14) PSN_PP_RIDE(15)
 #undef PSN_PP_RIDE
         });
     };
@@ -251,10 +219,6 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
         }                                                                                                                  \
         slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<0>());                                                           \
         slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<1>());                                                           \
-        if constexpr (KK > 2) {                                                                                            \
-            slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<(KK > 2 ? 2 : 0)>());                                        \
-            slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<(KK > 2 ? 3 : 0)>());                                        \
-        }                                                                                                                  \
         constexpr int KEEP = (NS - 2) * NX + ((J + 1) % 4 < NS - 2 ? WF::LOADS : 0);                                       \
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(KEEP) : "memory");                               \
         UNROLL for (int kk = HK; kk < KK; ++kk) { tie(xf[kk]); tie(wf[kk]); }                                              \
@@ -270,8 +234,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
 #undef PSN_PP_CHUNK
 #undef PSN_PP_STEP
     multiply(pf_int<HK>(), [](int) {});
-    if constexpr (KK > 2) multiply(pf_int<(KK > 2 ? HK + 1 : HK)>(), [](int) {});
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");       /* nothing is on its way into LDS any more */
     /* the last raw loads were for nothing, but their registers belong to them until they have landed */
     WF::template landed<NB>(wa);
     WF::template landed<NB>(wb);
@@ -280,28 +243,16 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
     int tid_out = threadIdx.x;
     asm volatile("" : "+v"(tid_out));
     const int wm_o = (tid_out >> 6) / WN, wn_o = (tid_out >> 6) % WN, lane_o = tid_out & 63;
-    UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int j = 0; j < TN; ++j) {
-        const int col = n0 + wn_o * (BN / WN) + MF * j + lane_o % MF;
-        UNROLL for (int r = 0; r < MMA::R; ++r) {
-            const int row = m0 + wm_o * (BM / WM) + MF * i + MMA::row(lane_o, r);
-            if (row < M && col < N) {
-                if (S == 1) a.Y[(int64_t)row * N + col] = acc[i][j][r];
-                else unsafeAtomicAdd(&a.Y[(int64_t)row * N + col], acc[i][j][r]);
-            }
-        }
-    }
+    UNROLL for (int i = 0; i < TM; ++i)
+        store_tiles<TN>(a, m0 + wm_o * (BM / WM) + MF * i, n0 + wn_o * (BN / WN), lane_o, acc[i], lds0 + (u32)((tid_out >> 6) * wave_out_bytes<TN>()));
 }
 
 
-#define PSN_PP(fmt, WF, BM, BN, WM, MF, NS)                                                                                  \
+#define PSN_PP(fmt, WF, BM, BN, WM, NS)                                                                                      \
     extern "C" __global__ void __launch_bounds__(512) psn_prefill_##fmt##_m##BM##_n##BN##_pp(const psn_prefill_args a) {    \
-        prefill_pp_body<WF, BM, BN, WM, MF, NS>(a);                                                                          \
+        prefill_pp_body<WF, BM, BN, WM, NS>(a);                                                                              \
     }
-#define PSN_PP_FAMILY(fmt, WF)           \
-    PSN_PP(fmt, WF, 64, 64, 2, 16, 4)    \
-    PSN_PP(fmt, WF, 64, 128, 2, 32, 4)   \
-    PSN_PP(fmt, WF, 128, 128, 2, 32, 4)  \
-    PSN_PP(fmt, WF, 256, 128, 4, 32, 4)
+#define PSN_PP_FAMILY(fmt, WF) PSN_PP(fmt, WF, 256, 128, 4, 4)
 
 #ifdef PSN_BUILD_PP_Q4_0
 PSN_PP_FAMILY(q4_0, PpQ4_0)
