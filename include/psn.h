@@ -294,9 +294,9 @@ int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32
  * 64x128, 128x128, 128x256, 256x128 or 256x256; family 8: below), into how many ranges K is cut (1, 2, 4 or 8; with more than one, Y is
  * zeroed by a fill kernel and the partial sums are added atomically, so their order -- and the last bit
  * of a sum -- can vary between runs), and the kernel family:
- *    4  the kernels that decode in their loop, every wave staging and multiplying (any tile): eight waves (two to a SIMD,
- *       the staging spread behind the MFMAs) for tiles of 64 and 128 columns, which are what the planner uses; four
- *       waves for tiles of 256 columns;
+ *    4  the kernels that decode in their loop (any tile): eight waves for tiles of 64 and 128 columns, which are what the
+ *       planner uses (up to 128 rows every wave decodes its own MFMA operands in registers; 256x128 tiles stage decoded
+ *       weights in LDS, spread behind the MFMAs); four waves for tiles of 256 columns;
  *   16  eight waves of which four only multiply and four only stage: X by direct-to-LDS loads three K
  *       steps ahead, weights decoded from registers one step ahead (64x64, 64x128, 128x128, 128x256);
  *   32  the wide kernel for large M (256x256 tiles only): four waves, each with all 256 rows x 64 columns
@@ -304,7 +304,8 @@ int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t qtype, int32
  *       a wave decodes the operand of its own columns one K slice ahead, interleaved with its MFMAs;
  *   64  the weight-streaming kernel for M <= 64 (64x64 tiles; every format, Q6_K only when K is a multiple of
  *       2048 so that its rows are whole 16-byte words): X and the raw GGUF bytes arrive in LDS rings by
- *       direct-to-LDS loads, every wave decodes its own MFMA operand, one barrier per 256 of K;
+ *       direct-to-LDS loads, every wave decodes its own MFMA operand, one barrier per 256 of K (Q4_0 and Q8_0; the
+ *       K-quants run family 4's 64x64 tile);
  *    8  the thin kernels for M <= 64 (every format and K): all of X, padded to 16, 32, 48 or 64 rows (tile_m >= M), by 16, 32 or
  *       64 rows of W (tile_n; 64 only with tile_m <= 48, Q8_0 16, and not for 16 rows of Q4_0, Q4_K and Q5_K), eight waves with chunks of
  *       K of their own and no barrier between them.  psn_qmatmul_prefill_plan and _plan_for never name them;
@@ -322,7 +323,8 @@ int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int32_t comput
  * psn_prefill_reserve (or an earlier dense call of that size) has sized it. */
 int32_t psn_qmatmul_prefill_plan_for(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t *tile_m,
                                      int32_t *tile_n, int32_t *ksplit, int32_t *waves);
-/* What psn_qmatmul_prefill runs, for any M: the plan above, or for M <= 64 a shape of family 8 where that is estimated to be faster.
+/* What psn_qmatmul_prefill runs, for any M: the plan above, or for M <= 64 a shape of family 8 (from 17 rows of X on and with more than 64 rows of W per compute unit also of family 4)
+ * where that is estimated to be faster.
  * workspace == 0: what it runs where the dense family's workspace is missing and cannot be allocated. */
 int32_t psn_qmatmul_prefill_choice(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t workspace, int32_t *tile_m,
                                    int32_t *tile_n, int32_t *ksplit, int32_t *waves);
@@ -333,7 +335,7 @@ int32_t psn_prefill_reserve(psn_stream *s, int64_t N, int64_t K);
  * into a caller-owned buffer of psn_prefill_packed_bytes(N, K) bytes (2 bytes per weight, rows padded to whole
  * 256-row panels; a deployment with HBM to spare keeps one per matrix beside the GGUF blocks the decode
  * matvec reads), psn_qmatmul_prefill_packed multiplies any number of X against it -- the same result as
- * psn_qmatmul_prefill_tiled(..., 256, 256, ksplit, 128) without the 35-48 us pass per call.  No stream
+ * psn_qmatmul_prefill_tiled(..., 256, 256, ksplit, 128), up to the order of sums, without the 35-48 us pass per call.  No stream
  * workspace is involved.  No counterpart in the reference, which dequantizes inside every call. */
 int64_t psn_prefill_packed_bytes(int64_t N, int64_t K);
 int32_t psn_prefill_pack(psn_module *mod, psn_stream *s, int32_t qtype, const psn_buf *W, psn_buf *packed, int64_t N, int64_t K);

@@ -311,11 +311,6 @@ template <int D0, int D1> PSN_DEV u32x2 lds_read2_b32(u32 addr) {
     asm volatile("ds_read2_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(v) : "v"(addr), "n"(D0), "n"(D1) : "memory");
     return v;
 }
-PSN_DEV u32 lds_read_u16(u32 addr) {
-    u32 v;
-    asm volatile("ds_read_u16 %0, %1" : "=v"(v) : "v"(addr) : "memory");
-    return v;
-}
 PSN_DEV void lds_write128(u32 addr, u32x4 v) { asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
 PSN_DEV void lds_write32(u32 addr, u32 v) { asm volatile("ds_write_b32 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
 PSN_DEV void lds_write16(u32 addr, u32 v) { asm volatile("ds_write_b16 %0, %1" ::"v"(addr), "v"(v) : "memory"); }

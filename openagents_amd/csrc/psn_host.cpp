@@ -1462,14 +1462,30 @@ extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int
                                             int32_t *waves) {
     return psn_qmatmul_prefill_plan_for(PSN_Q4_0, M, N, K, cus, tile_m, tile_n, ksplit, waves);
 }
+/* family 4: one tile's estimate; and the tile and the K split with the smallest one; K ranges hold at least two 256-wide chunks */
+static double in_loop_estimate(const prefill_cost &c, int32_t qtype, int64_t M, int64_t N, int64_t K, int sp, int32_t cus) {
+    const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
+    const int by_regs = qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu, by_lds = 160 * 1024 / in_loop_lds(qtype, bm, bn);
+    return tile_estimate(c.cost, c.step_us[format_index(qtype)], M, N, K, bm, bn, sp, by_regs < by_lds ? by_regs : by_lds, cus, false);
+}
+static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
+    double best = 1e300;
+    for (const prefill_cost &c : k_prefill_cost)
+        for (int sp = 1; sp <= 8; sp *= 2) {
+            if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
+            const double t = in_loop_estimate(c, qtype, M, N, K, sp, cus);
+            if (t < best) { best = t; *tile_m = k_prefill_tiles[c.tile][0]; *tile_n = k_prefill_tiles[c.tile][1]; *ksplit = sp; }
+        }
+    return best;
+}
+
 /* At most 64 rows: which kernel streams the weights.  psn_prefill_<fmt>_thin_<tm>_<rt> (psn_prefill_thin.hip, 16 tm rows of X and 16 rt
- * of W per workgroup) against the 64 x 64 kernel (psn_prefill_<fmt>_skinny; rt = 0 here; with Q6_K only for rows of whole 16-byte
- * words).  Checked on MI355X against every explicit plan over five formats, sixteen matrices and M = 1 .. 64 (11304 launches): what the estimates
- * pick is 1.3 % off the fastest on average and more than 10 % off in 35 of 720 shapes (a handful of rows of X on large matrices; the 64 x 64
- * kernel where family 4, which is considered here for Q6_K only, would do better).  An estimate is a launch, then per round of workgroups the first loads, a chain
- * per chunk of a wave, and the work that the waves of a SIMD share: decode per weight row, X per row of it.  The 64 x 64 kernel stays
- * the faster one from about 48 rows on where the matrix is large (Q4_0 8192 x 28672 M = 64: 62 us against 74), with Q8_0, whose raw
- * chunks leave no LDS for four tiles, from 17 on (14336 x 4096 M = 32: 23.0 against 25.4); it cuts K only while the weight rows
+ * of W per workgroup) against the 64 x 64 kernel: psn_prefill_<fmt>_skinny for Q4_0 and Q8_0, family 4's tile of that size for the K-quants (Q6_K only where rows are
+ * whole 16-byte words, as family 64 is documented; elsewhere family 4 competes by its own name).  Checked on MI355X against the explicit plans over five formats, eighteen matrices
+ * and M = 1 .. 64 (9800 launches): what the estimates pick is 1.3 % off the fastest on average and more than 10 % off in 21 of 700 shapes (family 4's estimates are
+ * raised by 1.3 and 1.22, the factors at which no shape gets slower that thin kernels serve well).  An
+ * estimate is a launch, then per round of workgroups the first loads and a chain per chunk of a wave, and the work that the waves of a SIMD
+ * share: decode per weight row, X per row of it.  The 64 x 64 kernel cuts K only while the weight rows
  * alone leave half of the compute units without a workgroup.  At rt = 4 a cut of K did not pay. */
 struct weight_stream_plan { int rt, ksplit; double us; };
 static bool may_cut_k(int64_t M, int64_t N, int64_t K, int sp) { return sp == 1 || ((M * N) % 4 == 0 && K / 256 >= 2 * sp); }
@@ -1479,7 +1495,7 @@ static int stream64_ksplit(int64_t M, int64_t N, int64_t K, int32_t cus) {
     return sp;
 }
 static const double k_thin_row_us[5] = {0.719, 1.348, 0.878, 1.062, 1.695};       /* decode of 16 rows x 256: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
-static const double k_stream64_chunk_us[5] = {0.963, 1.196, 1.175, 1.242, 1.519}; /* 64 rows x 256 in the 64 x 64 kernel */
+static const double k_skinny_chunk_us[2] = {0.934, 1.160};                        /* 64 rows x 256 in the 64 x 64 kernel of Q4_0, Q8_0 */
 static bool big_chunk(int32_t qtype) { return qtype == PSN_Q8_0 || qtype == PSN_Q6_K; }    /* raw chunks of five or six registers a lane instead of three */
 /* rt = 4: LDS and registers end at 48 rows of X (Q8_0: 16); at 16 rows the others' rt = 2 shares compute units */
 static bool thin_exists(int32_t qtype, int tm, int rt) {
@@ -1496,7 +1512,8 @@ static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N
         const int64_t nt = (N + 63) / 64;
         const int sp = stream64_ksplit(M, N, K, cus);
         const double rounds = (double)((nt * sp + cus - 1) / cus);
-        best = {0, sp, 0.97 * (3.8 + rounds * (double)((C + sp - 1) / sp) * k_stream64_chunk_us[f] + cut_us(sp) + 0.19 * y_mb)};
+        best = {0, sp, f >= 2 ? 1.3 * in_loop_estimate(k_prefill_cost[0], qtype, M, N, K, sp, cus)
+                              : 3.69 + rounds * (double)((C + sp - 1) / sp) * k_skinny_chunk_us[f] + 0.97 * cut_us(sp) + 0.184 * y_mb};
     }
     for (int rt = 1; rt <= 4; rt *= 2) {
         if (!thin_exists(qtype, tm, rt)) continue;
@@ -1508,20 +1525,6 @@ static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N
             const double us = 0.9 + rounds * (1.22 + 0.316 * rt * (double)((per + 7) / 8)) +
                               shared * (double)per * (rt * (k_thin_row_us[f] + 0.04 * tm) + 0.604 * tm) / 8 + cut_us(sp) + 1.52 * y_mb;
             if (us < best.us) best = {rt, sp, us};
-        }
-    }
-    return best;
-}
-/* family 4: the tile and the K split with the smallest estimate; K ranges hold at least two 256-wide chunks */
-static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
-    double best = 1e300;
-    for (const prefill_cost &c : k_prefill_cost) {
-        const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
-        const int by_regs = qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu, by_lds = 160 * 1024 / in_loop_lds(qtype, bm, bn);
-        for (int sp = 1; sp <= 8; sp *= 2) {
-            if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
-            const double t = tile_estimate(c.cost, c.step_us[format_index(qtype)], M, N, K, bm, bn, sp, by_regs < by_lds ? by_regs : by_lds, cus, false);
-            if (t < best) { best = t; *tile_m = bm; *tile_n = bn; *ksplit = sp; }
         }
     }
     return best;
@@ -1566,9 +1569,21 @@ static int32_t prefill_choice(int32_t qtype, int64_t M, int64_t N, int64_t K, in
     if (rc || M > 64) return rc;
     if (cus <= 0) cus = 256;
     const weight_stream_plan p = plan_weight_stream(qtype, M, N, K, cus);
+    /* Family 4 competes where it has to (Q6_K rows that are not whole 16-byte words) and where 64-row tiles need more than one round of workgroups, so that its tiles of 128
+     * rows of W pay (28672 x 8192, M = 64: Q4_K 47.5 us, 64 x 64 tiles 55.4; Q4_0 43.0, the skinny kernel 56.6); with fewer rows of W its 64 x 64 tile, or the kernel that stands for it, is the one that wins, and
+     * with up to 16 rows of X the thin kernels read W as fast as memory gives it (Q4_0 37 us there). */
     int32_t bm, bn, sp;
-    /* (Q6_K rows that are not whole 16-byte words: the kernels that decode in their loop are what it competes with) */
-    if (p.rt == 0 || (*waves == 4 && p.us >= plan_in_loop(qtype, M, N, K, cus, &bm, &bn, &sp))) return PSN_OK;
+    if (*waves == 4 || (M > 16 && N > 64 * (int64_t)cus)) {
+        const double t = 1.22 * plan_in_loop(qtype, M, N, K, cus, &bm, &bn, &sp);
+        if (t <= p.us) {
+            *tile_m = bm;
+            *tile_n = bn;
+            *ksplit = sp;
+            *waves = 4;
+            return PSN_OK;
+        }
+    }
+    if (p.rt == 0) return PSN_OK;
     *tile_m = 16 * (int32_t)((M + 15) / 16);
     *tile_n = 16 * p.rt;
     *ksplit = p.ksplit;
@@ -1714,11 +1729,14 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
     if (qtype != PSN_Q4_0 && qtype != PSN_Q8_0 && waves != 4 && waves != 64 && !(waves == 16 && bm == 128 && bn == 256 && qtype != PSN_Q6_K))
         return fail(PSN_E_UNSUPPORTED, "prefill: %s has families 4, 8 and 64 (M <= 64), 128%s", fmt_name(qtype),
                     qtype == PSN_Q6_K ? "" : " and 16 on the 128x256 tile");
-    /* waves == 64 selects the skinny kernel (M <= 64, 64 x 64 tiles, deep LDS rings) */
+    /* waves == 64 selects the 64 x 64 kernel for M <= 64: the skinny kernel (deep LDS rings) of Q4_0 and Q8_0, family 4's 64 x 64 tile of the K-quants */
+    if (waves == 64) {
+        if (bm != 64 || bn != 64 || M > 64) return fail(PSN_E_UNSUPPORTED, "prefill: the skinny kernel serves M <= 64 with a 64x64 tile");
+        /* (as the interface documents it; family 4 itself takes any row) */
+        if (qtype == PSN_Q6_K && K % 2048) return fail(PSN_E_UNSUPPORTED, "prefill: the skinny Q6_K kernel needs K to be a multiple of 2048 (K=%lld)", (long long)K);
+        if (qtype != PSN_Q4_0 && qtype != PSN_Q8_0) waves = 4;
+    }
     const bool skinny = waves == 64;
-    if (skinny && (bm != 64 || bn != 64 || M > 64)) return fail(PSN_E_UNSUPPORTED, "prefill: the skinny kernel serves M <= 64 with a 64x64 tile");
-    /* Q6_K super-blocks (210 bytes) are fetched as windows of aligned 16-byte words: the rows must start on one */
-    if (skinny && qtype == PSN_Q6_K && K % 2048) return fail(PSN_E_UNSUPPORTED, "prefill: the skinny Q6_K kernel needs K to be a multiple of 2048 (K=%lld)", (long long)K);
     /* waves == 32 selects the wide kernel: 256 x 256 tiles, four waves with 128 x 128 each, weights decoded
      * from raw bytes in LDS by the wave that multiplies them */
     const bool wide = waves == 32;
@@ -1732,9 +1750,9 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
     if (ksplit < 1 || ksplit > 64) return fail(PSN_E_UNSUPPORTED, "prefill: ksplit=%d outside 1..64", ksplit);
     if (ksplit > 1 && (M * N) % 4 != 0) return fail(PSN_E_UNSUPPORTED, "prefill: splitting K needs M*N to be a multiple of 4");
     /* the interleaved kernels carry their LDS as static arrays; the skinny kernel: rings of three X chunks
-     * (64 rows x 256 k fp16) and six (Q4_0, Q4_K), five (Q5_K), four (Q6_K) or three (Q8_0) raw weight chunks (64 rows, padded: SkinnyRings), reused for the final
+     * (64 rows x 256 k fp16) and six (Q4_0) or three (Q8_0) raw weight chunks (64 rows, padded: SkinnyRings), reused for the final
      * 8 x 16 KB reduction */
-    const int skinny_rings = 3 * 32768 + (qtype == PSN_Q4_0 || qtype == PSN_Q4_K ? 6 * 64 * 144 : qtype == PSN_Q5_K ? 5 * 64 * 176 : qtype == PSN_Q6_K ? 4 * 64 * 240 : 3 * 64 * 304);
+    const int skinny_rings = 3 * 32768 + (qtype == PSN_Q4_0 ? 6 * 64 * 144 : 3 * 64 * 304);
     const int wide_rings = 3 * (32768 + 256 * (qtype == PSN_Q4_0 ? 36 : 68));   /* three stages of X (256 rows x 64 k) and of raw blocks (two per row) */
     const bool pp = waves == 4 && bn <= 128;
     const int lds = pp ? in_loop_lds(qtype, bm, bn) : skinny ? (skinny_rings > 8 * 16384 ? skinny_rings : 8 * 16384) : wide ? wide_rings : waves == 16 ? 0 : 2 * (bm + bn) * 128;

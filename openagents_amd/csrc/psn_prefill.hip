@@ -1,6 +1,6 @@
 /*
  * psn_prefill.hip -- gfx950 quantized prefill matmul  Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k],
- * fp16 activations, fp32 accumulation on v_mfma_f32_32x32x16_f16: the weight-streaming kernels for M <= 64, the
+ * fp16 activations, fp32 accumulation on v_mfma_f32_32x32x16_f16: the 64-row streaming kernels of Q4_0 and Q8_0, the
  * dequantization pass of the dense family, and the kernels of explicit plans (producer / consumer, wide, and the four-wave tiles of 256
  * columns).  What the planner picks between 64 rows and the dense family is in psn_prefill_frag.hip and psn_prefill_pp.hip.
  *
@@ -566,7 +566,7 @@ PSN_DEV void prefill_body_ws(const psn_prefill_args &a) {
     }
 }
 
-/* ---- skinny variant (M <= 64) ---------------------------------------------------------------------
+/* ---- skinny variant (M <= 64; Q4_0 and Q8_0) ---------------------------------------------------------------------
  * With at most 64 activation rows the matmul is a weight stream (HBM-bound), and a workgroup's 64-wide K
  * step carries so little arithmetic (a 64 x 64 tile: 16 MFMAs) that the step time of the kernels above
  * is their per-step chain of barrier, decode and memory latency.  This kernel has no per-step
@@ -591,22 +591,19 @@ PSN_DEV void prefill_body_ws(const psn_prefill_args &a) {
  * every iteration issues the same number of loads and the outstanding-load count is a constant. */
 template <typename WF> struct SkinnyRings {
     static constexpr int XR = 3;                                /* X chunks in the ring */
-    /* DATA: the 16-byte words that hold a row's chunk.  Q6_K's 210-byte super-blocks start on 2-byte boundaries: what is
-     * loaded is the window of fourteen aligned words that holds the super-block (rows must be whole 16-byte words, K a
-     * multiple of 2048; chunk c then starts (210 c) mod 16 bytes into its window, the same for every row).
+    /* DATA: the 16-byte words that hold a row's chunk.
      * LROW: bytes between rows in LDS.  A wave reads the same 32-bit field of 32 different rows at a time; rows lie whole
      * 16-byte words apart, so those reads can reach only eight of the 32 banks (a four-way conflict) -- unless the rows
      * are ROTated against each other: row n is fetched from 4 rho(n) bytes before its chunk, rho(n) = (n >> RSH) & 3 (one
      * more word per row takes the bytes pushed out at the end; the bytes in front belong to the chunk or the row before).
-     * With 304 (Q8_0) or 240 (Q6_K) bytes between rows all 32 rows then hit different banks.  Q4_K / Q5_K read whole
-     * aligned words instead; Q4_0 stays unrotated (measured: with 160 bytes between rows its conflicts halve and the
-     * kernel gets 10 % slower -- the fetches that no longer start on 16-byte words and the extra word cost more than
-     * its few 32-bit reads per chunk). */
-    static constexpr int DATA = (WF::BYTES % 16 == 0 ? WF::BYTES : WF::BYTES + 14 + 15) / 16;
-    static constexpr bool ROT = DATA == 17 || DATA == 14;
-    static constexpr int LROW = !ROT ? WF::BYTES : DATA == 17 ? 304 : 240;
+     * With 304 (Q8_0) bytes between rows all 32 rows then hit different banks.  Q4_0 stays unrotated (measured: with 160
+     * bytes between rows its conflicts halve and the kernel gets 10 % slower -- the fetches that no longer start on 16-byte
+     * words and the extra word cost more than its few 32-bit reads per chunk). */
+    static constexpr int DATA = WF::BYTES / 16;
+    static constexpr bool ROT = DATA == 17;
+    static constexpr int LROW = ROT ? 304 : WF::BYTES;
     static constexpr int RSH = 3;
-    static constexpr int RS = LROW <= 160 ? 6 : LROW == 176 ? 5 : LROW == 240 ? 4 : 3;   /* raw weight chunks in the ring: what 160 KB hold beside X */
+    static constexpr int RS = ROT ? 3 : 6;                      /* raw weight chunks in the ring: what 160 KB hold beside X */
     static constexpr int XBYTES = 4 * 64 * 128, RBYTES = 64 * LROW;
     static constexpr int BYTES = XR * XBYTES + RS * RBYTES;
 };
@@ -615,26 +612,18 @@ template <typename WF> struct SkinnyRings {
  * multiply the block before, then decode); 2: waves 5..7.  EVEN: the wave's block index is even -- the
  * block starts on a dword (scale in the low half of its first dword, quants two bytes in: aligned dwords
  * are read and shifted; LDS reads that straddle dwords are very slow); an odd block starts two bytes
- * later (scale in the high half of the dword before, quants aligned).  Q4_K / Q5_K: the chunk is the row's
- * super-block and the wave's "block" its sub-block `wave` -- even ones sit in the low nibbles, odd ones in the
- * high nibbles of the same 32 bytes; sub-blocks 0..3 (LOADER 0) and 4..7 unpack their 6-bit scale and min
- * from different bytes of the 12-byte field; every LDS read is an aligned dword.  Q6_K: sub-block `wave` again
- * (LOADER 0: the super-block's first half; EVEN: the first 32 of a 64-byte group of ql); its fields start on
- * 2-byte boundaries, so three aligned dwords are read around each eight bytes and shifted with v_alignbyte. */
+ * later (scale in the high half of the dword before, quants aligned). */
 template <typename WF, int LOADER, bool EVEN>
 PSN_DEV void prefill_skinny_loop(const psn_prefill_args &a, int wave, int lane, int n0, int c_begin, int nq, int rot, bool rotate_rows,
                                  u32 xs_base, u32 raw_base, __attribute__((address_space(3))) char *lds_ptr, u32 lds0, float16_t (&acc)[2][2]) {
     typedef SkinnyRings<WF> R;
-    constexpr bool KQ = WF::KQ;                             /* Q4_K / Q5_K: the chunk is one super-block per row, wave w owns its sub-block w */
-    constexpr bool Q4 = !KQ && WF::DW == 36;
-    constexpr bool Q5K = KQ && WF::DW == 44;
-    constexpr bool Q6K = KQ && WF::DW == 53;
+    static_assert(!WF::KQ, "Q4_0 and Q8_0");
+    constexpr bool Q4 = WF::DW == 36;
     constexpr int XR = R::XR, RS = R::RS, XBYTES = R::XBYTES, RBYTES = R::RBYTES, LROW = R::LROW;
-    constexpr int RINSTR = RBYTES / 1024;                   /* wave-wide load instructions per raw chunk: 9, 10, 11, 15 or 19 */
+    constexpr int RINSTR = RBYTES / 1024;                   /* wave-wide load instructions per raw chunk: 9 or 19 */
     constexpr int CX = 8;                                   /* X loads per X wave and chunk (32 KB over 4 waves) */
     /* raw loads per weight wave and chunk: wave 4 takes the one load that does not divide over four waves; when
-     * three or two are left over (Q5_K, Q6_K) every wave issues the same number and the last waves repeat the chunk's
-     * last load */
+     * three are left over (Q8_0) every wave issues the same number and the last wave repeats the chunk's last load */
     constexpr bool EVEN_SHARE = RINSTR % 4 != 1;
     constexpr int CR = EVEN_SHARE ? (RINSTR + 3) / 4 : RINSTR / 4 + (LOADER == 1 ? 1 : 0);
     constexpr int DEPTH = LOADER == 0 ? XR : RS, PER = LOADER == 0 ? CX : CR;
@@ -662,8 +651,7 @@ PSN_DEV void prefill_skinny_loop(const psn_prefill_args &a, int wave, int lane, 
                 const int rho = R::ROT && rotate_rows ? ((row & 31) >> R::RSH) & 3 : 0;
                 /* words past the row's data (and past the one that takes the rotated-out bytes) repeat its last one */
                 const int wd = min(word % (LROW / 16), R::DATA - 1 + (rho > 0));
-                const int64_t coff = Q6K ? (int64_t)((c * WF::BYTES) & ~15) : (int64_t)c * WF::BYTES;
-                const uint8_t *src = a.W + (int64_t)min(n0 + row, N - 1) * a.row_bytes + coff + wd * 16 - 4 * rho;
+                const uint8_t *src = a.W + (int64_t)min(n0 + row, N - 1) * a.row_bytes + (int64_t)c * WF::BYTES + wd * 16 - 4 * rho;
                 __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(dst + i * 1024), 16, 0, 0);
             }
         }
@@ -674,77 +662,18 @@ PSN_DEV void prefill_skinny_loop(const psn_prefill_args &a, int wave, int lane, 
     const int h = lane >> 5;
     u32 xlane[2];
     UNROLL for (int sl = 0; sl < 2; ++sl) xlane[sl] = (u32)((wave >> 1) * 8192 + tile_off(lane & 31, 2 * (2 * (wave & 1) + sl) + h));
-    /* K-quants: the row's super-block; its quants of sub-block `wave` (bytes 32 (wave / 2) .. + 31 of the nibble
-     * array, this lane's eight at 8h and 16 + 8h); Q5_K: the fifth bits of the same elements (qh, bit `wave`) */
-    /* Q6_K, sub-block `wave` = half wave / 4, quarter t = wave % 4 of the super-block: low bits in ql[64 half + 32 (t & 1)
-     * + l] (high nibble for t >= 2), bits 4..5 in qh[32 half + l] >> 2 t, int8 scales[8 half + 2 t + l / 16], d at 208 */
     const u32 rho_lane = R::ROT && rotate_rows ? (u32)(((lane & 31) >> R::RSH) & 3) : 0u;
-    const u32 rlane = (KQ ? (u32)((lane & 31) * LROW) : (u32)((lane & 31) * LROW + wave * BB)) + 4u * rho_lane;
-    const u32 qlane = Q6K ? rlane + (u32)(64 * (LOADER != 0) + 32 * !EVEN + 8 * h)
-                    : KQ  ? rlane + (u32)((Q5K ? 48 : 16) + 32 * (wave >> 1) + 8 * h) : rlane + 8u * (u32)h;
-    const u32 hlane = Q6K ? rlane + (u32)(128 + 32 * (LOADER != 0) + 8 * h) : rlane + (u32)(16 + 8 * h);
+    const u32 rlane = (u32)((lane & 31) * LROW + wave * BB) + 4u * rho_lane, qlane = rlane + 8u * (u32)h;
     constexpr int ROW32 = 32 * LROW;
 
-    /* Q4_K / Q5_K: kh[j] = d | dmin << 16 and the three scale dwords, kv[j][0..1] = quants of slice 0, 1 (two dwords each),
-     * kv[j][2..3] = qh likewise; Q6_K, kq[j]: 0..5 = the aligned dwords around ql (three per slice), 6..11 = around qh,
-     * 12 = the two scales, 13 = d */
-    struct unit { u32x4 xf[2][2]; u32 raw[KQ ? 1 : NP][2][3], wd[2], kq[2][Q6K ? 14 : 1]; u32x4 kh[2]; u32x2 kv[2][4]; };
-    /* `o`: Q6_K only, where in its 16-byte-aligned window this chunk's super-block starts (even, wave-uniform) */
-    auto fetch = [&](u32 xst, u32 rst, unit &t, u32 o) {
+    struct unit { u32x4 xf[2][2]; u32 raw[NP][2][3], wd[2]; };
+    auto fetch = [&](u32 xst, u32 rst, unit &t) {
         const u32 xa0 = xst + xlane[0], xa1 = xst + xlane[1], rw = rst + rlane, rq = rst + qlane;
         t.xf[0][0] = lds_read128<0>(xa0);
         t.xf[0][1] = lds_read128<4096>(xa0);
         t.xf[1][0] = lds_read128<0>(xa1);
         t.xf[1][1] = lds_read128<4096>(xa1);
-        if constexpr (Q6K) {
-            /* every field starts o bytes into the record; o mod 4 is 0 or 2: aligned dwords are read and shifted in decode */
-            const u32 ob = o & ~3u, ql = rq + ob, qh = rst + hlane + ob;
-            const u32 sc = rw + (u32)(192 + 8 * (LOADER != 0)) + 2u * (u32)(wave & 3) + o, dd = rw + 208u + o;
-            t.kq[0][0] = lds_read32o<0>(ql);
-            t.kq[0][1] = lds_read32o<4>(ql);
-            t.kq[0][2] = lds_read32o<8>(ql);
-            t.kq[0][3] = lds_read32o<16>(ql);
-            t.kq[0][4] = lds_read32o<20>(ql);
-            t.kq[0][5] = lds_read32o<24>(ql);
-            t.kq[1][0] = lds_read32o<ROW32>(ql);
-            t.kq[1][1] = lds_read32o<ROW32 + 4>(ql);
-            t.kq[1][2] = lds_read32o<ROW32 + 8>(ql);
-            t.kq[1][3] = lds_read32o<ROW32 + 16>(ql);
-            t.kq[1][4] = lds_read32o<ROW32 + 20>(ql);
-            t.kq[1][5] = lds_read32o<ROW32 + 24>(ql);
-            t.kq[0][6] = lds_read32o<0>(qh);
-            t.kq[0][7] = lds_read32o<4>(qh);
-            t.kq[0][8] = lds_read32o<8>(qh);
-            t.kq[0][9] = lds_read32o<16>(qh);
-            t.kq[0][10] = lds_read32o<20>(qh);
-            t.kq[0][11] = lds_read32o<24>(qh);
-            t.kq[1][6] = lds_read32o<ROW32>(qh);
-            t.kq[1][7] = lds_read32o<ROW32 + 4>(qh);
-            t.kq[1][8] = lds_read32o<ROW32 + 8>(qh);
-            t.kq[1][9] = lds_read32o<ROW32 + 16>(qh);
-            t.kq[1][10] = lds_read32o<ROW32 + 20>(qh);
-            t.kq[1][11] = lds_read32o<ROW32 + 24>(qh);
-            t.kq[0][12] = lds_read_u16(sc);
-            t.kq[1][12] = lds_read_u16(sc + (u32)ROW32);
-            t.kq[0][13] = lds_read_u16(dd);
-            t.kq[1][13] = lds_read_u16(dd + (u32)ROW32);
-        } else if constexpr (KQ) {
-            /* a 32-bit read of 32 rows hits each LDS bank four times (rows are whole 16-byte words apart) and takes as long
-             * as a conflict-free 128-bit one: the header word (d, dmin, scales) is read whole, the quants 64 bits at a time */
-            const u32 rh = rst + hlane;
-            t.kh[0] = lds_read128<0>(rw);
-            t.kh[1] = lds_read128<ROW32>(rw);
-            t.kv[0][0] = lds_read64o<0>(rq);
-            t.kv[0][1] = lds_read64o<16>(rq);
-            t.kv[1][0] = lds_read64o<ROW32>(rq);
-            t.kv[1][1] = lds_read64o<ROW32 + 16>(rq);
-            if constexpr (Q5K) {
-                t.kv[0][2] = lds_read64o<0>(rh);
-                t.kv[0][3] = lds_read64o<16>(rh);
-                t.kv[1][2] = lds_read64o<ROW32>(rh);
-                t.kv[1][3] = lds_read64o<ROW32 + 16>(rh);
-            }
-        } else if constexpr (EVEN) {
+        if constexpr (EVEN) {
             t.wd[0] = lds_read32o<0>(rw);                                    /* scale | first two quant bytes */
             t.wd[1] = lds_read32o<ROW32>(rw);
             UNROLL for (int p = 0; p < NP; ++p) {
@@ -771,58 +700,14 @@ PSN_DEV void prefill_skinny_loop(const psn_prefill_args &a, int wave, int lane, 
     auto arrived = [&](unit &t) {
         tie(t.xf[0]);
         tie(t.xf[1]);
-        if constexpr (Q6K) {
-            UNROLL for (int j = 0; j < 2; ++j) UNROLL for (int i = 0; i < 14; ++i) tie1(t.kq[j][i]);
-        } else if constexpr (KQ) {
-            tie(t.kh);
-            UNROLL for (int j = 0; j < 2; ++j) UNROLL for (int i = 0; i < (Q5K ? 4 : 2); ++i) asm volatile("" : "+v"(t.kv[j][i]));
-        } else UNROLL for (int j = 0; j < 2; ++j) {
+        UNROLL for (int j = 0; j < 2; ++j) {
             tie1(t.wd[j]);
             UNROLL for (int p = 0; p < NP; ++p) { tie1(t.raw[p][j][0]); tie1(t.raw[p][j][1]); if (EVEN) tie1(t.raw[p][j][2]); }
         }
     };
     /* MFMA operands of the block's two slices, column blocks j = 0, 1 */
-    auto decode = [&](const unit &t, u32x4 (&wf)[2][2], u32 o) {
-        if constexpr (Q6K) {
-            const u32 sh = o & 2u;                          /* byte shift of every field against its aligned dwords */
-            const int tq = wave & 3;
-            UNROLL for (int j = 0; j < 2; ++j) {
-                const float d = h2f_lo(t.kq[j][13]);
-                UNROLL for (int sl = 0; sl < 2; ++sl) {
-                    const float ds = __fmul_rn(d, (float)(int)(int8_t)((t.kq[j][12] >> (8 * sl)) & 0xffu)), dm = ds * 32.f;
-                    u32 o4[4];
-                    UNROLL for (int e = 0; e < 2; ++e) {
-                        const u32 lo = __builtin_amdgcn_alignbyte(t.kq[j][3 * sl + e + 1], t.kq[j][3 * sl + e], sh);
-                        const u32 hi = __builtin_amdgcn_alignbyte(t.kq[j][6 + 3 * sl + e + 1], t.kq[j][6 + 3 * sl + e], sh);
-                        const u32 q = ((lo >> (4 * (tq >> 1))) & 0x0f0f0f0fu) | (((hi >> (2 * tq)) & 0x03030303u) << 4);
-                        pf_affine4(q, ds, dm, o4[2 * e], o4[2 * e + 1]);
-                    }
-                    wf[sl][j] = (u32x4){o4[0], o4[1], o4[2], o4[3]};
-                }
-            }
-        } else if constexpr (KQ) {
-            const int sh = 8 * (wave & 3);                  /* this sub-block's byte of the scale dwords */
-            UNROLL for (int j = 0; j < 2; ++j) {
-                u32 sc, mn;
-                if constexpr (LOADER == 0) {
-                    sc = (t.kh[j][1] >> sh) & 63u;
-                    mn = (t.kh[j][2] >> sh) & 63u;
-                } else {
-                    sc = ((t.kh[j][3] >> sh) & 0xfu) | (((t.kh[j][1] >> sh) >> 2) & 0x30u);
-                    mn = ((t.kh[j][3] >> (sh + 4)) & 0xfu) | (((t.kh[j][2] >> sh) >> 2) & 0x30u);
-                }
-                const float d1 = __fmul_rn(h2f_lo(t.kh[j][0]), (float)sc), m1 = __fmul_rn(h2f_hi(t.kh[j][0]), (float)mn);
-                UNROLL for (int sl = 0; sl < 2; ++sl) {
-                    u32 o[4];
-                    UNROLL for (int e = 0; e < 2; ++e) {
-                        u32 q = (EVEN ? t.kv[j][sl][e] : t.kv[j][sl][e] >> 4) & 0x0f0f0f0fu;
-                        if constexpr (Q5K) q |= ((t.kv[j][2 + sl][e] >> wave) & 0x01010101u) << 4;
-                        pf_affine4(q, d1, m1, o[2 * e], o[2 * e + 1]);
-                    }
-                    wf[sl][j] = (u32x4){o[0], o[1], o[2], o[3]};
-                }
-            }
-        } else UNROLL for (int j = 0; j < 2; ++j) {
+    auto decode = [&](const unit &t, u32x4 (&wf)[2][2]) {
+        UNROLL for (int j = 0; j < 2; ++j) {
             const half2_t w2 = bits_h2(t.wd[j]);
             const half2_t d2 = EVEN ? __builtin_shufflevector(w2, w2, 0, 0) : __builtin_shufflevector(w2, w2, 1, 1);
             u32 q[NP][2];
@@ -856,13 +741,12 @@ PSN_DEV void prefill_skinny_loop(const psn_prefill_args &a, int wave, int lane, 
     for (int q = 0; q < nq; ++q) {
         issue(q + DEPTH - 1);
         unit t;
-        const u32 o = Q6K ? (u32)((chunk_of(q) * WF::BYTES) & 15) : 0u;
-        fetch(xs_base + (u32)((q % XR) * XBYTES), raw_base + (u32)((q % RS) * RBYTES), t, o);
+        fetch(xs_base + (u32)((q % XR) * XBYTES), raw_base + (u32)((q % RS) * RBYTES), t);
         if constexpr (LOADER == 0) {
             u32x4 wf[2][2];
             lds_wait();
             arrived(t);
-            decode(t, wf, o);
+            decode(t, wf);
             __builtin_amdgcn_sched_barrier(0);
             multiply(t.xf, wf);
         } else {
@@ -870,7 +754,7 @@ PSN_DEV void prefill_skinny_loop(const psn_prefill_args &a, int wave, int lane, 
             __builtin_amdgcn_sched_barrier(0);
             lds_wait();
             arrived(t);
-            decode(t, wp, o);
+            decode(t, wp);
             UNROLL for (int sl = 0; sl < 2; ++sl) UNROLL for (int i = 0; i < 2; ++i) xp[sl][i] = t.xf[sl][i];
         }
         /* my share of chunk q+1: everything but the loads of the youngest DEPTH-2 iterations */
@@ -1317,9 +1201,6 @@ extern "C" __global__ void __launch_bounds__(256) psn_fill_zero(const psn_fill_a
 }
 PSN_PREFILL_KERNEL_SKINNY(q4_0, PfQ4_0)
 PSN_PREFILL_KERNEL_SKINNY(q8_0, PfQ8_0)
-PSN_PREFILL_KERNEL_SKINNY(q4_K, PfQ4_K)
-PSN_PREFILL_KERNEL_SKINNY(q5_K, PfQ5_K)
-PSN_PREFILL_KERNEL_SKINNY(q6_K, PfQ6_K)
 #endif
 #if !defined(PSN_BUILD_ONLY) || PSN_BUILD_PF == 2
 PSN_PREFILL_KERNEL_WIDE(q4_0, PfQ4_0)

@@ -499,3 +499,21 @@ def test_packed_multiply_at_tile_edges(hip, orc, m, n, k):
     hip.quantized_matmul_packed(packed, hip.upload(X), y, m, n, k)
     err = G.max_rel_err(y.download(np.float32, (m, n)), orc.prefill(orc.Q4_K, W, X, n, k))
     assert err < PARITY_TOL, (m, n, k, err)
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
+def test_few_rows_over_more_weight_rows_than_one_round_of_64(hip, orc, qname):
+    """64 rows of W per compute unit and one more: from there on psn_qmatmul_prefill may take family 4's tiles for M <= 64.  fp16 products are exact in fp32, so only the order
+    of at most 512 sums differs from the oracle: PARITY_TOL is far above 512 * 2^-24."""
+    t = getattr(orc, qname)
+    edge = 64 * hip.compute_units
+    for n, k in ((edge, 512), (edge + 1, 256), (edge + 4, 512)):
+        W = weights(orc, qname, 885, n, k)
+        w, X = hip.upload_weight(t, W, n, k), G.seeded_acts(886, 64, k).astype(np.float16)
+        ref = orc.prefill(t, W, X, n, k)
+        for m in (1, 33, 64):
+            say(f"few rows {qname} m={m} n={n} k={k} {backend.prefill_choice(m, n, k, t, hip.compute_units)}")
+            y = hip.upload(np.full((m, n), np.nan, np.float32))
+            hip.quantized_matmul(w, hip.upload(X[:m]), y, m)
+            err = G.max_rel_err(y.download(np.float32, (m, n)), ref[:m])
+            assert err < PARITY_TOL, (m, n, k, err)

@@ -189,6 +189,23 @@ def test_prefill_choice_is_the_plan_or_a_thin_kernel(lib):
     assert lib.psn_qmatmul_prefill_choice(_ffi.Q4_0, 1, 1, 256, 256, 1, None, None, None, None) == _ffi.E_INVALID_ARG
 
 
+def test_few_rows_over_wide_matrices_take_a_kernel_that_exists(lib):
+    """Host arithmetic, more weight rows than 64 per compute unit: the choice for M <= 64 is the 64 x 64 kernel, a thin one, or an eight-wave tile of family 4, with a K split
+    that leaves two whole chunks per range, and family 4 is taken somewhere in every format; up to 64 rows per unit it is not (Q6_K rows of odd sizes aside)."""
+    for qt in (_ffi.Q4_0, _ffi.Q8_0, _ffi.Q4_K, _ffi.Q5_K, _ffi.Q6_K):
+        families = set()
+        for k in (256, 768, 2048, 5120, 8192):
+            for n in (16384, 16385, 18176, 28672, 128256):
+                for m in (1, 16, 17, 33, 48, 64):
+                    tm, tn, sp, wv = c = backend.prefill_choice(m, n, k, qt)
+                    assert wv in (4, 8, 64) and sp in (1, 2, 4, 8), (qt, m, n, k, c)
+                    assert wv != 4 or ((tm, tn) in {(64, 64), (64, 128), (128, 128), (256, 128)} and (n > 16384 or (qt == _ffi.Q6_K and k % 2048))), (qt, m, n, k, c)
+                    assert wv != 64 or (c[:2] == (64, 64) and (qt != _ffi.Q6_K or k % 2048 == 0)), (qt, m, n, k, c)
+                    assert sp == 1 or ((m * n) % 4 == 0 and k // 256 >= 2 * sp), (qt, m, n, k, c)
+                    families.add(wv)
+        assert 4 in families and 8 in families, (qt, families)
+
+
 def test_null_handles_are_rejected_without_a_device(lib):
     assert lib.psn_stream_sync(None) == _ffi.E_INVALID_ARG
     assert lib.psn_buf_free(None) == _ffi.E_INVALID_ARG
