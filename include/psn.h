@@ -282,8 +282,8 @@ int32_t psn_selftest_arith(psn_module *mod, psn_stream *s, psn_buf *out);
 
 /* ---- prefill matmul ----------------------------------------------------------------------- */
 
-/* Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k]; X fp16 [M][K], Y fp32 [M][N], weight tiles are
- * dequantized to fp16 (h = round to nearest even) in LDS and fed to fp16 MFMA with fp32
+/* Y[m][n] = sum_k h(deq(W)[n][k]) * X[m][k]; X fp16 [M][K], Y fp32 [M][N], weights are
+ * dequantized to fp16 (h = round to nearest even) in registers or LDS and fed to fp16 MFMA with fp32
  * accumulation.  qtype PSN_Q4_0 or PSN_Q8_0 (every kernel family below), PSN_Q4_K, PSN_Q5_K or PSN_Q6_K
  * (families 4, 8, 64 and 128, and for Q4_K / Q5_K family 16 on the 128x256 tile; planned by psn_qmatmul_prefill_plan_for;
  * their fp32 dequantization is restated operation by operation before the rounding to fp16).  Replaces the CUDA backend's quantized prefill
