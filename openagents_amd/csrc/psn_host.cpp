@@ -1386,10 +1386,10 @@ static int32_t check_prefill(const char *what, psn_module *mod, psn_stream *s, i
  * compute unit slow each other down; then the store of Y, the weights from memory, and with K cut the zero fill and the adds. */
 static int format_index(int32_t t) { return t == PSN_Q4_0 ? 0 : t == PSN_Q8_0 ? 1 : t == PSN_Q4_K ? 2 : t == PSN_Q5_K ? 3 : 4; }
 struct tile_cost { double base_us, clock, busy_from, shared, prologue_steps, split_us, add_us_per_mb, y_us_per_mb, w_us_per_million; };     /* steps of 64 of K */
-static double tile_estimate(const tile_cost &c, double step_us, int64_t M, int64_t N, int64_t K, int bm, int bn, int sp, int per_cu, int32_t cus, bool in_turn) {
+static double tile_estimate(const tile_cost &c, double step_us, int64_t M, int64_t N, int64_t K, int bm, int bn, int sp, int per_cu, int32_t cus) {
     const double y_mb = (double)(M * N) * 4e-6;
     const int64_t per_xcd = cus < 8 ? 1 : cus / 8, mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn, slots = per_xcd * per_cu;
-    const int64_t most = in_turn ? (nt + 7) / 8 * mt * sp : (mt * nt * sp + 7) / 8;
+    const int64_t most = (mt * nt * sp + 7) / 8;
     const double share = (double)(mt * nt * sp) / (double)(8 * most) * (0.5 + 0.5 * (double)M / (double)(mt * bm));
     const double one = ((double)((K / 256 + sp - 1) / sp * 4) + c.prologue_steps) * step_us;
     const auto round_us = [&](int64_t wgs) {
@@ -1440,9 +1440,6 @@ static const dense_cost k_packed_cost[] = {
 static const double k_unpack_base_us = 7.03, k_unpack_us[5] = {0.400, 0.554, 0.385, 0.427, 0.530};      /* per million weights */
 struct dense_plan { int bm, bn, ksplit; double us; };
 static dense_plan plan_dense(int64_t M, int64_t N, int64_t K, int32_t cus, bool packed) {
-    /* A copy of more than 128 MiB is workspace that a stream holds for good: there the choice between the families stays what it was when N tiles were dealt to the XCDs in
-     * turn, so that shapes whose tiles come out uneven do not start to ask for it (5120 x 13824, M = 3072: 344 us, 389-428 in the loop). */
-    const bool in_turn = !packed && N * K * 2 > ((int64_t)128 << 20);
     dense_plan best = {256, 256, 1, 1e300};
     const dense_cost *const from = packed ? k_packed_cost : k_dense_cost, *const to = packed ? k_packed_cost + 5 : k_dense_cost + 2;
     for (const dense_cost *c = from; c != to; ++c) {
@@ -1450,7 +1447,7 @@ static dense_plan plan_dense(int64_t M, int64_t N, int64_t K, int32_t cus, bool 
         for (int sp = 1; sp <= (packed ? 8 : 4); sp *= 2) {
             if (sp > 1 && ((M * N) % 4 != 0 || K / 256 < 2 * sp)) continue;
             if (tiles * sp > (1 << 22)) continue;                          /* a launch holds fewer than 2^32 threads */
-            double t = tile_estimate(c->cost, c->step_us, M, N, K, c->bm, c->bn, sp, c->per_cu, cus, in_turn);
+            double t = tile_estimate(c->cost, c->step_us, M, N, K, c->bm, c->bn, sp, c->per_cu, cus);
             /* A fresh copy of more than 50 million values is no longer in the caches when it is read, and 128 rows read it twice as often per product: at 7168 x 18944, M = 606,
              * the multiply takes 257 us instead of 158 (family 4 in all: 243).  Fitted over eight matrices of 70 to 235 million weights, M = 300 .. 2500: 0.3 % off the fastest
              * plan on average and 4 % at most with this term, 5 % and 51 % without it. */
@@ -1470,7 +1467,7 @@ extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int
 static double in_loop_estimate(const prefill_cost &c, int32_t qtype, int64_t M, int64_t N, int64_t K, int sp, int32_t cus) {
     const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
     const int by_regs = qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu, by_lds = 160 * 1024 / in_loop_lds(qtype, bm, bn);
-    return tile_estimate(c.cost, c.step_us[format_index(qtype)], M, N, K, bm, bn, sp, by_regs < by_lds ? by_regs : by_lds, cus, false);
+    return tile_estimate(c.cost, c.step_us[format_index(qtype)], M, N, K, bm, bn, sp, by_regs < by_lds ? by_regs : by_lds, cus);
 }
 static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
     double best = 1e300;

@@ -332,13 +332,13 @@ def test_prefill_planner_counts_the_workgroups_a_compute_unit_can_hold():
             assert held(name, max(8 * (16 * rt * chunk[fmt] + tm * 2048), 8192 * rt * tm)) == (2 if two else 1), name
 
 
-def test_prefill_planner_knows_that_xcds_fill_unevenly(lib):
-    """Shapes whose N tiles do not spread evenly over the eight XCDs, or that fill every round, where a planner blind to it picked the slower family:
-    (measured us) dense 689 against 467 at 5120 x 13824 M = 3072, 329 against 283 at 32000 x 4096 M = 1024; family 4 150 against 135 at 4096 x 4096
-    M = 4096, and 40 instead of 31 for Q4_K at 1536 x 5632 M = 640."""
+def test_prefill_planner_knows_how_full_the_rounds_are(lib):
+    """Shapes on which a planner that takes another deal of the tiles than the kernels', or is blind to how full a round is, picks the slower family (measured us, weights from
+    memory): 5120 x 13824 M = 3072 dense 352 .. 367, in the loop 397 .. 453 (N tiles dealt to the XCDs in turn would make it two rounds); 32000 x 4096 M = 1024 in the loop 265,
+    dense 284; 4096 x 4096 M = 4096 dense 115, in the loop 133.  Without a workspace the dense family is out."""
     for qt in (_ffi.Q4_0, _ffi.Q8_0, _ffi.Q4_K, _ffi.Q5_K, _ffi.Q6_K):
-        for workspace in (True, False):
-            assert backend.prefill_choice(3072, 5120, 13824, qt, workspace=workspace) == (256, 128, 1, 4)
+        assert backend.prefill_choice(3072, 5120, 13824, qt) == (256, 256, 1, 128)
+        assert backend.prefill_choice(3072, 5120, 13824, qt, workspace=False) == (256, 128, 1, 4)
     assert backend.prefill_choice(1024, 32000, 4096, _ffi.Q4_0) == (256, 128, 1, 4)
     assert backend.prefill_choice(4096, 4096, 4096, _ffi.Q4_0) == (256, 256, 1, 128)
     for qt in (_ffi.Q4_0, _ffi.Q4_K, _ffi.Q5_K):
