@@ -1377,9 +1377,11 @@ static int32_t check_prefill(const char *what, psn_module *mod, psn_stream *s, i
     return PSN_OK;
 }
 
-/* Cost models of family 4 (psn_prefill_frag.hip, psn_prefill_pp.hip) and of the dense family, fitted to launches timed on MI355X.  Family 4 and the dense family against each other: five
- * formats, 14 matrices (1000 x 2560, 2048 x 2048 .. 32000 x 4096), M = 65 .. 4096, 13135 calls, zero fill and dequantization pass included; weight lies on plans near the
- * fastest, whose estimates are off by 4 % rms; what they pick is 0.4 % off the fastest plan on average over 910 shapes and more than 10 % off in 11.
+/* Cost models of family 4 (psn_prefill_frag.hip, psn_prefill_pp.hip) and of the dense family, fitted to launches timed on MI355X: five formats, 1650 matrices of drawn layers (hidden
+ * 1024 .. 8192, feed-forward 2.5 to 3.6 times that), M = 65 .. 4096, every plan, weights from memory (copies rotate through 320 MB, as the layers of a model do), zero fill and
+ * dequantization pass included.  Plans near the fastest are estimated 4 % off rms; over 1150 other matrices what the estimates pick is 0.3 % off the fastest plan on average, more
+ * than 5 % off in 18 and more than 10 % in 6.  (Fitted to one copy of the weights, which the caches then hold, 64 x 64 tiles without a K cut came out too cheap: 1280 x 2560
+ * M = 246 of Q4_0 13.7 us, with K in two 11.2.)
  *
  * Both families deal tiles evenly to the eight XCDs: rounds of workgroups on the XCD with most of them x (K steps + prologue) x a step cost per tile and format; a round in which nearly
  * every compute unit multiplies rows of its own (those past the end repeat the last one, and count half) runs at a lower clock than an emptier one; workgroups that share a
@@ -1417,27 +1419,27 @@ struct prefill_cost {
     double step_us[5];                /* per 64 of K: Q4_0, Q8_0, Q4_K, Q5_K, Q6_K */
 };
 static const prefill_cost k_prefill_cost[] = {
-    {0, 2, 2, {3.51, 0.194, 0.296, 0.667, 5.44, 1.90, 0.449, 0.109, 0.0082}, {0.176, 0.214, 0.200, 0.214, 0.226}},
-    {1, 2, 1, {4.17, 0.172, 0.160, 0.798, 4.28, 1.90, 0.520, 0.093, 0.0073}, {0.255, 0.319, 0.288, 0.329, 0.409}},
-    {2, 1, 1, {3.22, 0.224, 0.511, 0.100, 7.83, 1.90, 0.533, 0.112, 0.0125}, {0.354, 0.420, 0.387, 0.409, 0.481}},
-    {4, 1, 1, {3.83, 0.187, 0.630, 0.100, 5.90, 2.19, 0.544, 0.042, 0.0199}, {0.702, 0.806, 0.757, 0.782, 0.814}},
+    {0, 2, 2, {2.526, 0.067, 0.207, 0.585, 4.636, 1.757, 0.319, 0.0854, 0.0134}, {0.220, 0.254, 0.232, 0.245, 0.281}},
+    {1, 2, 1, {3.672, 0.185, 0.175, 0.785, 3.027, 2.009, 0.364, 0.0726, 0.0144}, {0.265, 0.339, 0.296, 0.328, 0.433}},
+    {2, 1, 1, {2.674, 0.231, 0.506, 0.073, 7.847, 2.067, 0.377, 0.0825, 0.0394}, {0.363, 0.438, 0.394, 0.419, 0.509}},
+    {4, 1, 1, {3.857, 0.194, 0.594, 0.104, 3.620, 2.584, 0.434, 0.0345, 0.0454}, {0.755, 0.851, 0.796, 0.822, 0.868}},
 };
 /* The dense family (psn_prefill_dense.hip) behind a pass that rewrites the matrix as fp16, and over packed weights: there all five tiles, fitted to 3175 launches of
  * the multiply alone (18 matrices, M = 16 .. 4096; what the estimates pick is 0.7 % off the fastest on average, more than 10 % off in 4 of 262 shapes).  The tiles below 256
  * columns are for packed weights only: explicit plans cannot name them, and a plan of psn_qmatmul_prefill is one that can be run explicitly. */
-struct dense_cost { int bm, bn, per_cu; tile_cost cost; double step_us; };
+struct dense_cost { int bm, bn, per_cu; tile_cost cost; double step_us, fresh_us_per_million; };
 static const dense_cost k_dense_cost[] = {
-    {256, 256, 1, {2.38, 0.430, 0.673, 0.016, 4.04, 4.03, 0.462, 0.126, 0.0791}, 0.920},
-    {128, 256, 1, {2.11, 0.517, 0.627, 0.890, 1.85, 4.32, 0.417, 0.162, 0.0058}, 0.512},
+    {256, 256, 1, {2.452, 0.397, 0.491, 0.014, 2.080, 4.137, 0.367, 0.1156, 0.0587}, 0.976, 0.22},
+    {128, 256, 1, {2.126, 0.479, 0.431, 0.905, 1.471, 4.139, 0.351, 0.1561, 0.0050}, 0.525, 0.64},
 };
 static const dense_cost k_packed_cost[] = {
-    {256, 256, 1, {2.04, 0.232, 0.688, 0.016, 9.23, 3.60, 0.543, 0.026, 0.0170}, 1.038},
-    {128, 256, 1, {2.23, 0.639, 0.328, 0.890, 7.57, 2.04, 0.539, 0.021, 0.0992}, 0.455},
-    {128, 128, 1, {2.15, 0.696, 0.318, 0.014, 9.71, 2.01, 0.452, 0.006, 0.0842}, 0.258},
-    {64, 128, 1, {2.04, 0.379, 0.198, 0.014, 8.71, 2.02, 0.434, 0.036, 0.1321}, 0.179},
-    {64, 64, 2, {2.60, 0.180, 0.442, 0.981, 2.28, 1.98, 0.499, 0.192, 0.1146}, 0.135},
+    {256, 256, 1, {2.04, 0.232, 0.688, 0.016, 9.23, 3.60, 0.543, 0.026, 0.0170}, 1.038, 0.0},
+    {128, 256, 1, {2.23, 0.639, 0.328, 0.890, 7.57, 2.04, 0.539, 0.021, 0.0992}, 0.455, 0.0},
+    {128, 128, 1, {2.15, 0.696, 0.318, 0.014, 9.71, 2.01, 0.452, 0.006, 0.0842}, 0.258, 0.0},
+    {64, 128, 1, {2.04, 0.379, 0.198, 0.014, 8.71, 2.02, 0.434, 0.036, 0.1321}, 0.179, 0.0},
+    {64, 64, 2, {2.60, 0.180, 0.442, 0.981, 2.28, 1.98, 0.499, 0.192, 0.1146}, 0.135, 0.0},
 };
-static const double k_unpack_base_us = 7.03, k_unpack_us[5] = {0.400, 0.554, 0.385, 0.427, 0.530};      /* per million weights */
+static const double k_unpack_base_us = 5.43, k_unpack_us[5] = {0.382, 0.571, 0.405, 0.467, 0.604};      /* per million weights */
 struct dense_plan { int bm, bn, ksplit; double us; };
 static dense_plan plan_dense(int64_t M, int64_t N, int64_t K, int32_t cus, bool packed) {
     dense_plan best = {256, 256, 1, 1e300};
@@ -1449,9 +1451,10 @@ static dense_plan plan_dense(int64_t M, int64_t N, int64_t K, int32_t cus, bool 
             if (tiles * sp > (1 << 22)) continue;                          /* a launch holds fewer than 2^32 threads */
             double t = tile_estimate(c->cost, c->step_us, M, N, K, c->bm, c->bn, sp, c->per_cu, cus);
             /* A fresh copy of more than 50 million values is no longer in the caches when it is read, and 128 rows read it twice as often per product: at 7168 x 18944, M = 606,
-             * the multiply takes 257 us instead of 158 (family 4 in all: 243).  Fitted over eight matrices of 70 to 235 million weights, M = 300 .. 2500: 0.3 % off the fastest
-             * plan on average and 4 % at most with this term, 5 % and 51 % without it. */
-            if (!packed && c->bm == 128 && N * K > 50000000) t += (double)(N * K - 50000000) * 1e-6;
+             * the multiply takes 257 us on them instead of 158 (family 4 in all: 243).  Over 150 drawn matrices of 45 to 230 million weights, M = 250 .. 4096, none of them fitted to, what
+             * the estimates pick is 0.5 % off the fastest plan on average.  It also drives out what the launches around it would have found in the caches: 4096 x 14336 of Q4_K, M = 2048, alone takes
+             * 222 us, 8 less than in the loop, but makes the seven launches of its layer 4 to 11 us longer; the 7 us count half of that (70 drawn layers: neither slower nor faster). */
+            if (!packed && N * K > 50000000) t += 7.0 + c->fresh_us_per_million * ((double)(N * K) * 1e-6 - 50.0);
             if (t < best.us) best = {c->bm, c->bn, sp, t};
         }
     }
@@ -1482,12 +1485,13 @@ static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32
 
 /* At most 64 rows: which kernel streams the weights.  psn_prefill_<fmt>_thin_<tm>_<rt> (psn_prefill_thin.hip, 16 tm rows of X and 16 rt
  * of W per workgroup) against the 64 x 64 kernel: psn_prefill_<fmt>_skinny for Q4_0 and Q8_0, family 4's tile of that size for the K-quants (Q6_K only where rows are
- * whole 16-byte words, as family 64 is documented; elsewhere family 4 competes by its own name).  Checked on MI355X against the explicit plans over five formats, eighteen matrices
- * and M = 1 .. 64 (9800 launches): what the estimates pick is 1.3 % off the fastest on average and more than 10 % off in 21 of 700 shapes (family 4's estimates are
- * raised by 1.3 and 1.22, the factors at which no shape gets slower that thin kernels serve well).  An
+ * whole 16-byte words, as family 64 is documented; elsewhere family 4 competes by its own name).  Checked on MI355X against the explicit plans over 1000 drawn
+ * matrices of five formats, M = 1 .. 64 (weights from memory): what the estimates pick is 1.6 % off the fastest on average and more than 10 % off in 54 (family 4's estimates, fitted to
+ * more than 64 rows, are raised by k_in_loop_bias: of 1.0 to 1.35 the factor at which fewest shapes are slower than a thin kernel makes them).  An
  * estimate is a launch, then per round of workgroups the first loads and a chain per chunk of a wave, and the work that the waves of a SIMD
  * share: decode per weight row, X per row of it.  The 64 x 64 kernel cuts K only while the weight rows
  * alone leave half of the compute units without a workgroup.  At rt = 4 a cut of K did not pay. */
+static const double k_in_loop_bias = 1.15;
 struct weight_stream_plan { int rt, ksplit; double us; };
 static bool may_cut_k(int64_t M, int64_t N, int64_t K, int sp) { return sp == 1 || ((M * N) % 4 == 0 && K / 256 >= 2 * sp); }
 static int stream64_ksplit(int64_t M, int64_t N, int64_t K, int32_t cus) {
@@ -1513,7 +1517,7 @@ static weight_stream_plan plan_weight_stream(int32_t qtype, int64_t M, int64_t N
         const int64_t nt = (N + 63) / 64;
         const int sp = stream64_ksplit(M, N, K, cus);
         const double rounds = (double)((nt * sp + cus - 1) / cus);
-        best = {0, sp, f >= 2 ? 1.3 * in_loop_estimate(k_prefill_cost[0], qtype, M, N, K, sp, cus)
+        best = {0, sp, f >= 2 ? k_in_loop_bias * in_loop_estimate(k_prefill_cost[0], qtype, M, N, K, sp, cus)
                               : 3.69 + rounds * (double)((C + sp - 1) / sp) * k_skinny_chunk_us[f] + 0.97 * cut_us(sp) + 0.184 * y_mb};
     }
     for (int rt = 1; rt <= 4; rt *= 2) {
@@ -1575,7 +1579,7 @@ static int32_t prefill_choice(int32_t qtype, int64_t M, int64_t N, int64_t K, in
      * with up to 16 rows of X the thin kernels read W as fast as memory gives it (Q4_0 37 us there). */
     int32_t bm, bn, sp;
     if (*waves == 4 || (M > 16 && N > 64 * (int64_t)cus)) {
-        const double t = 1.22 * plan_in_loop(qtype, M, N, K, cus, &bm, &bn, &sp);
+        const double t = k_in_loop_bias * plan_in_loop(qtype, M, N, K, cus, &bm, &bn, &sp);
         if (t <= p.us) {
             *tile_m = bm;
             *tile_n = bn;
