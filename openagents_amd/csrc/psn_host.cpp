@@ -1466,11 +1466,16 @@ extern "C" int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int
                                             int32_t *waves) {
     return psn_qmatmul_prefill_plan_for(PSN_Q4_0, M, N, K, cus, tile_m, tile_n, ksplit, waves);
 }
+/* 256 x 128 tiles that leave at least five of sixteen compute units without a workgroup run the kernels that multiply 32 x 32 x 16 (_pp32; psn_prefill_pp.hip has both sides) */
+static bool leaves_units_idle(int64_t workgroups, int32_t cus) { return workgroups * 16 <= (int64_t)cus * 11; }
 /* family 4: one tile's estimate; and the tile and the K split with the smallest one; K ranges hold at least two 256-wide chunks */
 static double in_loop_estimate(const prefill_cost &c, int32_t qtype, int64_t M, int64_t N, int64_t K, int sp, int32_t cus) {
     const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
     const int by_regs = qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu, by_lds = 160 * 1024 / in_loop_lds(qtype, bm, bn);
-    return tile_estimate(c.cost, c.step_us[format_index(qtype)], M, N, K, bm, bn, sp, by_regs < by_lds ? by_regs : by_lds, cus);
+    const int64_t wgs = (M + bm - 1) / bm * ((N + bn - 1) / bn) * sp;
+    /* (fitted to the 16 x 16 x 32 kernels; the others take less, least where fewer than nine of sixteen units have a workgroup) */
+    const double part = bm != 256 || !leaves_units_idle(wgs, cus) ? 1.0 : wgs * 16 <= (int64_t)cus * 9 ? 0.945 : 0.975;
+    return tile_estimate(c.cost, part * c.step_us[format_index(qtype)], M, N, K, bm, bn, sp, by_regs < by_lds ? by_regs : by_lds, cus);
 }
 static double plan_in_loop(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
     double best = 1e300;
@@ -1778,7 +1783,7 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
         snprintf(name, sizeof name, "psn_prefill_%s_wide", fmt_name(qtype));
         return launch(mod, s, name, (unsigned)blocks, 256, (unsigned)lds, &a);
     }
-    snprintf(name, sizeof name, "psn_prefill_%s_m%d_n%d%s", fmt_name(qtype), bm, bn, waves == 16 ? "_ws" : pp ? "_pp" : "");
+    snprintf(name, sizeof name, "psn_prefill_%s_m%d_n%d%s", fmt_name(qtype), bm, bn, waves == 16 ? "_ws" : !pp ? "" : bm == 256 && leaves_units_idle(nt * mt * ksplit, mod->ctx->compute_units) ? "_pp32" : "_pp");
     return launch(mod, s, name, (unsigned)blocks, (unsigned)(64 * (waves == 16 || pp ? 8 : 4)), (unsigned)lds, &a);
 }
 

@@ -97,32 +97,47 @@ PSN_DEV f32x4 mfma16(u32x4 w, u32x4 x, f32x4 c) {
  * MFMA's layout, 64 bytes of sixteen rows at a time: 4001 x 14336 x 4096 396 us instead of 389, 4001 x 1024 x 4096 on 256 x 256 tiles 87 instead of 78), else words: atomic adds
  * from the MFMA's layout take several times as long (512 x 1024 x 4096 in four ranges, 64 x 128 tiles: 33.3 us instead of 13.5). */
 template <int TN> constexpr int wave_out_bytes() { return 16 * (16 * TN + 4) * 4; }
-template <int TN> PSN_DEV void store_tiles(const psn_prefill_args &a, int row0, int col0, int lane, const f32x4 (&v)[TN], u32 out) {
-    constexpr int PITCH = (16 * TN + 4) * 4;
-    UNROLL for (int j = 0; j < TN; ++j) lds_write128(out + (u32)((lane & 15) * PITCH + 64 * j + 16 * (lane >> 4)), __builtin_bit_cast(u32x4, v[j]));
+/* the rows' second half of the way: COLS columns of ROWS rows, COLS + 4 words apart at `out`, written by this wave */
+template <int ROWS, int COLS> PSN_DEV void store_rows(const psn_prefill_args &a, int row0, int col0, int lane, u32 out) {
+    constexpr int PITCH = (COLS + 4) * 4, P16 = COLS / 4, T = ROWS * P16 / 64;
     lds_wait();
     if (a.ksplit == 1 && (a.N & 3) == 0) {
-        u32x4 w[TN];
-        UNROLL for (int t = 0; t < TN; ++t) w[t] = lds_read128<0>(out + (u32)((t * 64 + lane) / (4 * TN) * PITCH + (t * 64 + lane) % (4 * TN) * 16));
+        u32x4 w[T];
+        UNROLL for (int t = 0; t < T; ++t) w[t] = lds_read128<0>(out + (u32)((t * 64 + lane) / P16 * PITCH + (t * 64 + lane) % P16 * 16));
         lds_wait();
         tie(w);
-        UNROLL for (int t = 0; t < TN; ++t) {
-            const int row = row0 + (t * 64 + lane) / (4 * TN), col = col0 + (t * 64 + lane) % (4 * TN) * 4;
+        UNROLL for (int t = 0; t < T; ++t) {
+            const int row = row0 + (t * 64 + lane) / P16, col = col0 + (t * 64 + lane) % P16 * 4;
             if (row < a.M && col < a.N) *reinterpret_cast<u32x4 *>(a.Y + (int64_t)row * a.N + col) = w[t];
         }
         return;
     }
-    u32 w[4 * TN];
-    UNROLL for (int t = 0; t < 4 * TN; ++t) w[t] = lds_read32(out + (u32)((t * 64 + lane) / (16 * TN) * PITCH + (t * 64 + lane) % (16 * TN) * 4));
+    u32 w[4 * T];
+    UNROLL for (int t = 0; t < 4 * T; ++t) w[t] = lds_read32(out + (u32)((t * 64 + lane) / COLS * PITCH + (t * 64 + lane) % COLS * 4));
     lds_wait();
-    UNROLL for (int t = 0; t < 4 * TN; ++t) {
+    UNROLL for (int t = 0; t < 4 * T; ++t) {
         tie1(w[t]);
-        const int row = row0 + (t * 64 + lane) / (16 * TN), col = col0 + (t * 64 + lane) % (16 * TN);
+        const int row = row0 + (t * 64 + lane) / COLS, col = col0 + (t * 64 + lane) % COLS;
         if (row >= a.M || col >= a.N) continue;
         float *y = a.Y + (int64_t)row * a.N + col;
         if (a.ksplit == 1) *y = __uint_as_float(w[t]);
         else unsafeAtomicAdd(y, __uint_as_float(w[t]));
     }
+}
+template <int TN> PSN_DEV void store_tiles(const psn_prefill_args &a, int row0, int col0, int lane, const f32x4 (&v)[TN], u32 out) {
+    constexpr int PITCH = (16 * TN + 4) * 4;
+    UNROLL for (int j = 0; j < TN; ++j) lds_write128(out + (u32)((lane & 15) * PITCH + 64 * j + 16 * (lane >> 4)), __builtin_bit_cast(u32x4, v[j]));
+    store_rows<16, 16 * TN>(a, row0, col0, lane, out);
+}
+/* The same from 32 x 32 x 16 products: lane (h, m) = (lane / 32, lane % 32) holds columns 32 j + 8 g + 4 h .. + 3 of row m in registers 4 g .. 4 g + 3; 32 rows of 32 TN + 4 words. */
+template <int TN> constexpr int wave_out_bytes32() { return 32 * (32 * TN + 4) * 4; }
+template <int TN> PSN_DEV void store_tiles(const psn_prefill_args &a, int row0, int col0, int lane, const float16_t (&v)[TN], u32 out) {
+    constexpr int PITCH = (32 * TN + 4) * 4;
+    UNROLL for (int j = 0; j < TN; ++j) UNROLL for (int g = 0; g < 4; ++g) {
+        const f32x4 p = {v[j][4 * g], v[j][4 * g + 1], v[j][4 * g + 2], v[j][4 * g + 3]};
+        lds_write128(out + (u32)((lane & 31) * PITCH + 128 * j + 32 * g + 16 * (lane >> 5)), __builtin_bit_cast(u32x4, p));
+    }
+    store_rows<32, 32 * TN>(a, row0, col0, lane, out);
 }
 
 #endif

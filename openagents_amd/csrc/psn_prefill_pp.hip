@@ -15,8 +15,9 @@
  *
  * What bounds it, Q4_K 512 x 14336 x 4096: 69 us; 53 without the decode and its LDS writes, 53 without MFMAs, 57 without loads, so vector instructions, LDS traffic
  * (176 KB per step, 1.3 times as long as the MFMAs) and MFMAs add up; on a full chip power as well (on zero weights, the same instructions, a fifth faster), which is why the MFMAs
- * are 16 x 16 x 32: 32 x 32 x 16 took 70 us there and 275 at M = 2048 instead of 257, but 57 instead of 60 on half-filled rounds, which the smaller tiles
- * serve now.  Splitting the roles (eight multiplying and eight staging waves) measured 2-8 % slower, running the two waves of a SIMD in strictly opposite phases 10-15 %, sixteen
+ * are 16 x 16 x 32 there (275 us -> 257 at M = 2048).  With fewer than about 180 workgroups power does not bind, the MFMAs that ride shorter do, and the _pp32 kernels multiply
+ * 32 x 32 x 16, half as many: Q4_K, weights from memory, five formats and 110 matrices, geometric mean of 32 x 32 over 16 x 16 by workgroups (of 256 compute units): up to 100 1.07 x,
+ * 132 .. 150 1.06, 150 .. 165 1.04, 165 .. 180 1.03, 180 .. 195 1.00, 195 .. 256 0.985, more 0.99.  Splitting the roles (eight multiplying and eight staging waves) measured 2-8 % slower, running the two waves of a SIMD in strictly opposite phases 10-15 %, sixteen
  * waves with half the tile each 15 %.
  */
 #include "psn_args.h"
@@ -40,15 +41,31 @@ template <int OFF> PSN_DEV void lds_write128o(u32 addr, u32x4 v) { asm volatile(
 /* does piece p of a decode (see there) end in an LDS write? */
 constexpr bool pp_piece_writes(int p) { return p >= 2 && (p & 3) == 1; }
 
-template <typename WF, int BM, int BN, int WM, int NS>
+/* D = W X^T either way; KK: K slices per step */
+template <int MF> struct pp_mfma;
+template <> struct pp_mfma<16> {
+    typedef f32x4 acc;
+    static constexpr int KK = 2;
+    static PSN_DEV acc mul(u32x4 w, u32x4 x, acc c) { return mfma16(w, x, c); }
+    template <int TN> static constexpr int out_bytes() { return wave_out_bytes<TN>(); }
+};
+template <> struct pp_mfma<32> {
+    typedef float16_t acc;
+    static constexpr int KK = 4;
+    static PSN_DEV acc mul(u32x4 w, u32x4 x, acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, w), __builtin_bit_cast(half8_t, x), c, 0, 0, 0); }
+    template <int TN> static constexpr int out_bytes() { return wave_out_bytes32<TN>(); }
+};
+
+template <typename WF, int BM, int BN, int WM, int MF, int NS>
 PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
-    constexpr int MF = 16, WN = 8 / WM, TM = BM / WM / MF, TN = BN / WN / MF, KK = 2;     /* K slices per step */
+    typedef pp_mfma<MF> MMA;
+    constexpr int WN = 8 / WM, TM = BM / WM / MF, TN = BN / WN / MF, KK = MMA::KK;
     constexpr int NB = 8, PARTS = 4;                        /* quant bytes per thread and step, threads per weight row */
     static_assert(BN == 128, "512 threads, four to a row");
     constexpr int SPREAD = WF::SPREAD;
     constexpr int XBYTES = BM * 128, WBYTES = BN * 128;
     constexpr int NX = BM / 64;                             /* X loads per wave and step */
-    static_assert(TM >= 1 && TN >= 1 && NX >= 1 && NS * XBYTES + 2 * WBYTES <= 160 * 1024, "tile");
+    static_assert(TM >= 1 && TN >= 1 && NX >= 1 && NS * XBYTES + 2 * WBYTES <= 160 * 1024 && 8 * MMA::template out_bytes<TN>() <= NS * XBYTES, "tile");
     extern __shared__ uint4 psn_smem[];
     lds_char *const lds_ptr = (lds_char *)psn_smem;
     const u32 lds0 = (u32)(uintptr_t)lds_ptr;
@@ -61,8 +78,8 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
     if (!place_workgroup<BM, BN, 512>(a, at)) return;       /* whole workgroup leaves together */
     const int m0 = at.m0, n0 = at.n0, c_begin = at.c0, nq = at.chunks, nsteps = nq * 4;
 
-    f32x4 acc[TM][TN];
-    UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4)(0.f);
+    typename MMA::acc acc[TM][TN];
+    UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int j = 0; j < TN; ++j) acc[i][j] = (typename MMA::acc)(0.f);
 
     /* X: 16-byte word s of a stage in LDS order is row s / 8, position s % 8, which holds chunk (s % 8) ^ tile_swz(row) */
     u32 xoff[NX];
@@ -169,7 +186,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
         constexpr int kk = decltype(kc)::value;
         UNROLL for (int j = 0; j < TN; ++j) UNROLL for (int i = 0; i < TM; ++i) {
             __builtin_amdgcn_sched_barrier(0);
-            acc[i][j] = mfma16(wf[kk][j], xf[kk][i], acc[i][j]);
+            acc[i][j] = MMA::mul(wf[kk][j], xf[kk][i], acc[i][j]);
             __builtin_amdgcn_sched_barrier(0);
             behind(j * TM + i);
         }
@@ -219,6 +236,10 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
         }                                                                                                                  \
         slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<0>());                                                           \
         slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<1>());                                                           \
+        if constexpr (KK == 4) {                                                                                           \
+            slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<KK - 2>());                                                  \
+            slice(c, J == 3 ? wother : w, pf_int<J>(), pf_int<KK - 1>());                                                  \
+        }                                                                                                                  \
         constexpr int KEEP = (NS - 2) * NX + ((J + 1) % 4 < NS - 2 ? WF::LOADS : 0);                                       \
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(KEEP) : "memory");                               \
         UNROLL for (int kk = HK; kk < KK; ++kk) { tie(xf[kk]); tie(wf[kk]); }                                              \
@@ -234,6 +255,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
 #undef PSN_PP_CHUNK
 #undef PSN_PP_STEP
     multiply(pf_int<HK>(), [](int) {});
+    if constexpr (KK == 4) multiply(pf_int<KK - 1>(), [](int) {});
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");       /* nothing is on its way into LDS any more */
     /* the last raw loads were for nothing, but their registers belong to them until they have landed */
     WF::template landed<NB>(wa);
@@ -244,15 +266,15 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
     asm volatile("" : "+v"(tid_out));
     const int wm_o = (tid_out >> 6) / WN, wn_o = (tid_out >> 6) % WN, lane_o = tid_out & 63;
     UNROLL for (int i = 0; i < TM; ++i)
-        store_tiles<TN>(a, m0 + wm_o * (BM / WM) + MF * i, n0 + wn_o * (BN / WN), lane_o, acc[i], lds0 + (u32)((tid_out >> 6) * wave_out_bytes<TN>()));
+        store_tiles<TN>(a, m0 + wm_o * (BM / WM) + MF * i, n0 + wn_o * (BN / WN), lane_o, acc[i], lds0 + (u32)((tid_out >> 6) * MMA::template out_bytes<TN>()));
 }
 
 
-#define PSN_PP(fmt, WF, BM, BN, WM, NS)                                                                                      \
-    extern "C" __global__ void __launch_bounds__(512) psn_prefill_##fmt##_m##BM##_n##BN##_pp(const psn_prefill_args a) {    \
-        prefill_pp_body<WF, BM, BN, WM, NS>(a);                                                                              \
+#define PSN_PP(fmt, suffix, WF, BM, BN, WM, MF, NS)                                                                          \
+    extern "C" __global__ void __launch_bounds__(512) psn_prefill_##fmt##_m##BM##_n##BN##_pp##suffix(const psn_prefill_args a) { \
+        prefill_pp_body<WF, BM, BN, WM, MF, NS>(a);                                                                          \
     }
-#define PSN_PP_FAMILY(fmt, WF) PSN_PP(fmt, WF, 256, 128, 4, 4)
+#define PSN_PP_FAMILY(fmt, WF) PSN_PP(fmt, , WF, 256, 128, 4, 16, 4) PSN_PP(fmt, 32, WF, 256, 128, 4, 32, 4)
 
 #ifdef PSN_BUILD_PP_Q4_0
 PSN_PP_FAMILY(q4_0, PpQ4_0)

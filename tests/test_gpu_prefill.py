@@ -13,6 +13,7 @@ import pytest
 
 import ggufref as G
 from openagents_amd import _ffi, backend
+from openagents_amd.records import launched_kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -517,3 +518,26 @@ def test_few_rows_over_more_weight_rows_than_one_round_of_64(hip, orc, qname):
             hip.quantized_matmul(w, hip.upload(X[:m]), y, m)
             err = G.max_rel_err(y.download(np.float32, (m, n)), ref[:m])
             assert err < PARITY_TOL, (m, n, k, err)
+
+
+@pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
+def test_256_row_tiles_on_either_side_of_the_line_between_their_two_kernels(hip, orc, qname):
+    """11 of 16 compute units with a workgroup: up to there 256 x 128 tiles multiply 32 x 32 x 16, beyond 16 x 16 x 32.  Ragged rows and columns, rows of Y that are whole 16-byte words
+    and not, K cut and not.  fp16 products are exact in fp32, so what differs from float64 over the oracle's fp16 weights
+    is the rounding of at most 1280 sums: PARITY_TOL is far above sqrt(1280) * 2^-24."""
+    t = getattr(orc, qname)
+    line = hip.compute_units * 11 // 16
+    for m, k, ksplit in ((2041, 256, 1), (1793, 512, 1), (260, 1280, 4), (516, 1024, 2)):
+        rows = -(-m // 256) * ksplit
+        for n, name in ((line // rows * 128, "_pp32"), (line // rows * 128 - 127, "_pp32"), (line // rows * 128 + 1, "_pp"), (line // rows * 128 + 126, "_pp")):
+            if ksplit > 1 and (m * n) % 4:
+                continue
+            W = weights(orc, qname, 890, n, k)
+            w, X = hip.upload_weight(t, W, n, k), G.seeded_acts(891, m, k).astype(np.float16)
+            y = hip.upload(np.full((m, n), np.nan, np.float32))
+            x = hip.upload(X)
+            say(f"256-row tiles {qname} m={m} n={n} k={k} ksplit={ksplit}")
+            assert launched_kernels(hip, lambda: hip.quantized_matmul(w, x, y, m, (256, 128, ksplit, 4))).endswith(name), (m, n, k, ksplit)
+            ref = X.astype(np.float64) @ orc.dequantize(t, W, k).reshape(n, k).astype(np.float16).astype(np.float64).T
+            err = G.max_rel_err(y.download(np.float32, (m, n)), ref)
+            assert err < PARITY_TOL, (m, n, k, ksplit, err)
