@@ -78,6 +78,7 @@ struct psn_fill_args {
     uint32_t *p;          /* 16-byte aligned */
     int64_t n16;          /* number of 16-byte words to zero */
 };
+#define PSN_FILL_PLAIN_N16 8192   /* psn_fill_zero: up to here 16-byte stores, beyond 8-byte ones that go through to memory */
 
 struct psn_calib_args {
     const uint8_t *src;   /* 16-byte aligned */

@@ -1625,7 +1625,7 @@ static int32_t fill_zero_y(psn_module *mod, psn_stream *s, psn_buf *Y, int64_t M
     psn_fill_args f;
     f.p = (uint32_t *)Y->p;
     f.n16 = M * N / 4;
-    const int64_t fb = (f.n16 + 255) / 256;
+    const int64_t fb = ((f.n16 <= PSN_FILL_PLAIN_N16 ? f.n16 : 2 * f.n16) + 255) / 256;      /* a thread for every store, up to 4 MB */
     return launch(mod, s, "psn_fill_zero", (unsigned)(fb > 2048 ? 2048 : fb), 256, 0, &f);
 }
 static void prefill_args(psn_prefill_args *a, const void *W, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N, int64_t K, int32_t ksplit, int64_t row_bytes) {

@@ -1193,10 +1193,17 @@ PSN_DEV void prefill_unpack_body(const psn_unpack_args &a) {
  * 5 unpack kernels of all formats. */
 
 #if !defined(PSN_BUILD_ONLY) || PSN_BUILD_PF == 0
-/* zero fill with vector stores (graph-safe stand-in for a memset node).  The stores go through to memory: the adds that follow run at the device's coherence point, and a launch
- * that leaves nothing dirty in the eight L2s ends sooner (fill + K-cut kernel, 203 rows of Q5_K over 1024 x 4096: 11.60 us, 11.84 with plain stores, 12.03 with non-temporal ones). */
+/* zero fill with vector stores (graph-safe stand-in for a memset node).  Beyond 128 KB the stores go through to memory: the adds that follow run at the device's coherence point, and a
+ * launch that leaves nothing dirty in the eight L2s ends sooner; below, plain ones are the faster.  260 calls that cut K, fill and kernel together, plain against through stores with a
+ * thread for each: up to 64 KB 0.998, 64 .. 128 KB 0.999, 128 .. 256 KB 1.001, 0.25 .. 1 MB 1.003, 1 .. 4 MB 1.007 (with two stores to a thread the through stores lose 0.5 % up to
+ * 0.5 MB).  Non-temporal stores are slower than either. */
 extern "C" __global__ void __launch_bounds__(256) psn_fill_zero(const psn_fill_args a) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    if (a.n16 <= PSN_FILL_PLAIN_N16) {
+        uint4 *p = reinterpret_cast<uint4 *>(a.p);
+        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n16; i += stride) p[i] = make_uint4(0, 0, 0, 0);
+        return;
+    }
     unsigned long long *p = reinterpret_cast<unsigned long long *>(a.p);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < 2 * a.n16; i += stride) __hip_atomic_store(p + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

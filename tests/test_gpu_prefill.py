@@ -541,3 +541,16 @@ def test_256_row_tiles_on_either_side_of_the_line_between_their_two_kernels(hip,
             ref = X.astype(np.float64) @ orc.dequantize(t, W, k).reshape(n, k).astype(np.float16).astype(np.float64).T
             err = G.max_rel_err(y.download(np.float32, (m, n)), ref)
             assert err < PARITY_TOL, (m, n, k, ksplit, err)
+
+
+@pytest.mark.parametrize("m,n", [(4, 1), (64, 512), (64, 516), (1024, 1024), (1028, 1025)])
+def test_zero_fill_in_front_of_a_k_cut_at_the_lines_between_its_stores(hip, orc, m, n):
+    """One 16-byte word, 128 KB of Y (the last with plain stores) and a little more, 4 MB (the last with a thread for every store) and a little more: nothing of what Y held is left.
+    fp16 products are exact in fp32: PARITY_TOL is far above the rounding of 512 sums."""
+    k = 512
+    W = weights(orc, "Q4_0", 895, n, k)
+    X = G.seeded_acts(896, m, k).astype(np.float16)
+    w, x, y = hip.upload_weight(orc.Q4_0, W, n, k), hip.upload(X), hip.upload(np.full((m, n), np.nan, np.float32))
+    hip.quantized_matmul(w, x, y, m, (64, 64, 2, 4))
+    ref = X.astype(np.float64) @ orc.dequantize(orc.Q4_0, W, k).reshape(n, k).astype(np.float16).astype(np.float64).T
+    assert G.max_rel_err(y.download(np.float32, (m, n)), ref) < PARITY_TOL
