@@ -79,7 +79,7 @@ def build(jobs: int = 0, verbose: bool = True, reuse_device: bool = False) -> st
     jobs = jobs or min(8, os.cpu_count() or 1)
     todo = [(stem, src, defs) for stem, src, defs in CODE_OBJECTS if os.path.exists(os.path.join(CSRC, src))]
 
-    device_headers = ["psn_args.h", "psn_device.h", "psn_prefill_common.h", "psn_prefill_formats.h"]
+    device_headers = ["psn_args.h", "psn_device.h", "psn_prefill_common.h", "psn_prefill_formats.h", "psn_prefill_lds.h"]
 
     def compile_co(item):
         stem, src, defs = item

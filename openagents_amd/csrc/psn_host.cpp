@@ -7,6 +7,7 @@
  */
 #include "../../include/psn.h"
 #include "psn_args.h"
+#include "psn_prefill_lds.h"
 #include "psn_noalloc.h"
 
 #include <hip/hip_runtime_api.h>
@@ -1386,7 +1387,7 @@ static int32_t check_prefill(const char *what, psn_module *mod, psn_stream *s, i
  * Both families deal tiles evenly to the eight XCDs: rounds of workgroups on the XCD with most of them x (K steps + prologue) x a step cost per tile and format; a round in which nearly
  * every compute unit multiplies rows of its own (those past the end repeat the last one, and count half) runs at a lower clock than an emptier one; workgroups that share a
  * compute unit slow each other down; then the store of Y, the weights from memory, and with K cut the zero fill and the adds. */
-static int format_index(int32_t t) { return t == PSN_Q4_0 ? 0 : t == PSN_Q8_0 ? 1 : t == PSN_Q4_K ? 2 : t == PSN_Q5_K ? 3 : 4; }
+static int format_index(int32_t t) { return t == PSN_Q4_0 ? PSN_F_Q4_0 : t == PSN_Q8_0 ? PSN_F_Q8_0 : t == PSN_Q4_K ? PSN_F_Q4_K : t == PSN_Q5_K ? PSN_F_Q5_K : PSN_F_Q6_K; }
 struct tile_cost { double base_us, clock, busy_from, shared, prologue_steps, split_us, add_us_per_mb, y_us_per_mb, w_us_per_million; };     /* steps of 64 of K */
 static double tile_estimate(const tile_cost &c, double step_us, int64_t M, int64_t N, int64_t K, int bm, int bn, int sp, int per_cu, int32_t cus) {
     const double y_mb = (double)(M * N) * 4e-6;
@@ -1403,15 +1404,6 @@ static double tile_estimate(const tile_cost &c, double step_us, int64_t M, int64
     return sp > 1 ? t + c.split_us + (0.2 + c.add_us_per_mb * sp) * y_mb : t;
 }
 
-/* LDS of family 4's eight-wave kernels.  256 rows (psn_prefill_pp.hip): a ring of four stages of X and two fp16 weight tiles, 128 bytes per row.  Fewer
- * (psn_prefill_frag.hip): two stages of X of 256 bytes per row, two chunks of the weight rows in 1 KB pieces and one piece that nobody reads, Q6_K's last words of a row apart,
- * the unpacked scales of Q4_K and Q5_K. */
-static int in_loop_lds(int32_t qtype, int bm, int bn) {
-    static const int words[5] = {9, 17, 9, 11, 13};
-    const int f = format_index(qtype);
-    if (bm == 256) return (4 * bm + 2 * bn) * 128;
-    return 2 * (bm * 256 + ((bn * words[f] + 63) / 64 + 1) * 1024 + (f == 4 ? bn * 8 : 0)) + (f == 2 || f == 3 ? bn * 64 : 0);
-}
 /* Family 4.  per_cu: workgroups a compute unit holds by its registers, per_cu_q6_K of Q6_K's kernel. */
 struct prefill_cost {
     int tile, per_cu, per_cu_q6_K;    /* index into k_prefill_tiles */
@@ -1471,7 +1463,7 @@ static bool leaves_units_idle(int64_t workgroups, int32_t cus) { return workgrou
 /* family 4: one tile's estimate; and the tile and the K split with the smallest one; K ranges hold at least two 256-wide chunks */
 static double in_loop_estimate(const prefill_cost &c, int32_t qtype, int64_t M, int64_t N, int64_t K, int sp, int32_t cus) {
     const int bm = k_prefill_tiles[c.tile][0], bn = k_prefill_tiles[c.tile][1];
-    const int by_regs = qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu, by_lds = 160 * 1024 / in_loop_lds(qtype, bm, bn);
+    const int by_regs = qtype == PSN_Q6_K ? c.per_cu_q6_K : c.per_cu, by_lds = PSN_LDS_MAX / psn_lds_in_loop(format_index(qtype), bm, bn);
     const int64_t wgs = (M + bm - 1) / bm * ((N + bn - 1) / bn) * sp;
     /* (fitted to the 16 x 16 x 32 kernels; the others take less, least where fewer than nine of sixteen units have a workgroup) */
     const double part = bm != 256 || !leaves_units_idle(wgs, cus) ? 1.0 : wgs * 16 <= (int64_t)cus * 9 ? 0.945 : 0.975;
@@ -1641,10 +1633,7 @@ static void prefill_args(psn_prefill_args *a, const void *W, const psn_buf *X, p
 }
 static int32_t launch_thin(psn_module *mod, psn_stream *s, int32_t qtype, const psn_buf *W, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N,
                            int64_t K, int tm, int rt, int32_t ksplit) {
-    static const int lds_row[5] = {144, 272, 208, 240, 224};    /* a row's chunk in LDS, with the unpacked scales of Q4_K and Q5_K */
-    const int row = qtype == PSN_Q5_K && tm == 3 && rt == 4 ? 176 : lds_row[format_index(qtype)];      /* (no room for the scales there) */
-    const int rings = 8 * (16 * rt * row + tm * 2048), sums = 8 * 1024 * rt * tm;
-    const int lds = rings > sums ? rings : sums;
+    const int lds = psn_lds_thin(format_index(qtype), tm, rt);
     if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: %d x %d rows need %d bytes of LDS, device offers %d", 16 * tm, 16 * rt, lds, mod->ctx->max_lds);
     int32_t rc = bind(mod->ctx);
     if (rc) return rc;
@@ -1657,14 +1646,13 @@ static int32_t launch_thin(psn_module *mod, psn_stream *s, int32_t qtype, const 
 }
 static int32_t launch_dense(psn_module *mod, psn_stream *s, const void *packed, const psn_buf *X, psn_buf *Y, int64_t M, int64_t N, int64_t K,
                             int32_t bm, int32_t bn, int32_t ksplit) {
+    const int lds = psn_lds_dense(bm, bn);
+    if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: dense %dx%d tiles need %d bytes of LDS, device offers %d", bm, bn, lds, mod->ctx->max_lds);
     int32_t rc;
     if (ksplit > 1 && (rc = fill_zero_y(mod, s, Y, M, N))) return rc;
     const int64_t nt = (N + bn - 1) / bn, mt = (M + bm - 1) / bm;
     psn_prefill_args a;
     prefill_args(&a, packed, X, Y, M, N, K, ksplit, K * 2);
-    /* LDS: three stages of X (64 k) and four steps of W (32 k) with 256 columns, else a ring of four (64 x 64 tiles: five) stages of both */
-    const int lds = bn == 256 ? 3 * bm * 128 + 4 * bn * 64 : (bm + bn) * 128 * (bn == 64 ? 5 : 4);
-    if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: dense %dx%d tiles need %d bytes of LDS, device offers %d", bm, bn, lds, mod->ctx->max_lds);
     char name[96];
     if (bn == 256) snprintf(name, sizeof name, "psn_prefill_dense_f16%s", bm == 128 ? "_m128" : "");
     else snprintf(name, sizeof name, "psn_prefill_dense_f16_m%d_n%d", bm, bn);
@@ -1759,13 +1747,10 @@ extern "C" int32_t psn_qmatmul_prefill_tiled(psn_module *mod, psn_stream *s, int
     if (!skinny && !wide && waves != 4 && !(waves == 16 && has_ws)) return fail(PSN_E_UNSUPPORTED, "prefill: no kernel family %d for a %dx%d tile", waves, bm, bn);
     if (ksplit < 1 || ksplit > 64) return fail(PSN_E_UNSUPPORTED, "prefill: ksplit=%d outside 1..64", ksplit);
     if (ksplit > 1 && (M * N) % 4 != 0) return fail(PSN_E_UNSUPPORTED, "prefill: splitting K needs M*N to be a multiple of 4");
-    /* the interleaved kernels carry their LDS as static arrays; the skinny kernel: rings of three X chunks
-     * (64 rows x 256 k fp16) and six (Q4_0) or three (Q8_0) raw weight chunks (64 rows, padded: SkinnyRings), reused for the final
-     * 8 x 16 KB reduction */
-    const int skinny_rings = 3 * 32768 + (qtype == PSN_Q4_0 ? 6 * 64 * 144 : 3 * 64 * 304);
-    const int wide_rings = 3 * (32768 + 256 * (qtype == PSN_Q4_0 ? 36 : 68));   /* three stages of X (256 rows x 64 k) and of raw blocks (two per row) */
     const bool pp = waves == 4 && bn <= 128;
-    const int lds = pp ? in_loop_lds(qtype, bm, bn) : skinny ? (skinny_rings > 8 * 16384 ? skinny_rings : 8 * 16384) : wide ? wide_rings : waves == 16 ? 0 : 2 * (bm + bn) * 128;
+    const int f = format_index(qtype);
+    /* (the producer / consumer kernels carry their LDS as static arrays) */
+    const int lds = pp ? psn_lds_in_loop(f, bm, bn) : skinny ? psn_lds_skinny(f) : wide ? psn_lds_wide(f) : waves == 16 ? 0 : psn_lds_base(bm, bn);
     if (lds > mod->ctx->max_lds) return fail(PSN_E_UNSUPPORTED, "prefill: tile %dx%d needs %d bytes of LDS, device offers %d", bm, bn, lds, mod->ctx->max_lds);
     if ((rc = bind(mod->ctx))) return rc;
     if (ksplit > 1 && (rc = fill_zero_y(mod, s, Y, M, N))) return rc;

@@ -233,6 +233,7 @@ PSN_DEV void prefill_body(const psn_prefill_args &a) {
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;     /* 32x32 MFMA tiles per wave */
     constexpr int KCH = NT / BN;                            /* 256-wide K chunks held in registers per round */
     constexpr int XBYTES = BM * 128, WBYTES = BN * 128;
+    static_assert(2 * (XBYTES + WBYTES) == psn_lds_base(BM, BN), "LDS of the launch");
     extern __shared__ uint4 psn_smem[];
     char *smem = reinterpret_cast<char *>(psn_smem);
     char *xs[2] = {smem, smem + XBYTES};
@@ -770,6 +771,7 @@ template <typename WF>
 PSN_DEV void prefill_skinny_body(const psn_prefill_args &a) {
     typedef SkinnyRings<WF> R;
     constexpr int BN = 64;
+    static_assert(R::BYTES == psn_lds_skinny_rings(WF::DW == 36 ? PSN_F_Q4_0 : PSN_F_Q8_0), "LDS of the launch");
     extern __shared__ uint4 psn_smem[];
     typedef __attribute__((address_space(3))) char lds_char;
     lds_char *const lds_ptr = (lds_char *)psn_smem;
@@ -861,6 +863,7 @@ PSN_DEV void prefill_wide_body(const psn_prefill_args &a) {
     constexpr int XBYTES = BM * 128, RBYTES = BN * SB;
     constexpr int NX = XBYTES / 1024 / 4;                   /* X loads per wave and stage: 8 */
     constexpr int NR = RBYTES / 4 / 64 / 4;                 /* raw dword loads per wave and stage: 9 or 17 */
+    static_assert(NS * (XBYTES + RBYTES) == psn_lds_wide(Q4 ? PSN_F_Q4_0 : PSN_F_Q8_0), "LDS of the launch");
     extern __shared__ uint4 psn_smem[];
     typedef __attribute__((address_space(3))) char lds_char;
     lds_char *const lds_ptr = (lds_char *)psn_smem;

@@ -7,6 +7,7 @@
 
 #include "psn_args.h"
 #include "psn_device.h"
+#include "psn_prefill_lds.h"
 
 #define UNROLL _Pragma("unroll")
 

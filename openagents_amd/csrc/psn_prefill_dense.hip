@@ -44,7 +44,7 @@ template <int WM, int WN, int TM, int TN> PSN_DEV void dense_large_body(const ps
     constexpr int WAVES = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16, NX = 3, NW = 4;
     constexpr int XB = BM * 128, WB = BN * 64, W0 = NX * XB;
     constexpr int LXS = BM / 8 / WAVES, LX = LXS / 2, LW = BN / 16 / WAVES, NL = LX + LW;       /* loads per wave: X per stage and step, W per step */
-    static_assert(WAVES == 8 && LXS % 2 == 0 && LW >= 1 && W0 + NW * WB <= 160 * 1024 && 8 * wave_out_bytes<TN>() <= W0 + NW * WB, "tile");
+    static_assert(WAVES == 8 && LXS % 2 == 0 && LW >= 1 && W0 + NW * WB == psn_lds_dense(BM, BN) && W0 + NW * WB <= PSN_LDS_MAX && 8 * wave_out_bytes<TN>() <= W0 + NW * WB, "tile");
     extern __shared__ uint4 psn_smem[];
     lds_char *const lds_ptr = (lds_char *)psn_smem;
     const u32 lds0 = (u32)(uintptr_t)lds_ptr;
@@ -143,7 +143,7 @@ template <int WM, int WN, int TM, int TN> PSN_DEV void dense_large_body(const ps
 template <int WM, int WN, int TM, int TN, int NS> PSN_DEV void dense_small_body(const psn_prefill_args &a) {
     constexpr int BM = WM * TM * 16, BN = WN * TN * 16, XB = BM * 128, SB = (BM + BN) * 128;
     constexpr int LX = BM / 64, LW = BN / 64, NL = LX + LW;  /* loads per wave and stage */
-    static_assert(WM * WN == 4 && LX >= 1 && LW >= 1 && TM % 2 == 0 && NS * SB <= 160 * 1024 && 4 * TM * TN * 1024 + 8 * wave_out_bytes<TN>() <= NS * SB, "tile");
+    static_assert(WM * WN == 4 && LX >= 1 && LW >= 1 && TM % 2 == 0 && NS * SB == psn_lds_dense(BM, BN) && NS * SB <= PSN_LDS_MAX && 4 * TM * TN * 1024 + 8 * wave_out_bytes<TN>() <= NS * SB, "tile");
     extern __shared__ uint4 psn_smem[];
     lds_char *const lds_ptr = (lds_char *)psn_smem;
     const u32 lds0 = (u32)(uintptr_t)lds_ptr;

@@ -92,7 +92,7 @@ template <int J, bool FAR, class S> PSN_DEV void kq_scales1(u32x4 header, S &s) 
     }
 }
 struct PpQ4_K {
-    static constexpr int BYTES = 144, LOADS = 5;
+    static constexpr int FORMAT = PSN_F_Q4_K, BYTES = 144, LOADS = 5;
     template <int NB> struct raw { u32x4 h; typename raw_bytes<NB>::t q[4]; };
     template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
     template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
@@ -112,7 +112,7 @@ struct PpQ4_K {
     static constexpr int SPREAD = 3;
 };
 struct PpQ5_K {
-    static constexpr int BYTES = 176, LOADS = 6;
+    static constexpr int FORMAT = PSN_F_Q5_K, BYTES = 176, LOADS = 6;
     template <int NB> struct raw { u32x4 h; typename raw_bytes<NB>::t top, q[4]; };
     template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
     template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
@@ -136,7 +136,7 @@ struct PpQ5_K {
  * the half's 64 low-bit bytes, their low (J even) or high nibbles; bits 4..5 from the half's 32 high-bit bytes.  A
  * super-block (210 bytes) starts on a dword or two bytes behind one: `pick` takes four bytes out of two dwords accordingly. */
 struct PpQ6_K {
-    static constexpr int BYTES = 210, LOADS = 9;
+    static constexpr int FORMAT = PSN_F_Q6_K, BYTES = 210, LOADS = 9;
     template <int NB> struct raw { typename raw_bytes<NB + 4>::t ql[4], qh[2]; u32x4 sc; u32 sc4, d, pick; };
     template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
     template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
@@ -199,7 +199,7 @@ template <int PB, int NB> struct pp_blocks {               /* PB: bytes per part
     }
 };
 struct PpQ4_0 {
-    static constexpr int BYTES = 144, LOADS = 4;
+    static constexpr int FORMAT = PSN_F_Q4_0, BYTES = 144, LOADS = 4;
     template <int NB> struct raw { typename raw_bytes<NB + 4>::t q[4]; };
     template <int NB> static PSN_DEV int lane_off(int part) { return NB * part; }
     template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {
@@ -223,7 +223,7 @@ struct PpQ4_0 {
     static constexpr int SPREAD = 2;
 };
 struct PpQ8_0 {
-    static constexpr int BYTES = 272, LOADS = 8;
+    static constexpr int FORMAT = PSN_F_Q8_0, BYTES = 272, LOADS = 8;
     template <int NB> struct raw { typename raw_bytes<2 * NB>::t q[4]; u32 e[4]; };    /* e: the dword behind them */
     template <int NB> static PSN_DEV int lane_off(int part) { return 2 * NB * part; }
     template <int NB> static PSN_DEV void load(const uint8_t *row, int lane, raw<NB> &r) {

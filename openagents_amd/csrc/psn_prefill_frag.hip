@@ -147,7 +147,9 @@ PSN_DEV void prefill_frag_body(const psn_prefill_args &a) {
     constexpr int LX = BM / 32, LW = (BN * RF::WORDS + 511) / 512;    /* loads per wave: X per period, W per chunk */
     constexpr int NI = (BN * RF::WORDS + 63) / 64;                    /* 1 KB pieces of a chunk; loads of waves past them go to one more, which nothing reads */
     constexpr int W0 = 2 * XB, WBUF = (NI + 1) * 1024 + (RF::PASSED ? BN * 8 : 0), SC0 = W0 + 2 * WBUF, SCW = RF::SHARED ? TN * 512 : 0;
-    static_assert(TM % 4 == 0 && (TN == 1 || TN == 2) && SC0 + 8 * SCW <= 160 * 1024, "tile");
+    static_assert(TM % 4 == 0 && (TN == 1 || TN == 2) && SC0 + 8 * SCW <= PSN_LDS_MAX, "tile");
+    static_assert(SC0 + 8 * SCW == psn_lds_in_loop(F::FORMAT, BM, BN) && 4 * TM * TN * 1024 + 8 * wave_out_bytes<TN>() <= SC0 + 8 * SCW, "LDS of the launch; the sums and results at the end");
+    static_assert(RF::WORDS == psn_lds_words(F::FORMAT) && RF::SHARED == psn_lds_scales(F::FORMAT), "format");
     extern __shared__ uint4 psn_smem[];
     lds_char *const lds_ptr = (lds_char *)psn_smem;
     const u32 lds0 = (u32)(uintptr_t)lds_ptr;

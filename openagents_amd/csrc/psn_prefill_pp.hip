@@ -65,7 +65,7 @@ PSN_DEV void prefill_pp_body(const psn_prefill_args &a) {
     constexpr int SPREAD = WF::SPREAD;
     constexpr int XBYTES = BM * 128, WBYTES = BN * 128;
     constexpr int NX = BM / 64;                             /* X loads per wave and step */
-    static_assert(TM >= 1 && TN >= 1 && NX >= 1 && NS * XBYTES + 2 * WBYTES <= 160 * 1024 && 8 * MMA::template out_bytes<TN>() <= NS * XBYTES, "tile");
+    static_assert(TM >= 1 && TN >= 1 && NX >= 1 && NS * XBYTES + 2 * WBYTES == psn_lds_in_loop(WF::FORMAT, BM, BN) && psn_lds_in_loop(WF::FORMAT, BM, BN) <= PSN_LDS_MAX && 8 * MMA::template out_bytes<TN>() <= NS * XBYTES, "tile");
     extern __shared__ uint4 psn_smem[];
     lds_char *const lds_ptr = (lds_char *)psn_smem;
     const u32 lds0 = (u32)(uintptr_t)lds_ptr;

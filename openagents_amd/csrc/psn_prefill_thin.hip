@@ -87,9 +87,10 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
     constexpr int XD = RT * TM <= 3 ? 4 : RT * TM <= 8 ? 2 : 1;   /* steps of X on their way */
     constexpr bool AHEAD = TM * (RT + 2) < (BIG ? 16 : 24);       /* registers for the next step's fragments of X */
     constexpr int NI = (16 * F::WORDS + 63) / 64;           /* load instructions per 16 rows and chunk */
-    constexpr int WTILE = 16 * F::STRIDE, SHARED_BYTES = RT * (WTILE + F::SCALES) + TM * 2048;
-    constexpr bool SHARED = F::SCALES != 0 && 8 * SHARED_BYTES <= 160 * 1024;             /* (Q5_K's 48 rows of X by 64 of W are too large) */
-    constexpr int MINE = SHARED ? SHARED_BYTES : RT * WTILE + TM * 2048;
+    constexpr bool SHARED = psn_lds_thin_scales(WF::FORMAT, TM, RT);                      /* (Q5_K's 48 rows of X by 64 of W leave no room) */
+    constexpr int WTILE = 16 * F::STRIDE, MINE = RT * (WTILE + (SHARED ? F::SCALES : 0)) + TM * 2048;
+    static_assert(8 * MINE == psn_lds_thin_rings(WF::FORMAT, TM, RT, SHARED) && psn_lds_thin(WF::FORMAT, TM, RT) <= PSN_LDS_MAX && F::WORDS == psn_lds_words(WF::FORMAT) &&
+                  (F::SCALES != 0) == psn_lds_scales(WF::FORMAT), "LDS of the launch");
     extern __shared__ uint4 psn_smem[];
     const int tid = threadIdx.x, lane = tid & 63, row = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -260,6 +261,7 @@ PSN_DEV void prefill_thin_body(const psn_prefill_args &a) {
 
     /* partial tiles of the eight waves -> LDS ([wave][tile][register][lane]), then summed in the order of the waves */
     constexpr int TILE = 256, PER_WAVE = RT * TM * TILE;
+    static_assert(8 * PER_WAVE * 4 == psn_lds_thin_sums(TM, RT), "the sums at the end");
     float *const part_sums = reinterpret_cast<float *>(psn_smem);
     __syncthreads();
     UNROLL for (int t = 0; t < RT; ++t) UNROLL for (int i = 0; i < TM; ++i) UNROLL for (int r = 0; r < 4; ++r)

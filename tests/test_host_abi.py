@@ -310,26 +310,59 @@ def test_no_kernel_spills_registers_or_uses_scratch():
     assert not bad, bad
 
 
+def _prefill_lds(calls):
+    """what expressions of psn_prefill_lds.h come to: the sizes that the host launches with and that the kernels assert their layouts to equal"""
+    import subprocess
+    import tempfile
+    with tempfile.TemporaryDirectory() as d:
+        src = os.path.join(d, "lds.cpp")
+        with open(src, "w") as f:
+            f.write('#include "psn_prefill_lds.h"\n#include <cstdio>\nint main() {\n' + "".join(f'    std::printf("%d\\n", (int)({c}));\n' for c in calls) + "}\n")
+        subprocess.check_call(["g++", "-std=c++17", "-I", os.path.join(ROOT, "openagents_amd", "csrc"), "-o", os.path.join(d, "lds"), src])
+        return [int(v) for v in subprocess.check_output([os.path.join(d, "lds")], text=True).split()]
+
+
 def test_prefill_planner_counts_the_workgroups_a_compute_unit_can_hold():
-    """The cost models' workgroups per compute unit against the built kernels: 512 vector registers per lane and SIMD, given out in eights, two
-    waves of a workgroup on each of the four SIMDs; 160 KB of LDS, (4 rows + 2 columns) * 128 bytes of it for a family 4 tile."""
+    """The cost models' workgroups per compute unit against the built kernels: 512 vector registers per lane and SIMD, given out in eights, two waves of a workgroup on each of the four
+    SIMDs, and 160 KB of LDS.  Family 4's table holds what the registers allow (the planner takes the LDS of the format beside it), the dense family's and the thin kernels' rule
+    what both do."""
     src = open(os.path.join(ROOT, "openagents_amd", "csrc", "psn_host.cpp")).read()
+    table = lambda name: re.search(name + r"\[\] = \{(.*?)\n\};", src, re.S).group(1)
     tiles = re.findall(r"\{(\d+), (\d+)\}", re.search(r"k_prefill_tiles\[\]\[2\] = \{(.*)\};", src).group(1))
-    table = re.findall(r"\{(\d), (\d), (\d), ", re.search(r"k_prefill_cost\[\] = \{(.*?)\n\};", src, re.S).group(1))
-    assert len(table) == 4
     regs = _kernel_registers()
-    held = lambda name, lds: min(512 // (-(-regs[name] // 8) * 8) // 2, 160 * 1024 // lds)
-    for tile, others, q6_K in table:
+    by_registers = lambda name: 512 // (-(-regs[name] // 8) * 8) // 2
+    formats = ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K")
+    in_loop = re.findall(r"\{(\d), (\d), (\d), \{", table("k_prefill_cost"))
+    assert len(in_loop) == 4
+    for tile, others, q6_K in in_loop:
         m, n = map(int, tiles[int(tile)])
-        for fmt in ("q4_0", "q8_0", "q4_K", "q5_K", "q6_K"):
-            assert held(f"psn_prefill_{fmt}_m{m}_n{n}_pp", (4 * m + 2 * n) * 128) == int(q6_K if fmt == "q6_K" else others), (fmt, m, n)
-    chunk = {"q4_0": 144, "q8_0": 272, "q4_K": 144, "q5_K": 176, "q6_K": 224}
-    for name in regs:
-        thin = re.fullmatch(r"psn_prefill_(\w+)_thin_(\d)_(\d)", name)
-        if thin:
-            fmt, tm, rt = thin.group(1), int(thin.group(2)), int(thin.group(3))
-            two = tm == 1 and (rt == 1 or (rt == 2 and fmt not in ("q8_0", "q6_K")))
-            assert held(name, max(8 * (16 * rt * chunk[fmt] + tm * 2048), 8192 * rt * tm)) == (2 if two else 1), name
+        for fmt in formats:
+            for kernel in ("_pp", "_pp32") if m == 256 else ("_pp",):
+                assert by_registers(f"psn_prefill_{fmt}_m{m}_n{n}{kernel}") == int(q6_K if fmt == "q6_K" else others), (fmt, m, n)
+    assert re.search(r"by_lds = PSN_LDS_MAX / psn_lds_in_loop\(format_index\(qtype\), bm, bn\);", src)
+
+    dense = [tuple(map(int, t)) for name in ("k_dense_cost", "k_packed_cost") for t in re.findall(r"\{(\d+), (\d+), (\d), \{", table(name))]
+    assert len(dense) == 7
+    for (m, n, per_cu), lds in zip(dense, _prefill_lds(f"psn_lds_dense({m}, {n})" for m, n, _ in dense)):
+        name = "psn_prefill_dense_f16" + ("" if m == 256 else "_m128" if n == 256 else f"_m{m}_n{n}")
+        assert min(by_registers(name), 160 * 1024 // lds) == per_cu, (m, n)
+
+    thin = [(name, *re.fullmatch(r"psn_prefill_(\w+)_thin_(\d)_(\d)", name).groups()) for name in regs if "_thin_" in name]
+    assert len(thin) == 5 * 8 + 2 + 1 + 2 + 2 + 3
+    for (name, fmt, tm, rt), lds in zip(thin, _prefill_lds(f"psn_lds_thin({formats.index(fmt)}, {tm}, {rt})" for _, fmt, tm, rt in thin)):
+        two = tm == "1" and (rt == "1" or (rt == "2" and fmt not in ("q8_0", "q6_K")))
+        assert min(by_registers(name), 160 * 1024 // lds) == (2 if two else 1), name
+
+
+def test_prefill_lds_sizes_follow_from_the_layouts():
+    """Restated from what lies in LDS: 64 x 128 tiles of family 4 are where a format decides whether two workgroups share a compute unit, and one thin kernel has no room for scales."""
+    sizes = _prefill_lds([f"psn_lds_in_loop({f}, 64, 128)" for f in range(5)] + ["psn_lds_in_loop(2, 256, 128)", "psn_lds_thin(2, 3, 4)", "psn_lds_thin(3, 3, 4)", "psn_lds_thin_scales(3, 3, 4)",
+                          "psn_lds_dense(64, 64)", "psn_lds_dense(256, 256)"])
+    x = 2 * 64 * 256
+    raw = lambda words, extra: 2 * ((128 * words // 64 + 1) * 1024 + extra)
+    assert sizes[:5] == [x + raw(9, 0), x + raw(17, 0), x + raw(9, 0) + 8 * 1024, x + raw(11, 0) + 8 * 1024, x + raw(13, 128 * 8)]
+    assert [160 * 1024 // v for v in sizes[:5]] == [2, 1, 2, 1, 1]
+    assert sizes[5:] == [4 * 256 * 128 + 2 * 128 * 128, 8 * (64 * (144 + 64) + 3 * 2048), 8 * (64 * 176 + 3 * 2048), 0, 5 * 128 * 128, 160 * 1024]
 
 
 def test_prefill_planner_knows_how_full_the_rounds_are(lib):
