@@ -335,10 +335,12 @@ int32_t psn_prefill_reserve(psn_stream *s, int64_t N, int64_t K);
  * into a caller-owned buffer of psn_prefill_packed_bytes(N, K) bytes (2 bytes per weight, rows padded to whole
  * 256-row panels; a deployment with HBM to spare keeps one per matrix beside the GGUF blocks the decode
  * matvec reads), psn_qmatmul_prefill_packed multiplies any number of X against it -- the same result as
- * psn_qmatmul_prefill_tiled(..., 256, 256, ksplit, 128), up to the order of sums, without the 35-48 us pass per call.  No stream
- * workspace is involved.  No counterpart in the reference, which dequantizes inside every call. */
+ * psn_qmatmul_prefill_tiled(..., 256, 256, ksplit, 128), up to the order of sums, without the pass per call (33-45 us for 58 million weights).  No stream
+ * workspace is involved.  psn_qmatmul_prefill_packed_plan: which tile of the multiply it runs (64x64, 64x128, 128x128, 128x256 or 256x256) and into how many ranges K is cut (1, 2, 4
+ * or 8, as in psn_qmatmul_prefill_tiled); host arithmetic, compute_units <= 0 stands for 256.  No counterpart in the reference, which dequantizes inside every call. */
 int64_t psn_prefill_packed_bytes(int64_t N, int64_t K);
 int32_t psn_prefill_pack(psn_module *mod, psn_stream *s, int32_t qtype, const psn_buf *W, psn_buf *packed, int64_t N, int64_t K);
+int32_t psn_qmatmul_prefill_packed_plan(int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit);
 int32_t psn_qmatmul_prefill_packed(psn_module *mod, psn_stream *s, const psn_buf *packed, const psn_buf *X_f16, psn_buf *Y_f32,
                                    int64_t M, int64_t N, int64_t K);
 /* ... and the same matmul with a caller-chosen shape (auto-tuners, benchmarks). */

@@ -71,6 +71,13 @@ def prefill_choice(m: int, n: int, k: int, qtype: int, compute_units: int = 256,
     return int(tm.value), int(tn.value), int(sp.value), int(wv.value)
 
 
+def packed_plan(m: int, n: int, k: int, compute_units: int = 256):
+    """(tile_m, tile_n, ksplit) that quantized_matmul_packed runs."""
+    tm, tn, sp = C.c_int32(), C.c_int32(), C.c_int32()
+    _check(_ffi.load().psn_qmatmul_prefill_packed_plan(m, n, k, compute_units, C.byref(tm), C.byref(tn), C.byref(sp)))
+    return int(tm.value), int(tn.value), int(sp.value)
+
+
 def matvec_plan(qtype: int, scheme: int, n: int, k: int, batch: int, compute_units: int = 256, x_is_f32: bool = False) -> MatvecPlan:
     plan = MatvecPlan()
     _check(_ffi.load().psn_qmatvec_plan(qtype, scheme, n, k, batch, compute_units, int(x_is_f32), C.byref(plan)))

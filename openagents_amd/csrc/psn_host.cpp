@@ -1690,6 +1690,17 @@ extern "C" int32_t psn_qmatmul_prefill_packed(psn_module *mod, psn_stream *s, co
     return launch_dense(mod, s, packed->p, X, Y, M, N, K, d.bm, d.bn, d.ksplit);
 }
 
+extern "C" int32_t psn_qmatmul_prefill_packed_plan(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t *tile_m, int32_t *tile_n, int32_t *ksplit) {
+    if (!tile_m || !tile_n || !ksplit) return fail(PSN_E_INVALID_ARG, "psn_qmatmul_prefill_packed_plan: null output");
+    if (M <= 0 || M > (1 << 24) || N <= 0 || N > (1 << 30) || K <= 0 || K % 256 || K > (1 << 24))
+        return fail(PSN_E_SHAPE, "psn_qmatmul_prefill_packed_plan: M=%lld N=%lld K=%lld (K must be a multiple of 256)", (long long)M, (long long)N, (long long)K);
+    const dense_plan d = plan_dense(M, N, K, cus <= 0 ? 256 : cus, true);
+    *tile_m = d.bm;
+    *tile_n = d.bn;
+    *ksplit = d.ksplit;
+    return PSN_OK;
+}
+
 extern "C" int32_t psn_prefill_reserve(psn_stream *s, int64_t N, int64_t K) {
     if (!s) return fail(PSN_E_INVALID_ARG, "stream is null");
     if (N <= 0 || K <= 0 || K % 256 || N > (1 << 30) || K > (1 << 24)) return fail(PSN_E_SHAPE, "psn_prefill_reserve: N=%lld K=%lld", (long long)N, (long long)K);

@@ -338,7 +338,7 @@ def test_packed_weights_multiply_like_the_dense_family(hip, orc, qname):
     w = hip.upload_weight(t, W, n, k)
     packed = hip.pack_for_prefill(w)
     assert packed.nbytes >= 768 * k * 2
-    for m in (1, 260, 37, 384, 1100):                                                    # heights served by either tile of the multiply
+    for m in (1, 260, 37, 384, 1100):                                                    # (64 x 64 tiles at this width, with and without a K cut)
         X = G.seeded_acts(841 + m, m, k).astype(np.float16)
         y = hip.alloc(m * n * 4)
         hip.quantized_matmul_packed(packed, hip.upload(X), y, m, n, k)
@@ -490,8 +490,8 @@ def test_values_that_are_not_finite_stay_in_their_row_and_column(hip, orc, qname
 @pytest.mark.parametrize("m,n,k", [(1, 1, 256), (63, 65, 512), (64, 64, 2048), (65, 130, 768), (129, 127, 1280), (128, 1000, 2560), (257, 255, 256), (300, 2050, 512), (1025, 1021, 256),
                                    (2049, 4100, 256)])
 def test_packed_multiply_at_tile_edges(hip, orc, m, n, k):
-    """Every tile of the multiply (64 x 64 .. 256 x 256; the planner takes the larger ones as the shape grows) a row and a column either side of its edges, odd row lengths of Y
-    (stored word by word), and K in several ranges.  Products are exact in fp32, so only the order of at most 2560 sums differs from the oracle: PARITY_TOL is far above 2560 * 2^-24."""
+    """Shapes a row and a column either side of the tiles' edges, odd row lengths of Y (stored word by word), and K in several ranges; mostly 64 x 64 tiles, the last ones 64 x 128
+    and 256 x 256.  Products are exact in fp32, so only the order of at most 2560 sums differs from the oracle: PARITY_TOL is far above 2560 * 2^-24."""
     W = weights(orc, "Q4_K", 870, n, k)
     X = G.seeded_acts(871 + m, m, k).astype(np.float16)
     packed = hip.pack_for_prefill(hip.upload_weight(orc.Q4_K, W, n, k))
@@ -499,6 +499,26 @@ def test_packed_multiply_at_tile_edges(hip, orc, m, n, k):
     say(f"packed multiply m={m} n={n} k={k}")
     hip.quantized_matmul_packed(packed, hip.upload(X), y, m, n, k)
     err = G.max_rel_err(y.download(np.float32, (m, n)), orc.prefill(orc.Q4_K, W, X, n, k))
+    assert err < PARITY_TOL, (m, n, k, err)
+
+
+@pytest.mark.parametrize("m,n,k,plan", [(130, 129, 1280, (64, 64, 1)), (2, 2, 5120, (64, 64, 8)), (193, 4097, 1280, (64, 128, 1)), (193, 4100, 1280, (64, 128, 1)),
+                                        (1, 4100, 3840, (64, 128, 4)), (2052, 65, 5120, (64, 128, 4)), (1281, 1537, 1280, (128, 128, 1)), (2049, 1000, 1280, (128, 128, 1)),
+                                        (65, 4100, 5120, (128, 128, 4)), (1281, 3073, 1280, (128, 256, 1)), (4100, 1000, 1280, (128, 256, 1)), (4001, 2049, 1280, (256, 256, 1)),
+                                        (4001, 2052, 1280, (256, 256, 1))])
+def test_every_tile_of_the_packed_multiply(hip, orc, m, n, k, plan):
+    """Ragged rows and columns, K long enough that every slot of the rings is used again, rows of Y that are whole 16-byte words and not, K cut and not, on the tile that the plan
+    names and the launch runs.  fp16 products are exact in fp32: PARITY_TOL is far above the rounding of 5120 sums."""
+    assert backend.packed_plan(m, n, k, hip.compute_units) == plan
+    W = weights(orc, "Q8_0", 875, n, k)
+    X = G.seeded_acts(876, m, k).astype(np.float16)
+    packed = hip.pack_for_prefill(hip.upload_weight(orc.Q8_0, W, n, k))
+    x, y = hip.upload(X), hip.upload(np.full((m, n), np.nan, np.float32))
+    say(f"packed multiply m={m} n={n} k={k} plan={plan}")
+    name = "psn_prefill_dense_f16" + {(256, 256): "", (128, 256): "_m128"}.get(plan[:2], f"_m{plan[0]}_n{plan[1]}")
+    assert launched_kernels(hip, lambda: hip.quantized_matmul_packed(packed, x, y, m, n, k)) == ("psn_fill_zero + " if plan[2] > 1 else "") + name
+    ref = X.astype(np.float64) @ orc.dequantize(orc.Q8_0, W, k).reshape(n, k).astype(np.float16).astype(np.float64).T
+    err = G.max_rel_err(y.download(np.float32, (m, n)), ref)
     assert err < PARITY_TOL, (m, n, k, err)
 
 

@@ -398,6 +398,24 @@ def test_prefill_planner_picks_a_plan_near_the_fastest_where_weights_come_from_m
         assert us.get(chosen, 1e9) <= 1.05 * min(us.values()), (qt, m, n, k, chosen)
 
 
+def test_packed_plans_name_a_tile_of_the_multiply_and_a_cut_that_may_be_made(lib):
+    """Host arithmetic: every tile is taken somewhere, K is cut only where Y can be zeroed by 16-byte words and every range holds two chunks; what the call refuses, the plan refuses."""
+    taken = set()
+    for m in (1, 33, 64, 203, 512, 1281, 2048, 4001, 1 << 20):
+        for n in (1, 66, 1000, 1024, 4097, 14336, 1 << 20):
+            for k in (256, 1280, 4096, 14336):
+                tm, tn, sp = backend.packed_plan(m, n, k)
+                assert (tm, tn) in {(64, 64), (64, 128), (128, 128), (128, 256), (256, 256)}, (m, n, k)
+                assert sp == 1 or (sp in (2, 4, 8) and (m * n) % 4 == 0 and k // 256 >= 2 * sp), (m, n, k, sp)
+                taken.add((tm, tn))
+    assert len(taken) == 5
+    one = [C.c_int32() for _ in range(3)]
+    assert lib.psn_qmatmul_prefill_packed_plan(1, 1, 300, 256, *map(C.byref, one)) == _ffi.E_SHAPE
+    assert lib.psn_qmatmul_prefill_packed_plan(0, 1, 256, 256, *map(C.byref, one)) == _ffi.E_SHAPE
+    assert lib.psn_qmatmul_prefill_packed_plan(1, 1, 256, 256, None, None, None) == _ffi.E_INVALID_ARG
+    assert backend.packed_plan(512, 4096, 4096, 0) == backend.packed_plan(512, 4096, 4096, 256)
+
+
 def test_prefill_plans_take_the_dense_family_only_for_large_m():
     """Host arithmetic: from a few thousand rows of X on every format is dequantized once and multiplied as
     fp16 (family 128, 256 x 256 or 128 x 256 tiles); 64 rows and fewer never are."""
