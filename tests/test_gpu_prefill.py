@@ -524,20 +524,25 @@ def test_every_tile_of_the_packed_multiply(hip, orc, m, n, k, plan):
 
 @pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
 def test_few_rows_over_more_weight_rows_than_one_round_of_64(hip, orc, qname):
-    """64 rows of W per compute unit and one more: from there on psn_qmatmul_prefill may take family 4's tiles for M <= 64.  fp16 products are exact in fp32, so only the order
-    of at most 512 sums differs from the oracle: PARITY_TOL is far above 512 * 2^-24."""
+    """64 rows of W per compute unit and one more: from there on psn_qmatmul_prefill may take family 4's tiles for M <= 64, and in every format it does (Q4_0 and Q8_0 at K = 768).
+    fp16 products are exact in fp32, so only the order of at most 768 sums differs from the oracle: PARITY_TOL is far above 768 * 2^-24."""
     t = getattr(orc, qname)
     edge = 64 * hip.compute_units
-    for n, k in ((edge, 512), (edge + 1, 256), (edge + 4, 512)):
+    beyond = set()
+    for n, k in ((edge, 512), (edge + 1, 256), (edge + 4, 512), (edge + 4, 768)):
         W = weights(orc, qname, 885, n, k)
         w, X = hip.upload_weight(t, W, n, k), G.seeded_acts(886, 64, k).astype(np.float16)
         ref = orc.prefill(t, W, X, n, k)
         for m in (1, 33, 64):
-            say(f"few rows {qname} m={m} n={n} k={k} {backend.prefill_choice(m, n, k, t, hip.compute_units)}")
+            choice = backend.prefill_choice(m, n, k, t, hip.compute_units)
+            say(f"few rows {qname} m={m} n={n} k={k} {choice}")
+            if n > edge:
+                beyond.add((choice[3], m > 16))
             y = hip.upload(np.full((m, n), np.nan, np.float32))
             hip.quantized_matmul(w, hip.upload(X[:m]), y, m)
             err = G.max_rel_err(y.download(np.float32, (m, n)), ref[:m])
             assert err < PARITY_TOL, (m, n, k, err)
+    assert (4, True) in beyond and (8, False) in beyond, beyond
 
 
 @pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
