@@ -320,7 +320,8 @@ int32_t psn_qmatmul_prefill_plan(int64_t M, int64_t N, int64_t K, int32_t comput
  * available (psn_qmatmul_prefill_plan answers for Q4_0; the planner uses families 4 and 128 there), for M <= 64 the best shape of family 64 (Q6_K with
  * K not a multiple of 2048: of family 4), which every format can run.  While a stream is capturing, or while a captured graph refers to its workspace,
  * the workspace cannot grow: psn_qmatmul_prefill then takes the best plan without family 128 unless
- * psn_prefill_reserve (or an earlier dense call of that size) has sized it. */
+ * psn_prefill_reserve (or an earlier dense call of that size) has sized it.  So it does where the device has no memory left for the workspace; it does
+ * not ask for that size again on this stream until one has been allocated (psn_prefill_reserve). */
 int32_t psn_qmatmul_prefill_plan_for(int32_t qtype, int64_t M, int64_t N, int64_t K, int32_t compute_units, int32_t *tile_m,
                                      int32_t *tile_n, int32_t *ksplit, int32_t *waves);
 /* What psn_qmatmul_prefill runs, for any M: the plan above, or for M <= 64 a shape of family 8 (from 17 rows of X on and with more than 64 rows of W per compute unit also of family 4)

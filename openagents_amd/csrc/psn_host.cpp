@@ -190,6 +190,7 @@ struct psn_ctx {
 struct ws_state {
     void *p = nullptr;
     size_t bytes = 0;
+    size_t refused = 0;    /* the size that psn_qmatmul_prefill could not get: from there on it does not ask again (psn_prefill_reserve does) */
     int graph_refs = 0;    /* live graphs whose nodes hold p */
     int capture_refs = 0;  /* captures in progress that have recorded a node holding p */
     bool orphaned = false; /* the owning stream is gone; the last graph frees p */
@@ -436,11 +437,18 @@ static int32_t ensure_workspace(psn_stream *s, int64_t bytes) {
     HIP_TRY(hipStreamSynchronize(s->s));
     if (w.p) HIP_TRY(hipFree(w.p));
     w.p = nullptr;
+    const size_t had = w.bytes, want = (size_t)align_up(bytes, 1 << 20);
     w.bytes = 0;
-    const size_t want = (size_t)align_up(bytes, 1 << 20);
     hipError_t e = hipMalloc(&w.p, want);
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc(workspace)");
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        w.p = nullptr;
+        if (had && hipMalloc(&w.p, had) == hipSuccess) w.bytes = had;          /* what was there a moment ago */
+        else if (had) { (void)hipGetLastError(); w.p = nullptr; }
+        return hip_fail(e, "hipMalloc(workspace)");
+    }
     w.bytes = want;
+    w.refused = 0;
     return PSN_OK;
 }
 /* Called by every launch path that hands the workspace address to a kernel: if the stream is being captured
@@ -1797,9 +1805,19 @@ extern "C" int32_t psn_qmatmul_prefill(psn_module *mod, psn_stream *s, int32_t q
         if ((rc = is_capturing(s, &cap))) return rc;
         std::lock_guard<std::mutex> lk(g_cap_mu);
         const bool ws_pinned = s->ws->graph_refs > 0 || s->ws->capture_refs > 0;
-        dense_ok = s->ws->bytes >= (size_t)packed_bytes(N, K) || (!cap && !ws_pinned);
+        const size_t need = (size_t)packed_bytes(N, K);
+        dense_ok = s->ws->bytes >= need || (!cap && !ws_pinned && (!s->ws->refused || need < s->ws->refused));
     }
     if ((rc = prefill_choice(qtype, M, N, K, mod->ctx->compute_units, dense_ok, &bm, &bn, &sp, &wv))) return rc;
+    if (wv == 128 && s->ws->bytes < (size_t)packed_bytes(N, K)) {
+        if ((rc = bind(mod->ctx))) return rc;
+        rc = ensure_workspace(s, packed_bytes(N, K));
+        if (rc == PSN_E_OOM) {                               /* no room for the copy: the kernels that need none */
+            s->ws->refused = (size_t)packed_bytes(N, K);
+            rc = prefill_choice(qtype, M, N, K, mod->ctx->compute_units, false, &bm, &bn, &sp, &wv);
+        }
+        if (rc) return rc;
+    }
     return psn_qmatmul_prefill_tiled(mod, s, qtype, W, X, Y, M, N, K, bm, bn, sp, wv);
 }
 

@@ -6,6 +6,8 @@ fp32 accumulation.  The kernels form the fp16 weight bit-exactly (h(d*q); for th
 fp32 dequantization operation by operation, then h), so only the accumulation order differs.
 Gate (north_star): max|y - ref| / max|ref| <= 1e-3; asserted: PARITY_TOL.
 """
+import os
+import subprocess
 import sys
 
 import numpy as np
@@ -17,6 +19,7 @@ from openagents_amd.records import launched_kernels
 
 pytestmark = pytest.mark.gpu
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 GATE = 1e-3
 PARITY_TOL = 2e-5
 TILES = [(64, 64), (64, 128), (128, 128), (128, 256), (256, 128), (256, 256)]
@@ -326,6 +329,70 @@ def test_dense_family_in_graphs_needs_its_workspace_first(hip, orc):
             hip.destroy_graph(g)
     finally:
         hip.destroy_stream(s2)
+
+
+OUT_OF_MEMORY = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)          # its hipMalloc comes before the runtime's for what is loaded from here on
+import numpy as np
+from openagents_amd import _ffi, backend, quantize
+from openagents_amd.records import launched_kernels
+hip = backend.HipBackend(0)
+m, n, k, rng = 4096, 4096, 4096, np.random.default_rng(5)
+assert backend.prefill_choice(m, n, k, _ffi.Q4_0)[3] == 128
+w = hip.upload_weight(_ffi.Q4_0, quantize.quantize(_ffi.Q4_0, rng.standard_normal((n, k), dtype=np.float32), 8), n, k)
+x, y = hip.upload(rng.standard_normal((m, k), dtype=np.float32).astype(np.float16)), hip.alloc(m * n * 4)
+def out():
+    y.upload(np.full((m, n), np.nan, np.float32))
+    names = launched_kernels(hip, lambda: hip.quantized_matmul(w, x, y, m))
+    return names, y.download(np.float32, (m, n))
+hip.reserve(4096, 8)                                              # a small workspace, which stays
+copy = ctypes.c_size_t.in_dll(fake, "refuse_from")
+asked = ctypes.c_int.in_dll(fake, "refused")
+copy.value = n * k * 2
+names, got = out()
+assert asked.value == 1 and "dense" not in names, (asked.value, names)
+again, same = out()
+assert asked.value == 1 and again == names and np.array_equal(got, same)       # not asked for again
+assert hip.lib.hipGetLastError() == 0
+xv = hip.upload(rng.standard_normal((8, k), dtype=np.float32))
+yv = hip.alloc(8 * n * 4)
+hip.begin_capture()                                               # the small workspace is there: nothing has to grow while capturing
+hip.quantized_matvec(w, xv, yv, 8, _ffi.ACT_Q8)
+hip.destroy_graph(hip.end_capture())
+try:
+    hip.quantized_matmul(w, x, y, m, (256, 256, 1, 128))          # asked for by name: refused as before
+    raise SystemExit("no error")
+except backend.PsnError as e:
+    assert e.name == "PSN_E_OOM", e
+copy.value = 1 << 62
+hip.reserve_prefill(n, k)
+names, dense = out()
+assert "dense" in names and float(np.max(np.abs(dense - got)) / np.max(np.abs(got))) < 2e-6, names
+print("fell back")
+"""
+
+
+def test_a_copy_that_does_not_fit_the_device_leaves_the_kernels_that_need_none(hip, tmp_path):
+    """A process of its own in which hipMalloc answers out-of-memory from a size on: psn_qmatmul_prefill runs without the dequantized copy instead of failing, keeps the workspace it had,
+    leaves no error behind, does not ask for the copy at every call, and takes the dense family again once psn_prefill_reserve has got it."""
+    src, so = tmp_path / "fake.c", tmp_path / "fake.so"
+    src.write_text("""
+#include <dlfcn.h>
+#include <stddef.h>
+size_t refuse_from = (size_t)1 << 62;
+int refused = 0;
+int hipMalloc(void **p, size_t n) {
+    static int (*real)(void **, size_t);
+    if (!real) real = (int (*)(void **, size_t))dlsym(dlopen("libamdhip64.so", RTLD_NOW | RTLD_LOCAL), "hipMalloc");
+    if (n >= refuse_from) { ++refused; *p = 0; return 2; }
+    return real(p, n);
+}
+""")
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(src), "-ldl", "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib"])
+    say("prefill without room for the copy")
+    got = subprocess.run([sys.executable, "-c", OUT_OF_MEMORY, str(so)], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert got.returncode == 0 and got.stdout.strip().endswith("fell back"), got.stdout + got.stderr
 
 
 @pytest.mark.parametrize("qname", ["Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K"])
