@@ -1607,7 +1607,7 @@ extern "C" int32_t psn_qmatmul_prefill_choice(int32_t qtype, int64_t M, int64_t 
 
 static int32_t need(const psn_buf *b, int64_t bytes, const char *what, const char *name);
 /* the dense family's two steps: GGUF blocks -> fp16 MFMA fragments ([ceil(N/32)][K/16][64 lanes][8 halves], rows
- * padded to whole 256-row panels), and the fp16 multiply on 256 x 256 tiles over such a buffer */
+ * padded to whole 256-row panels, which every tile of the multiply divides), and the fp16 multiply over such a buffer */
 static int64_t packed_bytes(int64_t N, int64_t K) { return (N + 255) / 256 * 256 * K * 2; }
 static int32_t launch_unpack(psn_module *mod, psn_stream *s, int32_t qtype, const void *W, void *out, int64_t N, int64_t K) {
     psn_unpack_args u;

@@ -95,7 +95,7 @@ PSN_DEV f32x4 mfma16(u32x4 w, u32x4 x, f32x4 c) {
 }
 /* A wave's results of one row of MFMA tiles: lane (q, m) holds columns 16 j + 4 q .. + 3 of row m.  They go through LDS (16 rows of 16 TN + 4 words at `out`, this wave's own), so
  * that an instruction touches whole runs of a row of Y: 16-byte pieces of it where rows are whole 16-byte words and nothing has to be added (stored straight from the
- * MFMA's layout, 64 bytes of sixteen rows at a time: 4001 x 14336 x 4096 396 us instead of 389, 4001 x 1024 x 4096 on 256 x 256 tiles 87 instead of 78), else words: atomic adds
+ * MFMA's layout, 64 bytes of sixteen rows at a time: 4001 x 14336 x 4096 7 us more, 4001 x 1024 x 4096 on 256 x 256 tiles 9 more), else words: atomic adds
  * from the MFMA's layout take several times as long (512 x 1024 x 4096 in four ranges, 64 x 128 tiles: 33.3 us instead of 13.5). */
 template <int TN> constexpr int wave_out_bytes() { return 16 * (16 * TN + 4) * 4; }
 /* the rows' second half of the way: COLS columns of ROWS rows, COLS + 4 words apart at `out`, written by this wave */

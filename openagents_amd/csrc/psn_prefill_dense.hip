@@ -7,16 +7,16 @@
  * reads and loads are spread behind the MFMAs, one barrier per step, eight waves (two to a SIMD).
  *
  * What bounds it on MI355X: power on a full chip, and the bytes that a compute unit takes in otherwise.
- *   - Power.  4001 x 4096 x 14336 on 256 x 256 tiles takes 354 us on real data and 300 on zeros (same instructions); without its loads 288,
+ *   - Power.  4001 x 4096 x 14336 on 256 x 256 tiles, before X came in whole lines: 354 us on real data and 300 on zeros (same instructions); without its loads 288,
  *     without its LDS reads 331, the MFMAs alone 260.  So energy per product is what counts:
  *     16 x 16 x 32 MFMAs instead of 32 x 32 x 16 (384 against 423 us in one run), X fetched in whole 128-byte lines (64 k of a row per stage; a stage
- *     of 32 k fetches every line twice: 354 -> 336), and the order of the MFMAs within a step, boustrophedon, so that one operand stays put (1 %).
+ *     of 32 k fetches every line twice: 354 -> 336, which is what it takes now), and the order of the MFMAs within a step, boustrophedon, so that one operand stays put (1 %).
  *   - Intake.  A compute unit accepts about 40 bytes per cycle of direct-to-LDS loads, whatever the depth of the ring (128 x 128 tiles, rings of four
  *     and five stages: 81.5 and 81.4 us at 512 x 4096 x 14336): 256 x 256 tiles need 31 bytes per cycle of MFMA, 128 x 256 tiles 47, 128 x 128 tiles 63.
  * Against the kernels before (four waves, 32 x 32 x 16 MFMAs, weights from memory straight into registers), 256 x 256 tiles: 4001 x 14336 x 4096
  * 490 -> 393 us (1.20 PFLOP/s), 4001 x 4096 x 14336 410 -> 336 (1.40); 128 x 256: 2048 x 4096 x 4096 69 -> 60, 512 x 14336 x 4096 63 -> 55;
  * the smaller tiles, for few rows on either side: 4001 x 1024 x 4096 69 -> 36, 512 x 4096 x 4096 49 -> 23, 512 x 1024 x 4096 48 -> 13.5.
- * Storing Y costs 45 of the 393 us.  Tried without gain: workgroups that walk several tiles and ask for the next one's operands before they store (1-2 %
+ * (The largest one on other devices and days: 389 to 395 us, 407 under the profiler.)  Storing Y costs 45 of the 393 us.  Tried without gain: workgroups that walk several tiles and ask for the next one's operands before they store (1-2 %
  * on 128 x 256 tiles, spills on 256 x 256), K ranges rotated against each other per XCD, non-temporal stores.
  */
 #include "psn_args.h"

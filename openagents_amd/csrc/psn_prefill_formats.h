@@ -183,17 +183,17 @@ struct PpQ6_K {
  * part, and one v_perm selector per thread picks either. */
 template <int PB, int NB> struct pp_blocks {               /* PB: bytes per part (NB or 2 NB) */
     static constexpr int PARTS = 32 / NB;
+    static_assert(PARTS == 4, "a quad, or a part per sixteen lanes");
     static PSN_DEV bool second_block(int part) { return part >= PARTS / 2; }
     static PSN_DEV u32 pick(int part) { return second_block(part) ? 0x07060504u : 0x05040302u; }
     /* the block's scale in both halves.  FAR: the four parts of a row are the four sixteens of lanes, not neighbours */
     template <bool FAR> static PSN_DEV u32 scale(u32 first_dword, int part) {
         u32 v;
         if constexpr (FAR) {
-            static_assert(PARTS == 4, "a part per sixteen lanes");
             v = __builtin_amdgcn_permlane16_swap(first_dword, first_dword, false, false)[0];   /* lanes 16..31 get 0..15's, lanes 48..63 get 32..47's */
         } else {
-            /* quad_perm: lanes of a quad read their block's first part (parts 0, 0, 2, 2, or 0 of quads that are one block) */
-            v = (u32)__builtin_amdgcn_mov_dpp((int)first_dword, PARTS == 4 ? 0xA0 : 0x00, 0xf, 0xf, false);
+            /* quad_perm: lanes of a quad read their block's first part (parts 0, 0, 2, 2) */
+            v = (u32)__builtin_amdgcn_mov_dpp((int)first_dword, 0xA0, 0xf, 0xf, false);
         }
         return __builtin_amdgcn_perm(v, v, second_block(part) ? 0x03020302u : 0x01000100u);
     }
